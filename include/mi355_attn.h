@@ -577,6 +577,8 @@ int mi355_ssm_decode(const mi355_ssm_args* args, void* stream);
  *   mi355_moe_group   : pairs sorted by expert: order (n_pairs), offsets (n_experts + 1)
  *   mi355_moe_gate_up : act[i] = silu(Wg h) * (Wu h) for place i of the order; w (n_experts, 2 ff, k), gates first
  *   mi355_moe_down    : out[pair] = weights[pair] * (Wd act[i]); w (n_experts, n, ff)
+ *   mi355_moe_direct  : gate_up and down of a decode step's few pairs (up to 2048, bf16), without an order: act (n_pairs, ff)
+ *                       and out hold row `pair` for each pair
  * bf16 (fp32 sums): k and ff in multiples of 64, 16-byte aligned rows.  tiling AUTO chooses by pairs per expert.
  */
 enum { MI355_TILING_AUTO = 0, MI355_TILING_SKINNY = 1, MI355_TILING_LARGE = 2 };
@@ -590,6 +592,9 @@ int mi355_moe_gate_up(const void* h, const void* w, void* act, const int32_t* of
 int mi355_moe_down(const void* act, const void* w, const float* weights, void* out, const int32_t* offsets,
                    const int32_t* order, int64_t n_tokens, int64_t act_row_stride, int64_t out_row_stride, int n_experts,
                    int top, int ff, int n, int dtype, int tiling, void* stream);
+int mi355_moe_direct(const void* h, const void* w_gate_up, const void* w_down, const int32_t* ids, const float* weights,
+                     void* act, void* out, int64_t n_tokens, int64_t h_row_stride, int64_t out_row_stride, int n_experts,
+                     int top, int k, int ff, int n, void* stream);
 
 /*
  * Plain device-to-device copy of `bytes` bytes (16-byte aligned).  Measurement aid

@@ -9,10 +9,15 @@
 // needs the offsets alone, and a launch of n_pairs / BM + E row tiles covers every distribution of the tokens.  A row of a
 // product depends on its own token only, so neither the order inside an expert nor the tiling shows in a result.
 //   moe_gemm_kernel    128 x 128 tiles through LDS: prompts
-//   moe_skinny_kernel  16 rows x 16 (+ 16) weight rows, weights straight to registers, k dealt to the wavefronts: decoding
+//   moe_direct_kernel  32 weight rows, streamed through LDS, against an expert's rows, no grouping needed: decoding
+//   moe_skinny_kernel  16 rows x 16 (+ 16) weight rows, weights straight to registers: few pairs per expert, many experts
 //   moe_f32_kernel     fp32 on the vector unit
 #include "common.hpp"
 #include "launch.hpp"
+#include "weight_stream.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace mi355 {
 
@@ -76,54 +81,88 @@ __device__ __forceinline__ void choose_experts(const RouteParams& p, float* z, i
     }
 }
 
-// 16 tokens per workgroup; the wavefronts take the 32-wide steps of k in turn and meet in LDS.
+// Up to 64 logits: GROUP lanes per token, a lane owns one logit and counts those in front of it (larger, or as large with a
+// lower index), which is its place; 64 / GROUP tokens at a time.  The general form above walks the maxima one after the other,
+// six exchanges each: 16 of 23 us for 8192 tokens of 16 logits, four chosen, were spent there.  What is no number counts as
+// -inf, and a choice without a logit above -inf is expert E - 1, as there.
+template <int GROUP>
+__device__ __forceinline__ void choose_by_rank(const RouteParams& p, const float* z, int64_t t0, int lane, int wave, int n_waves) {
+    const int e = lane % GROUP;
+    for (int t = wave * (64 / GROUP) + lane / GROUP; t < 16; t += n_waves * (64 / GROUP)) {
+        const float* zt = z + t * p.n_logits;
+        float mine = e < p.E ? zt[e] : -INFINITY;
+        mine = mine > -INFINITY ? mine : -INFINITY;
+        float top1 = mine;
+#pragma unroll
+        for (int off = GROUP / 2; off >= 1; off >>= 1) top1 = fmaxf(top1, __shfl_xor(top1, off, 64));
+        int rank = 0;
+        for (int j = 0; j < p.E; ++j) {
+            float v = zt[j];
+            v = v > -INFINITY ? v : -INFINITY;
+            rank += v > mine || (v == mine && j < e);
+        }
+        const bool chosen = e < p.E && rank < p.top;
+        const float w = chosen ? expf(mine - top1) : 0.f;
+        float sum = w;
+#pragma unroll
+        for (int off = GROUP / 2; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (chosen && t0 + t < p.T) {
+            p.ids[(t0 + t) * p.top + rank] = mine > -INFINITY ? e : p.E - 1;
+            p.weights[(t0 + t) * p.top + rank] = w / sum;
+        }
+    }
+}
+
+// 16 tokens per workgroup; the wavefronts take the 32-wide steps of k in turn and meet in LDS.  TILES: 16-logit tiles per pass.
+// The loads of BATCH steps are in flight together: with one or two tiles, eight (k = 2048 in one go), which is what a launch
+// of few tokens is made of (32 tokens, 16 logits, k = 2048: 13.9 us with four tiles and four steps, 7.6 us like this).
 constexpr int kRouteWaves = 8;
+template <int TILES, int BATCH>
 __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(RouteParams p) {
     extern __shared__ __attribute__((aligned(16))) float route_lds[];
-    constexpr int kTiles = 4, kBatch = 4;         // 16 logits each
     f32x4* part = reinterpret_cast<f32x4*>(route_lds);                         // [wave][tile][lane]
-    float* z = route_lds + kRouteWaves * kTiles * 64 * 4;                              // [16][n_logits]
+    float* z = route_lds + kRouteWaves * TILES * 64 * 4;                              // [16][n_logits]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kg = lane >> 4;
     const int64_t t0 = (int64_t)blockIdx.x * 16;
     const __bf16* h = (const __bf16*)p.h + min(t0 + r, p.T - 1) * p.h_stride;
-    for (int l0 = 0; l0 < p.n_logits; l0 += 16 * kTiles) {
-        f32x4 acc[kTiles];
-        const __bf16* w[kTiles];
+    for (int l0 = 0; l0 < p.n_logits; l0 += 16 * TILES) {
+        f32x4 acc[TILES];
+        const __bf16* w[TILES];
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j) {
+        for (int j = 0; j < TILES; ++j) {
             acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
             w[j] = (const __bf16*)p.w + (int64_t)min(l0 + 16 * j + r, p.n_logits - 1) * p.w_stride;
         }
-        for (int k0 = 32 * wave; k0 < p.k; k0 += 32 * kRouteWaves * kBatch) {       // kBatch steps' loads, then their products
-            u32x4 hv[kBatch], wv[kTiles][kBatch];
+        for (int k0 = 32 * wave; k0 < p.k; k0 += 32 * kRouteWaves * BATCH) {       // BATCH steps' loads, then their products
+            u32x4 hv[BATCH], wv[TILES][BATCH];
 #pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
+            for (int i = 0; i < BATCH; ++i) {
                 const int col = k0 + 32 * kRouteWaves * i + 8 * kg;
                 const bool in = col < p.k;
                 hv[i] = u32x4{0u, 0u, 0u, 0u};
                 if (in) hv[i] = *reinterpret_cast<const u32x4*>(h + col);
 #pragma unroll
-                for (int j = 0; j < kTiles; ++j) {
+                for (int j = 0; j < TILES; ++j) {
                     wv[j][i] = u32x4{0u, 0u, 0u, 0u};
                     if (in && l0 + 16 * j < p.n_logits) wv[j][i] = *reinterpret_cast<const u32x4*>(w[j] + col);
                 }
             }
 #pragma unroll
-            for (int j = 0; j < kTiles; ++j)
+            for (int j = 0; j < TILES; ++j)
                 if (l0 + 16 * j < p.n_logits)
 #pragma unroll
-                    for (int i = 0; i < kBatch; ++i) acc[j] = mfma16(as_bf16x8(wv[j][i]), as_bf16x8(hv[i]), acc[j]);      // column r: token, rows 4 kg + i: logits
+                    for (int i = 0; i < BATCH; ++i) acc[j] = mfma16(as_bf16x8(wv[j][i]), as_bf16x8(hv[i]), acc[j]);      // column r: token, rows 4 kg + i: logits
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j) part[(wave * kTiles + j) * 64 + lane] = acc[j];
+        for (int j = 0; j < TILES; ++j) part[(wave * TILES + j) * 64 + lane] = acc[j];
         __syncthreads();
         // wavefront j sums tile j
-        if (wave < kTiles) {
+        if (wave < TILES) {
             f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int w8 = 0; w8 < kRouteWaves; ++w8) s += part[(w8 * kTiles + wave) * 64 + lane];
+            for (int w8 = 0; w8 < kRouteWaves; ++w8) s += part[(w8 * TILES + wave) * 64 + lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int l = l0 + 16 * wave + 4 * kg + i;
@@ -132,11 +171,12 @@ __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(RouteParams
         }
     }
     __syncthreads();
+    if (p.extra_logit && tid < 16 && t0 + tid < p.T) p.extra_logit[t0 + tid] = z[tid * p.n_logits + p.E];
+    if (p.E <= 16) return choose_by_rank<16>(p, z, t0, lane, wave, kRouteWaves);
+    if (p.E <= 64) return choose_by_rank<64>(p, z, t0, lane, wave, kRouteWaves);
     for (int t = wave; t < 16; t += kRouteWaves) {
         if (t0 + t >= p.T) break;
-        float* zt = z + t * p.n_logits;
-        if (p.extra_logit && lane == 0) p.extra_logit[t0 + t] = zt[p.E];
-        choose_experts(p, zt, t0 + t, lane);
+        choose_experts(p, z + t * p.n_logits, t0 + t, lane);
     }
 }
 
@@ -159,6 +199,14 @@ __global__ __launch_bounds__(256) void moe_route_f32_kernel(RouteParams p) {
     choose_experts(p, z, t, lane);
 }
 
+static void launch_route(const RouteParams& p, hipStream_t s) {
+    const dim3 grid((unsigned)((p.T + 15) / 16)), block(64 * kRouteWaves);
+    const auto lds = [&](int tiles) { return (kRouteWaves * tiles * 64 * 4 + 16 * p.n_logits) * sizeof(float); };
+    if (p.n_logits <= 16) hipLaunchKernelGGL((moe_route_kernel<1, 8>), grid, block, lds(1), s, p);
+    else if (p.n_logits <= 32) hipLaunchKernelGGL((moe_route_kernel<2, 8>), grid, block, lds(2), s, p);
+    else hipLaunchKernelGGL((moe_route_kernel<4, 4>), grid, block, lds(4), s, p);
+}
+
 // ---- pairs sorted by expert -----------------------------------------------------------------------
 // Workgroup e lists expert e's pairs: each of its 16 wavefronts counts the pairs of lower experts and of its own expert in
 // its share of the ids, the shares are summed, and a second pass writes.
@@ -167,11 +215,17 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* ids, int
     const int e = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int share = ((n_pairs + 15) / 16 + 63) / 64 * 64;
     const int i0 = min(n_pairs, wave * share), i1 = min(n_pairs, i0 + share);
+    constexpr int kAhead = 8;                     // loads in flight: one at a time, 32768 pairs took 23 us
     int n_below = 0, n_equal = 0;
-    for (int i = i0; i < i1; i += 64) {
-        const int id = i + lane < i1 ? ids[i + lane] : E;
-        n_below += __popcll(__builtin_amdgcn_ballot_w64(id < e));
-        n_equal += __popcll(__builtin_amdgcn_ballot_w64(id == e));
+    for (int i = i0; i < i1; i += 64 * kAhead) {
+        int id[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) id[j] = i + 64 * j + lane < i1 ? ids[i + 64 * j + lane] : E;
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            n_below += __popcll(__builtin_amdgcn_ballot_w64(id[j] < e));
+            n_equal += __popcll(__builtin_amdgcn_ballot_w64(id[j] == e));
+        }
     }
     if (lane == 0) {
         below[wave] = n_below;
@@ -184,11 +238,17 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int32_t* ids, int
         offsets[e] = at;
         if (e == E - 1) offsets[E] = n_pairs;
     }
-    for (int i = i0; i < i1; i += 64) {
-        const bool mine = i + lane < i1 && ids[i + lane] == e;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(mine);
-        if (mine) order[at + __popcll(m & ((1ull << lane) - 1))] = i + lane;
-        at += __popcll(m);
+    if (n_equal == 0) return;
+    for (int i = i0; i < i1; i += 64 * kAhead) {
+        int id[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) id[j] = i + 64 * j + lane < i1 ? ids[i + 64 * j + lane] : E;
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64(id[j] == e);
+            if (id[j] == e) order[at + __popcll(m & ((1ull << lane) - 1))] = i + 64 * j + lane;
+            at += __popcll(m);
+        }
     }
 }
 
@@ -204,18 +264,23 @@ struct MoeParams {
     int top;
 };
 
-// expert and first place of row tile `tile`; false: the tile has no rows
+// expert and first place of row tile `tile`; false: the tile has no rows.  A lane looks at one expert (64 at a time): one load
+// in front of a tile's first operand where a binary search has a chain of them.
 template <int BM>
 __device__ __forceinline__ bool find_tile(const MoeParams& p, int tile, int& e, int& first, int& end) {
-    int lo = 0, hi = p.E - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) / 2;
-        if (p.offsets[mid] / BM + mid <= tile) lo = mid;
-        else hi = mid - 1;
+    const int lane = threadIdx.x & 63;
+    int start = 0, stop = 0;
+    e = 0;
+    for (int e0 = 0; e0 < p.E; e0 += 64) {
+        const int mine = min(e0 + lane, p.E - 1), o0 = p.offsets[mine], o1 = p.offsets[mine + 1];
+        const uint64_t m = __builtin_amdgcn_ballot_w64(e0 + lane < p.E && o0 / BM + mine <= tile);
+        if (m == 0) break;                        // (the first tile numbers rise with the expert)
+        const int last = 63 - __builtin_clzll(m);
+        e = e0 + last;
+        start = __builtin_amdgcn_readlane(o0, last);
+        stop = __builtin_amdgcn_readlane(o1, last);
     }
-    e = __builtin_amdgcn_readfirstlane(lo);
-    const int start = __builtin_amdgcn_readfirstlane(p.offsets[e]);
-    end = min(__builtin_amdgcn_readfirstlane(p.offsets[e + 1]), p.n_pairs);
+    end = min(stop, p.n_pairs);
     first = start + (tile - (start / BM + e)) * BM;
     return first >= start && first < end;
 }
@@ -245,10 +310,10 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
 // LDS buffers filled by direct loads.  A 128-byte LDS row holds its eight 16-byte pieces in the order piece ^ (row % 8).
 // Wavefront (wm, wn) computes 64 x 64; weights are the MFMA's first operand, so that a lane ends with adjacent columns.
 template <bool GATE_UP>
-__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int m_tiles) {
+__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int m_tiles, int chunk) {
     constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];          // [buffer][rows | w]
-    const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, n_tiles);
+    const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, chunk);
     const int n_tile = id % n_tiles;
     int e, first, end;
     if (!find_tile<BM>(p, id / n_tiles, e, first, end)) return;
@@ -394,6 +459,104 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(MoeParams p, int n_tile
     }
 }
 
+// The same product for the few pairs of a decode step, without an order: a workgroup per expert and 32 rows of w (gate_up: 16
+// gates and their ups) looks through the ids for its expert's pairs itself, and row `pair` of the left and the output matrix
+// belongs to the pair.  The weights are read once for every 32 rows.  What it saves against group + skinny: a launch, and the
+// chain of dependent loads offsets -> order -> rows in front of the first weight.  Bound by the weights' stream (16 experts of
+// 2048 x 1024, 32 tokens: 134 + 67 MB in 31 + 14 us, 4.3 and 4.8 TB/s, where group + skinny took 3 + 34 + 21).
+constexpr int kDirectPairs = 2048;
+template <bool GATE_UP>
+__global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int32_t* ids, int n_tiles) {
+    constexpr int NW = GATE_UP ? 2 : 1;
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[4 * kStreamBytes];
+    __shared__ uint16_t mine[kDirectPairs];
+    __shared__ int counts[4];
+    // (an expert's tiles go round the XCDs: a step of one token uses few experts)
+    const int n0 = blockIdx.x % n_tiles * (GATE_UP ? 16 : 32), e = blockIdx.x / n_tiles;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    // wavefront w looks through pairs 64 (w + 4 i) + lane, kLook of them at a time
+    constexpr int kLook = kDirectPairs / 256;
+    uint64_t hit[kLook];
+    int found = 0;
+#pragma unroll
+    for (int i = 0; i < kLook; ++i) {
+        const int pair = 64 * (kLook * wave + i) + lane;
+        hit[i] = 0;
+        if (64 * (kLook * wave + i) < p.n_pairs) hit[i] = __builtin_amdgcn_ballot_w64(pair < p.n_pairs && ids[min(pair, p.n_pairs - 1)] == e);
+        found += __popcll(hit[i]);
+    }
+    if (lane == 0) counts[wave] = found;
+    __syncthreads();
+    int at = 0, n_rows = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        at += w < wave ? counts[w] : 0;
+        n_rows += counts[w];
+    }
+    if (n_rows == 0) return;
+#pragma unroll
+    for (int i = 0; i < kLook; ++i) {
+        if (hit[i] >> lane & 1) mine[at + __popcll(hit[i] & ((1ull << lane) - 1))] = (uint16_t)(64 * (kLook * wave + i) + lane);
+        at += __popcll(hit[i]);
+    }
+    __syncthreads();
+    const __bf16* w_base = (const __bf16*)p.w + (int64_t)e * (GATE_UP ? 2 : 1) * p.n * p.k;
+    const int piece = (lane & 7) ^ (lane >> 3);   // what a lane requests of its row's 128 bytes: see WeightStream
+    uint32_t w_off[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 8 * j + (lane >> 3);
+        const int64_t wr = GATE_UP ? (row < 16 ? min(n0 + row, p.n - 1) : p.n + min(n0 + row - 16, p.n - 1)) : min(n0 + row, p.n - 1);
+        w_off[j] = (uint32_t)((wr * p.k + piece * 8) * 2);
+    }
+    const auto rows = [&](int r0, auto tiles) {
+        constexpr int MT = decltype(tiles)::value;
+        uint32_t a_off[2 * MT];
+#pragma unroll
+        for (int j = 0; j < 2 * MT; ++j) {
+            const int pair = mine[min(r0 + 8 * j + (lane >> 3), n_rows - 1)];
+            a_off[j] = (uint32_t)(((int64_t)(GATE_UP ? pair / p.top : pair) * p.a_stride + piece * 8) * 2);
+        }
+        f32x4 acc[MT][2];
+        weight_stream<MT>(w_base, w_off, p.a, a_off, p.k / 64, wave, ring + wave * kStreamBytes, acc);
+        __syncthreads();                          // (the sums travel through the ring)
+        f32x4* part = reinterpret_cast<f32x4*>(ring);                           // [wave][row tile][16 rows of w][lane]
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) part[((wave * MT + m) * 2 + i) * 64 + lane] = acc[m][i];
+        __syncthreads();
+        // a wavefront sums one row tile (gate_up), or one row tile and 16 columns (down)
+        if (wave < (GATE_UP ? MT : 2 * MT)) {
+            const int m = GATE_UP ? wave : wave >> 1, half = GATE_UP ? 0 : wave & 1;
+            f32x4 sum[NW];
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+                sum[i] = part[(m * 2 + half + i) * 64 + lane];
+#pragma unroll
+                for (int w4 = 1; w4 < 4; ++w4) sum[i] += part[((w4 * MT + m) * 2 + half + i) * 64 + lane];
+            }
+            if (r0 + 16 * m + r < n_rows) {
+                const int pair = mine[r0 + 16 * m + r];
+                const float wgt = GATE_UP ? 1.f : p.weights[pair];
+                float v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if constexpr (GATE_UP) v[q] = silu_fast(sum[0][q]) * sum[NW - 1][q];
+                    else v[q] = wgt * sum[0][q];
+                }
+                store4(p, pair, n0 + 16 * half + 4 * kg, v);
+            }
+        }
+        __syncthreads();
+    };
+    for (int r0 = 0; r0 < n_rows; r0 += 32) {
+        if (n_rows - r0 <= 16) rows(r0, std::integral_constant<int, 1>{});
+        else rows(r0, std::integral_constant<int, 2>{});
+    }
+}
+
 // fp32: 16 rows x 64 columns per workgroup, a thread owns four rows of one column
 template <bool GATE_UP>
 __global__ __launch_bounds__(256) void moe_f32_kernel(MoeParams p, int n_tiles, int m_tiles) {
@@ -448,21 +611,27 @@ __global__ __launch_bounds__(256) void moe_f32_kernel(MoeParams p, int n_tiles, 
 
 template <bool GATE_UP>
 static int launch_moe(const MoeParams& p, int dtype, int tiling, hipStream_t s) {
-    const bool large = tiling == MI355_TILING_LARGE || (tiling == MI355_TILING_AUTO && p.n_pairs > 32 * (int64_t)p.E);
+    // From 8 pairs per expert on the large tiles, mostly padding then, still read the weights faster (2048 x 1024, 16 experts, both
+    // products: 8 pairs 44 us against 55, 32 pairs 49 against 109)
+    const bool large = tiling == MI355_TILING_LARGE || (tiling == MI355_TILING_AUTO && p.n_pairs > 8 * (int64_t)p.E);
     const int bm = dtype == MI355_BF16 && large ? 128 : 16;
     const int bn = dtype == MI355_FP32 ? 64 : (!large ? 16 : (GATE_UP ? 64 : 128));
     const int n_tiles = (p.n + bn - 1) / bn, m_tiles = p.n_pairs / bm + p.E;
     if ((int64_t)n_tiles * m_tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)(n_tiles * m_tiles)), block(256);
+    // An XCD takes as many neighbouring row tiles in turn as fill its 32 compute units twice: they mostly belong to one expert
+    // and share its weights in that L2.  (One row tile per turn, so that eight XCDs read eight tiles of one expert: 2048
+    // tokens, 16 experts of 2048 x 1024, top 4 176 us for both products, 146 us like this; 8192 tokens 518 against 511.)
+    const int chunk = n_tiles * std::max(1, 64 / n_tiles);
     if (dtype == MI355_FP32) hipLaunchKernelGGL(moe_f32_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
-    else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
+    else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles, chunk);
     else hipLaunchKernelGGL(moe_skinny_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     return (int)hipGetLastError();
 }
 
-static int moe_product(bool gate_up, const void* a, const void* w, void* out, const int32_t* offsets, const int32_t* order,
-                       const float* weights, int64_t a_stride, int64_t a_rows, int64_t out_stride, int64_t out_rows, int64_t n_pairs,
-                       int E, int top, int k, int n, int dtype, int tiling, void* stream) {
+static int moe_check(MoeParams& p, bool gate_up, const void* a, const void* w, void* out, const int32_t* offsets, const int32_t* order,
+                     const float* weights, int64_t a_stride, int64_t a_rows, int64_t out_stride, int64_t out_rows, int64_t n_pairs,
+                     int E, int top, int k, int n, int dtype, int tiling) {
     if (!a || !w || !out || !offsets || !order || (!gate_up && !weights)) return set_error(MI355_EINVAL, "moe: null pointer argument");
     if (dtype != MI355_BF16 && dtype != MI355_FP32) return set_error(MI355_EDTYPE, "moe: dtype must be MI355_BF16 or MI355_FP32");
     if (E <= 0 || E > kMaxExperts || top <= 0 || k <= 0 || n <= 0 || n_pairs < 0 || n_pairs > 0x3fffffffLL)
@@ -477,8 +646,6 @@ static int moe_product(bool gate_up, const void* a, const void* w, void* out, co
         if (a_rows * a_stride > 0x7fffffffLL || 2LL * n * k > 0x7fffffffLL)
             return set_error(MI355_EINVAL, "moe: an operand is too large for 32-bit byte offsets");
     }
-    if (n_pairs == 0) return MI355_OK;
-    MoeParams p;
     p.a = a;
     p.w = w;
     p.out = out;
@@ -494,6 +661,16 @@ static int moe_product(bool gate_up, const void* a, const void* w, void* out, co
     p.k = k;
     p.n = n;
     p.top = top;
+    return MI355_OK;
+}
+
+static int moe_product(bool gate_up, const void* a, const void* w, void* out, const int32_t* offsets, const int32_t* order,
+                       const float* weights, int64_t a_stride, int64_t a_rows, int64_t out_stride, int64_t out_rows, int64_t n_pairs,
+                       int E, int top, int k, int n, int dtype, int tiling, void* stream) {
+    MoeParams p;
+    if (int e = moe_check(p, gate_up, a, w, out, offsets, order, weights, a_stride, a_rows, out_stride, out_rows, n_pairs, E, top, k, n, dtype, tiling))
+        return e;
+    if (n_pairs == 0) return MI355_OK;
     const int rc = gate_up ? launch_moe<true>(p, dtype, tiling, (hipStream_t)stream) : launch_moe<false>(p, dtype, tiling, (hipStream_t)stream);
     if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
     return MI355_OK;
@@ -532,8 +709,7 @@ extern "C" int mi355_moe_route(const void* h, const void* w, const float* bias, 
     p.top = top;
     hipStream_t s = (hipStream_t)stream;
     if (dtype == MI355_BF16)
-        hipLaunchKernelGGL(moe_route_kernel, dim3((unsigned)((n_tokens + 15) / 16)), dim3(64 * kRouteWaves),
-                           (kRouteWaves * 4 * 64 * 4 + 16 * p.n_logits) * sizeof(float), s, p);
+        launch_route(p, s);
     else
         hipLaunchKernelGGL(moe_route_f32_kernel, dim3((unsigned)((n_tokens + 3) / 4)), dim3(256), 4 * p.n_logits * sizeof(float), s, p);
     const int rc = (int)hipGetLastError();
@@ -563,4 +739,27 @@ extern "C" int mi355_moe_down(const void* act, const void* w, const float* weigh
                               int dtype, int tiling, void* stream) {
     return moe_product(false, act, w, out, offsets, order, weights, act_row_stride, n_tokens * top, out_row_stride, n_tokens * top,
                        n_tokens * top, n_experts, top, ff, n, dtype, tiling, stream);
+}
+
+extern "C" int mi355_moe_direct(const void* h, const void* w_gate_up, const void* w_down, const int32_t* ids, const float* weights, void* act,
+                                void* out, int64_t n_tokens, int64_t h_row_stride, int64_t out_row_stride, int n_experts, int top, int k,
+                                int ff, int n, void* stream) {
+    if (!ids) return set_error(MI355_EINVAL, "moe_direct: null pointer argument");
+    if (n_tokens < 0 || top <= 0 || n_tokens * top > kDirectPairs) return set_error(MI355_EINVAL, "moe_direct: up to 2048 pairs");
+    // (ids stands in for the order, which these kernels do not read)
+    MoeParams p;
+    int rc = moe_check(p, true, h, w_gate_up, act, ids, ids, nullptr, h_row_stride, n_tokens, ff, n_tokens * top, n_tokens * top, n_experts, top,
+                       k, ff, MI355_BF16, MI355_TILING_AUTO);
+    if (rc != MI355_OK || n_tokens == 0) return rc;
+    hipStream_t s = (hipStream_t)stream;
+    int tiles = (ff + 15) / 16;
+    hipLaunchKernelGGL(moe_direct_kernel<true>, dim3((unsigned)(tiles * n_experts)), dim3(256), 0, s, p, ids, tiles);
+    if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
+    rc = moe_check(p, false, act, w_down, out, ids, ids, weights, ff, n_tokens * top, out_row_stride, n_tokens * top, n_tokens * top, n_experts,
+                   top, ff, n, MI355_BF16, MI355_TILING_AUTO);
+    if (rc != MI355_OK) return rc;
+    tiles = (n + 31) / 32;
+    hipLaunchKernelGGL(moe_direct_kernel<false>, dim3((unsigned)(tiles * n_experts)), dim3(256), 0, s, p, ids, tiles);
+    if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
+    return MI355_OK;
 }

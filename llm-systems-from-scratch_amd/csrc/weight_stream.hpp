@@ -1,0 +1,67 @@
+// 32 rows of a weight matrix against 16 or 32 rows of activations, as a wavefront's share of a product with few rows.
+//
+// Such a product reads every weight once, so what counts is how the weights come in.  16-byte loads straight into the
+// MFMA's operand layout touch 64 bytes of each of 16 rows per instruction, and the address unit takes four times as long for
+// one as for a load of whole lines; here a direct load to LDS brings 8 rows of 128 bytes.  Each wavefront has a ring of its own
+// (no barrier inside the stream) and takes every fourth 64-wide step of k; the caller adds the four up.
+#pragma once
+#include "common.hpp"
+
+namespace mi355 {
+
+constexpr int kStreamBytes = 12 * 1024;          // per wavefront: 2 steps of 32 + 16 rows, or one of 32 + 32; three workgroups per compute unit
+
+// w_off, a_off: byte offsets of this lane's 16 bytes in step 0: rows 8 j + lane / 8 of the weights (32) and of the activations
+// (16 * MT), piece (lane % 8) ^ (lane / 8) of the row's eight, so that the LDS row holds piece q at q ^ (row % 8).
+// acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
+template <int MT>
+__device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],
+                                              int n_steps, int wave, unsigned char* ring, f32x4 (&acc)[MT][2]) {
+    constexpr int kStep = (32 + 16 * MT) * 128, kDeep = MT == 1 ? 2 : 1, kLoads = 4 + 2 * MT;
+    static_assert(kDeep * kStep <= kStreamBytes, "ring");
+    const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
+    const uint32_t ring0 = lds_address(ring);
+    const auto request = [&](int t, int slot) {
+        const char* wt = (const char*)w + 128 * (int64_t)t;
+        const char* at = (const char*)a + 128 * (int64_t)t;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma_to_lds_16(wt, w_off[j], ring0 + slot * kStep + j * 1024);
+#pragma unroll
+        for (int j = 0; j < 2 * MT; ++j) dma_to_lds_16(at, a_off[j], ring0 + slot * kStep + (4 + j) * 1024);
+    };
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < kDeep; ++d)
+        if (wave + 4 * d < n_steps) request(wave + 4 * d, d);
+    int slot = 0;
+    for (int t = wave; t < n_steps; t += 4) {
+        if (t + 4 * (kDeep - 1) < n_steps) wait_vmcnt<(kDeep - 1) * kLoads>();
+        else wait_vmcnt<0>();                     // (the last steps are all on their way already)
+        const unsigned char* at = ring + slot * kStep;
+        bf16x8 wf[2][2], af[MT][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int piece = ((4 * s + kg) ^ (r & 7)) * 16;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wf[i][s] = as_bf16x8(*reinterpret_cast<const u32x4*>(at + (16 * i + r) * 128 + piece));
+#pragma unroll
+            for (int m = 0; m < MT; ++m) af[m][s] = as_bf16x8(*reinterpret_cast<const u32x4*>(at + (32 + 16 * m + r) * 128 + piece));
+        }
+        if (t + 4 * kDeep < n_steps) {
+            wait_lgkmcnt0();                      // the slot's bytes are in registers
+            request(t + 4 * kDeep, slot);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[m][i] = mfma16(wf[i][s], af[m][s], acc[m][i]);
+        slot = slot + 1 == kDeep ? 0 : slot + 1;
+    }
+}
+
+}  // namespace mi355

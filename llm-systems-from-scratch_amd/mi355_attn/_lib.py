@@ -222,6 +222,8 @@ def load():
     lib.mi355_moe_gate_up.argtypes = [vp, vp, vp, vp, vp, i64, i64, i64, i32, i32, i32, i32, i32, i32, vp]
     lib.mi355_moe_down.restype = i32
     lib.mi355_moe_down.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, i32, i32, i32, i32, i32, vp]
+    lib.mi355_moe_direct.restype = i32
+    lib.mi355_moe_direct.argtypes = [vp] * 7 + [i64, i64, i64, i32, i32, i32, i32, i32, vp]
     lib.mi355_calib_copy.restype = i32
     lib.mi355_calib_copy.argtypes = [vp, vp, sz, vp]
     lib.mi355_last_error.restype = C.c_char_p

@@ -1424,6 +1424,9 @@ def moe_route(h, w, bias, top: int, *, extra_row: bool = False):
     return ids, weights, extra
 
 
+_DIRECT_PAIRS = 2048        # the most pairs mi355_moe_direct takes
+
+
 def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
     """Gated feed-forward of each row's chosen experts: weights[t, c] * Wd (silu(Wg h_t) * (Wu h_t)) of expert ids[t, c] as row
     t * top + c of the result (T * top, n); their sum is left to the reader (residual_rms).  h (T,k), w_gate_up
@@ -1442,10 +1445,23 @@ def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
     out = torch.empty(T * top, n + (-n % 8), dtype=h.dtype, device=dev)[:, :n]            # (16-byte aligned rows)
     if T == 0:
         return out
+    act = torch.empty(T * top, ff, dtype=h.dtype, device=dev)
+    lib = _lib.load()
+    if tiling == "direct" and h.dtype != torch.bfloat16:
+        raise TypeError("the direct form is bfloat16")
+    # No order up to 16 pairs per expert: with 2048 x 1024 experts (16 of them, 128 pairs) 45 us against 55 (group + skinny) and
+    # 44 (128-row tiles), at 256 pairs 47 / 79 / 49, at 512 pairs 61 / 110 / 49.  Experts of a MB or less are bound by the
+    # launches, of which it saves one, up to 64 pairs (8 of 512 x 512: 18 us against 26).
+    few = (64 if E * k * ff <= 1 << 22 else 16) * E
+    if tiling == "direct" or (tiling == "auto" and h.dtype == torch.bfloat16 and T * top <= min(_DIRECT_PAIRS, few)):
+        with _on(h, ids, weights, w_gate_up, w_down) as stream:
+            rc = lib.mi355_moe_direct(h.data_ptr(), w_gate_up.data_ptr(), w_down.data_ptr(), ids.data_ptr(), weights.data_ptr(), act.data_ptr(),
+                                      out.data_ptr(), T, h.stride(0) if T > 1 else k, out.stride(0), E, top, k, ff, n, stream)
+        _lib.check(rc, "mi355_moe_direct")
+        return out
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
     order = torch.empty(T * top, dtype=torch.int32, device=dev)
-    act = torch.empty(T * top, ff, dtype=h.dtype, device=dev)
-    lib, tl = _lib.load(), _lib.TILINGS[tiling]
+    tl = _lib.TILINGS[tiling]
     with _on(h, ids, weights, w_gate_up, w_down) as stream:
         rc = lib.mi355_moe_group(ids.data_ptr(), T * top, E, offsets.data_ptr(), order.data_ptr(), stream)
         _lib.check(rc, "mi355_moe_group")

@@ -418,6 +418,52 @@ def test_experts(ops, T, E, top, k, ff, n, tiling, dtype):
         rows_close(got, ref, dtype, what=f"{tiling}")
 
 
+@pytest.mark.parametrize("tiling,T,E,top,k,ff,n", [
+    ("direct", 1, 8, 2, 64, 64, 40), ("direct", 33, 4, 1, 192, 128, 72), ("direct", 50, 8, 3, 1088, 192, 130), ("direct", 512, 8, 4, 64, 64, 8)])
+def test_expert_tilings(ops, tiling, T, E, top, k, ff, n):
+    """The decode form that finds its pairs itself: one row, edges of 16 and 32 rows, the most pairs it takes, k of one step and of a remainder
+    of the four wavefronts' turns; also against the 128 x 128 tiles on the same operands: the same bf16 products in another order of the fp32
+    sums, so results agree to one rounding of the activations (2^-8) in either product."""
+    print(f"case: expert tilings {tiling} {T} {E} {top} {k} {ff} {n}", flush=True)
+    bf = torch.bfloat16
+    h, wg = rnd(T, k, seed=1, dtype=bf).cuda(), rnd(E, 2 * ff, k, seed=2, std=k ** -0.5, dtype=bf).cuda()
+    wd, wt = rnd(E, n, ff, seed=3, std=ff ** -0.5, dtype=bf).cuda(), torch.rand(T, top, generator=gen(4)).cuda()
+    scattered = torch.stack([torch.randperm(E, generator=gen(t))[:top] for t in range(T)]).int().cuda()
+    crowded = torch.arange(top).repeat(T, 1).int().cuda()
+    for ids in (scattered, crowded):
+        got = ops.moe_experts(h, ids, wt, wg, wd, tiling=tiling)
+        act = torch.empty(T, top, 2 * ff, device="cuda")
+        for e in range(E):
+            act[ids == e] = (h.float() @ wg[e].float().T)[:, None].expand(T, top, 2 * ff)[ids == e]
+        act = zo.silu(act[..., :ff]) * act[..., ff:]
+        ref = torch.empty(T, top, n, device="cuda")
+        for e in range(E):
+            ref[ids == e] = act[ids == e] @ wd[e].float().T
+        # rounding of the activations and of the results: 2^-9 of each at most, so 2^-8 of the whole (a row of eight sums that cancel may be further off)
+        ref = (wt[..., None] * ref).view(T * top, n)
+        assert bool(torch.isfinite(got).all()) and float((got.float() - ref).norm()) <= 2 ** -8 * float(ref.norm())
+        other = ops.moe_experts(h, ids, wt, wg, wd, tiling="large")
+        assert float((got.float() - other.float()).norm()) <= 2 ** -8 * float(other.float().norm())
+
+
+@pytest.mark.parametrize("E,top", [(5, 5), (16, 4), (33, 7), (64, 64)])
+def test_router_places_choices(ops, E, top):
+    """Experts that are switched off by a bias of -inf, ties, and infinities that leave too few choices."""
+    T, k = 35, 64
+    h, w = rnd(T, k, seed=1, dtype=torch.bfloat16), rnd(E, k, seed=2, std=k ** -0.5, dtype=torch.bfloat16)
+    b = torch.randn(E, generator=gen(3))
+    b[::3] = -float("inf")
+    ids, wt, _ = ops.moe_route(h.cuda(), w.cuda(), b.cuda(), top)
+    z = h.float() @ w.float().T + b
+    live = min(top, int(torch.isfinite(b).sum()))
+    val, idx = torch.sort(z, dim=1, descending=True, stable=True)
+    assert torch.equal(ids.cpu()[:, :live].long(), idx[:, :live])
+    assert bool((ids[:, live:] == E - 1).all()) and bool((wt[:, live:] == 0).all())
+    assert torch.allclose(wt.cpu()[:, :live], torch.softmax(val[:, :live], 1), atol=2e-6)
+    ids, wt, _ = ops.moe_route(torch.zeros(2, k, dtype=torch.bfloat16).cuda(), w.cuda(), torch.zeros(E).cuda(), top)
+    assert torch.equal(ids.cpu(), torch.arange(top).repeat(2, 1).int()) and torch.allclose(wt.cpu(), torch.full((2, top), 1.0 / top))
+
+
 # ---- the model ---------------------------------------------------------------------------------------------------------
 def attn(window, keep, **kw):
     return {"type": "attention", "mixer": dict(dict(heads=4, kv_heads=2, dim=24, vdim=24, rot={"base": 300.0, "dims": 24}, scale=0.25,
