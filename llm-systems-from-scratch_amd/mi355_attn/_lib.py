@@ -65,6 +65,7 @@ EXPORTS = (
     "mi355_moe_group",
     "mi355_moe_gate_up",
     "mi355_moe_down",
+    "mi355_moe_direct",
     "mi355_calib_copy",
     "mi355_last_error",
     "mi355_version",
