@@ -597,6 +597,36 @@ int mi355_moe_direct(const void* h, const void* w_gate_up, const void* w_down, c
                      int top, int k, int ff, int n, void* stream);
 
 /*
+ * Linear layers of a decode step: n_rows (up to 32) rows of x against w (n, k), both bf16, fp32 sums, with what stands in front
+ * of and behind the product.  x_rows (int64, optional): row i of the operand is row x_rows[i] of the x_count rows of x.  norm
+ * (fp32 (k), optional): the operand is x / sqrt(mean(x^2) + eps) * norm.  k in multiples of 8 (up to 4096 with a norm).
+ *   STORE   : out (n_rows, n) bf16
+ *   F32     : out (n_rows, n) fp32
+ *   ADD     : out = bf16(product + resid[i]), or resid[resid_rows[i]] (out may be resid when there are no resid_rows)
+ *   GATE_UP : w (2 n, k), gates first: out (n_rows, n) = bf16(silu(gate) * up)
+ *   QKV     : n = (n_q_heads + 2 n_kv_heads) * head_dim: queries and keys rotated as in mi355_rope_and_cache, queries to out,
+ *             keys and values to the slots of a bf16 cache (outside the cache: not written)
+ */
+enum { MI355_ROWS_STORE = 0, MI355_ROWS_F32 = 1, MI355_ROWS_ADD = 2, MI355_ROWS_GATE_UP = 3, MI355_ROWS_QKV = 4 };
+typedef struct mi355_rows_args {
+    const void* x;
+    const int64_t* x_rows;
+    const float* norm;
+    const void* w;
+    void* out;
+    const void* resid;
+    const int64_t* resid_rows;
+    void *k_cache, *v_cache;
+    const int64_t* slots;
+    const int32_t* positions;
+    const float* freq_cache;
+    int64_t x_count, x_row_stride, out_row_stride, resid_count, resid_row_stride, num_blocks;
+    float eps;
+    int n_rows, n, k, n_q_heads, n_kv_heads, head_dim, context_length;
+} mi355_rows_args;
+int mi355_rows_linear(const mi355_rows_args* args, int mode, void* stream);
+
+/*
  * Plain device-to-device copy of `bytes` bytes (16-byte aligned).  Measurement aid
  * with no counterpart in the reference: a copy of known size whose FETCH_SIZE /
  * WRITE_SIZE counter readings calibrate the HBM-traffic figures of the kernels above.

@@ -519,7 +519,7 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
             a_off[j] = (uint32_t)(((int64_t)(GATE_UP ? pair / p.top : pair) * p.a_stride + piece * 8) * 2);
         }
         f32x4 acc[MT][2];
-        weight_stream<MT>(w_base, w_off, p.a, a_off, p.k / 64, wave, ring + wave * kStreamBytes, acc);
+        weight_stream<MT>(w_base, w_off, p.a, a_off, p.k, wave, ring + wave * kStreamBytes, acc, [] {}, [](int, int, int, bf16x8&) {});
         __syncthreads();                          // (the sums travel through the ring)
         f32x4* part = reinterpret_cast<f32x4*>(ring);                           // [wave][row tile][16 rows of w][lane]
 #pragma unroll

@@ -13,21 +13,26 @@ constexpr int kStreamBytes = 12 * 1024;          // per wavefront: 2 steps of 32
 
 // w_off, a_off: byte offsets of this lane's 16 bytes in step 0: rows 8 j + lane / 8 of the weights (32) and of the activations
 // (16 * MT), piece (lane % 8) ^ (lane / 8) of the row's eight, so that the LDS row holds piece q at q ^ (row % 8).
+// k: row length in elements, a multiple of 8; meanwhile() runs when the first steps have been requested; on_rows(t, s, m, fragment) may change a fragment of activations: lane holds row
+// 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
 // acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
-template <int MT>
+template <int MT, typename G, typename F>
 __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],
-                                              int n_steps, int wave, unsigned char* ring, f32x4 (&acc)[MT][2]) {
+                                              int k, int wave, unsigned char* ring, f32x4 (&acc)[MT][2], G&& meanwhile, F&& on_rows) {
     constexpr int kStep = (32 + 16 * MT) * 128, kDeep = MT == 1 ? 2 : 1, kLoads = 4 + 2 * MT;
     static_assert(kDeep * kStep <= kStreamBytes, "ring");
     const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
     const uint32_t ring0 = lds_address(ring);
+    const int n_steps = (k + 63) / 64;
     const auto request = [&](int t, int slot) {
         const char* wt = (const char*)w + 128 * (int64_t)t;
         const char* at = (const char*)a + 128 * (int64_t)t;
+        // (pieces behind the end of a row: its first piece of this step once more)
+        const uint32_t piece = (lane & 7) ^ (lane >> 3), back = 8 * (int)piece >= k - 64 * t ? 16 * piece : 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dma_to_lds_16(wt, w_off[j], ring0 + slot * kStep + j * 1024);
+        for (int j = 0; j < 4; ++j) dma_to_lds_16(wt, w_off[j] - back, ring0 + slot * kStep + j * 1024);
 #pragma unroll
-        for (int j = 0; j < 2 * MT; ++j) dma_to_lds_16(at, a_off[j], ring0 + slot * kStep + (4 + j) * 1024);
+        for (int j = 0; j < 2 * MT; ++j) dma_to_lds_16(at, a_off[j] - back, ring0 + slot * kStep + (4 + j) * 1024);
     };
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -36,6 +41,7 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
 #pragma unroll
     for (int d = 0; d < kDeep; ++d)
         if (wave + 4 * d < n_steps) request(wave + 4 * d, d);
+    meanwhile();
     int slot = 0;
     for (int t = wave; t < n_steps; t += 4) {
         if (t + 4 * (kDeep - 1) < n_steps) wait_vmcnt<(kDeep - 1) * kLoads>();
@@ -50,10 +56,21 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
 #pragma unroll
             for (int m = 0; m < MT; ++m) af[m][s] = as_bf16x8(*reinterpret_cast<const u32x4*>(at + (32 + 16 * m + r) * 128 + piece));
         }
+        if (k - 64 * t < 64) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s)
+                if (32 * s + 8 * kg >= k - 64 * t)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) af[m][s] = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
+        }
         if (t + 4 * kDeep < n_steps) {
             wait_lgkmcnt0();                      // the slot's bytes are in registers
             request(t + 4 * kDeep, slot);
         }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) on_rows(t, s, m, af[m][s]);
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll

@@ -23,6 +23,7 @@ llm-core/llm_core/model.py:308-325 and the SDPA slot at model.py:382):
     ff_act(a, b)                                        # silu(a) * b, or gelu(a)
     gated_norm(y, z, weight, groups, eps)               # y silu(z) with a norm per group
     ssm_mix(proj, ...)                                  # Mamba-2: causal convolution + selective state, prompts and decode
+    rows_linear(x, w, norm=, resid=, gate_up=), rows_qkv(...)              # linear layers of a decode step with their surroundings
     moe_route(h, w, bias, top), moe_experts(h, ids, weights, w_gate_up, w_down)         # mixture of experts
 
 Models (paged cache, batched prefill and decode, sampling): load_model(folder), CachedTransformerLM, ZuzelornLM,
@@ -48,6 +49,8 @@ from .ops import (  # noqa: F401
     ssm_mix,
     moe_route,
     moe_experts,
+    rows_linear,
+    rows_qkv,
     kv_cache_write,
     paged_attention_any,
     flash_attn_paged_prefill,

@@ -19,6 +19,8 @@ STATIC_SCRATCH_BYTES = 16 << 20          # MI355_STATIC_SCRATCH_BYTES
 SCANS = {"auto": 0, "serial": 1, "chunked": 2}
 TILINGS = {"auto": 0, "skinny": 1, "large": 2}
 
+ROWS_STORE, ROWS_F32, ROWS_ADD, ROWS_GATE_UP, ROWS_QKV = range(5)
+
 _i64x3 = C.c_int64 * 3
 _i64x2 = C.c_int64 * 2
 _lib = None
@@ -66,6 +68,7 @@ EXPORTS = (
     "mi355_moe_gate_up",
     "mi355_moe_down",
     "mi355_moe_direct",
+    "mi355_rows_linear",
     "mi355_calib_copy",
     "mi355_last_error",
     "mi355_version",
@@ -79,6 +82,15 @@ class SsmArgs(C.Structure):
                 [(n, C.c_int64) for n in ("proj_row_stride", "xbc_col", "dt_col", "y_row_stride", "n_rows")] +
                 [(n, C.c_int) for n in ("batch", "heads", "vdim", "state", "groups", "taps", "n_slots", "dtype")] +
                 [("seg_state", C.c_void_p), ("seg_decay", C.c_void_p), ("seg_len", C.c_int)])
+
+
+class RowsArgs(C.Structure):
+    """mi355_rows_args"""
+    _fields_ = ([(n, C.c_void_p) for n in ("x", "x_rows", "norm", "w", "out", "resid", "resid_rows", "k_cache", "v_cache", "slots", "positions",
+                                           "freq_cache")] +
+                [(n, C.c_int64) for n in ("x_count", "x_row_stride", "out_row_stride", "resid_count", "resid_row_stride", "num_blocks")] +
+                [("eps", C.c_float)] +
+                [(n, C.c_int) for n in ("n_rows", "n", "k", "n_q_heads", "n_kv_heads", "head_dim", "context_length")])
 
 
 class LibraryMissing(RuntimeError):
@@ -225,6 +237,8 @@ def load():
     lib.mi355_moe_down.argtypes = [vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, i32, i32, i32, i32, i32, vp]
     lib.mi355_moe_direct.restype = i32
     lib.mi355_moe_direct.argtypes = [vp] * 7 + [i64, i64, i64, i32, i32, i32, i32, i32, vp]
+    lib.mi355_rows_linear.restype = i32
+    lib.mi355_rows_linear.argtypes = [C.POINTER(RowsArgs), i32, vp]
     lib.mi355_calib_copy.restype = i32
     lib.mi355_calib_copy.argtypes = [vp, vp, sz, vp]
     lib.mi355_last_error.restype = C.c_char_p

@@ -482,7 +482,22 @@ class PagedAttentionEngine:
         returns its attention output (B,Hq,D), written into `out` when given (rows may be strided)."""
         if q.shape[0] != plan.positions.shape[0]:
             raise ValueError("one query token per sequence expected")
-        q = self._write_cache(layer, plan, q, k, v)
+        return self._decode_attention(layer, plan, self._write_cache(layer, plan, q, k, v), out)
+
+    def project_decode(self, layer: int, plan: DecodePlan, x, w_qkv, norm, eps: float = 1e-5, x_rows=None):
+        """attend_decode from the layer's input on: x (B,d) bf16 (or rows x_rows of it), normed, times the merged projection w_qkv, in
+        one launch with rotation and cache write.  For a layer with RoPE of its own cache in bf16 (`fuses_projection`)."""
+        q = ops.rows_qkv(x, w_qkv, plan.positions, self.freq_caches[layer], self.k_caches[layer], self.v_caches[layer], plan.slots,
+                         self.layers[layer].n_q_heads, norm=norm, eps=eps, x_rows=x_rows)
+        return self._decode_attention(layer, plan, q, None)
+
+    def fuses_projection(self, layer: int) -> bool:
+        ly, dims = self.layers[layer], self.cache_dims[layer]
+        return (isinstance(ly, AttentionLayer) and self.kv_dtype == "bf16" and ly.rope and ly.kv_from is None and bool(self.mfma[layer])
+                and dims == (ly.head_dim, ly.v_dim or ly.head_dim) and dims[0] == dims[1])
+
+    def _decode_attention(self, layer: int, plan: DecodePlan, q, out):
+        """The step's attention of a layer whose new keys and values are in its cache."""
         terms = dict(self._score_terms(layer), out=out)
         kc, vc = self.k_caches[layer], self.v_caches[layer]
         if not self.mfma[layer]:

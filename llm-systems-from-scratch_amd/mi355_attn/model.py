@@ -22,7 +22,7 @@ import json
 import torch
 
 from . import ops
-from .engine import BLOCK, PagedAttentionEngine
+from .engine import BLOCK, DecodePlan, PagedAttentionEngine
 from .weights import load_state_dict
 
 
@@ -271,6 +271,9 @@ class CachedTransformerLM(CachedLM):
             self.layers.append(dict(wqkv=wqkv, wo=w(pre + "attn.output_proj.weight"), wgu=wgu, wdown=wdown,
                                     attn_norm=w(pre + "attn_norm.weight", torch.float32),
                                     ffn_norm=w(pre + "ffn_norm.weight", torch.float32)))
+        # what rows_linear takes: rows of whole 16-byte pieces, a norm of up to 4096 columns, operands of up to 4 GB
+        biggest = max(3 * d * d, 2 * self.d_ff * d, *(t.numel() for t in (self.emb, self.lm_head)))
+        self._rows_fuse = d <= 4096 and self.d_ff % 8 == 0 and biggest < 1 << 31
         if num_blocks is None:
             num_blocks = max_batch * ((self.context_length + BLOCK - 1) // BLOCK)
         self._serve(PagedAttentionEngine(num_blocks, H, H, self.d_head, self.context_length, rope_theta=config["rope_theta"],
@@ -283,6 +286,8 @@ class CachedTransformerLM(CachedLM):
         Returns logits of rows `out_rows` (default: all rows), fp32."""
         H, dh, d, ff = self.num_heads, self.d_head, self.d_model, self.d_ff
         T = token_ids.shape[0]
+        if self._rows_fuse and T <= ops.MAX_LINEAR_ROWS and isinstance(plan, DecodePlan) and out_rows is None:
+            return self._forward_rows(token_ids, plan, attend)
         resid = self.emb[token_ids]                                   # model.py:50
         h = ops.rms_norm(resid, self.layers[0]["attn_norm"])
         for i, ly in enumerate(self.layers):
@@ -297,3 +302,19 @@ class CachedTransformerLM(CachedLM):
         if out_rows is not None:
             h = h[out_rows]
         return (h @ self.lm_head.T).float()                            # model.py:185
+
+    def _forward_rows(self, token_ids, plan, attend):
+        """The same for the few rows of a decode step, a layer in five launches: norm + projection + rotation + cache write,
+        attention, output projection + residual, norm + gate/up + activation, down projection + residual."""
+        H, dh, d = self.num_heads, self.d_head, self.d_model
+        x, rows = self.emb, token_ids                                 # the residual stream: rows of the embedding, then of its own
+        for i, ly in enumerate(self.layers):
+            if self.engine.fuses_projection(i):
+                a = self.engine.project_decode(i, plan, x, ly["wqkv"], ly["attn_norm"], x_rows=rows)
+            else:
+                qkv = ops.rows_linear(x, ly["wqkv"], norm=ly["attn_norm"], x_rows=rows).view(-1, 3, H, dh)
+                a = attend(i, plan, qkv[:, 0], qkv[:, 1], qkv[:, 2])
+            x, rows = ops.rows_linear(a.reshape(-1, d), ly["wo"], resid=x, resid_rows=rows), None
+            f = ops.rows_linear(x, ly["wgu"], norm=ly["ffn_norm"], gate_up=True)
+            x = ops.rows_linear(f, ly["wdown"], resid=x)
+        return ops.rows_linear(x, self.lm_head, norm=self.final_norm, x_rows=rows, out_dtype=torch.float32)

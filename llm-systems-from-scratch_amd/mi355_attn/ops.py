@@ -1472,3 +1472,85 @@ def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
                                 order.data_ptr(), T, ff, out.stride(0), E, top, ff, n, code, tl, stream)
         _lib.check(rc, "mi355_moe_down")
     return out
+
+
+MAX_LINEAR_ROWS = 32        # the most rows rows_linear and rows_qkv take
+
+
+def _row_ids(name, t, T):
+    if t is not None and (t.dtype != torch.int64 or t.shape != (T,) or not t.is_contiguous()):
+        raise TypeError(f"{name} must be a contiguous int64 ({T},) tensor")
+
+
+def _bf16_rows(name, t, cols):
+    if t.dtype != torch.bfloat16 or t.dim() != 2 or t.shape[1] != cols or t.stride(1) != 1:
+        raise ValueError(f"{name} must be a bfloat16 matrix of {cols} columns with unit column stride")
+    return t.stride(0) if t.shape[0] > 1 else cols
+
+
+def rows_linear(x, w, *, norm=None, eps: float = 1e-5, x_rows=None, resid=None, resid_rows=None, gate_up=False, out_dtype=torch.bfloat16):
+    """A linear layer of a decode step: up to 32 rows of x (T,k) against w (n,k), both bf16, fp32 sums, in one launch with
+
+        x_rows (T,) int64: row i of the operand is x[x_rows[i]]        norm (k,) fp32: the operand is x / sqrt(mean(x^2) + eps) * norm
+        resid (.,n) bf16: + resid[i], or resid[resid_rows[i]]          gate_up: w (2n,k), gates first; the result is silu(gate) * up
+
+    Returns (T,n) in bf16, or with out_dtype float32 the fp32 sums (no resid, no gate_up)."""
+    T = x.shape[0] if x_rows is None else x_rows.numel()
+    w_rows, k = w.shape
+    n = w_rows // 2 if gate_up else w_rows
+    x_stride = _bf16_rows("x", x, k)
+    _row_ids("x_rows", x_rows, T)
+    _row_ids("resid_rows", resid_rows, T)
+    if w.dtype != torch.bfloat16 or not w.is_contiguous() or (gate_up and w_rows % 2):
+        raise ValueError("w must be a contiguous bfloat16 (n, k) matrix (2n rows with gate_up)")
+    _vector("norm", norm, k)
+    f32 = out_dtype == torch.float32
+    if (resid is not None) + gate_up + f32 > 1 or (not f32 and out_dtype != torch.bfloat16):
+        raise ValueError("a residual, gate_up and fp32 results exclude each other")
+    r_stride = 0
+    if resid is not None:
+        r_stride = _bf16_rows("resid", resid, n)
+        if resid_rows is None and resid.shape[0] != T:
+            raise ValueError("one residual row per row expected")
+    out = torch.empty(T, n, dtype=out_dtype, device=x.device)
+    if T == 0:
+        return out
+    mode = _lib.ROWS_ADD if resid is not None else _lib.ROWS_GATE_UP if gate_up else _lib.ROWS_F32 if f32 else _lib.ROWS_STORE
+    ptr = [None if t is None else t.data_ptr() for t in (x, x_rows, norm, w, out, resid, resid_rows)]
+    with _on(x, x_rows, norm, w, resid, resid_rows) as stream:
+        args = _lib.RowsArgs(*ptr, None, None, None, None, None, x.shape[0], x_stride, n, 0 if resid is None else resid.shape[0], r_stride, 0,
+                             float(eps), T, n, k, 0, 0, 0, 0)
+        _lib.check(_lib.load().mi355_rows_linear(args, mode, stream), "mi355_rows_linear")
+    return out
+
+
+def rows_qkv(x, w, positions, freq_cache, k_cache, v_cache, slot_mapping, n_q_heads: int, *, norm=None, eps: float = 1e-5, x_rows=None):
+    """The merged query/key/value projection of a decode step (rows_linear) and rope_and_cache of its result, in one launch.  w
+    ((Hq + 2 Hkv) D, k); k_cache, v_cache (num_blocks,Hkv,16,D) bf16; the rest as there.  Returns the rotated queries (T,Hq,D)."""
+    T = x.shape[0] if x_rows is None else x_rows.numel()
+    n, k = w.shape
+    x_stride = _bf16_rows("x", x, k)
+    _row_ids("x_rows", x_rows, T)
+    _row_ids("slot_mapping", slot_mapping, T)
+    _vector("norm", norm, k)
+    nb, Hkv, bs, D = k_cache.shape
+    for name, c in (("k_cache", k_cache), ("v_cache", v_cache)):
+        if c.dtype != torch.bfloat16 or tuple(c.shape) != (nb, Hkv, _BLOCK, D) or not c.is_contiguous():
+            raise ValueError(f"{name} must be a contiguous bf16 (num_blocks, kv_heads, {_BLOCK}, d_head) tensor")
+    if w.dtype != torch.bfloat16 or not w.is_contiguous() or n != (n_q_heads + 2 * Hkv) * D:
+        raise ValueError(f"w must be a contiguous bfloat16 ({(n_q_heads + 2 * Hkv) * D}, k) matrix")
+    if freq_cache.dtype != torch.float32 or freq_cache.dim() != 3 or freq_cache.shape[0] != 2 or freq_cache.shape[2] * 2 != D \
+            or not freq_cache.is_contiguous():
+        raise ValueError("freq_cache must be a contiguous float32 tensor (2, context_length, d_head/2)")
+    if positions.dtype != torch.int32 or positions.shape != (T,) or not positions.is_contiguous():
+        raise TypeError("positions must be a contiguous int32 (tokens,) tensor")
+    out = torch.empty(T, n_q_heads, D, dtype=torch.bfloat16, device=x.device)
+    if T == 0:
+        return out
+    with _on(x, x_rows, norm, w, k_cache, v_cache, slot_mapping, positions, freq_cache) as stream:
+        args = _lib.RowsArgs(x.data_ptr(), None if x_rows is None else x_rows.data_ptr(), None if norm is None else norm.data_ptr(), w.data_ptr(),
+                             out.data_ptr(), None, None, k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(), positions.data_ptr(),
+                             freq_cache.data_ptr(), x.shape[0], x_stride, n_q_heads * D, 0, 0, nb, float(eps), T, n, k, n_q_heads, Hkv, D,
+                             freq_cache.shape[1])
+        _lib.check(_lib.load().mi355_rows_linear(args, _lib.ROWS_QKV, stream), "mi355_rows_linear")
+    return out

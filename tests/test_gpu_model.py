@@ -322,3 +322,61 @@ def test_from_pretrained_reads_reference_files(ops, tmp_path):
     _logit_close(model.forward(ids), mo.transformer_lm_reference(bf, CFG, ids))
     with pytest.raises(ValueError):
         ops.CachedTransformerLM(dict(CFG, num_heads=8), bf)            # d_head 16 is not supported by the kernels
+
+
+# ---- linear layers of a decode step ----------------------------------------------------------------------
+def _close_rows(got, ref, rounded, what):
+    """Products of bf16 operands with fp32 sums: what is rounded to bf16 on the way (the normed operand, the result) is off by 2^-9 of itself at
+    most, a sum of k roundings of random sign by no more of its norm."""
+    got, ref = got.double().cpu(), ref.double().cpu()
+    assert bool(torch.isfinite(got).all()), what
+    assert float((got - ref).norm()) <= (rounded * 2 ** -8 + 1e-6) * float(ref.norm()), what
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 32])
+@pytest.mark.parametrize("k,n", [(8, 4), (64, 30), (72, 129), (512, 96), (1344, 512), (4096, 36)])
+def test_rows_linear(ops, T, k, n):
+    """Edges of the row tiles, of the 32 weight rows of a workgroup and of the 64-wide steps of k (fewer than four of them, remainders)."""
+    g = torch.Generator().manual_seed(T * 1000 + k)
+
+    def t(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g) * std).to(torch.bfloat16).cuda()
+
+    table, w, norm = t(50, k + 8), t(2 * n, k, std=k ** -0.5), (torch.randn(k, generator=g) * 0.3 + 1).cuda()
+    ids = torch.randint(0, 50, (T,), generator=g).cuda()
+    rows, resid = table[:, :k], t(40, n + 4)[:, :n]
+    x = rows[ids].double()
+    normed = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5) * norm.double()
+    wd = w.double()
+    _close_rows(ops.rows_linear(rows[:T].contiguous(), w[:n].contiguous()), rows[:T].double() @ wd[:n].T, 1, "plain")
+    _close_rows(ops.rows_linear(rows, w[:n].contiguous(), x_rows=ids, out_dtype=torch.float32), x @ wd[:n].T, 0, "fp32")
+    _close_rows(ops.rows_linear(rows, w[:n].contiguous(), x_rows=ids, norm=norm, out_dtype=torch.float32), normed @ wd[:n].T, 1, "norm")
+    pick = torch.randint(0, 40, (T,), generator=g).cuda()
+    _close_rows(ops.rows_linear(rows, w[:n].contiguous(), x_rows=ids, resid=resid, resid_rows=pick), x @ wd[:n].T + resid[pick].double(), 1, "add")
+    gate, up = (normed @ wd.T).split(n, 1)
+    _close_rows(ops.rows_linear(rows, w, x_rows=ids, norm=norm, gate_up=True), torch.nn.functional.silu(gate) * up, 3, "gate_up")
+    with pytest.raises(ValueError):
+        ops.rows_linear(t(33, k), w)
+
+
+@pytest.mark.parametrize("T,H,G,D", [(1, 2, 2, 32), (17, 4, 1, 64), (32, 8, 2, 128)])
+def test_rows_qkv(ops, T, H, G, D):
+    """Projection, rotation and cache write in one launch against the product and rope_and_cache: the product is rounded once less."""
+    g = torch.Generator().manual_seed(D)
+    k, nb = 200, 9
+
+    def t(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g) * std).to(torch.bfloat16).cuda()
+
+    x, w = t(T, k), t((H + 2 * G) * D, k, std=k ** -0.5)
+    pos = torch.randint(0, 70, (T,), generator=g).int().cuda()                  # (some beyond the table: clamped into it)
+    slots = torch.randperm(nb * 16, generator=g)[:T].cuda()
+    slots[0] = -1 if T > 1 else slots[0]
+    freq = ops.build_rope_cache(64, D)
+    pools = [torch.full((nb, G, 16, D), 3.0, dtype=torch.bfloat16).cuda() for _ in range(4)]
+    q = ops.rows_qkv(x, w, pos, freq, pools[0], pools[1], slots, H)
+    qkv = (x.float() @ w.float().T).to(torch.bfloat16).view(T, H + 2 * G, D)
+    ref = ops.rope_and_cache(qkv[:, :H], qkv[:, H:H + G], qkv[:, H + G:], pos, freq, pools[2], pools[3], slots)
+    for got, want, what in ((q, ref, "q"), (pools[0], pools[2], "k"), (pools[1], pools[3], "v")):
+        _close_rows(got, want, 2, what)
+        assert torch.equal(got.float().cpu() == 3.0, want.float().cpu() == 3.0) or what == "q"       # the same rows are written
