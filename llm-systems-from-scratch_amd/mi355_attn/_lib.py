@@ -248,11 +248,11 @@ def load():
 
 
 def strides3(values):
-    return _i64x3(*[int(v) for v in values])
+    return _i64x3(*values)
 
 
 def strides2(values):
-    return _i64x2(*[int(v) for v in values])
+    return _i64x2(*values)
 
 
 def floats4(values):

@@ -18,8 +18,10 @@ flash_attn_paged_prefill, paged_attention_decode, paged_attention_any, ssm_mix);
 from __future__ import annotations
 
 import math
+from array import array
 from dataclasses import dataclass, field
 
+import numpy as np
 import torch
 
 from . import ops
@@ -138,40 +140,41 @@ class StaticDecodeStep:
     """Device tensors of one decode step at fixed addresses, refreshed from the host by one copy.
 
     Layout of the int32 buffer: token ids (int64), slots (int64), positions, context lengths,
-    state slots, block tables (batch x max_blocks)."""
+    state slots, block tables (batch x max_blocks).  The host side is two such buffers in turn, so that a step is written
+    while the copy of the one in front may still wait on the stream."""
 
     def __init__(self, batch: int, max_blocks: int, device):
         B, M = batch, max_blocks
         self.batch, self.max_blocks = B, M
         n = 7 * B + B * M
         self._dev = torch.zeros(n, dtype=torch.int32, device=device)
-        self._host = torch.zeros(n, dtype=torch.int32, pin_memory=True)
-        self._copied = torch.cuda.Event()
-        self._pending = False
         self.tokens = self._dev[0:2 * B].view(torch.int64)
         slots = self._dev[2 * B:4 * B].view(torch.int64)
         positions = self._dev[4 * B:5 * B]
         context_lens = self._dev[5 * B:6 * B]
         tables = self._dev[7 * B:].view(B, M)
         self.plan = DecodePlan(positions, slots, tables, context_lens, M * BLOCK, self._dev[6 * B:7 * B])
-        h = self._host
-        self._h_tokens, self._h_slots = h[0:2 * B].view(torch.int64), h[2 * B:4 * B].view(torch.int64)
-        self._h_positions, self._h_ctx, self._h_state = h[4 * B:5 * B], h[5 * B:6 * B], h[6 * B:7 * B]
-        self._h_tables = h[7 * B:].view(B, M)
+        self._turn = 0
+        self._staging = []
+        for host in torch.zeros(2, n, dtype=torch.int32, pin_memory=True):         # (one allocation: it is a millisecond's work)
+            h = host.numpy()
+            self._staging.append((host, torch.cuda.Event(), h[0:2 * B].view(np.int64), h[2 * B:4 * B].view(np.int64), h[4 * B:5 * B],
+                                  h[5 * B:6 * B], h[6 * B:7 * B], h[7 * B:].reshape(B, M)))
+        self._pending = [False, False]
 
-    def fill(self, tokens, slots, positions, context_lens, block_lists, state_slots) -> None:
-        if self._pending:
-            self._copied.synchronize()              # the previous copy has left the staging buffer
-        self._h_tokens.copy_(torch.tensor(tokens, dtype=torch.int64))
-        self._h_slots.copy_(torch.tensor(slots, dtype=torch.int64))
-        self._h_positions.copy_(torch.tensor(positions, dtype=torch.int32))
-        self._h_ctx.copy_(torch.tensor(context_lens, dtype=torch.int32))
-        self._h_state.copy_(torch.tensor(state_slots, dtype=torch.int32))
-        for i, blocks in enumerate(block_lists):
-            self._h_tables[i, :len(blocks)] = torch.tensor(blocks, dtype=torch.int32)
-        self._dev.copy_(self._host, non_blocking=True)
-        self._copied.record()
-        self._pending = True
+    def fill(self, tokens, slots, positions, context_lens, block_rows, state_slots) -> None:
+        """block_rows: each sequence's blocks as an array of int32."""
+        turn = self._turn
+        host, copied, h_tokens, h_slots, h_positions, h_ctx, h_state, h_tables = self._staging[turn]
+        if self._pending[turn]:
+            copied.synchronize()                    # the copy of the step before last has left the buffer
+        h_tokens[:], h_slots[:], h_positions[:], h_ctx[:], h_state[:] = tokens, slots, positions, context_lens, state_slots
+        for i, blocks in enumerate(block_rows):
+            h_tables[i, :len(blocks)] = blocks
+        self._dev.copy_(host, non_blocking=True)
+        copied.record()
+        self._pending[turn] = True
+        self._turn = 1 - turn
 
 
 class PagedAttentionEngine:
@@ -266,6 +269,7 @@ class PagedAttentionEngine:
                              for d in {dims[0] for dims in self.cache_dims if dims}} if kv_dtype == "fp8" else None
         self.allocator = BlockAllocator(num_blocks)
         self.blocks: dict[int, list[int]] = {}      # sequence id -> physical blocks
+        self._block_rows: dict[int, array] = {}     # the same as int32 arrays: a table row is one copy, not a conversion per block
         self.lengths: dict[int, int] = {}           # sequence id -> tokens in the cache
         self.state_slots: dict[int, int] = {}       # sequence id -> state slot (models with state layers)
         self._free_slots = list(range(max_batch - 1, -1, -1))
@@ -295,31 +299,50 @@ class PagedAttentionEngine:
                 raise OutOfBlocks(f"all {self.max_batch} state slots are taken")
             self.state_slots[seq_id] = self._free_slots.pop()
         self.blocks[seq_id] = []
+        self._block_rows[seq_id] = array("i")
         self.lengths[seq_id] = 0
 
     def remove_sequence(self, seq_id: int) -> None:
         self.allocator.free(self.blocks.pop(seq_id))
-        del self.lengths[seq_id]
+        del self.lengths[seq_id], self._block_rows[seq_id]
         if seq_id in self.state_slots:
             self._free_slots.append(self.state_slots.pop(seq_id))       # (a new sequence starts from zero whatever the slot holds)
 
-    def _slots_of(self, seq_ids) -> torch.Tensor | None:
-        return torch.tensor([self.state_slots[s] for s in seq_ids], dtype=torch.int32, device=self.device) if self.conv_states else None
-
-    def _reserve(self, seq_id: int, n_new: int) -> list[int]:
-        """Slots for the next n_new tokens of a sequence (allocates blocks as needed)."""
+    def _reserve(self, seq_id: int, n_new: int):
+        """Slots for the next n_new tokens of a sequence (allocates blocks as needed), as an int64 array."""
         length = self.lengths[seq_id]
         if length + n_new > self.context_length:
             raise ValueError(f"sequence {seq_id} would exceed context_length {self.context_length}")
-        blocks = self.blocks[seq_id]
+        blocks, row = self.blocks[seq_id], self._block_rows[seq_id]
         need = (length + n_new + BLOCK - 1) // BLOCK - len(blocks)
         if need > self.allocator.num_free:
             raise OutOfBlocks(f"sequence {seq_id} needs {need} blocks, {self.allocator.num_free} free")
         for _ in range(need):
             blocks.append(self.allocator.allocate())
-        slots = [blocks[t // BLOCK] * BLOCK + t % BLOCK for t in range(length, length + n_new)]
+            row.append(blocks[-1])
         self.lengths[seq_id] = length + n_new
-        return slots
+        if n_new == 1:
+            return [blocks[length // BLOCK] * BLOCK + length % BLOCK]
+        t = np.arange(length, length + n_new, dtype=np.int64)
+        return np.array(row, dtype=np.int64)[t // BLOCK] * BLOCK + t % BLOCK
+
+    def _tables_of(self, seq_ids) -> torch.Tensor:
+        """Block tables of these sequences on the host, as wide as the longest."""
+        rows = np.zeros((len(seq_ids), max(len(self.blocks[s]) for s in seq_ids)), dtype=np.int32)
+        for i, s in enumerate(seq_ids):
+            rows[i, :len(self.blocks[s])] = self._block_rows[s]
+        return torch.from_numpy(rows)
+
+    def _on_device(self, *parts) -> list[torch.Tensor]:
+        """Host integers as device tensors, (values, dtype) each, in one copy.  The int64 ones come first."""
+        arrays = [np.asarray(v, dtype=dt) for v, dt in parts]
+        flat = torch.from_numpy(np.concatenate([a.view(np.int32) for a in arrays])).to(self.device)
+        out, at = [], 0
+        for a in arrays:
+            words = a.size * (a.itemsize // 4)
+            out.append(flat[at:at + words].view(torch.int64 if a.itemsize == 8 else torch.int32))
+            at += words
+        return out
 
     # ---- planning (once per step) ---------------------------------------------
     def plan_prefill(self, seq_ids, lens) -> PrefillPlan:
@@ -341,29 +364,24 @@ class PagedAttentionEngine:
         slots, positions, cu = [], [], [0]
         for sid, n in zip(seq_ids, lens):
             start = self.lengths[sid]
-            slots += self._reserve(sid, n)
-            positions += list(range(start, start + n))
+            slots.append(self._reserve(sid, n))
+            positions.append(np.arange(start, start + n, dtype=np.int32))
             cu.append(cu[-1] + n)
-        dev = self.device
-        plan = PrefillPlan(torch.tensor(positions, dtype=torch.int32, device=dev),
-                           torch.tensor(slots, dtype=torch.int64, device=dev),
-                           torch.tensor(cu, dtype=torch.int32, device=dev), max(lens),
-                           torch.tensor([c - 1 for c in cu[1:]], dtype=torch.int64, device=dev),
-                           state_slots=self._slots_of(seq_ids))
+        context = [self.lengths[sid] for sid in seq_ids]
+        i64, i32 = np.int64, np.int32
+        slots, last, pos, cu_seqlens, ctx, state = self._on_device(
+            (np.concatenate(slots), i64), ([c - 1 for c in cu[1:]], i64), (np.concatenate(positions), i32), (cu, i32), (context, i32),
+            ([self.state_slots.get(s, 0) for s in seq_ids], i32))
+        plan = PrefillPlan(pos, slots, cu_seqlens, max(lens), last, state_slots=state if self.conv_states else None)
         if chunked or self.always_tables:
-            max_blk = max(len(self.blocks[sid]) for sid in seq_ids)
-            rows = torch.zeros(len(seq_ids), max_blk, dtype=torch.int32)
-            for i, sid in enumerate(seq_ids):
-                b = self.blocks[sid]
-                rows[i, :len(b)] = torch.tensor(b, dtype=torch.int32)
-            plan.tables = rows.to(dev)
-            plan.context_lens = torch.tensor([self.lengths[sid] for sid in seq_ids], dtype=torch.int32, device=dev)
+            plan.tables = self._tables_of(seq_ids).to(self.device)
+            plan.context_lens = ctx
             plan.total_context = sum(self.lengths[sid] for sid in seq_ids)
             if self.kv_dtype == "fp8":
                 run = [0]
                 for sid in seq_ids:
                     run.append(run[-1] + self.lengths[sid])
-                plan.cu_context = torch.tensor(run, dtype=torch.int32, device=dev)
+                plan.cu_context = torch.tensor(run, dtype=torch.int32, device=self.device)
         return plan
 
     def _reserve_decode(self, seq_ids):
@@ -389,19 +407,12 @@ class PagedAttentionEngine:
         """Reserves the slot of one new token for each running sequence in `seq_ids`."""
         B = len(seq_ids)
         positions, slots = self._reserve_decode(seq_ids)
-        dev = self.device
-        max_len = max(self.lengths[s] for s in seq_ids)
-        max_blk = (max_len + BLOCK - 1) // BLOCK
-        rows = torch.zeros(B, max_blk, dtype=torch.int32)
-        for i, s in enumerate(seq_ids):
-            b = self.blocks[s]
-            rows[i, :len(b)] = torch.tensor(b, dtype=torch.int32)
-        tables = self._tables[:B, :max_blk]
+        rows = self._tables_of(seq_ids)
+        tables = self._tables[:B, :rows.shape[1]]
         tables.copy_(rows, non_blocking=False)
-        return DecodePlan(torch.tensor(positions, dtype=torch.int32, device=dev),
-                          torch.tensor(slots, dtype=torch.int64, device=dev), tables,
-                          torch.tensor([p + 1 for p in positions], dtype=torch.int32, device=dev), max_blk * BLOCK,
-                          self._slots_of(seq_ids))
+        slots, positions, context_lens, state = self._on_device(
+            (slots, np.int64), (positions, np.int32), ([p + 1 for p in positions], np.int32), ([self.state_slots.get(s, 0) for s in seq_ids], np.int32))
+        return DecodePlan(positions, slots, tables, context_lens, rows.shape[1] * BLOCK, state if self.conv_states else None)
 
     def make_static_decode(self, batch: int) -> "StaticDecodeStep":
         """Fixed device tensors for decode steps of `batch` sequences (what a captured HIP graph needs:
@@ -419,7 +430,7 @@ class PagedAttentionEngine:
             raise ValueError("seq_ids, tokens and the static buffers disagree on the batch size")
         positions, slots = self._reserve_decode(seq_ids)
         static.fill([int(t) for t in tokens], slots, positions, [p + 1 for p in positions],
-                    [self.blocks[s] for s in seq_ids], [self.state_slots.get(s, 0) for s in seq_ids])
+                    [self._block_rows[s] for s in seq_ids], [self.state_slots.get(s, 0) for s in seq_ids])
         return static.plan
 
     # ---- attention calls (once per layer) -----------------------------------------

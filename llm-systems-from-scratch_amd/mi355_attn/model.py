@@ -60,6 +60,14 @@ class CachedLM:
             raise ValueError(f"token ids must be in 0..{self.vocab_size - 1}")
         return ids
 
+    def _token_list(self, tokens) -> list[int]:
+        """_token_ids as a list; a list of ints is looked at as it is."""
+        if type(tokens) is not list or not all(type(t) is int for t in tokens):
+            return self._token_ids(tokens).tolist()
+        if tokens and not 0 <= min(tokens) <= max(tokens) < self.vocab_size:
+            raise ValueError(f"token ids must be in 0..{self.vocab_size - 1}")
+        return tokens
+
     # ---- sequence-level API ---------------------------------------------------------------------
     def new_sequence(self) -> int:
         sid = self._next_id
@@ -87,7 +95,7 @@ class CachedLM:
         """Appends one token to each running sequence; returns the next-token logits (n_seq, vocab) fp32."""
         seq_ids = list(seq_ids)
         if self.decode_graphs:
-            return self._decode_graphed(seq_ids, self._token_ids(tokens).tolist())
+            return self._decode_graphed(seq_ids, self._token_list(tokens))
         ids = self._token_ids(tokens).to(self.device)
         if ids.numel() != len(seq_ids):
             raise ValueError("one token per sequence expected")

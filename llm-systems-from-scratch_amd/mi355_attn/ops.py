@@ -18,24 +18,32 @@ _BLOCK = 16
 
 class _on:
     """`with _on(t0, t1, ...) as stream:` -- checks that every given tensor lives on one GPU, makes that GPU
-    the current device for the launch and yields its current stream (as the integer the C ABI takes)."""
+    the current device for the launch and yields its current stream (as the integer the C ABI takes).
+    The switch of devices is left out where the GPU is current already, and the stream's number is asked for without a Stream
+    object around it: 2 of the 13.6 us that a call of a 7 us kernel took."""
+
+    __slots__ = ("device", "_guard")
 
     def __init__(self, *tensors):
-        ts = [t for t in tensors if t is not None]
-        self.device = ts[0].device
-        for t in ts:
-            if t.device != self.device:
-                raise ValueError(f"all tensors of one call must be on one device (got {self.device} and {t.device})")
+        self.device = None
+        for t in tensors:
+            if t is not None:
+                if self.device is None:
+                    self.device = t.device
+                elif t.device != self.device:
+                    raise ValueError(f"all tensors of one call must be on one device (got {self.device} and {t.device})")
         if self.device.type != "cuda":
             raise ValueError(f"tensors must live on the GPU (got {self.device}); this library has no CPU path")
-        self._guard = torch.cuda.device(self.device)
 
     def __enter__(self):
-        self._guard.__enter__()
-        return torch.cuda.current_stream(self.device).cuda_stream
+        index = self.device.index
+        self._guard = None if torch.cuda.current_device() == index else torch.cuda.device(index)
+        if self._guard is not None:
+            self._guard.__enter__()
+        return torch._C._cuda_getCurrentRawStream(index)
 
     def __exit__(self, *exc):
-        return self._guard.__exit__(*exc)
+        return None if self._guard is None else self._guard.__exit__(*exc)
 
 
 def _require_gpu_bf16(name, t):
