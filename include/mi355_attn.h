@@ -220,6 +220,16 @@ int mi355_prefill_bwd_mask(const void* q, const void* k, const void* v, const vo
                            const int64_t lse_strides[2], const uint8_t* mask, const int64_t mask_strides[3],
                            int B, int Hq, int Hkv, int Sq, int Sk, int D, float softmax_scale, int dtype,
                            void* stream);
+/* Both of the above, with gradients of either type: bit 0, 1, 2 of f32_grads makes dq, dk, dv fp32 (strides in elements).
+ * mask and mask_strides are read with MI355_MASK_BOOL only. */
+int mi355_prefill_bwd_typed(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,
+                            float* delta, void* dq, void* dk, void* dv, const int64_t q_strides[3], const int64_t k_strides[3],
+                            const int64_t v_strides[3], const int64_t o_strides[3], const int64_t do_strides[3],
+                            const int64_t dq_strides[3], const int64_t dk_strides[3], const int64_t dv_strides[3],
+                            const int64_t lse_strides[2], const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                            const uint8_t* mask, const int64_t mask_strides[3], int f32_grads, int B, int Hq, int Hkv, int Sq_max,
+                            int Sk_max, int D, float softmax_scale, int mask_mode, int dtype, void* stream);
+
 
 /*
  * Paged-KV decode attention, one query token per sequence (split-K + combine).

@@ -5,8 +5,8 @@
 //   P_ij    = exp(scale * q_i.k_j - lse_i)                 (recomputed, never stored)
 //   dV_j    = sum_i P_ij dO_i                              (bwd_dkv_kernel: one workgroup per key tile,
 //   dP_ij   = dO_i . v_j                                    summing over the query heads of a GQA group;
-//   dS_ij   = P_ij (dP_ij - delta_i)                        dV on half of its wavefronts, dK on the other half)
-//   dK_j    = scale * sum_i dS_ij q_i
+//   dS_ij   = P_ij (dP_ij - delta_i)                        dV on half of its wavefronts, dK on the other half;
+//   dK_j    = scale * sum_i dS_ij q_i                       head sizes 32 and 64: bwd_dkv_one_kernel)
 //   dQ_i    = scale * sum_j dS_ij k_j                      (bwd_dq_kernel: one workgroup per query tile)
 //
 // Both kernels work on transposed problems, like the forward: the wavefront owns 32 columns
@@ -40,9 +40,10 @@ struct BwdParams {
     const __bf16* dout;
     const float* lse;
     float* delta;
-    __bf16* dq;
-    __bf16* dk;
-    __bf16* dv;
+    void* dq;                     // bf16 or fp32
+    void* dk;
+    void* dv;
+    bool dq_f32, dk_f32, dv_f32;
     int64_t qs[3], ks[3], vs[3], os[3], dos[3], dqs[3], dks[3], dvs[3];   // batch, head, row strides (elements)
     int64_t ls[2];                                                          // lse / delta: batch, head strides
     const int32_t* cu_q;
@@ -53,6 +54,20 @@ struct BwdParams {
     float scale, scale_log2;
     int n_qtiles, n_ktiles;
 };
+
+// Gradients leave in bf16, or in fp32 for an fp32 input: the sums as they are, where a conversion behind the kernel would
+// read and write them once more (64 x 16 heads x 256 x 32: 8.8 us each for dq and dk).
+// Four adjacent elements at element offset `at`.
+__device__ __forceinline__ void store_grad4(void* grad, bool f32, int64_t at, float a, float b, float c, float d) {
+    if (f32) {
+        *reinterpret_cast<f32x4*>((float*)grad + at) = f32x4{a, b, c, d};
+    } else {
+        u32x2 w;
+        w[0] = pack_bf16(a, b);
+        w[1] = pack_bf16(c, d);
+        *reinterpret_cast<u32x2*>((__bf16*)grad + at) = w;
+    }
+}
 
 // Loader of a 64-row tile (rows of D bf16, row stride `stride` elements) into swizzled LDS:
 // wavefront w, instruction j covers LDS chunks (w*NI + j)*64 .. +63; rows past `last` re-read row `last`.
@@ -320,16 +335,13 @@ __global__ __launch_bounds__(kBwWaves * 64, 1) void bwd_dq_kernel(BwdParams p) {
 
         // store: lane owns query qi, d = 32dt + 8(i/4) + 4kg + i%4
         if (q_ok) {
-            __bf16* row = p.dq + dq_base + (int64_t)qi * p.dqs[2];
+            const int64_t row = dq_base + (int64_t)qi * p.dqs[2];
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    u32x2 w;
-                    w[0] = pack_bf16(dq[dt][4 * g + 0] * p.scale, dq[dt][4 * g + 1] * p.scale);
-                    w[1] = pack_bf16(dq[dt][4 * g + 2] * p.scale, dq[dt][4 * g + 3] * p.scale);
-                    *reinterpret_cast<u32x2*>(row + 32 * dt + 8 * g + 4 * kg) = w;
-                }
+                for (int g = 0; g < 4; ++g)
+                    store_grad4(p.dq, p.dq_f32, row + 32 * dt + 8 * g + 4 * kg, dq[dt][4 * g + 0] * p.scale, dq[dt][4 * g + 1] * p.scale,
+                                dq[dt][4 * g + 2] * p.scale, dq[dt][4 * g + 3] * p.scale);
         }
     }
 }
@@ -651,34 +663,280 @@ __global__ __launch_bounds__(2 * kFuPairs * 64, 1) void bwd_dkv_kernel(BwdParams
         // store: lane owns key kj, d = 32dt + 8(i/4) + 4kg + i%4
         if (k_ok) {
             const float f = role_b ? p.scale : 1.0f;
-            __bf16* row = role_b ? p.dk + dk_base + (int64_t)kj * p.dks[2] : p.dv + dv_base + (int64_t)kj * p.dvs[2];
+            const int64_t row = role_b ? dk_base + (int64_t)kj * p.dks[2] : dv_base + (int64_t)kj * p.dvs[2];
+            void* const grad = role_b ? p.dk : p.dv;
+            const bool f32 = role_b ? p.dk_f32 : p.dv_f32;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    store_grad4(grad, f32, row + 32 * dt + 8 * g + 4 * kg, acc[dt][4 * g + 0] * f, acc[dt][4 * g + 1] * f, acc[dt][4 * g + 2] * f,
+                                acc[dt][4 * g + 3] * f);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// dK and dV at head sizes 32 and 64, where one wavefront has the registers for both: it holds the K and V fragments of 32
+// keys and both accumulators, so that P need not travel.  Workgroups of four wavefronts (128 keys) with 16 or 32 KB of LDS:
+// two to four of them on a compute unit fill each other's barriers and load latencies, which is what the kernel with two
+// roles (87 / 107 KB: one workgroup) spends most of its time in at these sizes.
+template <int D, int MODE>
+__global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdParams p) {
+    constexpr bool CAUSAL = MODE == MI355_MASK_CAUSAL, BOOLM = MODE == MI355_MASK_BOOL;
+    constexpr int NWV = kFuPairs;
+    using R = TileReads<D>;
+    constexpr int NS = R::NS, NDT = R::NDT, kRow = R::kRow, kTile = kBwRows * kRow;
+    // [Q buffer 0][Q buffer 1][dO buffer 0][dO buffer 1]
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];
+    __shared__ __attribute__((aligned(16))) float lse_lds2[2 * kBwRows];
+    __shared__ __attribute__((aligned(16))) float delta_lds2[2 * kBwRows];       // -delta
+
+    // (key-tile pairs as in the kernel with two roles: equal work, and one (batch, kv head) on one XCD.  Single tiles, the dearest
+    // first, for launches of up to one round: 4 x 32 / 8 heads x 4096 1218 us against 1001)
+    const int n_pairs = (p.n_ktiles + 1) / 2;
+    const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, n_pairs);
+    const int pair = lid % n_pairs;
+    const int hk = (lid / n_pairs) % p.Hkv;
+    const int b = lid / (n_pairs * p.Hkv);
+    const int G = p.Hq / p.Hkv;
+    int sq, sk;
+    int64_t q_base, do_base, l_base, k_base, v_base, dk_base, dv_base;           // (q, dO, lse, delta: of the batch; heads are added)
+    if (p.cu_q) {
+        const int q_start = p.cu_q[b], k_start = p.cu_k[b];
+        sq = p.cu_q[b + 1] - q_start;
+        sk = p.cu_k[b + 1] - k_start;
+        q_base = (int64_t)q_start * p.qs[2];
+        do_base = (int64_t)q_start * p.dos[2];
+        l_base = q_start;
+        k_base = (int64_t)k_start * p.ks[2] + (int64_t)hk * p.ks[1];
+        v_base = (int64_t)k_start * p.vs[2] + (int64_t)hk * p.vs[1];
+        dk_base = (int64_t)k_start * p.dks[2] + (int64_t)hk * p.dks[1];
+        dv_base = (int64_t)k_start * p.dvs[2] + (int64_t)hk * p.dvs[1];
+    } else {
+        sq = p.Sq;
+        sk = p.Sk;
+        q_base = (int64_t)b * p.qs[0];
+        do_base = (int64_t)b * p.dos[0];
+        l_base = (int64_t)b * p.ls[0];
+        k_base = (int64_t)b * p.ks[0] + (int64_t)hk * p.ks[1];
+        v_base = (int64_t)b * p.vs[0] + (int64_t)hk * p.vs[1];
+        dk_base = (int64_t)b * p.dks[0] + (int64_t)hk * p.dks[1];
+        dv_base = (int64_t)b * p.dvs[0] + (int64_t)hk * p.dvs[1];
+    }
+    const int nk = (sk + kFuCols - 1) / kFuCols;
+    if (2 * pair >= nk) return;                                         // (a sequence without queries still gets dk = dv = 0 written)
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, kg = lane >> 5;
+    const int coff = sk - sq;
+
+    TileLoader<D, NWV> ld;
+    ld.init(wave, lane);
+    R rd;
+    rd.init(lane);
+    const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_address(lds) + wave * TileLoader<D, NWV>::NI * 1024);
+    const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    for (int half = 0; half < 2; ++half) {
+        const int ktile = half == 0 ? pair : nk - 1 - pair;
+        if (half == 1 && ktile == pair) break;                          // odd tile count: the middle tile has no partner
+        const int k0 = ktile * kFuCols;
+        const int kw0 = k0 + 32 * wave;
+        const int kj = kw0 + n;
+        const bool k_ok = kj < sk;
+        __syncthreads();                                                // the previous half's readers are done with the LDS buffers
+
+        // fragments of this lane's key column: step s covers d = 16s + 8kg + j
+        bf16x8 kf[NS], vf[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            u32x4 a = {0u, 0u, 0u, 0u}, c = {0u, 0u, 0u, 0u};
+            if (k_ok) {
+                a = *reinterpret_cast<const u32x4*>(p.k + k_base + (int64_t)kj * p.ks[2] + 16 * s + 8 * kg);
+                c = *reinterpret_cast<const u32x4*>(p.v + v_base + (int64_t)kj * p.vs[2] + 16 * s + 8 * kg);
+            }
+            kf[s] = as_bf16x8(a);
+            vf[s] = as_bf16x8(c);
+        }
+        f32x16 dk[NDT], dv[NDT];
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) dk[i] = dv[i] = zero16;
+
+        int first_tile = 0;
+        if (CAUSAL) first_tile = max(0, k0 - coff) / kBwRows;
+        const int n_tiles = (sq + kBwRows - 1) / kBwRows;
+        const int n_steps = G * max(0, n_tiles - first_tile);           // (row tile, query head of the group), heads innermost
+        struct Pos {
+            int r0, hq;
+        };
+        const int r_step = half == 0 ? -kBwRows : kBwRows;
+        const auto advance = [&](Pos ps) {
+            ++ps.hq;
+            if (ps.hq == G) {
+                ps.hq = 0;
+                ps.r0 += r_step;
+            }
+            return ps;
+        };
+        float pend_lse = 0.f, pend_delta = 0.f;
+        const auto issue = [&](int st, Pos ps) {
+            const int h = hk * G + ps.hq, r0 = ps.r0, buf = (st & 1) * kTile;
+            ld.issue(p.q + q_base + (int64_t)h * p.qs[1] + (int64_t)r0 * p.qs[2], (int)p.qs[2], sq - 1 - r0, dst + buf);
+            ld.issue(p.dout + do_base + (int64_t)h * p.dos[1] + (int64_t)r0 * p.dos[2], (int)p.dos[2], sq - 1 - r0, dst + 2 * kTile + buf);
+            if (tid < kBwRows) {
+                const int64_t at = l_base + (int64_t)h * p.ls[1] + r0 + min(tid, sq - 1 - r0);
+                pend_lse = p.lse[at];
+                pend_delta = p.delta[at];
+            }
+        };
+        // (a causal row that sees no key has out = NaN, hence delta = NaN, and P = 0 everywhere: any finite delta gives the
+        // dS = 0 it must have)
+        const auto publish = [&](int st, Pos ps) {
+            if (tid < kBwRows) {
+                const bool in = ps.r0 + tid < sq;
+                lse_lds2[(st & 1) * kBwRows + tid] = in ? pend_lse * kLog2e : INFINITY;
+                delta_lds2[(st & 1) * kBwRows + tid] = in && pend_delta == pend_delta ? -pend_delta : 0.f;
+            }
+        };
+        // fragments read kDepth MFMAs ahead, in order, as in the other kernels
+        constexpr int kDepth = 2;
+        const auto scores = [&](const unsigned char* a_lds, const bf16x8 (&bfr)[NS], const f32x16& c0) {
+            u32x4 a[NS];
+#pragma unroll
+            for (int s = 0; s < kDepth && s < NS; ++s) a[s] = *reinterpret_cast<const u32x4*>(a_lds + rd.row_off[s]);
+            f32x16 r = c0;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                if (s + kDepth < NS) a[s + kDepth] = *reinterpret_cast<const u32x4*>(a_lds + rd.row_off[s + kDepth]);
+                r = mfma32(as_bf16x8(a[s]), bfr[s], r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            return r;
+        };
+        // acc^T (D x 32 keys) += tile^T . w over 32 rows of the tile
+        const auto update = [&](f32x16 (&acc)[NDT], const unsigned char* a_lds, const u32x4 (&w)[2]) {
+            constexpr int NC = 2 * NDT;
+            i16x4 lo[NC], hi[NC];
+            const auto read = [&](int c) {
+                const int u = c / NDT, dt = c % NDT;
+                lo[c] = lds_read_tr16(a_lds + 16 * u * kRow + rd.tr_off[0][dt]);
+                hi[c] = lds_read_tr16(a_lds + 16 * u * kRow + rd.tr_off[1][dt]);
+            };
+#pragma unroll
+            for (int c = 0; c < kDepth && c < NC; ++c) read(c);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                if (c + kDepth < NC) read(c + kDepth);
+                acc[c % NDT] = mfma32(join_bf16x8(lo[c], hi[c]), as_bf16x8(w[c / NDT]), acc[c % NDT]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        const auto step = [&](int st, Pos ps) {
+            const unsigned char* q_lds = lds + (st & 1) * kTile;
+            const unsigned char* do_lds = q_lds + 2 * kTile;
+            const float* lse_lds = lse_lds2 + (st & 1) * kBwRows;
+            const float* delta_lds = delta_lds2 + (st & 1) * kBwRows;
+            const int row_lim = CAUSAL ? kj - coff - ps.r0 - 4 * kg : -1;
+            // one 32-row half at a time: element i of this lane is query row r0 + 32t + 8(i/4) + 4kg + i%4, key kj
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                uint8_t mb[16] = {};
+                if constexpr (BOOLM) {           // (a row or key past the end re-reads the last one, see bwd_dkv_kernel)
+                    const uint8_t* mcol = p.mask + (int64_t)b * p.ms[0] + (int64_t)(hk * G + ps.hq) * p.ms[1] + min(kj, sk - 1);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        mb[e] = mcol[(int64_t)min(ps.r0 + 32 * t + 8 * (e >> 2) + 4 * kg + (e & 3), sq - 1) * p.ms[2]];
+                }
+                f32x16 c0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(delta_lds + 32 * t + 8 * j + 4 * kg);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) c0[4 * j + r] = d4[r];
+                }
+                const f32x16 s_acc = scores(q_lds + t * 32 * kRow, kf, zero16);
+                const f32x16 dp_acc = scores(do_lds + t * 32 * kRow, vf, c0);              // dP - delta
+                u32x4 pw[2], dsw[2];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_lds + 32 * t + 8 * j + 4 * kg);
+                    float x[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        x[r] = fast_exp2(fmaf(s_acc[4 * j + r], p.scale_log2, -l4[r]));
+                        // kept iff kj <= row + coff, i.e. the tile-relative row (compile-time part) >= row_lim
+                        if constexpr (CAUSAL || BOOLM) {
+                            bool keep = 32 * t + 8 * j + r >= row_lim;
+                            if constexpr (BOOLM) keep = keep & (mb[4 * j + r] != 0);
+                            x[r] = keep ? x[r] : 0.f;
+                        }
+                    }
+                    pw[j >> 1][2 * (j & 1)] = pack_bf16(x[0], x[1]);
+                    pw[j >> 1][2 * (j & 1) + 1] = pack_bf16(x[2], x[3]);
+                    dsw[j >> 1][2 * (j & 1)] = pack_bf16(x[0] * dp_acc[4 * j], x[1] * dp_acc[4 * j + 1]);          // dS without the scale factor
+                    dsw[j >> 1][2 * (j & 1) + 1] = pack_bf16(x[2] * dp_acc[4 * j + 2], x[3] * dp_acc[4 * j + 3]);
+                }
+                update(dv, do_lds + 32 * t * kRow, pw);
+                update(dk, q_lds + 32 * t * kRow, dsw);
+            }
+        };
+
+        Pos ps = {(half == 0 ? n_tiles - 1 : first_tile) * kBwRows, 0};
+        if (n_steps > 0) {
+            issue(0, ps);
+            publish(0, ps);
+        }
+        for (int i = 0; i < n_steps; ++i) {
+            const Pos next = advance(ps);
+            wait_vmcnt<0>();                                   // this wavefront's share of the step's tiles has landed
+            __syncthreads();                                   // ... and everybody's; lse and delta are visible; the other buffers are free
+            if (i + 1 < n_steps) issue(i + 1, next);
+            // (a step whose rows all lie above this wavefront's first key column has nothing for it)
+            if (!CAUSAL || kw0 <= ps.r0 + kBwRows - 1 + coff) step(i, ps);
+            if (i + 1 < n_steps) publish(i + 1, next);
+            ps = next;
+        }
+
+        // store: lane owns key kj, d = 32dt + 8(i/4) + 4kg + i%4
+        if (k_ok) {
+            const int64_t k_row = dk_base + (int64_t)kj * p.dks[2], v_row = dv_base + (int64_t)kj * p.dvs[2];
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
-                    u32x2 w;
-                    w[0] = pack_bf16(acc[dt][4 * g + 0] * f, acc[dt][4 * g + 1] * f);
-                    w[1] = pack_bf16(acc[dt][4 * g + 2] * f, acc[dt][4 * g + 3] * f);
-                    *reinterpret_cast<u32x2*>(row + 32 * dt + 8 * g + 4 * kg) = w;
+                    const int d = 32 * dt + 8 * g + 4 * kg;
+                    store_grad4(p.dk, p.dk_f32, k_row + d, dk[dt][4 * g] * p.scale, dk[dt][4 * g + 1] * p.scale, dk[dt][4 * g + 2] * p.scale,
+                                dk[dt][4 * g + 3] * p.scale);
+                    store_grad4(p.dv, p.dv_f32, v_row + d, dv[dt][4 * g], dv[dt][4 * g + 1], dv[dt][4 * g + 2], dv[dt][4 * g + 3]);
                 }
         }
     }
 }
 
+template <int D, int MODE>
+static void launch_bwd_mode(const BwdParams& p, hipStream_t stream) {
+    const dim3 grid_q((unsigned)((p.n_qtiles + 1) / 2 * p.Hq * p.B)), grid_k((unsigned)((p.n_ktiles + 1) / 2 * p.Hkv * p.B));
+    hipLaunchKernelGGL((bwd_dq_kernel<D, MODE>), grid_q, dim3(kBwWaves * 64), 0, stream, p);             // dQ, writes delta
+    // dK and dV, reads delta.  Head sizes 32 and 64: one role per wavefront up to a workgroup per compute unit, where a workgroup's
+    // own chain is what counts (one sequence of 8192 tokens, 8 / 1 heads of 64: 1.56 ms against 1.75; 8 x 1024, 32 / 8 heads 192
+    // us against 199), both roles in each wavefront beyond (4 x 4096, 32 / 8 heads of 64 1.14 -> 1.00 ms, of 32 0.89 -> 0.69;
+    // 64 x 256, 16 heads of 64 129 -> 110 us, of 32 the kernel alone 56 -> 34)
+    if constexpr (D <= 64) {
+        if (grid_k.x > 256) {
+            hipLaunchKernelGGL((bwd_dkv_one_kernel<D, MODE>), grid_k, dim3(kFuPairs * 64), 0, stream, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((bwd_dkv_kernel<D, MODE>), grid_k, dim3(2 * kFuPairs * 64), 0, stream, p);
+}
+
 template <int D>
 static int launch_bwd(const BwdParams& p, int mask_mode, hipStream_t stream) {
-    const dim3 block(kBwWaves * 64), block_kv(2 * kFuPairs * 64);
-    const dim3 grid_q((unsigned)((p.n_qtiles + 1) / 2 * p.Hq * p.B)), grid_k((unsigned)((p.n_ktiles + 1) / 2 * p.Hkv * p.B));
-    if (mask_mode == MI355_MASK_CAUSAL) {
-        hipLaunchKernelGGL((bwd_dq_kernel<D, MI355_MASK_CAUSAL>), grid_q, block, 0, stream, p);        // dQ, writes delta
-        hipLaunchKernelGGL((bwd_dkv_kernel<D, MI355_MASK_CAUSAL>), grid_k, block_kv, 0, stream, p);    // dK and dV, reads delta
-    } else if (mask_mode == MI355_MASK_BOOL) {
-        hipLaunchKernelGGL((bwd_dq_kernel<D, MI355_MASK_BOOL>), grid_q, block, 0, stream, p);
-        hipLaunchKernelGGL((bwd_dkv_kernel<D, MI355_MASK_BOOL>), grid_k, block_kv, 0, stream, p);
-    } else {
-        hipLaunchKernelGGL((bwd_dq_kernel<D, MI355_MASK_NONE>), grid_q, block, 0, stream, p);
-        hipLaunchKernelGGL((bwd_dkv_kernel<D, MI355_MASK_NONE>), grid_k, block_kv, 0, stream, p);
-    }
+    if (mask_mode == MI355_MASK_CAUSAL) launch_bwd_mode<D, MI355_MASK_CAUSAL>(p, stream);
+    else if (mask_mode == MI355_MASK_BOOL) launch_bwd_mode<D, MI355_MASK_BOOL>(p, stream);
+    else launch_bwd_mode<D, MI355_MASK_NONE>(p, stream);
     return (int)hipGetLastError();
 }
 
@@ -693,7 +951,7 @@ static int prefill_bwd_common(const void* q, const void* k, const void* v, const
                               const int64_t dk_strides[3], const int64_t dv_strides[3], const int64_t lse_strides[2],
                               const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const uint8_t* mask,
                               const int64_t* mask_strides, int B, int Hq, int Hkv, int Sq_max, int Sk_max, int D,
-                              float softmax_scale, int mask_mode, int dtype, void* stream) {
+                              float softmax_scale, int mask_mode, int dtype, void* stream, int f32_grads = 0) {
     if (!q || !k || !v || !out || !dout || !lse || !delta || !dq || !dk || !dv)
         return set_error(MI355_EINVAL, "prefill_bwd: null pointer argument");
     if (!q_strides || !k_strides || !v_strides || !o_strides || !do_strides || !dq_strides || !dk_strides || !dv_strides ||
@@ -735,9 +993,12 @@ static int prefill_bwd_common(const void* q, const void* k, const void* v, const
     p.dout = (const __bf16*)dout;
     p.lse = lse;
     p.delta = delta;
-    p.dq = (__bf16*)dq;
-    p.dk = (__bf16*)dk;
-    p.dv = (__bf16*)dv;
+    p.dq = dq;
+    p.dk = dk;
+    p.dv = dv;
+    p.dq_f32 = f32_grads & 1;
+    p.dk_f32 = f32_grads & 2;
+    p.dv_f32 = f32_grads & 4;
     for (int i = 0; i < 3; ++i) {
         p.qs[i] = q_strides[i];
         p.ks[i] = k_strides[i];
@@ -799,4 +1060,18 @@ extern "C" int mi355_prefill_bwd_mask(const void* q, const void* k, const void* 
     return prefill_bwd_common(q, k, v, out, dout, lse, delta, dq, dk, dv, q_strides, k_strides, v_strides, o_strides,
                               do_strides, dq_strides, dk_strides, dv_strides, lse_strides, nullptr, nullptr, mask,
                               mask_strides, B, Hq, Hkv, Sq, Sk, D, softmax_scale, MI355_MASK_BOOL, dtype, stream);
+}
+
+extern "C" int mi355_prefill_bwd_typed(const void* q, const void* k, const void* v, const void* out, const void* dout,
+                                       const float* lse, float* delta, void* dq, void* dk, void* dv,
+                                       const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
+                                       const int64_t o_strides[3], const int64_t do_strides[3], const int64_t dq_strides[3],
+                                       const int64_t dk_strides[3], const int64_t dv_strides[3],
+                                       const int64_t lse_strides[2], const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                       const uint8_t* mask, const int64_t mask_strides[3], int f32_grads, int B, int Hq, int Hkv,
+                                       int Sq_max, int Sk_max, int D, float softmax_scale, int mask_mode, int dtype, void* stream) {
+    if (f32_grads < 0 || f32_grads > 7) return set_error(MI355_EINVAL, "prefill_bwd: f32_grads has three bits");
+    return prefill_bwd_common(q, k, v, out, dout, lse, delta, dq, dk, dv, q_strides, k_strides, v_strides, o_strides,
+                              do_strides, dq_strides, dk_strides, dv_strides, lse_strides, cu_seqlens_q, cu_seqlens_k, mask,
+                              mask_strides, B, Hq, Hkv, Sq_max, Sk_max, D, softmax_scale, mask_mode, dtype, stream, f32_grads);
 }

@@ -8,7 +8,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmi355attn.so")
 # the same library without the training kernels: what a served model needs, built by the command line tools in a fresh checkout
 SERVING_LIB_PATH = os.path.join(_HERE, "libmi355attn_serving.so")
-TRAINING_ONLY = ("mi355_prefill_bwd", "mi355_prefill_bwd_mask")
+TRAINING_ONLY = ("mi355_prefill_bwd", "mi355_prefill_bwd_mask", "mi355_prefill_bwd_typed")
 
 MI355_BF16 = 0
 MI355_FP8_E4M3 = 1
@@ -31,6 +31,7 @@ EXPORTS = (
     "mi355_prefill_bwd",
     "mi355_prefill_fwd_mask_lse",
     "mi355_prefill_bwd_mask",
+    "mi355_prefill_bwd_typed",
     "mi355_paged_decode_fwd",
     "mi355_paged_decode_fwd_static",
     "mi355_paged_decode_workspace_bytes",
@@ -148,6 +149,9 @@ def load():
     lib.mi355_prefill_bwd_mask.restype = i32
     lib.mi355_prefill_bwd_mask.argtypes = [vp] * 10 + [_i64x3] * 8 + [_i64x2, vp, _i64x3,
                                                                       i32, i32, i32, i32, i32, i32, f32, i32, vp]
+    lib.mi355_prefill_bwd_typed.restype = i32
+    lib.mi355_prefill_bwd_typed.argtypes = [vp] * 10 + [_i64x3] * 8 + [_i64x2, vp, vp, vp, _i64x3, i32,
+                                                                       i32, i32, i32, i32, i32, i32, f32, i32, i32, vp]
     lib.mi355_prefill_paged_fwd.restype = i32
     lib.mi355_prefill_paged_fwd.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp, i64, i64, vp,
                                             i32, i32, i32, i32, i32, i32, i64, f32, i32, i32, i64, vp, sz, vp]

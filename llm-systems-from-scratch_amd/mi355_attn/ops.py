@@ -60,12 +60,12 @@ def _autocast_on() -> bool:
         return torch.is_autocast_enabled()
 
 
-def _to_bf16(q, k, v):
-    """The kernels compute on bf16 operands.  Inputs may be bfloat16 or float32 in any mix -- at
+def _out_dtype(q, k, v):
+    """Checks the inputs' types and returns the result's.  The kernels compute on bf16 operands.  Inputs may be bfloat16 or float32 in any mix -- at
     llm-core/llm_core/model.py:382 the reference passes float32 Q and K (RoPE multiplies the bf16 projections by its
     float32 table, model.py:93-104) with a bfloat16 V under `--amp` (train.py:215), and three float32 tensors
-    without it.  float32 inputs are rounded to bf16 (what autocast does to them in front of PyTorch's SDPA; the cast
-    is differentiable).  Returns (q, k, v, out_dtype): float32 only when all three inputs are float32 and autocast
+    without it.  float32 inputs are rounded to bf16 (what autocast does to them in front of PyTorch's SDPA), their
+    gradients are float32.  The result is float32 only when all three inputs are float32 and autocast
     is off -- the case in which the reference's next operator expects float32 -- bfloat16 otherwise."""
     for n, t in (("q", q), ("k", k), ("v", v)):
         if not t.is_cuda:
@@ -73,9 +73,7 @@ def _to_bf16(q, k, v):
         if t.dtype not in (torch.bfloat16, torch.float32):
             raise TypeError(f"{n} must be bfloat16 or float32 (got {t.dtype})")
     all_f32 = all(t.dtype == torch.float32 for t in (q, k, v))
-    out_dtype = torch.float32 if all_f32 and not _autocast_on() else torch.bfloat16
-    q, k, v = (t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16) for t in (q, k, v))
-    return q, k, v, out_dtype
+    return torch.float32 if all_f32 and not _autocast_on() else torch.bfloat16
 
 
 def _rows16(name, t):
@@ -232,20 +230,20 @@ def _dense(q, k, v, mask, mode, softmax_scale, want_lse=False, kv_splits=1, work
     return (out, lse) if want_lse else out
 
 
-def _grad_like(t):
+def _grad_like(t, dtype):
     """Gradient buffer with t's shape and, where t is dense, t's memory layout (so the gradient of the
     reference's strided V view lands in the layout of the projection it is a view of)."""
-    g = torch.empty_like(t)
+    g = torch.empty_like(t, dtype=dtype)
     ok = g.stride(-1) == 1 and all(s % 8 == 0 for s in g.stride()[:-1])
-    return g if ok else torch.empty(t.shape, dtype=t.dtype, device=t.device)
+    return g if ok else torch.empty(t.shape, dtype=dtype, device=t.device)
 
 
-def _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, Sq, Sk, scale, mode, mask=None):
-    """dq, dk, dv through mi355_prefill_bwd (mi355_prefill_bwd_mask with an explicit (B,H,Sq,Sk) uint8 mask);
+def _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, Sq, Sk, scale, mode, mask=None, dtypes=(torch.bfloat16,) * 3):
+    """dq, dk, dv of the given types (bf16 or fp32) through mi355_prefill_bwd_typed (mask: an explicit (B,H,Sq,Sk) uint8 mask);
     tensors dense (B,H,S,D) or packed (T,H,D)."""
     packed = cu_q is not None
     q, k, v, out, dout = (_rows16(n, t) for n, t in (("q", q), ("k", k), ("v", v), ("out", out), ("dout", dout)))
-    dq, dk, dv = _grad_like(q), _grad_like(k), _grad_like(v)
+    dq, dk, dv = (_grad_like(t, dt) for t, dt in zip((q, k, v), dtypes))
     if q.numel() == 0 or k.numel() == 0:
         return dq.zero_(), dk.zero_(), dv.zero_()
     delta = torch.empty_like(lse)
@@ -256,29 +254,30 @@ def _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, Sq, Sk, scale, mode, 
         (B, Hq, _, D), Hkv = q.shape, k.shape[1]
         ls = lse.stride()[:2]
     st = [_lib.strides3(_packed_or_dense_strides(t, packed)) for t in (q, k, v, out, dout, dq, dk, dv)]
-    if mask is not None:
-        with _on(q, k, v, out, dout, lse, mask) as stream:
-            rc = _lib.load().mi355_prefill_bwd_mask(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *st, _lib.strides2(ls), mask.data_ptr(),
-                _lib.strides3(mask.stride()[:3]), B, Hq, Hkv, int(Sq), int(Sk), D, float(scale), _lib.MI355_BF16, stream)
-        _lib.check(rc, "mi355_prefill_bwd_mask")
-        return dq, dk, dv
-    with _on(q, k, v, out, dout, lse, cu_q, cu_k) as stream:
-        rc = _lib.load().mi355_prefill_bwd(
+    f32 = sum(1 << i for i, dt in enumerate(dtypes) if dt == torch.float32)
+    with _on(q, k, v, out, dout, lse, cu_q, cu_k, mask) as stream:
+        rc = _lib.load().mi355_prefill_bwd_typed(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(), lse.data_ptr(), delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), *st, _lib.strides2(ls),
             None if cu_q is None else cu_q.data_ptr(), None if cu_k is None else cu_k.data_ptr(),
+            None if mask is None else mask.data_ptr(), _lib.strides3((0, 0, 0) if mask is None else mask.stride()[:3]), f32,
             B, Hq, Hkv, int(Sq), int(Sk), D, float(scale), mode, _lib.MI355_BF16, stream)
-    _lib.check(rc, "mi355_prefill_bwd")
+    _lib.check(rc, "mi355_prefill_bwd_typed")
     return dq, dk, dv
 
 
+def _bf16(*tensors):
+    return tuple(t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16) for t in tensors)
+
+
 class _DensePrefillFn(torch.autograd.Function):
-    """out = attention(q, k, v) on the HIP forward; backward on the HIP backward kernels."""
+    """out = attention(q, k, v) on the HIP forward; backward on the HIP backward kernels.  float32 inputs are rounded here, and
+    their gradients come out of the kernels in float32."""
 
     @staticmethod
     def forward(ctx, q, k, v, causal, softmax_scale):
+        ctx.dtypes = (q.dtype, k.dtype, v.dtype)
+        q, k, v = _bf16(q, k, v)
         mode = _lib.MASK_CAUSAL if causal else _lib.MASK_NONE
         out, lse = _dense(q, k, v, None, mode, softmax_scale, want_lse=True)
         ctx.save_for_backward(q, k, v, out, lse)
@@ -289,7 +288,8 @@ class _DensePrefillFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse = ctx.saved_tensors
-        dq, dk, dv = _prefill_backward(q, k, v, out, dout, lse, None, None, q.shape[2], k.shape[2], ctx.scale, ctx.mode)
+        dq, dk, dv = _prefill_backward(q, k, v, out, dout, lse, None, None, q.shape[2], k.shape[2], ctx.scale, ctx.mode,
+                                       dtypes=ctx.dtypes)
         return dq, dk, dv, None, None
 
 
@@ -313,6 +313,8 @@ class _MaskedPrefillFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, m4):
+        ctx.dtypes = (q.dtype, k.dtype, v.dtype)
+        q, k, v = _bf16(q, k, v)
         out, lse = _dense(q, k, v, m4, _lib.MASK_BOOL, None, want_lse=True)
         ctx.save_for_backward(q, k, v, out, lse, m4)
         return out
@@ -321,13 +323,15 @@ class _MaskedPrefillFn(torch.autograd.Function):
     def backward(ctx, dout):
         q, k, v, out, lse, m4 = ctx.saved_tensors
         dq, dk, dv = _prefill_backward(q, k, v, out, dout, lse, None, None, q.shape[2], k.shape[2],
-                                       1.0 / math.sqrt(q.shape[-1]), _lib.MASK_BOOL, mask=m4)
+                                       1.0 / math.sqrt(q.shape[-1]), _lib.MASK_BOOL, mask=m4, dtypes=ctx.dtypes)
         return dq, dk, dv, None
 
 
 class _VarlenPrefillFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, cu_q, cu_k, max_q, max_k, causal, softmax_scale):
+        ctx.dtypes = (q.dtype, k.dtype, v.dtype)
+        q, k, v = _bf16(q, k, v)
         out, lse = _varlen(q, k, v, cu_q, cu_k, max_q, max_k, causal, softmax_scale, want_lse=True)
         ctx.save_for_backward(q, k, v, out, lse, cu_q, cu_k)
         ctx.args = (int(max_q), int(max_k), _lib.MASK_CAUSAL if causal else _lib.MASK_NONE,
@@ -338,7 +342,7 @@ class _VarlenPrefillFn(torch.autograd.Function):
     def backward(ctx, dout):
         q, k, v, out, lse, cu_q, cu_k = ctx.saved_tensors
         max_q, max_k, mode, scale = ctx.args
-        dq, dk, dv = _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, max_q, max_k, scale, mode)
+        dq, dk, dv = _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, max_q, max_k, scale, mode, dtypes=ctx.dtypes)
         return dq, dk, dv, None, None, None, None, None, None
 
 
@@ -352,7 +356,7 @@ def flash_attn_prefill(q, k, v, *, causal=True, softmax_scale=None, kv_splits=No
     Fills the slot of torch.nn.functional.scaled_dot_product_attention(Q, K, V,
     is_causal=True) at llm-core/llm_core/model.py:382.  With Sk > Sq the causal
     diagonal is bottom-right aligned (the queries are the last Sq positions).
-    Inputs are bfloat16 or float32 in any mix (see _to_bf16: bf16 math either way; the result is
+    Inputs are bfloat16 or float32 in any mix (see _out_dtype: bf16 math either way; the result is
     float32 only for three float32 inputs outside autocast, bfloat16 otherwise).
     Differentiable: when an input requires grad, dq/dk/dv come from the HIP backward kernels
     (what autograd computes behind model.py:382 during train.py's loss.backward()).
@@ -361,10 +365,11 @@ def flash_attn_prefill(q, k, v, *, causal=True, softmax_scale=None, kv_splits=No
     per pair of 256-row query tiles would leave most of the GPU idle.  None chooses (1 whenever the plain
     launch already fills the GPU); `workspace` may carry a prefill_splitkv_workspace() tensor to reuse.
     """
-    q, k, v, out_dtype = _to_bf16(q, k, v)
+    out_dtype = _out_dtype(q, k, v)
     if _needs_grad(q, k, v):
         out = _DensePrefillFn.apply(q, k, v, bool(causal), softmax_scale)
     else:
+        q, k, v = _bf16(q, k, v)
         out = _dense(q, k, v, None, _lib.MASK_CAUSAL if causal else _lib.MASK_NONE, softmax_scale,
                      kv_splits=kv_splits, workspace=workspace)
     return out if out.dtype == out_dtype else out.to(out_dtype)
@@ -383,7 +388,7 @@ def scaled_dot_product_attention(Q, K, V, mask=None):
     scale is 1/sqrt(d_k).  A query row whose keys are all masked yields NaN, as
     the reference softmax (llm-core/llm_core/nn_functional.py:8-11) does.
     Restrictions of the HIP path: d_v == d_k in {32, 64, 128}; bfloat16 or float32 tensors (bf16 math, see
-    _to_bf16).  Differentiable with and without a mask (dq/dk/dv from the HIP backward kernels), so the reference's
+    _out_dtype).  Differentiable with and without a mask (dq/dk/dv from the HIP backward kernels), so the reference's
     non-flash training branch (model.py:384-385: the tril mask rebuilt per call) runs through it unchanged; the
     explicit-mask kernels read the mask element by element, so flash_attn_prefill(causal=True) remains the fast way
     to train with a causal mask.  A fully masked query row gives NaN outputs like the reference but zero gradients
@@ -406,7 +411,7 @@ def scaled_dot_product_attention(Q, K, V, mask=None):
             return t.reshape((1,) * (4 - t.dim()) + tuple(t.shape))
         return t.reshape(-1, *t.shape[-3:])
 
-    Q, K, V, out_dtype = _to_bf16(Q, K, V)
+    out_dtype = _out_dtype(Q, K, V)
     q4, k4, v4 = as4(Q, nq), as4(K, nk), as4(V, nk)
     m4 = None
     mode = _lib.MASK_NONE
@@ -421,7 +426,7 @@ def scaled_dot_product_attention(Q, K, V, mask=None):
         else:
             out = _DensePrefillFn.apply(q4, k4, v4, False, None)
         return out.reshape(*lead, nq, d).to(out_dtype)
-    out = _dense(q4, k4, v4, m4, mode, None, kv_splits=None)
+    out = _dense(*_bf16(q4, k4, v4), m4, mode, None, kv_splits=None)
     return out.reshape(*lead, nq, d).to(out_dtype)
 
 
@@ -488,7 +493,7 @@ def flash_attn_varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
     window, keep_first (causal, forward only): query i sees key j when i - j < window or j < keep_first (window 0: every
     earlier key).  out: (Tq,Hq,D) bf16 to write into, rows may be strided.
     """
-    q, k, v, out_dtype = _to_bf16(q, k, v)
+    out_dtype = _out_dtype(q, k, v)
     window, keep_first = _window(window, keep_first)
     if window and not causal:
         raise ValueError("a window is causal")
@@ -498,6 +503,7 @@ def flash_attn_varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
         out = _VarlenPrefillFn.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, bool(causal),
                                      softmax_scale)
     else:
+        q, k, v = _bf16(q, k, v)
         out = _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, softmax_scale,
                       kv_splits=kv_splits, workspace=workspace, head_scale=head_scale, sinks=sinks, window=window,
                       keep_first=keep_first, out=out)

@@ -319,3 +319,58 @@ def test_masked_sdpa_backward_of_a_fully_masked_row(ops):
     check_grad("dq", qg.grad[:, :, keep], dq)
     check_grad("dk", kg.grad, dk)
     check_grad("dv", vg.grad, dv)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("Sq,Sk,causal", [(1, 1, True), (33, 33, True), (64, 129, True), (130, 130, False), (257, 300, True)])
+def test_backward_of_many_short_heads(ops, D, Sq, Sk, causal):
+    """More than 256 workgroups: the kernel with both roles in a wavefront; edges of the 32 keys of a wavefront, of the 64-row tiles
+    and of the 128-key workgroups, pairs of key tiles and a middle one, two query heads per key head."""
+    print(f"case: backward many heads D={D} {Sq} {Sk} {causal}", flush=True)
+    run_dense(ops, 65, 8, 4, Sq, Sk, D, causal, seed=D + Sq)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+def test_backward_of_many_packed_sequences_and_masks(ops, D):
+    """The same kernel on packed sequences (some empty) against its dense runs, and under a mask of every element kept against no mask."""
+    lens = [0, 1, 200, 17, 128, 0, 129] * 10
+    H, G = 8, 4
+    T = sum(lens)
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    q, k, v, do = (rnd(T, h, D, seed=s).cuda() for s, h in ((1, H), (2, G), (3, G), (4, H)))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    grads = torch.autograd.grad(ops.flash_attn_varlen_prefill(q, k, v, cu, cu, 200, 200), leaves, do)
+    at = 0
+    for n in lens[:7]:
+        if n:
+            part = [t.detach()[at:at + n].transpose(0, 1)[None] for t in (q, k, v)]
+            dq, dk, dv, _ = orc.prefill_backward_reference(*(t.cpu() for t in part), do[at:at + n].transpose(0, 1)[None].cpu(), causal=True)
+            for name, got, ref in (("dq", grads[0], dq), ("dk", grads[1], dk), ("dv", grads[2], dv)):
+                check_grad(name, got[at:at + n].transpose(0, 1)[None], ref)
+        at += n
+    B, S = 65, 100
+    q, k, v, do = (rnd(B, 4, S, D, seed=s).cuda() for s in (5, 6, 7, 8))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    keep = torch.ones(S, S, dtype=torch.bool, device="cuda")
+    masked = torch.autograd.grad(ops.scaled_dot_product_attention(q, k, v, keep), leaves, do)
+    plain = torch.autograd.grad(ops.scaled_dot_product_attention(q, k, v), leaves, do)
+    for a, b in zip(masked, plain):          # (the two forwards differ in their exponent reference, so in the log-sum-exp's last bits)
+        assert float((a.float() - b.float()).norm()) <= 2 ** -8 * float(b.float().norm())
+
+
+@pytest.mark.parametrize("D,B", [(32, 65), (64, 65), (64, 1), (128, 1)])
+def test_gradients_of_float32_inputs(ops, D, B):
+    """float32 inputs are rounded to bf16 and get the float32 gradients that the bf16 ones are the rounding of."""
+    H, S = 4, 70
+    q, k = (torch.randn(B, H, S, D, generator=torch.Generator().manual_seed(s)).cuda() for s in (1, 2))
+    v, do = rnd(B, S, H, D, seed=3).cuda().permute(0, 2, 1, 3), rnd(B, H, S, D, seed=4).cuda()
+    mixed = [t.detach().clone().requires_grad_() for t in (q, k, v)]
+    out = ops.sdpa_slot(*mixed)
+    grads = torch.autograd.grad(out, mixed, do)
+    half = [t.detach().to(torch.bfloat16).requires_grad_() for t in (q, k, v)]
+    ref = ops.sdpa_slot(*half)
+    want = torch.autograd.grad(ref, half, do)
+    assert out.dtype == torch.bfloat16 and torch.equal(out, ref)
+    assert [g.dtype for g in grads] == [torch.float32, torch.float32, torch.bfloat16] and grads[2].stride() == v.stride()
+    for g, w in zip(grads, want):
+        assert torch.equal(g.to(torch.bfloat16), w)
