@@ -95,29 +95,6 @@ struct TileLoader {
     }
 };
 
-// Per-lane LDS offsets of the two read patterns of a swizzled 64 x D tile.
-template <int D>
-struct TileReads {
-    static constexpr int NS = D / 16, NDT = D / 32, kRow = D * 2;
-    int row_off[NS];        // A fragment "row n of the tile, k = 16s + 8kg ..": add 32*t*kRow
-    int tr_off[2][NDT];     // transposed fragment of d-tile dt for a 16-row slice: add 16*u*kRow
-    __device__ __forceinline__ void init(int lane) {
-        const int n = lane & 31, kg = lane >> 5;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) row_off[s] = n * kRow + (((2 * s + kg) ^ swz<D>(n)) << 4);
-        const int g16 = lane >> 4, s16 = lane & 15;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int row = 4 * (g16 >> 1) + (s16 >> 2) + 8 * e;
-#pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
-                const int d = 32 * dt + 16 * (g16 & 1) + 4 * (s16 & 3);
-                tr_off[e][dt] = row * kRow + (((d >> 3) ^ swz<D>(row)) << 4) + (d & 7) * 2;
-            }
-        }
-    }
-};
-
 // ---------------------------------------------------------------------------------------------
 // dQ: one workgroup per tile of 128 queries of one (batch, query head); K/V stream through LDS.
 // Per wavefront: Q and dO fragments of its 32 query columns in registers (64), dQ^T accumulators (64).

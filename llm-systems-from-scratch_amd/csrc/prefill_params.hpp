@@ -52,4 +52,8 @@ struct PrefillParams {
 bool prefill_w64_takes(const PrefillParams& p);
 int launch_prefill_w64(const PrefillParams& p, hipStream_t stream);
 
+// Up to 256 keys at head sizes 32 and 64, dense layout: prefill_short.hip.
+bool prefill_short_takes(const PrefillParams& p, int D);
+int launch_prefill_short(const PrefillParams& p, int D, hipStream_t stream);
+
 }  // namespace mi355

@@ -394,6 +394,30 @@ def test_prefill_head_dim_64_32_preset_reference_against_tracked_maxima(ops, D, 
         check(shared, ref, what=f"preset reference, keys split, D={D} seed {seed} #{case}")
 
 
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("Sq,Sk,causal", [(1, 1, True), (31, 32, True), (33, 33, True), (64, 97, True), (129, 129, True), (160, 160, False),
+                                          (256, 256, True), (225, 256, True), (100, 224, False), (300, 200, False), (513, 17, False)])
+def test_prefill_of_short_heads(ops, D, Sq, Sk, causal):
+    """Up to 256 keys (224 without a mask) at head sizes 32 and 64: edges of the 32-row blocks and of the 32 keys of a diagonal step, an
+    uneven number of blocks, several query tiles; keys that outgrow each other by tens of binary orders; the log-sum-exp too."""
+    print(f"case: short heads D={D} {Sq} {Sk} {causal}", flush=True)
+    q, k, v = rnd(3, 4, Sq, D, seed=Sk), rnd(3, 2, Sk, D, seed=Sk + 1), rnd(3, 2, Sk, D, seed=Sk + 2)
+    k[1] *= torch.exp2(torch.linspace(0, 4, Sk))[:, None].to(torch.bfloat16)        # (later keys draw ever larger scores)
+    k[2, :, Sk // 2:] = k[2, :, Sk // 2:] * 8
+    ref = orc.prefill_reference(q, k, v, causal=causal)
+    check(ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=causal, kv_splits=1), ref, what="out")
+    strided = q.transpose(1, 2).contiguous().transpose(1, 2).cuda().requires_grad_()       # rows of one head far apart, and with the lse
+    check(ops.flash_attn_prefill(strided, k.cuda(), v.cuda(), causal=causal).detach(), ref, what="out, strided")
+
+
+def test_prefill_of_short_heads_without_keys(ops):
+    """Causal with fewer keys than queries: the rows in front of the first key are NaN, as the reference's softmax gives them."""
+    q, k, v = rnd(1, 2, 40, 32, seed=1), rnd(1, 2, 7, 32, seed=2), rnd(1, 2, 7, 32, seed=3)
+    out = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=True, kv_splits=1).cpu()
+    assert bool(torch.isnan(out[:, :, :33]).all())
+    check(out[:, :, 33:], orc.prefill_reference(q, k, v, causal=True)[:, :, 33:])
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("splits", [2, 5, 64])
 def test_prefill_split_keys_dense(ops, D, splits):
