@@ -589,9 +589,10 @@ int mi355_ssm_decode(const mi355_ssm_args* args, void* stream);
  *   mi355_moe_down    : out[pair] = weights[pair] * (Wd act[i]); w (n_experts, n, ff)
  *   mi355_moe_direct  : gate_up and down of a decode step's few pairs (up to 2048, bf16), without an order: act (n_pairs, ff)
  *                       and out hold row `pair` for each pair
- * bf16 (fp32 sums): k and ff in multiples of 64, 16-byte aligned rows.  tiling AUTO chooses by pairs per expert.
+ * bf16 (fp32 sums): k and ff in multiples of 64, 16-byte aligned rows.  tiling AUTO chooses by pairs and experts; WIDE needs
+ * 16-byte aligned output rows (and is LARGE without them).
  */
-enum { MI355_TILING_AUTO = 0, MI355_TILING_SKINNY = 1, MI355_TILING_LARGE = 2 };
+enum { MI355_TILING_AUTO = 0, MI355_TILING_SKINNY = 1, MI355_TILING_LARGE = 2, MI355_TILING_WIDE = 3 };
 int mi355_moe_route(const void* h, const void* w, const float* bias, int32_t* ids, float* weights, float* extra_logit,
                     int64_t n_tokens, int64_t h_row_stride, int64_t w_row_stride, int k, int n_experts, int top, int dtype,
                     void* stream);

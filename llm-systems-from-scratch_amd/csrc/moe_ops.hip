@@ -5,9 +5,10 @@
 //   group   pairs sorted by expert: order[], and offsets[e] = first place of expert e's pairs in it
 //   gate_up act[i] = silu(Wg h_i) * (Wu h_i) for place i of the order, h_i the pair's token
 //   down    out[pair] = weight[pair] * (Wd act[i])
-// The products are tiled per expert.  Tiles of expert e start at number offsets[e] / BM + e, so the tile -> expert search
-// needs the offsets alone, and a launch of n_pairs / BM + E row tiles covers every distribution of the tokens.  A row of a
-// product depends on its own token only, so neither the order inside an expert nor the tiling shows in a result.
+// The products are tiled per expert.  Tiles of expert e start at number offsets[e] / BM + e (the large tiles: where those of
+// e - 1 end), so the tile -> expert search needs the offsets alone, and a launch of n_pairs / BM + E row tiles covers every
+// distribution of the tokens.  A row of a product depends on its own token only, so neither the order inside an expert nor the tiling shows in a result.
+//   moe_wide_kernel    256 x 256 tiles through LDS: long prompts
 //   moe_gemm_kernel    128 x 128 tiles through LDS: prompts
 //   moe_direct_kernel  32 weight rows, streamed through LDS, against an expert's rows, no grouping needed: decoding
 //   moe_skinny_kernel  16 rows x 16 (+ 16) weight rows, weights straight to registers: few pairs per expert, many experts
@@ -17,6 +18,7 @@
 #include "weight_stream.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace mi355 {
@@ -285,6 +287,34 @@ __device__ __forceinline__ bool find_tile(const MoeParams& p, int tile, int& e, 
     return first >= start && first < end;
 }
 
+// The same with the tiles numbered without gaps, so that the ones that have rows are the launch's first and none of the eight XCDs
+// has more of them than its share: the large tiles, where a round of the chip counts more than a scan over the experts (16 experts
+// of 2048 x 1024, top 4, 128 x 128 tiles, 1800 tokens: both products 138 -> 115 us; 32 of 2048 x 2048, 512 pairs: 240 -> 200).
+template <int BM>
+__device__ __forceinline__ bool find_dense_tile(const MoeParams& p, int tile, int& e, int& first, int& end) {
+    const int lane = threadIdx.x & 63;
+    for (int e0 = 0, before = 0; e0 < p.E; e0 += 64) {
+        const int mine = min(e0 + lane, p.E - 1), o0 = p.offsets[mine], o1 = p.offsets[mine + 1];
+        const int n = e0 + lane < p.E ? (max(o1 - o0, 0) + BM - 1) / BM : 0;
+        int sum = n;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int left = __shfl_up(sum, d);
+            sum += lane >= d ? left : 0;
+        }
+        const uint64_t m = __builtin_amdgcn_ballot_w64(tile < before + sum);
+        if (m != 0) {
+            const int at = __builtin_ctzll(m), start = __builtin_amdgcn_readlane(o0, at);
+            e = e0 + at;
+            first = start + (tile - before - __builtin_amdgcn_readlane(sum - n, at)) * BM;
+            end = min(__builtin_amdgcn_readlane(o1, at), p.n_pairs);
+            return first >= start && first < end;
+        }
+        before += __builtin_amdgcn_readlane(sum, 63);
+    }
+    return false;
+}
+
 // row of the left operand for place i of the order
 template <bool GATE_UP>
 __device__ __forceinline__ int64_t left_row(const MoeParams& p, int i) {
@@ -316,7 +346,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
     const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, chunk);
     const int n_tile = id % n_tiles;
     int e, first, end;
-    if (!find_tile<BM>(p, id / n_tiles, e, first, end)) return;
+    if (!find_dense_tile<BM>(p, id / n_tiles, e, first, end)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, r = lane & 15, kg = lane >> 4;
     const int n0 = n_tile * (GATE_UP ? 64 : 128);
@@ -390,6 +420,154 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
                 for (int q = 0; q < 4; ++q) v[q] = wgt * acc[i][j][q];
                 store4(p, pair, n0 + 64 * wn + 16 * i + 4 * kg, v);
             }
+        }
+    }
+}
+
+// 256 rows x 256 rows of w per workgroup (gate_up: 128 gates and the 128 ups of the same columns): four wavefronts of
+// 128 x 128 on 32x32x16 MFMAs, k in steps of 64 through two LDS buffers (128 KB, one workgroup per compute unit).  A byte
+// that is brought into LDS feeds twice, a byte read from it 1.5 times the MFMAs it feeds in the 128 x 128 kernel, which is bound
+// by the requests (a compute unit takes in about 40 bytes per cycle, that kernel wants 62 at the full MFMA rate).  One
+// wavefront per SIMD hides nothing of another, and a request that waits for its turn holds up the MFMAs behind it: so the
+// buffers change hands at three quarters of a step, and the next step's 16 requests of a wavefront go out one behind every third
+// MFMA from there on, the fragments of the next quarter one in front of each of the first eight.  (All requests in front of the
+// last quarter: 40 % more cycles.)  Results leave through LDS in whole rows.
+// 32768 pairs, 16 experts, 2048 x 1024: 307-320 -> 258-268 us (1.05 PFLOP/s; MFMAs busy 53 % of 1.9 GHz, the clock this load
+// settles at; the library's product of that size 1.05-1.3), down 201-212 -> 169-172.  Lines touched ahead for the L2: 3 % slower.
+__device__ __forceinline__ int wide_swz(int row) { return (((row >> 1) & 3) << 1) | ((row >> 3) & 1); }       // (banks repeat every 256 bytes)
+template <bool GATE_UP>
+__global__ __launch_bounds__(256, 1) void moe_wide_kernel(MoeParams p, int n_tiles, int m_tiles, int chunk) {
+    constexpr int BM = 256, BK = 64, kTile = 256 * BK * 2;
+    constexpr int kCols = GATE_UP ? 128 : 256, kOutRow = kCols * 2 + 16;           // output columns; bytes of a padded LDS row of them
+    constexpr int kLds = 4 * kTile > BM * kOutRow ? 4 * kTile : BM * kOutRow;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];               // [buffer][rows | w]
+    const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, chunk);
+    const int n_tile = id % n_tiles;
+    int e, first, end;
+    if (!find_dense_tile<BM>(p, id / n_tiles, e, first, end)) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, r = lane & 31, kg = lane >> 5;
+    const int n0 = n_tile * kCols;
+    const __bf16* a_base = (const __bf16*)p.a;
+    const __bf16* w_base = (const __bf16*)p.w + (int64_t)e * (GATE_UP ? 2 : 1) * p.n * p.k;
+    // wavefront w fills rows 64 w .. 64 w + 63 of both tiles, 8 rows per load
+    uint32_t a_off[8], w_off[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int row = 64 * wave + 8 * j + (lane >> 3), piece = (lane & 7) ^ wide_swz(row);
+        a_off[j] = (uint32_t)((left_row<GATE_UP>(p, min(first + row, end - 1)) * p.a_stride + piece * 8) * 2);
+        const int64_t wr = GATE_UP ? (row < 128 ? min(n0 + row, p.n - 1) : p.n + min(n0 + row - 128, p.n - 1)) : min(n0 + row, p.n - 1);
+        w_off[j] = (uint32_t)((wr * p.k + piece * 8) * 2);
+    }
+    const uint32_t lds0 = lds_address(lds);
+    const auto issue1 = [&](int k0, int buf, int j) {        // the wavefront's 16 requests of a step
+        if (j < 8) dma_to_lds_16(a_base + k0, a_off[j], lds0 + (2 * buf) * kTile + (64 * wave + 8 * j) * 128);
+        else dma_to_lds_16(w_base + k0, w_off[j - 8], lds0 + (2 * buf + 1) * kTile + (64 * wave + 8 * (j - 8)) * 128);
+    };
+    f32x16 acc[4][4];                             // [32 rows of w][32 rows]
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
+    // 32-row groups of w of this wavefront: gate_up: gates 64 wn, 64 wn + 32, then the ups of these columns
+    const auto w_group = [&](int i) { return GATE_UP ? (i >> 1) * 128 + 64 * wn + (i & 1) * 32 : 128 * wn + 32 * i; };
+    bf16x8 wf[2][4], af[2][4];
+    // One fragment of quarter step s of buffer buf: four of the weights, then four of the rows
+    const auto fetch1 = [&](int buf, int s, int f) {
+        const unsigned char* at = lds + (2 * buf) * kTile;
+        const int piece = ((2 * s + kg) ^ wide_swz(r)) * 16;
+        if (f < 4) wf[s & 1][f] = as_bf16x8(*reinterpret_cast<const u32x4*>(at + kTile + (w_group(f) + r) * 128 + piece));
+        else af[s & 1][f - 4] = as_bf16x8(*reinterpret_cast<const u32x4*>(at + (128 * wm + 32 * (f - 4) + r) * 128 + piece));
+    };
+    // The 16 MFMAs of quarter s, with the reads of the next quarter's fragments (fetch: its buffer and number, or -1) between the
+    // first eight and a request (of step k_ahead into buffer to, numbers first .. first + n - 1; n 0: none) after every third
+    const auto quarter = [&](int s, int fbuf, int fs, int k_ahead, int to, int first, int n) {
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            if (fs >= 0 && m < 8) fetch1(fbuf, fs, m);
+            acc[m & 3][m >> 2] = mfma32(wf[s & 1][m & 3], af[s & 1][m >> 2], acc[m & 3][m >> 2]);
+            if (m % 3 == 2 && m / 3 < n) issue1(k_ahead, to, first + m / 3);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // step at k0 in buffer buf; next: a step follows, half requested in the step in front; ahead: another one follows that
+    const auto step = [&](int k0, int buf, auto next_c, auto ahead_c) {
+        constexpr bool next = decltype(next_c)::value, ahead = decltype(ahead_c)::value;
+        quarter(0, buf, 1, k0 + BK, buf ^ 1, 6, next ? 5 : 0);
+        quarter(1, buf, 2, k0 + BK, buf ^ 1, 11, next ? 5 : 0);
+        quarter(2, buf, 3, 0, 0, 0, 0);
+        if constexpr (next) {
+            wait_lgkmcnt0();                      // the last fragments of this buffer are in registers,
+            wait_vmcnt<0>();                      // the other buffer has landed
+            __syncthreads();
+            quarter(3, buf ^ 1, 0, k0 + 2 * BK, buf, 0, ahead ? 5 : 0);
+            if constexpr (ahead) issue1(k0 + 2 * BK, buf, 5);
+        } else {
+            quarter(3, 0, -1, 0, 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < 16; ++j) issue1(0, 0, j);
+    if (BK < p.k) {
+#pragma unroll
+        for (int j = 0; j < 6; ++j) issue1(BK, 1, j);
+        wait_vmcnt<6>();
+    } else {
+        wait_vmcnt<0>();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < 8; ++f) fetch1(0, 0, f);
+    constexpr std::integral_constant<bool, true> yes{};
+    constexpr std::integral_constant<bool, false> no{};
+    int k0 = 0, buf = 0;
+    for (; k0 + 2 * BK < p.k; k0 += BK, buf ^= 1) step(k0, buf, yes, yes);
+    if (k0 + BK < p.k) {
+        step(k0, buf, yes, no);
+        k0 += BK;
+        buf ^= 1;
+    }
+    step(k0, buf, no, no);
+    __syncthreads();
+    // lane: row 128 wm + 32 j + r, columns 8 g + 4 kg + q of a 32-column group
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int row = 128 * wm + 32 * j + r;
+        float wgt = 1.f;
+        if constexpr (!GATE_UP) wgt = p.weights[min(max(p.order[min(first + row, end - 1)], 0), p.n_pairs - 1)];
+#pragma unroll
+        for (int i = 0; i < (GATE_UP ? 2 : 4); ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                float v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if constexpr (GATE_UP) v[q] = silu_fast(acc[i][j][4 * g + q]) * acc[i + 2][j][4 * g + q];
+                    else v[q] = wgt * acc[i][j][4 * g + q];
+                }
+                const int col = (GATE_UP ? 64 : 128) * wn + 32 * i + 8 * g + 4 * kg;
+                *reinterpret_cast<u32x2*>(lds + row * kOutRow + col * 2) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+            }
+    }
+    __syncthreads();
+    constexpr int kLanes = kCols / 8;             // 16-byte pieces of a row
+    const int col = tid % kLanes * 8;
+#pragma unroll 4
+    for (int row = tid / kLanes; row < BM; row += 256 / kLanes) {
+        const int place = first + row;
+        if (place >= end || n0 + col >= p.n) break;
+        const int64_t out_row = GATE_UP ? place : min(max(p.order[place], 0), p.n_pairs - 1);
+        const u32x4 v = *reinterpret_cast<const u32x4*>(lds + row * kOutRow + col * 2);
+        __bf16* o = (__bf16*)p.out + out_row * p.out_stride + n0 + col;
+        if (n0 + col + 8 <= p.n) {
+            *reinterpret_cast<u32x4*>(o) = v;
+        } else {
+            const bf16x8 b = as_bf16x8(v);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (n0 + col + i < p.n) o[i] = b[i];
         }
     }
 }
@@ -609,21 +787,37 @@ __global__ __launch_bounds__(256) void moe_f32_kernel(MoeParams p, int n_tiles, 
     }
 }
 
+// The 256 x 256 tiles are a fifth faster where they fill whole rounds of the 256 compute units, and lose that to a round that is
+// mostly empty.  With one and a half full tiles per expert or more, an expert's last tile is half full on average: about (pairs / 256
+// + experts / 2) row tiles, give or take sqrt(experts / 12); with fewer most of a tile is padding.  Measured, both products, against
+// 128 x 128 (16 experts of 2048 x 1024, top 4): 3400 tokens (0.95 of two rounds) 197 against 227 us, 8192 (0.85 of five) 454 / 516,
+// 2600 (0.76 of two) 184 / 174; 32 experts of 2048 x 2048: 3400 tokens (0.86 of five) 397 / 477, 512 (64 pairs an expert) 224 / 208.
+// With a short k a tile is mostly its beginning and its end (512 x 512, 8 experts, 4096 tokens: 64 / 57).
+static bool wide_pays(const MoeParams& p, bool gate_up) {
+    const double n_tiles = (p.n + (gate_up ? 127 : 255)) / (gate_up ? 128 : 256);
+    const double tiles = (p.n_pairs / 256.0 + 0.5 * p.E) * n_tiles;
+    const double rounds = std::ceil((tiles + n_tiles * std::sqrt(p.E / 12.0)) / 256.0);
+    return p.k >= 1024 && p.n_pairs >= 384LL * p.E && tiles >= 0.79 * 256.0 * rounds;
+}
+
 template <bool GATE_UP>
 static int launch_moe(const MoeParams& p, int dtype, int tiling, hipStream_t s) {
     // From 8 pairs per expert on the large tiles, mostly padding then, still read the weights faster (2048 x 1024, 16 experts, both
     // products: 8 pairs 44 us against 55, 32 pairs 49 against 109)
-    const bool large = tiling == MI355_TILING_LARGE || (tiling == MI355_TILING_AUTO && p.n_pairs > 8 * (int64_t)p.E);
-    const int bm = dtype == MI355_BF16 && large ? 128 : 16;
-    const int bn = dtype == MI355_FP32 ? 64 : (!large ? 16 : (GATE_UP ? 64 : 128));
+    const bool large = tiling >= MI355_TILING_LARGE || (tiling == MI355_TILING_AUTO && p.n_pairs > 8 * (int64_t)p.E);
+    const bool fits = p.out_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+    const bool wide = dtype == MI355_BF16 && fits && (tiling == MI355_TILING_WIDE || (tiling == MI355_TILING_AUTO && large && wide_pays(p, GATE_UP)));
+    const int bm = dtype == MI355_BF16 && large ? (wide ? 256 : 128) : 16;
+    const int bn = dtype == MI355_FP32 ? 64 : (!large ? 16 : (GATE_UP ? 64 : 128) * (wide ? 2 : 1));
     const int n_tiles = (p.n + bn - 1) / bn, m_tiles = p.n_pairs / bm + p.E;
     if ((int64_t)n_tiles * m_tiles > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)(n_tiles * m_tiles)), block(256);
     // An XCD takes as many neighbouring row tiles in turn as fill its 32 compute units twice: they mostly belong to one expert
     // and share its weights in that L2.  (One row tile per turn, so that eight XCDs read eight tiles of one expert: 2048
     // tokens, 16 experts of 2048 x 1024, top 4 176 us for both products, 146 us like this; 8192 tokens 518 against 511.)
-    const int chunk = n_tiles * std::max(1, 64 / n_tiles);
+    const int chunk = n_tiles * std::max(1, (wide ? 32 : 64) / n_tiles);
     if (dtype == MI355_FP32) hipLaunchKernelGGL(moe_f32_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
+    else if (wide) hipLaunchKernelGGL(moe_wide_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles, chunk);
     else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles, chunk);
     else hipLaunchKernelGGL(moe_skinny_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     return (int)hipGetLastError();
@@ -636,7 +830,7 @@ static int moe_check(MoeParams& p, bool gate_up, const void* a, const void* w, v
     if (dtype != MI355_BF16 && dtype != MI355_FP32) return set_error(MI355_EDTYPE, "moe: dtype must be MI355_BF16 or MI355_FP32");
     if (E <= 0 || E > kMaxExperts || top <= 0 || k <= 0 || n <= 0 || n_pairs < 0 || n_pairs > 0x3fffffffLL)
         return set_error(MI355_EINVAL, "moe: experts, top, k, n, n_pairs out of range");
-    if (tiling < MI355_TILING_AUTO || tiling > MI355_TILING_LARGE) return set_error(MI355_EINVAL, "moe: unknown tiling");
+    if (tiling < MI355_TILING_AUTO || tiling > MI355_TILING_WIDE) return set_error(MI355_EINVAL, "moe: unknown tiling");
     if (a_stride < k || out_stride < n) return set_error(MI355_EINVAL, "moe: row strides shorter than a row");
     if (a_rows < (gate_up ? (n_pairs + top - 1) / top : n_pairs) || out_rows < n_pairs) return set_error(MI355_EINVAL, "moe: too few rows");
     if (dtype == MI355_BF16) {

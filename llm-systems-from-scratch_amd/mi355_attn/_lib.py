@@ -17,7 +17,7 @@ MASK_NONE, MASK_CAUSAL, MASK_BOOL = 0, 1, 2
 STATIC_SCRATCH_BYTES = 16 << 20          # MI355_STATIC_SCRATCH_BYTES
 
 SCANS = {"auto": 0, "serial": 1, "chunked": 2}
-TILINGS = {"auto": 0, "skinny": 1, "large": 2}
+TILINGS = {"auto": 0, "skinny": 1, "large": 2, "wide": 3}
 
 ROWS_STORE, ROWS_F32, ROWS_ADD, ROWS_GATE_UP, ROWS_QKV = range(5)
 

@@ -419,11 +419,15 @@ def test_experts(ops, T, E, top, k, ff, n, tiling, dtype):
 
 
 @pytest.mark.parametrize("tiling,T,E,top,k,ff,n", [
-    ("direct", 1, 8, 2, 64, 64, 40), ("direct", 33, 4, 1, 192, 128, 72), ("direct", 50, 8, 3, 1088, 192, 130), ("direct", 512, 8, 4, 64, 64, 8)])
+    ("direct", 1, 8, 2, 64, 64, 40), ("direct", 33, 4, 1, 192, 128, 72), ("direct", 50, 8, 3, 1088, 192, 130), ("direct", 512, 8, 4, 64, 64, 8),
+    ("wide", 1, 2, 1, 64, 64, 40), ("wide", 257, 3, 1, 192, 192, 264), ("wide", 300, 5, 2, 128, 320, 130), ("wide", 1024, 2, 2, 64, 128, 520),
+    ("wide", 300, 70, 3, 64, 64, 40),
+    ("auto", 1024, 2, 2, 1024, 3072, 200)])
 def test_expert_tilings(ops, tiling, T, E, top, k, ff, n):
     """The decode form that finds its pairs itself: one row, edges of 16 and 32 rows, the most pairs it takes, k of one step and of a remainder
-    of the four wavefronts' turns; also against the 128 x 128 tiles on the same operands: the same bf16 products in another order of the fp32
-    sums, so results agree to one rounding of the activations (2^-8) in either product."""
+    of the four wavefronts' turns.  The 256 x 256 tiles: edges of rows and columns, one, two and three steps of k, more experts than lanes;
+    "auto": where these tiles fill the chip.  Both also against the 128 x 128 tiles on the same operands: the same bf16 products in another
+    order of the fp32 sums, so results agree to one rounding of the activations (2^-8) in either product."""
     print(f"case: expert tilings {tiling} {T} {E} {top} {k} {ff} {n}", flush=True)
     bf = torch.bfloat16
     h, wg = rnd(T, k, seed=1, dtype=bf).cuda(), rnd(E, 2 * ff, k, seed=2, std=k ** -0.5, dtype=bf).cuda()
