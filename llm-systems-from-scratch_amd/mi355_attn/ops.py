@@ -1463,10 +1463,14 @@ def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
     lib = _lib.load()
     if tiling == "direct" and h.dtype != torch.bfloat16:
         raise TypeError("the direct form is bfloat16")
-    # No order up to 16 pairs per expert: with 2048 x 1024 experts (16 of them, 128 pairs) 45 us against 55 (group + skinny) and
-    # 44 (128-row tiles), at 256 pairs 47 / 79 / 49, at 512 pairs 61 / 110 / 49.  Experts of a MB or less are bound by the
-    # launches, of which it saves one, up to 64 pairs (8 of 512 x 512: 18 us against 26).
-    few = (64 if E * k * ff <= 1 << 22 else 16) * E
+    # The form without an order saves a launch and most of the padding, but reads the rows once per 32 weight rows: the larger all
+    # weights together, the fewer pairs it pays for.  Us against the 128-row tiles, at 8, 16, 32, 64 pairs per expert: 16 experts of
+    # 512 x 512 15, 14, 14, 19 / 21; 8 of 1024 x 1024 15, 16, 20, 29 / 28, 29, 30, 31; 32 of 512 x 512 16, 19, 24, 33 / 21, 21, 23, 24; 16
+    # of 1024 x 1024 22, 24, 34, 50 / 31, 31, 33, 35; 32 of 1024 x 1024 40, 47, 56 / 39, 40, 42; 8 of 2048 x 2048 44, 41, 59 / 49, 50, 51;
+    # 32 of 2048 x 1024 88, 93, 123 / 97, 98, 102.
+    weight = E * k * ff
+    few = 64 * E if weight <= 1 << 22 else max(16 * E, 512) if weight <= 1 << 23 else 320 if weight <= 1 << 24 \
+        else min(16 * E, 256) if weight <= 1 << 25 else 16 * E
     if tiling == "direct" or (tiling == "auto" and h.dtype == torch.bfloat16 and T * top <= min(_DIRECT_PAIRS, few)):
         with _on(h, ids, weights, w_gate_up, w_down) as stream:
             rc = lib.mi355_moe_direct(h.data_ptr(), w_gate_up.data_ptr(), w_down.data_ptr(), ids.data_ptr(), weights.data_ptr(), act.data_ptr(),
