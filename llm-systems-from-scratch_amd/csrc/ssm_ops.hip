@@ -18,6 +18,8 @@
 #include "common.hpp"
 #include "launch.hpp"
 
+#include <type_traits>
+
 namespace mi355 {
 
 constexpr int kConvTile = 16;        // tokens per thread of the convolution
@@ -294,12 +296,8 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(SsmParams<T> p) {
 
 // two values -> their bf16 parts and the bf16 parts of what those leave: v = hi + lo to 16 bits
 __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint32_t& lo) {
-    const __bf16 ha = (__bf16)a, hb = (__bf16)b;
-    bf16x2 t;
-    t[0] = ha;
-    t[1] = hb;
-    hi = __builtin_bit_cast(uint32_t, t);
-    lo = pack_bf16(a - (float)ha, b - (float)hb);
+    hi = pack_bf16(a, b);
+    lo = pack_bf16(a - __builtin_bit_cast(float, hi << 16), b - __builtin_bit_cast(float, hi & 0xffff0000u));
 }
 
 // Chunked form for bf16 prompts.  With c_t = a_1 + .. + a_t inside a chunk of 64 tokens and S the state in front of it:
@@ -307,8 +305,8 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 //     S  <- exp(c_last) S + sum_s B_s (exp(c_last - c_s) dt_s x_s)^T
 // One workgroup of four wavefronts per (sequence, head, 64 columns of vdim) walks the chunks; wavefront w owns 16 columns
 // and keeps its part of S, all 32 * NT rows of it, in MFMA accumulators.  v_mfma_f32_16x16x32_bf16 throughout:
-//   G^T (s x t)   = B C^T         rows from LDS, wavefront w takes tokens t = 16w .. 16w + 15 and only s tiles up to its own;
-//                                 weighted in fp32, it goes to LDS as the row t of bracketed factors
+//   G^T (s x t)   = B C^T         rows from LDS, the ten 16 x 16 tiles that hold an s <= t shared out over the wavefronts;
+//                                 weighted in fp32, they go to LDS as the rows t of bracketed factors
 //   Y^T (p x t)   = S^T C^T       S^T is the accumulator itself: the MFMA's k order is that of the accumulator's rows, which
 //                                 the reads of C mirror; scaled by exp(c_t), then
 //                 + X^T F^T       X^T fragments through the transposed LDS read
@@ -319,16 +317,24 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 // kWhole: a workgroup walks its whole sequence.  Few sequences and heads leave most of the chip idle then, so their segments
 // of seg_len tokens go side by side: kSegState leaves what each segment but the last adds to the state, ssd_carry_kernel turns
 // these into the states in front of the segments, and kSegOut computes every segment's outputs from there.
+//
+// Bound by the chain through a chunk -- three barriers, products that wait for LDS -- with two wavefronts per SIMD (NT 4: 220 registers,
+// 66 KB of LDS per workgroup).  What keeps it short: no branch inside a phase (one around each factor took half the VALU cycles),
+// four accumulators side by side in each product, one wavefront that prepares the next chunk's decays while the others take its
+// share of G, exponentials once per token instead of once per use.  4 sequences of 2048 tokens, 64 heads, state 128: states 50 -> 37
+// us, outputs 136 -> 108.  (Four heads per workgroup with shared B C^T: 108 to 124 before that, but one workgroup per compute unit: a
+// fifth slower where its rounds do not come out even.)
 enum { kWhole, kSegState, kSegOut };
 template <int NT, int MODE>
-__global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
+__global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmParams<__bf16> p) {
     constexpr int Q = 64, NP = 32 * NT;
     constexpr int kBRow = NP * 2 + 32, kCRow = NP * 2 + 16, kXRow = 64 * 2 + 32, kFRow = Q * 2 + 16;
     __shared__ __attribute__((aligned(16))) unsigned char b_lds[Q * kBRow];
     __shared__ __attribute__((aligned(16))) unsigned char c_lds[Q * kCRow];
     __shared__ __attribute__((aligned(16))) unsigned char x_lds[Q * kXRow];
     __shared__ __attribute__((aligned(16))) unsigned char f_lds[2][Q * kFRow];        // leading parts, remainders
-    __shared__ float cum_lds[Q], dt_lds[Q];
+    // per token, of this chunk and the next one: c_t, dt_t, exp(c_t), exp(c_last - c_t) dt_t
+    __shared__ __attribute__((aligned(16))) float cum_lds[2][Q], dt_lds[2][Q], grow_lds[2][Q], left_lds[2][Q];
 
     const int h = blockIdx.x / p.slices % p.H;
     const int col0 = (blockIdx.x % p.slices) * 64;
@@ -372,9 +378,9 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
             S[j][i] = resumed && n < p.N && pc + r < p.P ? from[(int64_t)n * p.Pp] : 0.f;
         }
 
-    // one chunk's loads: NT 16-byte pieces of B and C and two of x per thread, dt of token `lane`
+    // one chunk's loads: NT 16-byte pieces of B and C and two of x per thread
     u32x4 rb[NT], rc[NT], rx[2];
-    float rdt = 0.f, total = 0.f;                        // total: log2 of the decay so far
+    float total = 0.f;                                   // log2 of the decay so far
     const auto fetch = [&](int t0) {
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -393,19 +399,39 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
             if (t0 + row < len && col0 + col < p.P)
                 rx[j] = *reinterpret_cast<const u32x4*>(xsrc + (int64_t)(first + t0 + row) * p.channels + col);
         }
-        rdt = t0 + lane < len ? (float)p.proj[(int64_t)(first + t0 + lane) * p.proj_stride + p.dt_at + h] : 0.f;
     };
-    fetch(0);
-    for (int t0 = 0; t0 < len; t0 += Q) {
-        const float dt = t0 + lane < len ? softplus(rdt + bias) : 0.f;
+    // dt of token t0 + lane, and what follows from it, by one wavefront
+    const auto fetch_dt = [&](int t0) {
+        return p.proj[(int64_t)(first + min(t0 + lane, len - 1)) * p.proj_stride + p.dt_at + h];
+    };
+    const auto decays = [&](__bf16 raw, int t0, int buf) {
+        const float dt = t0 + lane < len ? softplus((float)raw + bias) : 0.f;
         float cum = na2 * dt;                            // running sum of the log2 decays, per lane = token
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
             const float up = __shfl_up(cum, off, 64);
-            if (lane >= off) cum += up;
+            cum += lane >= off ? up : 0.f;
         }
-        const float cum_last = __shfl(cum, 63, 64);
-        total += cum_last;
+        cum_lds[buf][lane] = cum;
+        dt_lds[buf][lane] = dt;
+        grow_lds[buf][lane] = fast_exp2(cum);
+        left_lds[buf][lane] = fast_exp2(__shfl(cum, 63, 64) - cum) * dt;
+    };
+    __bf16 rdt = (__bf16)0.f;
+    fetch(0);
+    if (wave == 0) {
+        const __bf16 dt0 = fetch_dt(0);
+        rdt = fetch_dt(Q);
+        decays(dt0, 0, 0);
+    }
+    if constexpr (MODE != kSegState) {                   // the tiles of the factors that are read but have no s <= t
+        if (wave % 2 == 0)
+#pragma unroll
+            for (int part = 0; part < 2; ++part)
+                *reinterpret_cast<u32x2*>(f_lds[part] + (16 * wave + r) * kFRow + (16 * wave + 16 + 4 * kg) * 2) = u32x2{0u, 0u};
+    }
+    int buf = 0;
+    for (int t0 = 0; t0 < len; t0 += Q, buf ^= 1) {
         __syncthreads();                                 // everybody has read the chunk before
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -418,40 +444,57 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
             const int idx = j * 256 + tid;
             *reinterpret_cast<u32x4*>(x_lds + (idx / 8) * kXRow + (idx % 8) * 16) = rx[j];
         }
-        if (wave == 0) {
-            cum_lds[lane] = cum;
-            dt_lds[lane] = dt;
-        }
         if (t0 + Q < len) fetch(t0 + Q);
         __syncthreads();
+        const float cum_last = cum_lds[buf][Q - 1];
+        total += cum_last;
+        if (wave == 0 && t0 + Q < len) {                 // (it has the least to do below)
+            decays(rdt, t0 + Q, buf ^ 1);
+            rdt = fetch_dt(t0 + 2 * Q);
+        }
 
-        // ---- bracketed factors of tokens 16 wave + r ------------------------------------------
+        // ---- bracketed factors: n tiles of 16 s from 16 s0 on of the tokens t = 16 tt + r ----------
         if constexpr (MODE != kSegState) {
-            const int t = 16 * wave + r;
-            const float ct = cum_lds[t];
-            bf16x8 cf[NT];
+            const auto factors = [&](int tt, int s0, auto n_c) {
+                constexpr int n = decltype(n_c)::value;
+                const int t = 16 * tt + r;
+                const float ct = cum_lds[buf][t];
+                f32x4 acc[n];
 #pragma unroll
-            for (int u = 0; u < NT; ++u)
-                cf[u] = as_bf16x8(*reinterpret_cast<const u32x4*>(c_lds + t * kCRow + (32 * u + 8 * kg) * 2));
-            // (tiles behind the wavefront's own come out as zeros: four independent chains are shorter than a branch per tile)
+                for (int m = 0; m < n; ++m) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s0 = 0; s0 < 4; ++s0) {
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int u = 0; u < NT; ++u) {
+                    const bf16x8 cf = as_bf16x8(*reinterpret_cast<const u32x4*>(c_lds + t * kCRow + (32 * u + 8 * kg) * 2));
 #pragma unroll
-                for (int u = 0; u < NT; ++u)
-                    acc = mfma16(as_bf16x8(*reinterpret_cast<const u32x4*>(b_lds + (16 * s0 + r) * kBRow + (32 * u + 8 * kg) * 2)),
-                                 cf[u], acc);
-                float f[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int s = 16 * s0 + 4 * kg + i;
-                    f[i] = s <= t ? acc[i] * (fast_exp2(ct - cum_lds[s]) * dt_lds[s]) : 0.f;
+                    for (int m = 0; m < n; ++m)
+                        acc[m] = mfma16(as_bf16x8(*reinterpret_cast<const u32x4*>(b_lds + (16 * (s0 + m) + r) * kBRow + (32 * u + 8 * kg) * 2)),
+                                        cf, acc[m]);
                 }
-                uint32_t h0, h1, l0, l1;
-                split_bf16(f[0], f[1], h0, l0);
-                split_bf16(f[2], f[3], h1, l1);
-                *reinterpret_cast<u32x2*>(f_lds[0] + t * kFRow + (16 * s0 + 4 * kg) * 2) = u32x2{h0, h1};
-                *reinterpret_cast<u32x2*>(f_lds[1] + t * kFRow + (16 * s0 + 4 * kg) * 2) = u32x2{l0, l1};
+#pragma unroll
+                for (int m = 0; m < n; ++m) {
+                    const int s = 16 * (s0 + m) + 4 * kg;
+                    const f32x4 cs = *reinterpret_cast<const f32x4*>(cum_lds[buf] + s);
+                    const f32x4 ds = *reinterpret_cast<const f32x4*>(dt_lds[buf] + s);
+                    float f[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = acc[m][i] * (fast_exp2(ct - cs[i]) * ds[i]);
+                        f[i] = s + i <= t ? v : 0.f;
+                    }
+                    uint32_t h0, h1, l0, l1;
+                    split_bf16(f[0], f[1], h0, l0);
+                    split_bf16(f[2], f[3], h1, l1);
+                    *reinterpret_cast<u32x2*>(f_lds[0] + t * kFRow + s * 2) = u32x2{h0, h1};
+                    *reinterpret_cast<u32x2*>(f_lds[1] + t * kFRow + s * 2) = u32x2{l0, l1};
+                }
+            };
+            if (wave == 0) {
+                factors(0, 0, std::integral_constant<int, 1>{});
+            } else if (wave == 1) {
+                factors(1, 0, std::integral_constant<int, 2>{});
+                factors(3, 3, std::integral_constant<int, 1>{});
+            } else {
+                factors(wave, 0, std::integral_constant<int, 3>{});
             }
             __syncthreads();
         }
@@ -467,7 +510,9 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
         }
         // ---- Y^T -------------------------------------------------------------------------------
         if constexpr (MODE != kSegState) {
-            bf16x8 sh[NT], sl[NT];
+            f32x4 acc[4];                                // tokens 16 tt + r: four chains side by side
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int u = 0; u < NT; ++u) {
                 u32x4 hi, lo;
@@ -478,52 +523,53 @@ __global__ __launch_bounds__(256) void ssd_chunk_kernel(SsmParams<__bf16> p) {
                     hi[e] = a;
                     lo[e] = c;
                 }
-                sh[u] = as_bf16x8(hi);
-                sl[u] = as_bf16x8(lo);
+                bf16x8 cf[4];
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    const unsigned char* src = c_lds + (16 * tt + r) * kCRow + (32 * u + 4 * kg) * 2;
+                    const u32x2 c0 = *reinterpret_cast<const u32x2*>(src), c1 = *reinterpret_cast<const u32x2*>(src + 32);
+                    cf[tt] = as_bf16x8(u32x4{c0[0], c0[1], c1[0], c1[1]});
+                }
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(as_bf16x8(hi), cf[tt], acc[tt]);
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) acc[tt] = mfma16(as_bf16x8(lo), cf[tt], acc[tt]);
             }
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) acc[tt] *= grow_lds[buf][16 * tt + r];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int part = 0; part < 2; ++part)
+#pragma unroll
+                    for (int tt = 2 * u; tt < 4; ++tt)
+                        acc[tt] = mfma16(xf[u], as_bf16x8(*reinterpret_cast<const u32x4*>(f_lds[part] + (16 * tt + r) * kFRow + (32 * u + 8 * kg) * 2)), acc[tt]);
 #pragma unroll
             for (int tt = 0; tt < 4; ++tt) {
                 const int t = 16 * tt + r;
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int u = 0; u < NT; ++u) {
-                    const unsigned char* src = c_lds + t * kCRow + (32 * u + 4 * kg) * 2;
-                    const u32x2 c0 = *reinterpret_cast<const u32x2*>(src), c1 = *reinterpret_cast<const u32x2*>(src + 32);
-                    const bf16x8 cf = as_bf16x8(u32x4{c0[0], c0[1], c1[0], c1[1]});
-                    acc = mfma16(sh[u], cf, acc);
-                    acc = mfma16(sl[u], cf, acc);
-                }
-                acc *= fast_exp2(cum_lds[t]);
-#pragma unroll
-                for (int u = 0; u <= tt / 2; ++u) {
-#pragma unroll
-                    for (int part = 0; part < 2; ++part)
-                        acc = mfma16(xf[u], as_bf16x8(*reinterpret_cast<const u32x4*>(f_lds[part] + t * kFRow + (32 * u + 8 * kg) * 2)), acc);
-                }
-                if (t0 + t < len && pc + 4 * kg < p.P) {
-                    const u32x2 xw = *reinterpret_cast<const u32x2*>(x_lds + t * kXRow + (16 * wave + 4 * kg) * 2);
-                    const uint32_t x01 = xw[0], x23 = xw[1];
-                    const bf16x2 xa = __builtin_bit_cast(bf16x2, x01), xb = __builtin_bit_cast(bf16x2, x23);
-                    u32x2 o;
-                    o[0] = pack_bf16(fmaf(skip, (float)xa[0], acc[0]), fmaf(skip, (float)xa[1], acc[1]));
-                    o[1] = pack_bf16(fmaf(skip, (float)xb[0], acc[2]), fmaf(skip, (float)xb[1], acc[3]));
+                const u32x2 xw = *reinterpret_cast<const u32x2*>(x_lds + t * kXRow + (16 * wave + 4 * kg) * 2);
+                const uint32_t x01 = xw[0], x23 = xw[1];
+                const bf16x2 xa = __builtin_bit_cast(bf16x2, x01), xb = __builtin_bit_cast(bf16x2, x23);
+                u32x2 o;
+                o[0] = pack_bf16(fmaf(skip, (float)xa[0], acc[tt][0]), fmaf(skip, (float)xa[1], acc[tt][1]));
+                o[1] = pack_bf16(fmaf(skip, (float)xb[0], acc[tt][2]), fmaf(skip, (float)xb[1], acc[tt][3]));
+                if (t0 + t < len && pc + 4 * kg < p.P)
                     *reinterpret_cast<u32x2*>(p.y + (int64_t)(first + t0 + t) * p.y_stride + h * p.P + pc + 4 * kg) = o;
-                }
             }
         }
         // ---- S --------------------------------------------------------------------------------
-        {
+        if (MODE != kSegOut || last || t0 + Q < len) {   // (nobody reads what a segment's last chunk would leave)
             const float decay = fast_exp2(cum_last);
             bf16x8 wh[2], wl[2];
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 u32x4 hi, lo;
+                const f32x4* left = reinterpret_cast<const f32x4*>(left_lds[buf] + 32 * u + 8 * kg);
+                const f32x4 w0 = left[0], w1 = left[1];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int s = 32 * u + 8 * kg + 2 * e;
                     uint32_t a, c;
-                    split_bf16((float)xf[u][2 * e] * (fast_exp2(cum_last - cum_lds[s]) * dt_lds[s]),
-                               (float)xf[u][2 * e + 1] * (fast_exp2(cum_last - cum_lds[s + 1]) * dt_lds[s + 1]), a, c);
+                    split_bf16((float)xf[u][2 * e] * (e < 2 ? w0 : w1)[2 * e % 4], (float)xf[u][2 * e + 1] * (e < 2 ? w0 : w1)[2 * e % 4 + 1], a, c);
                     hi[e] = a;
                     lo[e] = c;
                 }
