@@ -1352,12 +1352,19 @@ def gated_norm(y, z, weight, groups: int, eps: float, *, out=None):
     return out
 
 
-def ssm_segment_length(n_tokens: int, n_sequences: int, heads: int, vdim: int) -> int:
-    """Tokens per segment of the chunked scan (0: whole sequences): enough workgroups to fill the chip, of 256 tokens or more."""
+def ssm_segment_length(n_tokens: int, n_sequences: int, heads: int, vdim: int, state: int = 128) -> int:
+    """Tokens per segment of the chunked scan (0: whole sequences).
+
+    Segments cost a second pass and the states between them, so whole sequences from 512 workgroups on, two per compute unit (8 x
+    1000 tokens, 64 heads: 117 us against 164; 16 x 1000, 32 heads: 125 / 179).  Below, segments of 256 to 512 tokens that make as
+    many workgroups as are resident at once, three per compute unit up to a state of 64 (4 x 2048, 32 heads: 512 tokens 101 us, 256
+    tokens 111; 8 x 2000, 16 heads, state 64: 384 tokens 77, 256 83, 512 87); longer ones when there is work for two rounds."""
     per_unit = heads * ((vdim + 63) // 64)
-    if n_sequences * per_unit >= 1024 or n_tokens < 768 * n_sequences:
+    if n_sequences * per_unit >= 512 or n_tokens < 768 * n_sequences:
         return 0
-    return max(256, -(-n_tokens * per_unit // 1024) // 64 * 64)
+    resident = 512 if state > 64 else 768
+    fill = -(-n_tokens * per_unit // resident)
+    return max(256, min(512, -(-fill // 64) * 64), -(-n_tokens * per_unit // 1024) // 64 * 64)
 
 
 def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positions, cu_seqlens=None, *, heads, vdim, state, groups,
@@ -1398,7 +1405,7 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
     xbc = None if cu_seqlens is None else torch.empty(T, channels, dtype=proj.dtype, device=proj.device)
     seg_len, seg_state, seg_decay = 0, None, None
     if cu_seqlens is not None and scan != "serial" and proj.dtype == torch.bfloat16 and state % 8 == 0 and vdim % 8 == 0 and state <= 256:
-        seg_len = ssm_segment_length(T, B, heads, vdim) if segment is None else int(segment)
+        seg_len = ssm_segment_length(T, B, heads, vdim, state) if segment is None else int(segment)
     if seg_len:
         units = T // seg_len + B
         seg_state = torch.empty(units, heads, state, vdim, dtype=torch.float32, device=proj.device)
