@@ -47,9 +47,11 @@ def _traffic(key):
         return None
 
 
-def _prefill_kernel(head_dim):
-    """Name of the kernel a causal, unsplit prefill of this head_dim runs on."""
-    return "prefill_fwd_w64_kernel<causal>" if head_dim == 128 else "prefill_fwd_kernel<%d, causal>" % head_dim
+def _prefill_kernel(head_dim, keys=1 << 30):
+    """Name of the kernel a causal, unsplit, dense prefill of this head_dim and so many keys runs on."""
+    if head_dim == 128:
+        return "prefill_fwd_w64_kernel<causal>"
+    return ("prefill_short_kernel<%d, causal>" if keys <= 256 else "prefill_fwd_kernel<%d, causal>") % head_dim
 
 
 BURN_MS = 40.0      # untimed launches for about this long in front of the warm-up of every leg but the two decode legs
@@ -870,10 +872,10 @@ def bench_prefill_small(args, with_cpu):
         nbytes = 4 * b * h * n * d * 2                  # q, k, v read and out written once, bf16
         # which roofline binds: S/4 flops per byte (causal) against the part's 312 -- at these sizes the HBM one
         if nbytes / HBM_PEAK_GBPS / 1e9 >= flops / MFMA_BF16_PEAK_TFLOPS / 1e12:
-            roof = {"bound": "hbm", "kernel": _prefill_kernel(d), "achieved": nbytes / dev_ms / 1e6, "peak": HBM_PEAK_GBPS,
+            roof = {"bound": "hbm", "kernel": _prefill_kernel(d, n), "achieved": nbytes / dev_ms / 1e6, "peak": HBM_PEAK_GBPS,
                     "unit": "GB/s", "frac": nbytes / dev_ms / 1e6 / HBM_PEAK_GBPS}
         else:
-            roof = {"bound": "mfma", "kernel": _prefill_kernel(d), "achieved": flops / dev_ms / 1e9,
+            roof = {"bound": "mfma", "kernel": _prefill_kernel(d, n), "achieved": flops / dev_ms / 1e9,
                     "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": flops / dev_ms / 1e9 / MFMA_BF16_PEAK_TFLOPS}
         roof.update({"device_ms": dev_ms, "traffic": None, "algorithmic_bytes": nbytes,
                      "mfma_frac": flops / dev_ms / 1e9 / MFMA_BF16_PEAK_TFLOPS,
