@@ -939,21 +939,20 @@ extern "C" int mi355_moe_direct(const void* h, const void* w_gate_up, const void
                                 void* out, int64_t n_tokens, int64_t h_row_stride, int64_t out_row_stride, int n_experts, int top, int k,
                                 int ff, int n, void* stream) {
     if (!ids) return set_error(MI355_EINVAL, "moe_direct: null pointer argument");
-    if (n_tokens < 0 || top <= 0 || n_tokens * top > kDirectPairs) return set_error(MI355_EINVAL, "moe_direct: up to 2048 pairs");
-    // (ids stands in for the order, which these kernels do not read)
-    MoeParams p;
-    int rc = moe_check(p, true, h, w_gate_up, act, ids, ids, nullptr, h_row_stride, n_tokens, ff, n_tokens * top, n_tokens * top, n_experts, top,
+    if (n_tokens < 0 || top <= 0 || n_tokens > kDirectPairs || n_tokens * top > kDirectPairs) return set_error(MI355_EINVAL, "moe_direct: up to 2048 pairs");
+    // (ids stands in for the order, which these kernels do not read; nothing is launched before both products' arguments are checked)
+    MoeParams up, down;
+    int rc = moe_check(up, true, h, w_gate_up, act, ids, ids, nullptr, h_row_stride, n_tokens, ff, n_tokens * top, n_tokens * top, n_experts, top,
                        k, ff, MI355_BF16, MI355_TILING_AUTO);
+    if (rc == MI355_OK)
+        rc = moe_check(down, false, act, w_down, out, ids, ids, weights, ff, n_tokens * top, out_row_stride, n_tokens * top, n_tokens * top,
+                       n_experts, top, ff, n, MI355_BF16, MI355_TILING_AUTO);
     if (rc != MI355_OK || n_tokens == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
-    int tiles = (ff + 15) / 16;
-    hipLaunchKernelGGL(moe_direct_kernel<true>, dim3((unsigned)(tiles * n_experts)), dim3(256), 0, s, p, ids, tiles);
+    const int up_tiles = (ff + 15) / 16, down_tiles = (n + 31) / 32;
+    hipLaunchKernelGGL(moe_direct_kernel<true>, dim3((unsigned)(up_tiles * n_experts)), dim3(256), 0, s, up, ids, up_tiles);
     if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
-    rc = moe_check(p, false, act, w_down, out, ids, ids, weights, ff, n_tokens * top, out_row_stride, n_tokens * top, n_tokens * top, n_experts,
-                   top, ff, n, MI355_BF16, MI355_TILING_AUTO);
-    if (rc != MI355_OK) return rc;
-    tiles = (n + 31) / 32;
-    hipLaunchKernelGGL(moe_direct_kernel<false>, dim3((unsigned)(tiles * n_experts)), dim3(256), 0, s, p, ids, tiles);
+    hipLaunchKernelGGL(moe_direct_kernel<false>, dim3((unsigned)(down_tiles * n_experts)), dim3(256), 0, s, down, ids, down_tiles);
     if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
     return MI355_OK;
 }

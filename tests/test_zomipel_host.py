@@ -273,3 +273,19 @@ def test_operator_arguments_are_checked_on_the_host():
     assert lib.mi355_moe_route(z, z, z, z, z, z, 1, 64, 64, 64, 4, 1, 0, z) == -1
     assert lib.mi355_moe_group(z, 1, 4, z, z, z) == -1
     assert lib.mi355_ssm_decode(z, z) == -1 and lib.mi355_ssm_prefill(z, 0, z) == -1
+
+
+def test_expert_products_check_both_operands_before_any_launch():
+    """mi355_moe_direct is two products; what is wrong with the second is an argument error too (-1), not met after the first has been launched
+    (a launch without a GPU gives the runtime's own, positive status)."""
+    lib = mi355_attn.load()
+    buf = torch.zeros(64, dtype=torch.bfloat16)
+    at = (buf.data_ptr() + 15) // 16 * 16
+
+    def call(w_down=at, weights=at, out=at, stride=64, n=64, tokens=1):
+        return lib.mi355_moe_direct(at, at, w_down, at, weights, at, out, tokens, 64, stride, 2, 1, 64, 64, n, None)
+
+    assert call(tokens=0) == 0
+    for kw in (dict(w_down=None), dict(w_down=at + 2), dict(weights=None), dict(out=None), dict(out=at + 2), dict(stride=32), dict(stride=66), dict(n=0),
+               dict(tokens=1 << 62)):
+        assert call(**kw) == -1, kw
