@@ -267,7 +267,16 @@ def _prefill_backward(q, k, v, out, dout, lse, cu_q, cu_k, Sq, Sk, scale, mode, 
 
 
 def _bf16(*tensors):
-    return tuple(t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16) for t in tensors)
+    """The tensors in bf16.  What is broadcast (stride 0) is rounded once and stays broadcast: `to` alone writes every copy out, and the kernels
+    then read every copy."""
+    def rounded(t):
+        if t.dtype == torch.bfloat16:
+            return t
+        if 0 not in t.stride():
+            return t.to(torch.bfloat16)
+        return t[tuple(slice(0, 1) if st == 0 else slice(None) for st in t.stride())].to(torch.bfloat16).expand(t.shape)
+
+    return tuple(rounded(t) for t in tensors)
 
 
 class _DensePrefillFn(torch.autograd.Function):
@@ -411,7 +420,9 @@ def scaled_dot_product_attention(Q, K, V, mask=None):
             return t.reshape((1,) * (4 - t.dim()) + tuple(t.shape))
         return t.reshape(-1, *t.shape[-3:])
 
-    out_dtype = _out_dtype(Q, K, V)
+    out_dtype, grad = _out_dtype(Q, K, V), _needs_grad(Q, K, V)
+    if not grad:
+        Q, K, V = _bf16(Q, K, V)
     q4, k4, v4 = as4(Q, nq), as4(K, nk), as4(V, nk)
     m4 = None
     mode = _lib.MASK_NONE
@@ -420,13 +431,13 @@ def scaled_dot_product_attention(Q, K, V, mask=None):
         if m4.stride(-1) != 1:
             m4 = m4.contiguous()
         mode = _lib.MASK_BOOL
-    if _needs_grad(Q, K, V):
+    if grad:
         if mask is not None:
             out = _MaskedPrefillFn.apply(q4, k4, v4, _mask_words(m4))
         else:
             out = _DensePrefillFn.apply(q4, k4, v4, False, None)
         return out.reshape(*lead, nq, d).to(out_dtype)
-    out = _dense(*_bf16(q4, k4, v4), m4, mode, None, kv_splits=None)
+    out = _dense(q4, k4, v4, m4, mode, None, kv_splits=None)
     return out.reshape(*lead, nq, d).to(out_dtype)
 
 

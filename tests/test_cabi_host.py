@@ -243,3 +243,23 @@ def test_committed_assembly_include_is_what_the_generator_writes(tmp_path):
     subprocess.run([sys.executable, gen, str(out)], check=True, capture_output=True, env=env)
     assert out.read_bytes() == open(os.path.join(csrc, "prefill_w64_asm.inc"), "rb").read()
     assert "environ" not in open(gen).read()
+
+
+def test_float32_broadcast_inputs_are_rounded_once(monkeypatch):
+    """One key head shared by many query heads, in float32: the rounding must not write a copy per head."""
+    ops = mi355_attn.ops
+    seen = []
+    monkeypatch.setattr(ops, "_out_dtype", lambda *t: torch.float32)
+    monkeypatch.setattr(ops, "_dense", lambda q, k, v, *a, **kw: seen.append((q, k, v)) or torch.zeros(q.shape))
+    q, k, v = torch.randn(2, 6, 5, 32), torch.randn(2, 1, 7, 32), torch.randn(1, 1, 7, 32)
+    ops.scaled_dot_product_attention(q, k, v)
+    ops.scaled_dot_product_attention(q[None], k[None], v[None])                  # (five dimensions become four by a copy, of bf16)
+    for got, (k_strides, v_strides) in zip(seen, (((7 * 32, 0, 32, 1), (0, 0, 32, 1)), (None, None))):
+        for t, ref in zip(got, (q, k.expand(2, 6, 7, 32), v.expand(2, 6, 7, 32))):
+            assert t.dtype == torch.bfloat16 and torch.equal(t, ref.to(torch.bfloat16))
+        if k_strides:
+            assert got[1].stride() == k_strides and got[2].stride() == v_strides
+    for t in (q, k.expand(2, 6, 7, 32), v.expand(2, 6, 7, 32), torch.randn(3, 1, 4).expand(3, 0, 4), q.transpose(1, 2)):        # in front of the gradients too
+        b, = ops._bf16(t)
+        assert b.dtype == torch.bfloat16 and torch.equal(b, t.to(torch.bfloat16))
+        assert all(sb == 0 for sb, st, n in zip(b.stride(), t.stride(), t.shape) if st == 0 and n > 1)
