@@ -16,6 +16,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "weight_stream.hpp"
+#include "xcd_order.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -287,21 +288,44 @@ __device__ __forceinline__ bool find_tile(const MoeParams& p, int tile, int& e, 
     return first >= start && first < end;
 }
 
-// The same with the tiles numbered without gaps, so that the ones that have rows are the launch's first and none of the eight XCDs
-// has more of them than its share: the large tiles, where a round of the chip counts more than a scan over the experts (16 experts
-// of 2048 x 1024, top 4, 128 x 128 tiles, 1800 tokens: both products 138 -> 115 us; 32 of 2048 x 2048, 512 pairs: 240 -> 200).
+// Sum over the lanes up to this one: shifts inside rows of 16 lanes, then row ends into the rows behind them
+__device__ __forceinline__ int running_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);        // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);        // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);        // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// The same for workgroup `bid` of a launch with n_tiles columns of tiles, for the large tiles, where a round of the chip counts more
+// than a scan over the experts: the tiles are numbered without gaps and dealt to the XCDs by how many of them have rows, not by the
+// launch's bound, so that no XCD gets more workgroups than the others (16 experts of 2048 x 1024, top 4, 128 x 128 tiles, 1800
+// tokens: both products 138 -> 115 us; 32 of 2048 x 2048, 512 pairs: 240 -> 200.  Numbered without gaps but dealt by the bound, what
+// came behind the last whole round fell on some of the XCDs: 16 experts, 512 tokens, uniform ids 61 us and 55 like this, skewed ones
+// 68 and 57; 32 experts of 1024 x 512, top 2, 1500 tokens 36 and 31).
 template <int BM>
-__device__ __forceinline__ bool find_dense_tile(const MoeParams& p, int tile, int& e, int& first, int& end) {
+__device__ __forceinline__ bool find_dense_tile(const MoeParams& p, int bid, int n_tiles, int chunk, int& n_tile, int& e, int& first, int& end) {
     const int lane = threadIdx.x & 63;
+    int o0, o1, n, sum, total = 0;
+    const auto scan = [&](int e0) {               // tiles of the 64 experts from e0 on; sum: with those in front of each
+        const int mine = min(e0 + lane, p.E - 1);
+        o0 = p.offsets[mine];
+        o1 = p.offsets[mine + 1];
+        n = e0 + lane < p.E ? (max(o1 - o0, 0) + BM - 1) / BM : 0;
+        sum = running_sum(n);
+    };
+    for (int e0 = 0; e0 < p.E; e0 += 64) {
+        scan(e0);
+        total += __builtin_amdgcn_readlane(sum, 63);
+    }
+    total = min(total, p.n_pairs / BM + p.E);     // (the launch's bound, whatever the offsets are)
+    if (bid >= total * n_tiles) return false;
+    const int id = __builtin_amdgcn_readfirstlane(xcd_even_id(bid, total * n_tiles, chunk)), tile = id / n_tiles;
+    n_tile = id - tile * n_tiles;
     for (int e0 = 0, before = 0; e0 < p.E; e0 += 64) {
-        const int mine = min(e0 + lane, p.E - 1), o0 = p.offsets[mine], o1 = p.offsets[mine + 1];
-        const int n = e0 + lane < p.E ? (max(o1 - o0, 0) + BM - 1) / BM : 0;
-        int sum = n;
-#pragma unroll
-        for (int d = 1; d < 64; d *= 2) {
-            const int left = __shfl_up(sum, d);
-            sum += lane >= d ? left : 0;
-        }
+        if (p.E > 64) scan(e0);
         const uint64_t m = __builtin_amdgcn_ballot_w64(tile < before + sum);
         if (m != 0) {
             const int at = __builtin_ctzll(m), start = __builtin_amdgcn_readlane(o0, at);
@@ -340,13 +364,11 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
 // LDS buffers filled by direct loads.  A 128-byte LDS row holds its eight 16-byte pieces in the order piece ^ (row % 8).
 // Wavefront (wm, wn) computes 64 x 64; weights are the MFMA's first operand, so that a lane ends with adjacent columns.
 template <bool GATE_UP>
-__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int m_tiles, int chunk) {
+__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int chunk) {
     constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];          // [buffer][rows | w]
-    const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, chunk);
-    const int n_tile = id % n_tiles;
-    int e, first, end;
-    if (!find_dense_tile<BM>(p, id / n_tiles, e, first, end)) return;
+    int n_tile, e, first, end;
+    if (!find_dense_tile<BM>(p, blockIdx.x, n_tiles, chunk, n_tile, e, first, end)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, r = lane & 15, kg = lane >> 4;
     const int n0 = n_tile * (GATE_UP ? 64 : 128);
@@ -436,15 +458,13 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
 // settles at; the library's product of that size 1.05-1.3), down 201-212 -> 169-172.  Lines touched ahead for the L2: 3 % slower.
 __device__ __forceinline__ int wide_swz(int row) { return (((row >> 1) & 3) << 1) | ((row >> 3) & 1); }       // (banks repeat every 256 bytes)
 template <bool GATE_UP>
-__global__ __launch_bounds__(256, 1) void moe_wide_kernel(MoeParams p, int n_tiles, int m_tiles, int chunk) {
+__global__ __launch_bounds__(256, 1) void moe_wide_kernel(MoeParams p, int n_tiles, int chunk) {
     constexpr int BM = 256, BK = 64, kTile = 256 * BK * 2;
     constexpr int kCols = GATE_UP ? 128 : 256, kOutRow = kCols * 2 + 16;           // output columns; bytes of a padded LDS row of them
     constexpr int kLds = 4 * kTile > BM * kOutRow ? 4 * kTile : BM * kOutRow;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];               // [buffer][rows | w]
-    const int id = xcd_chunked_id(blockIdx.x, n_tiles * m_tiles, chunk);
-    const int n_tile = id % n_tiles;
-    int e, first, end;
-    if (!find_dense_tile<BM>(p, id / n_tiles, e, first, end)) return;
+    int n_tile, e, first, end;
+    if (!find_dense_tile<BM>(p, blockIdx.x, n_tiles, chunk, n_tile, e, first, end)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, r = lane & 31, kg = lane >> 5;
     const int n0 = n_tile * kCols;
@@ -817,8 +837,8 @@ static int launch_moe(const MoeParams& p, int dtype, int tiling, hipStream_t s) 
     // tokens, 16 experts of 2048 x 1024, top 4 176 us for both products, 146 us like this; 8192 tokens 518 against 511.)
     const int chunk = n_tiles * std::max(1, (wide ? 32 : 64) / n_tiles);
     if (dtype == MI355_FP32) hipLaunchKernelGGL(moe_f32_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
-    else if (wide) hipLaunchKernelGGL(moe_wide_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles, chunk);
-    else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles, chunk);
+    else if (wide) hipLaunchKernelGGL(moe_wide_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, chunk);
+    else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, chunk);
     else hipLaunchKernelGGL(moe_skinny_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     return (int)hipGetLastError();
 }

@@ -1,7 +1,10 @@
 """Host logic around the Zomipel model, on the CPU: order of looped layers, registry and configuration, weight layout (stacked
 projections, padded heads, turned pairs, experts), state slots, argument checks -- and the oracle itself against closed forms."""
+import ctypes
 import json
 import math
+import os
+import subprocess
 
 import pytest
 import torch
@@ -289,3 +292,30 @@ def test_expert_products_check_both_operands_before_any_launch():
     for kw in (dict(w_down=None), dict(w_down=at + 2), dict(weights=None), dict(out=None), dict(out=at + 2), dict(stride=32), dict(stride=66), dict(n=0),
                dict(tokens=1 << 62)):
         assert call(**kw) == -1, kw
+
+
+# ---- order of workgroups -------------------------------------------------------------------------------------------------
+def test_workgroups_with_work_are_dealt_evenly_to_the_xcds(tmp_path):
+    """Every workgroup with work gets an id of its own, and no XCD (id modulo 8 of the launch) gets more than one of them more than another,
+    beyond the whole rounds, which are even by themselves; whole chunks of neighbouring ids stay on one XCD."""
+    src, lib = tmp_path / "order.cpp", tmp_path / "order.so"
+    src.write_text('#include "xcd_order.hpp"\n'
+                   'extern "C" void ids(int n, int chunk, int* out) { for (int i = 0; i < n; ++i) out[i] = mi355::xcd_even_id(i, n, chunk); }\n')
+    csrc = os.path.join(os.path.dirname(os.path.dirname(mi355_attn.__file__)), "csrc")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
+    fn = ctypes.CDLL(str(lib)).ids
+    # 336: 21 row tiles of 16 columns, where a launch of 32 row tiles dealt in chunks of 64 gave 64, 64, 64, 64, 64, 16, 0, 0
+    for n, chunk in ((336, 64), (1, 64), (7, 16), (8, 1), (9, 1), (511, 64), (512, 64), (513, 64), (1300, 48), (4096, 64), (4100, 32), (77, 33)):
+        out = (ctypes.c_int * n)()
+        fn(n, chunk, out)
+        assert sorted(out) == list(range(n)), (n, chunk)
+        whole = n // (8 * chunk) * 8 * chunk
+        assert sorted(out[:whole]) == list(range(whole))
+        counts = [len(out[whole + x::8]) for x in range(8)]
+        assert max(counts) - min(counts) <= 1
+        for x in range(8):
+            mine = out[whole + x::8]
+            assert list(mine) == list(range(mine[0], mine[0] + len(mine))) if mine else True
+            for turn in range(whole // (8 * chunk)):
+                run = out[x:whole:8][turn * chunk:(turn + 1) * chunk]
+                assert list(run) == list(range(run[0], run[0] + chunk)) and run[0] % chunk == 0
