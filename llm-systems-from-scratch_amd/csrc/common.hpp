@@ -137,6 +137,17 @@ __device__ __forceinline__ void dma_to_lds_16(const void* gbase, uint32_t voff, 
                  : "v"(voff), "s"(gbase), "{m0}"(lds_addr)
                  : "memory");
 }
+// Sum over the lanes up to this one: shifts inside rows of 16 lanes, then row ends into the rows behind them
+__device__ __forceinline__ int running_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);        // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);        // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);        // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // Logical id of workgroup `bid` of a one-dimensional grid whose ids come in chunks of `chunk` that read the same
 // tensor rows (e.g. the query tiles and query heads of one K/V head).  Workgroup ids are dealt round-robin to the 8
 // XCDs, each with an L2 of its own; the XCDs take whole chunks in turn, so the workgroups of a chunk are resident on

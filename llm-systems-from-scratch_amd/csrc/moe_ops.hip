@@ -288,17 +288,6 @@ __device__ __forceinline__ bool find_tile(const MoeParams& p, int tile, int& e, 
     return first >= start && first < end;
 }
 
-// Sum over the lanes up to this one: shifts inside rows of 16 lanes, then row ends into the rows behind them
-__device__ __forceinline__ int running_sum(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);        // row_shr:1, 2, 4, 8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);        // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);        // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
 // The same for workgroup `bid` of a launch with n_tiles columns of tiles, for the large tiles, where a round of the chip counts more
 // than a scan over the experts: the tiles are numbered without gaps and dealt to the XCDs by how many of them have rows, not by the
 // launch's bound, so that no XCD gets more workgroups than the others (16 experts of 2048 x 1024, top 4, 128 x 128 tiles, 1800

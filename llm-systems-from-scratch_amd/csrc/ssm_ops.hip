@@ -41,7 +41,7 @@ struct SsmParams {
     int B, H, P, Pp, N, G, taps, channels, n_slots;
     int np4, slices;                 // scan: 4-wide pieces of vdim per workgroup, and workgroups per head
     float *seg_state, *seg_decay;    // segments: (segment, head) states (N x Pp), log2 of the decay across a segment
-    int seg_len, n_segs;
+    int seg_len, n_segs, whole_len;  // whole_len: sequences of up to so many tokens are one segment
 };
 
 template <typename T>
@@ -294,6 +294,48 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(SsmParams<T> p) {
     }
 }
 
+// ---- segments of the chunked scan ----
+// Segments are numbered without gaps, sequence by sequence, so that the workgroups that have one are a launch's first: one that has
+// none still holds 66 KB of LDS while it finds out (32 sequences of 1000 tokens, 16 heads, two of three numbers without a segment
+// 199 us, like this 133; 125 where the caller says that nothing need be cut).
+__device__ __forceinline__ int segments_of(const SsmParams<__bf16>& p, int b) {
+    int first, len;
+    seq_rows(p, b, first, len);
+    return len <= max(p.seg_len, p.whole_len) ? len > 0 : (len + p.seg_len - 1) / p.seg_len;
+}
+// Walks the sequences 64 at a time, a lane each; at(e0, n, sum) with the segments of this lane's sequence and of all up to it (of
+// this walk's 64) says whether to go on.
+template <typename F>
+__device__ __forceinline__ void walk_segments(const SsmParams<__bf16>& p, F&& at) {
+    const int lane = threadIdx.x & 63;
+    for (int e0 = 0; e0 < p.B; e0 += 64) {
+        const int n = e0 + lane < p.B ? segments_of(p, e0 + lane) : 0;
+        if (!at(e0, n, running_sum(n))) return;
+    }
+}
+// The sequence of segment `unit` of the segments that have `skip` behind them in their sequence, its place there and the number of
+// the sequence's first segment; false: there are not so many
+__device__ __forceinline__ bool find_segment(const SsmParams<__bf16>& p, int unit, int skip, int& b, int& place, int& seg0) {
+    bool found = false;
+    int before = 0, before_all = 0;
+    walk_segments(p, [&](int e0, int n, int sum) {
+        const int mine = max(n - skip, 0), mine_sum = skip == 0 ? sum : running_sum(mine);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(unit < before + mine_sum);
+        if (m != 0) {
+            const int at = __builtin_ctzll(m);
+            b = e0 + at;
+            place = unit - before - __builtin_amdgcn_readlane(mine_sum - mine, at);
+            seg0 = before_all + __builtin_amdgcn_readlane(sum - n, at);
+            found = true;
+            return false;
+        }
+        before += __builtin_amdgcn_readlane(mine_sum, 63);
+        before_all += __builtin_amdgcn_readlane(sum, 63);
+        return true;
+    });
+    return found;
+}
+
 // two values -> their bf16 parts and the bf16 parts of what those leave: v = hi + lo to 16 bits
 __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint32_t& lo) {
     hi = pack_bf16(a, b);
@@ -316,7 +358,8 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 //
 // kWhole: a workgroup walks its whole sequence.  Few sequences and heads leave most of the chip idle then, so their segments
 // of seg_len tokens go side by side: kSegState leaves what each segment but the last adds to the state, ssd_carry_kernel turns
-// these into the states in front of the segments, and kSegOut computes every segment's outputs from there.
+// these into the states in front of the segments, and kSegOut computes every segment's outputs from there.  A sequence of up to
+// seg_len or whole_len tokens is one segment, which only kSegOut sees.
 //
 // Bound by the chain through a chunk -- three barriers, products that wait for LDS -- with two wavefronts per SIMD (NT 4: 220 registers,
 // 66 KB of LDS per workgroup).  What keeps it short: no branch inside a phase (one around each factor took half the VALU cycles),
@@ -339,18 +382,21 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
     const int h = blockIdx.x / p.slices % p.H;
     const int col0 = (blockIdx.x % p.slices) * 64;
     const int unit = blockIdx.x / (p.slices * p.H);
-    const int b = MODE == kWhole ? unit : seq_of_unit(p, unit, p.seg_len);
+    int b = unit, place = 0, seg = 0;
+    if constexpr (MODE != kWhole) {
+        if (!find_segment(p, unit, MODE == kSegState ? 1 : 0, b, place, seg)) return;       // (nobody comes after a last one)
+        seg += place;
+        if (seg >= p.n_segs) return;                     // (sequences that overlap: no scratch beyond the caller's)
+    }
     int first, len;
     seq_rows(p, b, first, len);
     if (len <= 0) return;
-    bool last = true;
+    bool last = true, alone = true;                      // the sequence's last segment, its only one
     if constexpr (MODE != kWhole) {
-        const int s0 = (unit - (first / p.seg_len + b)) * p.seg_len;
-        if (s0 < 0 || s0 >= len) return;
-        last = s0 + p.seg_len >= len;
-        if (MODE == kSegState && last) return;           // nobody comes after it
-        first += s0;
-        len = min(p.seg_len, len - s0);
+        alone = len <= max(p.seg_len, p.whole_len);
+        last = alone || (place + 1) * p.seg_len >= len;
+        first += place * p.seg_len;
+        len = last ? len - place * p.seg_len : p.seg_len;
     }
     const int g = h / (p.H / p.G), inner = p.H * p.P;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -360,7 +406,7 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
     const bool has_cols = pc < p.P;
     const int slot = state_slot(p, b);
     float* st = p.ssm_state + ((int64_t)slot * p.H + h) * p.N * p.Pp + pc + r;
-    float* seg_st = MODE == kWhole ? nullptr : p.seg_state + ((int64_t)unit * p.H + h) * p.N * p.Pp + pc + r;
+    float* seg_st = MODE == kWhole ? nullptr : p.seg_state + ((int64_t)seg * p.H + h) * p.N * p.Pp + pc + r;
     const float bias = p.dt_bias[h], na2 = p.neg_a[h] * kLog2e, skip = p.d_skip[h];
     const __bf16* xsrc = p.xbc + h * p.P + col0;
     const __bf16* bsrc = p.xbc + inner + g * p.N;
@@ -368,8 +414,8 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
 
     // S: lane holds column pc + r, rows 16 j + 4 kg + i
     f32x4 S[2 * NT];
-    const float* from = MODE == kWhole ? st : seg_st;
-    const bool resumed = MODE == kSegOut || (MODE == kWhole && p.positions[first] > 0);
+    const float* from = alone ? st : seg_st;
+    const bool resumed = MODE != kSegState && (!alone || p.positions[first] > 0);
 #pragma unroll
     for (int j = 0; j < 2 * NT; ++j)
 #pragma unroll
@@ -590,7 +636,7 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
         }
     }
     if constexpr (MODE == kSegState) {
-        if (tid == 0 && col0 == 0) p.seg_decay[(int64_t)unit * p.H + h] = total;
+        if (tid == 0 && col0 == 0) p.seg_decay[(int64_t)seg * p.H + h] = total;
     }
     if (MODE == kSegOut && !last) return;
     float* to = MODE == kSegState ? seg_st : st;
@@ -610,11 +656,17 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsmParams<__bf16> p) {
     const int64_t size = (int64_t)p.N * p.Pp, at = 4 * (blockIdx.y * 256LL + threadIdx.x);
     int first, len;
     seq_rows(p, b, first, len);
-    if (len <= 0 || at >= size) return;
+    const int n = segments_of(p, b);
+    if (n <= 1) return;
+    int64_t seg0 = 0;
+    walk_segments(p, [&](int e0, int, int sum) {
+        const int end = __builtin_amdgcn_readlane(sum, min(b - e0, 63));
+        seg0 += b - e0 <= 63 ? end - n : end;
+        return b - e0 > 63;
+    });
+    if (at >= size || seg0 + n > p.n_segs) return;
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
     if (p.positions[first] > 0) S = *reinterpret_cast<const f32x4*>(p.ssm_state + ((int64_t)state_slot(p, b) * p.H + h) * size + at);
-    const int64_t seg0 = first / p.seg_len + b;
-    const int n = (len + p.seg_len - 1) / p.seg_len;
     float* seg = p.seg_state + (seg0 * p.H + h) * size + at;
     const float* decay = p.seg_decay + seg0 * p.H + h;
     for (int i = 0; i < n; i += kAhead) {
@@ -697,12 +749,15 @@ static int launch_chunks(const SsmParams<__bf16>& p, int64_t units, hipStream_t 
 static int launch_chunked(SsmParams<__bf16> p, hipStream_t s) {
     p.slices = (p.P + 63) / 64;
     if (p.seg_len == 0) return launch_chunks<kWhole>(p, p.B, s);
-    p.n_segs = (int)(p.n_rows / p.seg_len) + p.B;
-    if (int e = launch_chunks<kSegState>(p, p.n_segs, s)) return e;
-    const int64_t pieces = ((int64_t)p.N * p.Pp / 4 + 255) / 256, heads = (int64_t)p.B * p.H;
-    if (pieces > 65535 || heads > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    hipLaunchKernelGGL(ssd_carry_kernel, dim3((unsigned)heads, (unsigned)pieces), dim3(256), 0, s, p);
-    if (int e = (int)hipGetLastError()) return e;
+    // (of a sequence's segments all but the last are full ones)
+    const int64_t full = p.n_rows / p.seg_len, pieces = ((int64_t)p.N * p.Pp / 4 + 255) / 256, heads = (int64_t)p.B * p.H;
+    p.n_segs = (int)full + p.B;
+    if (full > 0) {
+        if (int e = launch_chunks<kSegState>(p, full, s)) return e;
+        if (pieces > 65535 || heads > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+        hipLaunchKernelGGL(ssd_carry_kernel, dim3((unsigned)heads, (unsigned)pieces), dim3(256), 0, s, p);
+        if (int e = (int)hipGetLastError()) return e;
+    }
     return launch_chunks<kSegOut>(p, p.n_segs, s);
 }
 
@@ -739,6 +794,7 @@ static SsmParams<T> ssm_params(const mi355_ssm_args& a) {
     p.seg_state = a.seg_state;
     p.seg_decay = a.seg_decay;
     p.seg_len = a.seg_len;
+    p.whole_len = a.whole_len;
     return p;
 }
 
@@ -769,7 +825,7 @@ extern "C" int mi355_ssm_prefill(const mi355_ssm_args* args, int scan, void* str
     if (!args->xbc) return set_error(MI355_EINVAL, "ssm_prefill: null xbc buffer");
     if (!args->cu_seqlens && args->n_rows != args->batch) return set_error(MI355_EINVAL, "ssm_prefill: one row per sequence without cu_seqlens");
     if (scan < MI355_SCAN_AUTO || scan > MI355_SCAN_CHUNKED) return set_error(MI355_EINVAL, "ssm_prefill: unknown scan");
-    if (args->seg_len < 0 || args->seg_len % 64 ||
+    if (args->seg_len < 0 || args->seg_len % 64 || args->whole_len < 0 ||
         (args->seg_len > 0 && (!args->seg_state || !args->seg_decay || (reinterpret_cast<uintptr_t>(args->seg_state) & 15))))
         return set_error(MI355_EINVAL, "ssm_prefill: segments are multiples of 64 tokens and need their buffers");
     if (args->n_rows == 0) return MI355_OK;

@@ -82,7 +82,7 @@ class SsmArgs(C.Structure):
                                            "slots", "positions", "cu_seqlens", "xbc", "y")] +
                 [(n, C.c_int64) for n in ("proj_row_stride", "xbc_col", "dt_col", "y_row_stride", "n_rows")] +
                 [(n, C.c_int) for n in ("batch", "heads", "vdim", "state", "groups", "taps", "n_slots", "dtype")] +
-                [("seg_state", C.c_void_p), ("seg_decay", C.c_void_p), ("seg_len", C.c_int)])
+                [("seg_state", C.c_void_p), ("seg_decay", C.c_void_p), ("seg_len", C.c_int), ("whole_len", C.c_int)])
 
 
 class RowsArgs(C.Structure):

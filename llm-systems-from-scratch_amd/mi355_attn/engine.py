@@ -524,9 +524,9 @@ class PagedAttentionEngine:
         ly = self.layers[layer]
         if proj.shape[0] != plan.positions.shape[0]:
             raise ValueError("the plan and the projection disagree on the number of tokens")
+        cu, longest = (plan.cu_seqlens, plan.max_len) if isinstance(plan, PrefillPlan) else (None, None)
         return ops.ssm_mix(proj, xbc_col, dt_col, ly.params, self.conv_states[layer], self.ssm_states[layer], plan.state_slots,
-                           plan.positions, plan.cu_seqlens if isinstance(plan, PrefillPlan) else None, heads=ly.heads, vdim=ly.vdim,
-                           state=ly.state, groups=ly.groups, out=out)
+                           plan.positions, cu, heads=ly.heads, vdim=ly.vdim, state=ly.state, groups=ly.groups, out=out, longest=longest)
 
     # ---- single-layer convenience ----------------------------------------------------
     def prefill(self, seq_ids, lens, q, k, v):

@@ -1378,8 +1378,23 @@ def ssm_segment_length(n_tokens: int, n_sequences: int, heads: int, vdim: int, s
     return max(256, min(512, -(-fill // 64) * 64), -(-n_tokens * per_unit // 1024) // 64 * 64)
 
 
+def ssm_segments(n_tokens: int, n_sequences: int, heads: int, vdim: int, state: int = 128, longest: int | None = None):
+    """(tokens per segment of the chunked scan or 0, tokens up to which a sequence stays whole all the same).
+
+    Between 512 and 1024 workgroups whole sequences pay only if they are about equally long: the longest one is what the call waits for.
+    So those of more than twice the mean are cut, on the device, where the lengths are; `longest` saves the two launches that
+    look for them where there are none.  64 heads, state 128, all whole / the long ones cut: 8192 tokens and 7 x 64 490 / 181 us, 4096
+    and 7 x 512 262 / 149, 3000 and 7 x 500 200 / 142; 400 to 1800 tokens 161 / 176 (with a line at 1.5); 16 x 1000, 32
+    heads 120 / 128, which is the two launches."""
+    seg = ssm_segment_length(n_tokens, n_sequences, heads, vdim, state)
+    whole = 2 * n_tokens // n_sequences
+    if seg or n_tokens < 768 * n_sequences or n_sequences * heads * ((vdim + 63) // 64) >= 1024 or (longest is not None and longest <= whole):
+        return seg, 0
+    return 512, whole
+
+
 def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positions, cu_seqlens=None, *, heads, vdim, state, groups,
-            out=None, scan="auto", segment: int | None = None):
+            out=None, scan="auto", segment: int | None = None, longest: int | None = None):
     """Mamba-2 mixer between its projections: causal convolution + silu of the channels (x | B | C) at column xbc_col of proj's
     rows, then S <- exp(A dt) S + dt B x^T, y = S^T C + D x with dt = softplus(columns dt_col .. + dt_bias).
 
@@ -1388,7 +1403,7 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
     to 4) fp32, updated in place at slots (B,) int32; positions (T,) int32 (a sequence whose first row has position 0 starts from
     zero).  With cu_seqlens (int32 (B+1,)) sequence b owns those rows; without it each owns one and everything is one launch.
     scan: "auto", "serial" or "chunked" (see mi355_ssm_prefill); segment: tokens per segment of the chunked scan (0: whole
-    sequences, None: chosen by size).  Returns y (T, heads * vdim), into `out` when given."""
+    sequences, None: chosen by size, which the longest sequence's length helps).  Returns y (T, heads * vdim), into `out` when given."""
     code = _dtype_code("proj", proj)
     T, width = _matrix("proj", proj, proj.dtype).shape
     channels, inner = heads * vdim + 2 * groups * state, heads * vdim
@@ -1414,9 +1429,9 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
     if T == 0:
         return out
     xbc = None if cu_seqlens is None else torch.empty(T, channels, dtype=proj.dtype, device=proj.device)
-    seg_len, seg_state, seg_decay = 0, None, None
+    seg_len, whole_len, seg_state, seg_decay = 0, 0, None, None
     if cu_seqlens is not None and scan != "serial" and proj.dtype == torch.bfloat16 and state % 8 == 0 and vdim % 8 == 0 and state <= 256:
-        seg_len = ssm_segment_length(T, B, heads, vdim, state) if segment is None else int(segment)
+        seg_len, whole_len = ssm_segments(T, B, heads, vdim, state, longest) if segment is None else (int(segment), 0)
     if seg_len:
         units = T // seg_len + B
         seg_state = torch.empty(units, heads, state, vdim, dtype=torch.float32, device=proj.device)
@@ -1427,7 +1442,7 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
                             None if cu_seqlens is None else cu_seqlens.data_ptr(), None if xbc is None else xbc.data_ptr(),
                             out.data_ptr(), proj.stride(0) if T > 1 else width, xbc_col, dt_col, out.stride(0) if T > 1 else inner, T,
                             B, heads, vdim, state, groups, taps, n_slots, code, None if seg_state is None else seg_state.data_ptr(),
-                            None if seg_decay is None else seg_decay.data_ptr(), seg_len)
+                            None if seg_decay is None else seg_decay.data_ptr(), seg_len, whole_len)
         if cu_seqlens is None:
             rc = _lib.load().mi355_ssm_decode(args, stream)
         else:

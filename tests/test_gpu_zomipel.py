@@ -361,6 +361,38 @@ def test_segment_lengths(ops):
     assert length(700, 1, 6, 40) == 0 and length(1100, 1, 6, 40) == 256 and length(10 ** 6, 1, 24, 200) % 64 == 0
 
 
+@pytest.mark.parametrize("longest", [None, 3000, 1000])
+def test_scan_of_unequal_sequences(ops, longest):
+    """512 workgroups, one sequence far longer than the others: cut where it is known to be, or the lengths are not known, and whole otherwise;
+    the others, which stay whole, have the same bits as without segments.  Resumed once; all of it against whole sequences and the float64 scan."""
+    m = dict(heads=64, vdim=8, state=16, groups=1, taps=2)
+    kw = {k: m[k] for k in ("heads", "vdim", "state", "groups")}
+    lens, slots = [460, 3000, 400, 450, 460, 500, 450, 430], [7, 1, 2, 0, 6, 5, 4, 3]
+    print(f"case: ssm unequal, longest {longest}", flush=True)
+    assert ops.ops.ssm_segments(sum(lens), 8, 64, 8, 16, longest) == ((0, 0) if longest == 1000 else (512, 1537))
+    case, params, xbc_at, dt_at = ssm_case(m, 8, 3, torch.bfloat16)
+    params["neg_a"] = params["neg_a"] * 0.1                               # long memories: what crosses a segment's edge shows
+    projs = [rnd(2 * n, case.shape[1], seed=n, dtype=torch.bfloat16) for n in lens]
+    pc, sl = {k: v.cuda() for k, v in params.items()}, torch.tensor(slots, dtype=torch.int32).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+
+    def both_halves(**how):
+        conv, state = ssm_pools(m, 9, torch.bfloat16)
+        halves = [ops.ssm_mix(torch.cat([p[i * n:i * n + n] for p, n in zip(projs, lens)]).cuda(), xbc_at, dt_at, pc, conv, state, sl,
+                              torch.cat([torch.arange(i * n, i * n + n) for n in lens]).int().cuda(), cu, **how, **kw) for i in range(2)]
+        assert bool((state[8] == 1e6).all())
+        return [torch.cat([torch.split(h, lens)[i] for h in halves]) for i in range(len(lens))], state
+
+    got, state = both_halves(longest=longest)
+    ref, ref_state = both_halves(segment=0)
+    for i in range(len(lens)):
+        if i != 1 or longest == 1000:
+            assert torch.equal(got[i], ref[i]) and torch.equal(state[slots[i]], ref_state[slots[i]]), i
+    want, S = ssm_oracle(m, projs[1], params, xbc_at, dt_at, True)
+    rows_close(got[1], want, torch.bfloat16, what="the long one")
+    assert float((state[1].cpu() - S).pow(2).mean().sqrt() / S.pow(2).mean().sqrt()) <= 1.5e-3
+
+
 def test_chunked_scan_forgets_and_remembers(ops):
     """Decays from almost none to complete within a token: chunks agree with the token-by-token form."""
     m = SSM[2]

@@ -294,6 +294,21 @@ def test_expert_products_check_both_operands_before_any_launch():
         assert call(**kw) == -1, kw
 
 
+# ---- segments of the scan ----------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("heads,lens", [(64, [8192] + [64] * 7), (64, [16384] + [16] * 7), (64, [3000] + [500] * 7), (16, [4000] + [1000] * 31),
+                                        (64, [1000] * 8), (32, [2000, 1000] * 8), (64, [1700] + [1500] * 8)])
+def test_no_sequence_of_a_scan_is_waited_for_alone(heads, lens):
+    """The longest walk over a sequence, in tokens: at most twice the mean, however the lengths are spread and whether the caller knows
+    the longest or not; equal lengths stay whole."""
+    mean = sum(lens) / len(lens)
+    for longest in (None, max(lens)):
+        seg, whole = mi355_attn.ops.ssm_segments(sum(lens), len(lens), heads, 64, 128, longest)
+        walks = [n if not seg or n <= max(seg, whole) else seg for n in lens]
+        assert max(walks) <= max(512, 2 * mean)
+    if len(set(lens)) == 1:
+        assert walks == lens and seg == 0
+
+
 # ---- order of workgroups -------------------------------------------------------------------------------------------------
 def test_workgroups_with_work_are_dealt_evenly_to_the_xcds(tmp_path):
     """Every workgroup with work gets an id of its own, and no XCD (id modulo 8 of the launch) gets more than one of them more than another,
