@@ -1474,6 +1474,17 @@ def moe_route(h, w, bias, top: int, *, extra_row: bool = False):
 _DIRECT_PAIRS = 2048        # the most pairs mi355_moe_direct takes
 
 
+def _direct_pairs(experts: int, k: int, ff: int, n: int) -> int:
+    """Up to how many pairs the expert products run without an order.  That saves a launch and the padding of 128-row tiles, and costs
+    what the pairs' rows take up: each 32 weight rows read those of their expert (k wide, then ff wide, and n out), and the weights once
+    more for every 32 of them.  So the line is drawn at 1.2 M elements in all pairs' rows, but not below 12 nor above 64 pairs per expert,
+    where one expert with more than its share would be waited for.  Us without and with an order, uniform ids: 8 experts of 1024 x 1024
+    (line at 48 pairs per expert) 32 pairs 20 / 30, 48 26 / 31, 64 31 / 32; 16 of 1024 x 1024 (24) 16 25 / 31, 24 28 / 31, 32 34 / 32; 32 of
+    512 x 512 (24) 16 20 / 22, 24 22 / 23, 32 24 / 23; 24 of 1536 x 768 (12.8) 12 36 / 38, 16 38 / 39, 20 44 / 39; 16 of 2048 x 1024 (14.4) 8
+    44 / 43, 12 44 / 42, 20 47 / 43; 8 of 2048 x 2048 (24) 24 46 / 50, 32 55 / 51; 8 of 1024 x 3072 (29) 24 34 / 51, 48 58 / 54."""
+    return min(_DIRECT_PAIRS, 64 * experts, max(12 * experts, (9 << 17) // (k + ff + n)))
+
+
 def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
     """Gated feed-forward of each row's chosen experts: weights[t, c] * Wd (silu(Wg h_t) * (Wu h_t)) of expert ids[t, c] as row
     t * top + c of the result (T * top, n); their sum is left to the reader (residual_rms).  h (T,k), w_gate_up
@@ -1496,15 +1507,7 @@ def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):
     lib = _lib.load()
     if tiling == "direct" and h.dtype != torch.bfloat16:
         raise TypeError("the direct form is bfloat16")
-    # The form without an order saves a launch and most of the padding, but reads the rows once per 32 weight rows: the larger all
-    # weights together, the fewer pairs it pays for.  Us against the 128-row tiles, at 8, 16, 32, 64 pairs per expert: 16 experts of
-    # 512 x 512 15, 14, 14, 19 / 21; 8 of 1024 x 1024 15, 16, 20, 29 / 28, 29, 30, 31; 32 of 512 x 512 16, 19, 24, 33 / 21, 21, 23, 24; 16
-    # of 1024 x 1024 22, 24, 34, 50 / 31, 31, 33, 35; 32 of 1024 x 1024 40, 47, 56 / 39, 40, 42; 8 of 2048 x 2048 44, 41, 59 / 49, 50, 51;
-    # 32 of 2048 x 1024 88, 93, 123 / 97, 98, 102.
-    weight = E * k * ff
-    few = 64 * E if weight <= 1 << 22 else max(16 * E, 512) if weight <= 1 << 23 else 320 if weight <= 1 << 24 \
-        else min(16 * E, 256) if weight <= 1 << 25 else 16 * E
-    if tiling == "direct" or (tiling == "auto" and h.dtype == torch.bfloat16 and T * top <= min(_DIRECT_PAIRS, few)):
+    if tiling == "direct" or (tiling == "auto" and h.dtype == torch.bfloat16 and T * top <= _direct_pairs(E, k, ff, n)):
         with _on(h, ids, weights, w_gate_up, w_down) as stream:
             rc = lib.mi355_moe_direct(h.data_ptr(), w_gate_up.data_ptr(), w_down.data_ptr(), ids.data_ptr(), weights.data_ptr(), act.data_ptr(),
                                       out.data_ptr(), T, h.stride(0) if T > 1 else k, out.stride(0), E, top, k, ff, n, stream)

@@ -294,6 +294,19 @@ def test_expert_products_check_both_operands_before_any_launch():
         assert call(**kw) == -1, kw
 
 
+# ---- expert products without an order -----------------------------------------------------------------------------------
+def test_line_of_the_expert_products_without_an_order():
+    """Wider experts never take more pairs, and a few columns more do not move the line by much; never below 12 pairs per expert."""
+    line = mi355_attn.ops._direct_pairs
+    widths = range(128, 4096 + 1, 64)
+    for E in (1, 8, 12, 24, 64, 170):
+        for square in (lambda d: (d, d, d), lambda d: (1024, d, 1024), lambda d: (d, 512, d), lambda d: (1024, 1024, d)):
+            at = [line(E, *square(d)) for d in widths]
+            assert all(12 * E <= x <= min(64 * E, 2048) for x in at)
+            assert all(b <= a <= 1.5 * b + 1 for a, b in zip(at, at[1:]))
+    assert line(400, 64, 64, 64) == 2048
+
+
 # ---- segments of the scan ----------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("heads,lens", [(64, [8192] + [64] * 7), (64, [16384] + [16] * 7), (64, [3000] + [500] * 7), (16, [4000] + [1000] * 31),
                                         (64, [1000] * 8), (32, [2000, 1000] * 8), (64, [1700] + [1500] * 8)])
