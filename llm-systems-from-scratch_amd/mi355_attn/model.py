@@ -315,9 +315,11 @@ class CachedTransformerLM(CachedLM):
         """The same for the few rows of a decode step, a layer in five launches: norm + projection + rotation + cache write,
         attention, output projection + residual, norm + gate/up + activation, down projection + residual."""
         H, dh, d = self.num_heads, self.d_head, self.d_model
+        # (project_decode is attend_decode with the projection in front; another attend is asked for every layer)
+        own = getattr(attend, "__func__", None) is PagedAttentionEngine.attend_decode
         x, rows = self.emb, token_ids                                 # the residual stream: rows of the embedding, then of its own
         for i, ly in enumerate(self.layers):
-            if self.engine.fuses_projection(i):
+            if own and self.engine.fuses_projection(i):
                 a = self.engine.project_decode(i, plan, x, ly["wqkv"], ly["attn_norm"], x_rows=rows)
             else:
                 qkv = ops.rows_linear(x, ly["wqkv"], norm=ly["attn_norm"], x_rows=rows).view(-1, 3, H, dh)

@@ -237,6 +237,22 @@ def test_decode_steps_replayed_from_a_hip_graph_equal_eager_steps(ops, kv_dtype)
     assert bool((err <= (0.15 if kv_dtype == "fp8" else 8e-2) + 5e-2 * ref.abs()).all()), float(err.max())
 
 
+def test_decode_steps_ask_the_attention_they_are_given(ops):
+    """An engine whose attend_decode is replaced (to look at queries and keys, say) is asked in every layer of a decode step."""
+    print("case: replaced attend_decode", flush=True)
+    params = _bf16_params(CFG, seed=3)
+    model = ops.CachedTransformerLM(CFG, params, max_batch=2)
+    twin = ops.CachedTransformerLM(CFG, params, max_batch=2)
+    seen, attend = [], model.engine.attend_decode
+    model.engine.attend_decode = lambda layer, plan, q, k, v: seen.append((layer, q.shape, k.shape)) or attend(layer, plan, q, k, v)
+    for m in (model, twin):
+        m.sids = [m.new_sequence()]
+        m.prefill(m.sids, [torch.arange(5)])
+    got, ref = model.decode(model.sids, [7]), twin.decode(twin.sids, [7])
+    assert seen == [(i, (1, 4, 32), (1, 4, 32)) for i in range(CFG["num_layers"])]
+    assert bool(((got - ref).abs() <= 3e-2 + 2e-2 * ref.abs()).all())               # (queries and keys are rounded once more in front of the rotation)
+
+
 def _check_greedy(params, cfg, prompt, toks, margin=0.15):
     """Every generated token must be (nearly) the oracle's argmax given the tokens before it, with the
     reference's sliding window (model.py:215)."""
