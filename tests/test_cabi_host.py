@@ -263,3 +263,15 @@ def test_float32_broadcast_inputs_are_rounded_once(monkeypatch):
         b, = ops._bf16(t)
         assert b.dtype == torch.bfloat16 and torch.equal(b, t.to(torch.bfloat16))
         assert all(sb == 0 for sb, st, n in zip(b.stride(), t.stride(), t.shape) if st == 0 and n > 1)
+
+
+def test_stream_number_without_torchs_private_shorthand(monkeypatch):
+    """The public way to a stream's number gives what the shorthand gives; which of them is used is decided at import."""
+    ops = mi355_attn.ops
+
+    class Stream:
+        cuda_stream = 17
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda index: Stream() if index == 1 else None)
+    assert ops._current_stream(1) == 17
+    assert ops._raw_stream in (ops._current_stream, getattr(torch._C, "_cuda_getCurrentRawStream", None))
