@@ -59,9 +59,12 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
         if (k - 64 * t < 64) {
 #pragma unroll
             for (int s = 0; s < 2; ++s)
-                if (32 * s + 8 * kg >= k - 64 * t)
+                if (32 * s + 8 * kg >= k - 64 * t) {          // (the weights too: zero times an infinity is no zero)
 #pragma unroll
                     for (int m = 0; m < MT; ++m) af[m][s] = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) wf[i][s] = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
+                }
         }
         if (t + 4 * kDeep < n_steps) {
             wait_lgkmcnt0();                      // the slot's bytes are in registers

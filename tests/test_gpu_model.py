@@ -375,6 +375,23 @@ def test_rows_linear(ops, T, k, n):
         ops.rows_linear(t(33, k), w)
 
 
+@pytest.mark.parametrize("T", [3, 20])
+@pytest.mark.parametrize("k", [72, 200, 256])
+def test_rows_linear_with_infinities(ops, T, k):
+    """Infinite and NaN weights and rows give what the product gives, also in the last, partial step of k."""
+    g = torch.Generator().manual_seed(k)
+    x, w = torch.rand(T, k, generator=g).to(torch.bfloat16) + 0.5, torch.randn(40, k, generator=g).to(torch.bfloat16)
+    last = k // 64 * 64 if k % 64 else k - 64                           # where the last step of k begins
+    w[1, last], w[2, last + 7], w[3, k - 1], w[4, 0], w[5, last], w[6, last + 1] = float("inf"), -float("inf"), float("inf"), -float("inf"), float("nan"), 3e38
+    x[1, k - 1] = float("inf")
+    x[2, last] = float("nan")
+    ref = x.float() @ w.float().T
+    got = ops.rows_linear(x.cuda(), w.cuda(), out_dtype=torch.float32).cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)]) and torch.allclose(got[fine], ref[fine], rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("T,H,G,D", [(1, 2, 2, 32), (17, 4, 1, 64), (32, 8, 2, 128)])
 def test_rows_qkv(ops, T, H, G, D):
     """Projection, rotation and cache write in one launch against the product and rope_and_cache: the product is rounded once less."""
