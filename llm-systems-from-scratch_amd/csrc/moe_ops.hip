@@ -668,9 +668,9 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
     int found = 0;
 #pragma unroll
     for (int i = 0; i < kLook; ++i) {
-        const int pair = 64 * (kLook * wave + i) + lane;
+        const int pair = 64 * (wave + 4 * i) + lane;
         hit[i] = 0;
-        if (64 * (kLook * wave + i) < p.n_pairs) hit[i] = __builtin_amdgcn_ballot_w64(pair < p.n_pairs && ids[min(pair, p.n_pairs - 1)] == e);
+        if (64 * (wave + 4 * i) < p.n_pairs) hit[i] = __builtin_amdgcn_ballot_w64(pair < p.n_pairs && ids[min(pair, p.n_pairs - 1)] == e);
         found += __popcll(hit[i]);
     }
     if (lane == 0) counts[wave] = found;
@@ -684,12 +684,12 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
     if (n_rows == 0) return;
 #pragma unroll
     for (int i = 0; i < kLook; ++i) {
-        if (hit[i] >> lane & 1) mine[at + __popcll(hit[i] & ((1ull << lane) - 1))] = (uint16_t)(64 * (kLook * wave + i) + lane);
+        if (hit[i] >> lane & 1) mine[at + __popcll(hit[i] & ((1ull << lane) - 1))] = (uint16_t)(64 * (wave + 4 * i) + lane);
         at += __popcll(hit[i]);
     }
     __syncthreads();
     const __bf16* w_base = (const __bf16*)p.w + (int64_t)e * (GATE_UP ? 2 : 1) * p.n * p.k;
-    const int piece = (lane & 7) ^ (lane >> 3);   // what a lane requests of its row's 128 bytes: see WeightStream
+    const int piece = (lane & 7) ^ (lane >> 3);   // what a lane requests of its row's 128 bytes: see weight_stream
     uint32_t w_off[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
