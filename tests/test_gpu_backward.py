@@ -374,3 +374,75 @@ def test_gradients_of_float32_inputs(ops, D, B):
     assert [g.dtype for g in grads] == [torch.float32, torch.float32, torch.bfloat16] and grads[2].stride() == v.stride()
     for g, w in zip(grads, want):
         assert torch.equal(g.to(torch.bfloat16), w)
+
+
+@pytest.mark.parametrize("lead", ["none", "batch", "full"])
+@pytest.mark.parametrize("D,Sq,Sk", [(32, 77, 301), (64, 130, 212), (64, 67, 33)])
+def test_masked_backward_of_many_short_heads(ops, D, Sq, Sk, lead):
+    """Above 256 workgroups at head sizes 32 and 64: random keep-masks whose rows, columns, heads and sequences all differ (or are broadcast),
+    odd sizes, a query row and a key that the mask leaves out altogether; against autograd through the oracle."""
+    print(f"case: masked backward many heads D={D} {Sq} {Sk} {lead}", flush=True)
+    B, H = 65, 4
+    q, k, v, dout = (rnd(B, H, n, D, seed=600 + i + Sq) for i, n in enumerate((Sq, Sk, Sk, Sq)))
+    mask = torch.rand(*{"none": (), "batch": (B, 1), "full": (B, H)}[lead], Sq, Sk, generator=torch.Generator().manual_seed(604)) < 0.6
+    rows = torch.arange(Sq)
+    mask[..., rows, rows % (Sk - 1)] = True
+    mask[..., Sk - 1] = False                                             # nobody sees the last key
+    mask[..., 17, :] = False                                              # a row that sees nothing
+    leaves = [t.cuda().requires_grad_() for t in (q, k, v)]
+    out = ops.scaled_dot_product_attention(*leaves, mask.cuda())
+    dq, dk, dv = torch.autograd.grad(out, leaves, dout.cuda())
+    assert bool(torch.isnan(out[:, :, 17].float()).all()) and bool((dq[:, :, 17] == 0).all())
+    assert bool((dk[:, :, Sk - 1] == 0).all()) and bool((dv[:, :, Sk - 1] == 0).all())
+    keep = [i for i in range(Sq) if i != 17]
+    ref, rq, rk, rv = oracle_masked_grads(q[:, :, keep], k, v, mask[..., keep, :], dout[:, :, keep])
+    torch.testing.assert_close(out.detach()[:, :, keep].float().cpu(), ref, atol=2e-2, rtol=1e-2)
+    check_grad("dq", dq[:, :, keep], rq)
+    check_grad("dk", dk, rk)
+    check_grad("dv", dv, rv)
+
+
+@pytest.mark.parametrize("D,copies", [(32, 1), (64, 1), (64, 33), (128, 1)])
+def test_gradients_of_float32_inputs_packed_and_masked(ops, D, copies):
+    """All three inputs float32, packed sequences (one of them empty) and explicit masks, fewer and more than 256 workgroups: the float32
+    gradients are those that the bf16 inputs' gradients are the rounding of."""
+    print(f"case: fp32 gradients packed and masked D={D} x{copies}", flush=True)
+    lens = [70, 0, 33, 1, 130] * copies
+    T, H, G = sum(lens), 4, 2
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+
+    def both(call, q, k, v, do):
+        full = [t.cuda().requires_grad_() for t in (q, k, v)]
+        half = [t.detach().to(torch.bfloat16).requires_grad_() for t in full]
+        out, ref = call(*full), call(*half)
+        assert out.dtype == torch.float32 and torch.equal(out, ref.float())
+        got, want = torch.autograd.grad(out, full, do.float().cuda()), torch.autograd.grad(ref, half, do.cuda())
+        for name, g, w in zip(("dq", "dk", "dv"), got, want):
+            assert g.dtype == torch.float32 and w.dtype == torch.bfloat16 and bool(torch.isfinite(g).all()), name
+            assert torch.equal(g.to(torch.bfloat16), w), name
+            assert not torch.equal(g, w.float()), name                    # (not rounded on the way)
+
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(T, h, D, generator=g) for h in (H, G, G))
+    both(lambda *t: ops.flash_attn_varlen_prefill(*t, cu, cu, 130, 130), q, k, v, rnd(T, H, D, seed=5))
+    B, Sq, Sk = 3 * copies, 45, 67
+    mask = (torch.rand(B, 1, Sq, Sk, generator=g) < 0.7).cuda()
+    mask[..., 0] = True
+    q, k, v = (torch.randn(B, H, n, D, generator=g) for n in (Sq, Sk, Sk))
+    both(lambda *t: ops.scaled_dot_product_attention(*t, mask), q, k, v, rnd(B, H, Sq, D, seed=6))
+
+
+def test_gradients_of_broadcast_float32_inputs(ops):
+    """One float32 key and value head behind several query heads, as views: the gradients of what is shared are the sums over who shares it."""
+    print("case: fp32 broadcast gradients", flush=True)
+    B, H, S, D = 2, 4, 50, 64
+    g = torch.Generator().manual_seed(9)
+    q, k, v = torch.randn(B, H, S, D, generator=g), torch.randn(B, 1, S, D, generator=g), torch.randn(1, 1, S, D, generator=g)
+    do = rnd(B, H, S, D, seed=4)
+    leaves = [t.cuda().requires_grad_() for t in (q, k, v)]
+    dq, dk, dv = torch.autograd.grad(ops.scaled_dot_product_attention(*leaves), leaves, do.float().cuda())
+    b = [t.to(torch.bfloat16).float().requires_grad_() for t in (q, k, v)]
+    ref = torch.autograd.grad(torch.softmax(b[0] @ b[1].transpose(-1, -2) / D ** 0.5, -1) @ b[2], b, do.float())
+    assert dk.shape == k.shape and dv.shape == v.shape
+    for name, got, want in zip(("dq", "dk", "dv"), (dq, dk, dv), ref):
+        check_grad(name, got, want)

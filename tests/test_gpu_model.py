@@ -327,6 +327,36 @@ def test_generate_batch_continuous_batching(ops):
         model.generate_batch([[1]] * 9, 1)
 
 
+@pytest.mark.parametrize("d_ff", [352, 356])
+@pytest.mark.parametrize("graphs", [False, True])
+def test_decode_across_the_row_limit_of_the_fused_layers(ops, d_ff, graphs):
+    """35 sequences that end one after the other: steps of more than 32 rows (and, with a d_ff that is no multiple of 8, all steps) run library
+    products and separate operators, the others rows_linear; a sequence that sees both follows the oracle.  Eager and replayed."""
+    print(f"case: decode across 32 rows, d_ff {d_ff} graphs {graphs}", flush=True)
+    cfg = dict(CFG, d_ff=d_ff)
+    params = _bf16_params(cfg, seed=31)
+    model = ops.CachedTransformerLM(cfg, params, max_batch=36, decode_graphs=graphs)
+    assert model._rows_fuse == (d_ff % 8 == 0)
+    g = torch.Generator().manual_seed(32)
+    seqs = [torch.randint(0, cfg["vocab_size"], (8 + (3 * i + 7) % 17 + (12 if i < 4 else 0),), generator=g) for i in range(35)]
+    sids = [model.new_sequence() for _ in seqs]
+    logits = model.prefill(sids, [s[:5] for s in seqs])
+    rows, live, widths = [[logits[i]] for i in range(35)], list(range(35)), []
+    for t in range(5, 40):
+        live = [i for i in live if t < len(seqs[i])]
+        if not live:
+            break
+        widths.append(len(live))
+        logits = model.decode([sids[i] for i in live], [int(seqs[i][t]) for i in live])
+        for j, i in enumerate(live):
+            rows[i].append(logits[j])
+    assert widths[0] == 35 and min(widths) <= 4 and widths.count(35) >= 2 and any(1 < w <= 32 for w in widths)
+    for i, s in enumerate(seqs):
+        _logit_close(torch.stack(rows[i])[None], mo.transformer_lm_reference(params, cfg, s[None])[:, 4:])
+    for s in sids:
+        model.free_sequence(s)
+
+
 def test_from_pretrained_reads_reference_files(ops, tmp_path):
     print("case: from_pretrained", flush=True)
     params = mo.random_lm_params(CFG, seed=22)

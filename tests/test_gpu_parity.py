@@ -408,6 +408,34 @@ def test_prefill_of_short_heads(ops, D, Sq, Sk, causal):
     check(ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=causal, kv_splits=1), ref, what="out")
     strided = q.transpose(1, 2).contiguous().transpose(1, 2).cuda().requires_grad_()       # rows of one head far apart, and with the lse
     check(ops.flash_attn_prefill(strided, k.cuda(), v.cuda(), causal=causal).detach(), ref, what="out, strided")
+    # log-sum-exp: the weights are summed as rounded to bf16, each off by 2^-9 of itself at most, so the sum's logarithm by 2^-9, and the
+    # scores in fp32 (sums of D products, off by D 2^-24 of their parts' sizes)
+    _, lse = ops.ops._dense(strided.detach(), k.cuda(), v.cuda(), None, ops._lib.MASK_CAUSAL if causal else ops._lib.MASK_NONE, None, want_lse=True)
+    scores = q.double() @ k.double().repeat_interleave(2, 1).transpose(-1, -2) / D ** 0.5
+    size = q.double().abs() @ k.double().abs().repeat_interleave(2, 1).transpose(-1, -2) / D ** 0.5
+    sees = torch.ones(Sq, Sk, dtype=torch.bool).tril(Sk - Sq) if causal else torch.ones(Sq, Sk, dtype=torch.bool)
+    want = torch.logsumexp(scores.masked_fill(~sees, -float("inf")), -1)
+    assert bool(((lse.double().cpu() - want).abs() <= 2.0 ** -9 + 1e-5 + D * 2.0 ** -24 * size.amax(-1)).all())
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("Sq,Sk,causal", [(70, 70, True), (33, 100, True), (130, 65, False)])
+def test_prefill_of_short_heads_with_infinities_and_nan(ops, D, Sq, Sk, causal):
+    """A key or query with an infinity makes scores of +inf (a NaN row), -inf (a weight of zero) or NaN; a value with one shows in the rows
+    that give it weight.  Rows come out as the reference softmax has them, NaN for NaN; a key behind the diagonal shows nowhere in front."""
+    print(f"case: short heads, infinities D={D} {Sq} {Sk} {causal}", flush=True)
+    q, k, v = rnd(5, 2, Sq, D, seed=1), rnd(5, 2, Sk, D, seed=2), rnd(5, 2, Sk, D, seed=3)
+    inf, nan = float("inf"), float("nan")
+    at = Sk * 2 // 3
+    k[0, :, at, 3], k[1, :, at, 5], k[2, :, 1, 0] = inf, nan, -inf
+    q[3, :, Sq // 2, 1], q[3, :, Sq // 3, 2] = inf, nan
+    v[4, :, 0, 7], v[4, :, 0, 9] = inf, nan                                  # (key 0, which every row gives weight)
+    ref = orc.prefill_reference(q, k, v, causal=causal)
+    got = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=causal, kv_splits=1).float().cpu()
+    assert 0 < int(torch.isnan(ref).any(-1).sum()) < ref[..., 0].numel() and torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    check(torch.where(fine, got, 0.0), torch.where(fine, ref.float(), 0.0))
 
 
 def test_prefill_of_short_heads_without_keys(ops):
