@@ -298,34 +298,39 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(SsmParams<T> p) {
 // Segments are numbered without gaps, sequence by sequence, so that the workgroups that have one are a launch's first: one that has
 // none still holds 66 KB of LDS while it finds out (32 sequences of 1000 tokens, 16 heads, two of three numbers without a segment
 // 199 us, like this 133; 125 where the caller says that nothing need be cut).
-__device__ __forceinline__ int segments_of(const SsmParams<__bf16>& p, int b) {
-    int first, len;
-    seq_rows(p, b, first, len);
-    return len <= max(p.seg_len, p.whole_len) ? len > 0 : (len + p.seg_len - 1) / p.seg_len;
-}
-// Walks the sequences 64 at a time, a lane each; at(e0, n, sum) with the segments of this lane's sequence and of all up to it (of
-// this walk's 64) says whether to go on.
+// Walks the sequences 64 at a time, a lane each: at(e0, rows, sum) with this lane's sequence and the segments of all up to it (of this
+// walk's 64) says whether to go on.
+struct SeqSegments {
+    int first, len, n;           // rows; segments
+};
 template <typename F>
 __device__ __forceinline__ void walk_segments(const SsmParams<__bf16>& p, F&& at) {
     const int lane = threadIdx.x & 63;
     for (int e0 = 0; e0 < p.B; e0 += 64) {
-        const int n = e0 + lane < p.B ? segments_of(p, e0 + lane) : 0;
-        if (!at(e0, n, running_sum(n))) return;
+        SeqSegments q = {0, 0, 0};
+        if (e0 + lane < p.B) {
+            seq_rows(p, e0 + lane, q.first, q.len);
+            q.n = q.len <= max(p.seg_len, p.whole_len) ? q.len > 0 : (q.len + p.seg_len - 1) / p.seg_len;
+        }
+        if (!at(e0, q, running_sum(q.n))) return;
     }
 }
-// The sequence of segment `unit` of the segments that have `skip` behind them in their sequence, its place there and the number of
-// the sequence's first segment; false: there are not so many
-__device__ __forceinline__ bool find_segment(const SsmParams<__bf16>& p, int unit, int skip, int& b, int& place, int& seg0) {
+// The sequence of segment `unit` of the segments that have `skip` behind them in their sequence, its rows, the segment's place
+// there and its number among all; false: there are not so many
+template <int SKIP>
+__device__ __forceinline__ bool find_segment(const SsmParams<__bf16>& p, int unit, int& b, int& first, int& len, int& place, int& seg) {
     bool found = false;
     int before = 0, before_all = 0;
-    walk_segments(p, [&](int e0, int n, int sum) {
-        const int mine = max(n - skip, 0), mine_sum = skip == 0 ? sum : running_sum(mine);
+    walk_segments(p, [&](int e0, const SeqSegments& q, int sum) {
+        const int mine = max(q.n - SKIP, 0), mine_sum = SKIP == 0 ? sum : running_sum(mine);
         const uint64_t m = __builtin_amdgcn_ballot_w64(unit < before + mine_sum);
         if (m != 0) {
             const int at = __builtin_ctzll(m);
             b = e0 + at;
+            first = __builtin_amdgcn_readlane(q.first, at);
+            len = __builtin_amdgcn_readlane(q.len, at);
             place = unit - before - __builtin_amdgcn_readlane(mine_sum - mine, at);
-            seg0 = before_all + __builtin_amdgcn_readlane(sum - n, at);
+            seg = before_all + __builtin_amdgcn_readlane(sum - q.n, at) + place;
             found = true;
             return false;
         }
@@ -382,15 +387,14 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
     const int h = blockIdx.x / p.slices % p.H;
     const int col0 = (blockIdx.x % p.slices) * 64;
     const int unit = blockIdx.x / (p.slices * p.H);
-    int b = unit, place = 0, seg = 0;
-    if constexpr (MODE != kWhole) {
-        if (!find_segment(p, unit, MODE == kSegState ? 1 : 0, b, place, seg)) return;       // (nobody comes after a last one)
-        seg += place;
+    int b = unit, first, len, place = 0, seg = 0;
+    if constexpr (MODE == kWhole) {
+        seq_rows(p, b, first, len);
+        if (len <= 0) return;
+    } else {
+        if (!find_segment<MODE == kSegState ? 1 : 0>(p, unit, b, first, len, place, seg)) return;       // (nobody comes after a last one)
         if (seg >= p.n_segs) return;                     // (sequences that overlap: no scratch beyond the caller's)
     }
-    int first, len;
-    seq_rows(p, b, first, len);
-    if (len <= 0) return;
     bool last = true, alone = true;                      // the sequence's last segment, its only one
     if constexpr (MODE != kWhole) {
         alone = len <= max(p.seg_len, p.whole_len);
@@ -654,16 +658,19 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsmParams<__bf16> p) {
     constexpr int kAhead = 4;
     const int h = blockIdx.x % p.H, b = blockIdx.x / p.H;
     const int64_t size = (int64_t)p.N * p.Pp, at = 4 * (blockIdx.y * 256LL + threadIdx.x);
-    int first, len;
-    seq_rows(p, b, first, len);
-    const int n = segments_of(p, b);
-    if (n <= 1) return;
+    int first = 0, n = 0;
     int64_t seg0 = 0;
-    walk_segments(p, [&](int e0, int, int sum) {
-        const int end = __builtin_amdgcn_readlane(sum, min(b - e0, 63));
-        seg0 += b - e0 <= 63 ? end - n : end;
-        return b - e0 > 63;
+    walk_segments(p, [&](int e0, const SeqSegments& q, int sum) {
+        if (b - e0 > 63) {
+            seg0 += __builtin_amdgcn_readlane(sum, 63);
+            return true;
+        }
+        first = __builtin_amdgcn_readlane(q.first, b - e0);
+        n = __builtin_amdgcn_readlane(q.n, b - e0);
+        seg0 += __builtin_amdgcn_readlane(sum, b - e0) - n;
+        return false;
     });
+    if (n <= 1) return;
     if (at >= size || seg0 + n > p.n_segs) return;
     f32x4 S = {0.f, 0.f, 0.f, 0.f};
     if (p.positions[first] > 0) S = *reinterpret_cast<const f32x4*>(p.ssm_state + ((int64_t)state_slot(p, b) * p.H + h) * size + at);
