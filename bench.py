@@ -327,7 +327,7 @@ def bench_decode_few_sequences(args):
 def bench_decode_loop(args):
     """Decode steps of the KV-cached decoder at the reference's sample model (configures/sample.yaml:
     vocab 10000, context 256, d_model 512, 4 layers, 16 heads, d_ff 1344; random weights), batch 8:
-    launched eagerly (about ten launches per layer from Python) and replayed from a captured HIP graph."""
+    launched eagerly (five launches per layer from Python) and replayed from a captured HIP graph."""
     import torch
     import mi355_attn
 

@@ -10,8 +10,11 @@
 // rotation and the attention.  All of them are a few microseconds of latency in a small model (8 rows, width 512: products 6.1,
 // norms 3.9, rotation 4.1, activation 3.0 us), so fewer launches is what counts there; in a large one the weights' stream is,
 // see weight_stream.hpp.  GPU time of a whole step, this against library products and separate operators: 4 layers of width 512,
-// 8 rows 86 / 181 us, 32 rows 106 / 226; 4 layers of 2048, 8 rows 226 / 382, 32 rows 307 / 378; 2 layers of 4096, 16 rows
-// 297 / 363, 32 rows 378 / 379, which is where the line is drawn (32 rows).  A workgroup takes 32 weight rows; its four wavefronts share k and meet in LDS.
+// 8 rows 84 / 180 us, 32 rows 104 / 225; 4 layers of 2048, 8 rows 212 / 349, 32 rows 284 / 392; 2 layers of 4096, 16 rows
+// 265 / 375, 32 rows 335 / 340.  The line at 32 rows is not where it breaks even but what the ring and the accumulators are laid out
+// for, two tiles of 16 rows: a small model's step doubles behind it (width 512, 33 rows 227 us), a wide one's does not (4096: 350).  What
+// is slower than the library's product by itself is a long k at 17 rows and more, where the ring holds one step (ADD of 4096 x 14336,
+// 32 rows: 34 us against 22).  A workgroup takes 32 weight rows; its four wavefronts share k and meet in LDS.
 #include "common.hpp"
 #include "launch.hpp"
 #include "weight_stream.hpp"

@@ -9,12 +9,13 @@
 
 namespace mi355 {
 
-constexpr int kStreamBytes = 12 * 1024;          // per wavefront: 2 steps of 32 + 16 rows, or one of 32 + 32; three workgroups per compute unit
+// per wavefront: 2 steps of 32 + 16 rows, or one of 32 + 32; three workgroups of four per compute unit, two where a norm's 16 KB come on top
+constexpr int kStreamBytes = 12 * 1024;
 
 // w_off, a_off: byte offsets of this lane's 16 bytes in step 0: rows 8 j + lane / 8 of the weights (32) and of the activations
 // (16 * MT), piece (lane % 8) ^ (lane / 8) of the row's eight, so that the LDS row holds piece q at q ^ (row % 8).
-// k: row length in elements, a multiple of 8; meanwhile() runs when the first steps have been requested; on_rows(t, s, m, fragment) may change a fragment of activations: lane holds row
-// 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
+// k: row length in elements, a multiple of 8; meanwhile() runs when the first steps have been requested; on_rows(t, s, m, fragment) may
+// change a fragment of activations: lane holds row 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
 // acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
 template <int MT, typename G, typename F>
 __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],

@@ -268,7 +268,7 @@ class PagedAttentionEngine:
         self._no_rotation = {d: torch.stack((torch.ones(1, d // 2), torch.zeros(1, d // 2))).to(self.device)
                              for d in {dims[0] for dims in self.cache_dims if dims}} if kv_dtype == "fp8" else None
         self.allocator = BlockAllocator(num_blocks)
-        self.blocks: dict[int, list[int]] = {}      # sequence id -> physical blocks
+        self.blocks: dict[int, list[int]] = {}      # sequence id -> physical blocks (to be read; _reserve adds to both forms)
         self._block_rows: dict[int, array] = {}     # the same as int32 arrays: a table row is one copy, not a conversion per block
         self.lengths: dict[int, int] = {}           # sequence id -> tokens in the cache
         self.state_slots: dict[int, int] = {}       # sequence id -> state slot (models with state layers)
@@ -422,8 +422,8 @@ class PagedAttentionEngine:
         return StaticDecodeStep(batch, self.max_blocks_per_seq, self.device)
 
     def plan_decode_into(self, seq_ids, tokens, static: "StaticDecodeStep") -> DecodePlan:
-        """plan_decode whose tensors (and the new token ids) are written into `static`: one pinned staging
-        buffer, one asynchronous copy on the current stream.  Tables have their full width and
+        """plan_decode whose tensors (and the new token ids) are written into `static`: two pinned staging
+        buffers in turn, one asynchronous copy on the current stream.  Tables have their full width and
         max_context is the context length, so nothing about the step's shapes depends on the data."""
         B = len(seq_ids)
         if B != static.batch or len(tokens) != B:

@@ -245,8 +245,9 @@ class CachedTransformerLM(CachedLM):
         feed-forward weights.  num_blocks sizes the KV pool of every layer (default: max_batch full
         contexts); kv_dtype "fp8" keeps the pool as e4m3 bytes with per-(block, head) scales (half the
         cache bytes per decode step; d_head 64 or 128).  decode_graphs=True replays every decode step
-        after the first of a batch size from a captured HIP graph (about ten launches per layer become one
-        graph launch; the step's tensors then live at fixed addresses and tables have their full width)."""
+        after the first of a batch size from a captured HIP graph (five launches per layer up to 32 sequences, about
+        ten beyond, become one graph launch; the step's tensors then live at fixed addresses and tables have their
+        full width)."""
         self.config = dict(config)
         self.device = torch.device(device)
         self.context_length = config["context_length"]
