@@ -650,7 +650,7 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(MoeParams p, int n_tile
 // gates and their ups) looks through the ids for its expert's pairs itself, and row `pair` of the left and the output matrix
 // belongs to the pair.  The weights are read once for every 32 rows.  What it saves against group + skinny: a launch, and the
 // chain of dependent loads offsets -> order -> rows in front of the first weight.  Bound by the weights' stream (16 experts of
-// 2048 x 1024, 32 tokens: 134 + 67 MB in 31 + 14 us, 4.3 and 4.8 TB/s, where group + skinny took 3 + 34 + 21).
+// 2048 x 1024, 32 tokens: 134 + 67 MB in 31 + 13 us, 4.4 and 5.0 TB/s, where group + skinny took 3 + 34 + 21).
 constexpr int kDirectPairs = 2048;
 template <bool GATE_UP>
 __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int32_t* ids, int n_tiles) {
@@ -799,8 +799,9 @@ __global__ __launch_bounds__(256) void moe_f32_kernel(MoeParams p, int n_tiles, 
 // The 256 x 256 tiles are a fifth faster where they fill whole rounds of the 256 compute units, and lose that to a round that is
 // mostly empty.  With one and a half full tiles per expert or more, an expert's last tile is half full on average: about (pairs / 256
 // + experts / 2) row tiles, give or take sqrt(experts / 12); with fewer most of a tile is padding.  Measured, both products, against
-// 128 x 128 (16 experts of 2048 x 1024, top 4): 3400 tokens (0.95 of two rounds) 197 against 227 us, 8192 (0.85 of five) 454 / 516,
-// 2600 (0.76 of two) 184 / 174; 32 experts of 2048 x 2048: 3400 tokens (0.86 of five) 397 / 477, 512 (64 pairs an expert) 224 / 208.
+// 128 x 128 (16 experts of 2048 x 1024, top 4): 3400 tokens (0.95 of two rounds) 187 against 220 us, 8192 (0.85 of five) 446 / 503,
+// 2600 (0.76 of two) 167 / 168, 2048 (0.63) 159 / 141; 32 experts of 2048 x 2048: 3400 tokens (0.86 of five) 396 / 493, 512 (64 pairs
+// an expert) 224 / 208.
 // With a short k a tile is mostly its beginning and its end (512 x 512, 8 experts, 4096 tokens: 64 / 57).
 static bool wide_pays(const MoeParams& p, bool gate_up) {
     const double n_tiles = (p.n + (gate_up ? 127 : 255)) / (gate_up ? 128 : 256);

@@ -369,8 +369,8 @@ __device__ __forceinline__ void split_bf16(float a, float b, uint32_t& hi, uint3
 // Bound by the chain through a chunk -- three barriers, products that wait for LDS -- with two wavefronts per SIMD (NT 4: 220 registers,
 // 66 KB of LDS per workgroup).  What keeps it short: no branch inside a phase (one around each factor took half the VALU cycles),
 // four accumulators side by side in each product, one wavefront that prepares the next chunk's decays while the others take its
-// share of G, exponentials once per token instead of once per use.  4 sequences of 2048 tokens, 64 heads, state 128: states 50 -> 37
-// us, outputs 136 -> 108.  (Four heads per workgroup with shared B C^T: 108 to 124 before that, but one workgroup per compute unit: a
+// share of G, exponentials once per token instead of once per use.  4 sequences of 2048 tokens, 64 heads, state 128: states 50 -> 33
+// us, outputs 136 -> 105.  (Four heads per workgroup with shared B C^T: 108 to 124 before that, but one workgroup per compute unit: a
 // fifth slower where its rounds do not come out even.)
 enum { kWhole, kSegState, kSegOut };
 template <int NT, int MODE>
