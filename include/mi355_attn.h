@@ -576,7 +576,7 @@ typedef struct mi355_ssm_args {
     int batch, heads, vdim, state, groups, taps, n_slots, dtype;
     float *seg_state, *seg_decay; /* chunked scan in segments: scratch */
     int seg_len;                 /* tokens per segment, 0: none */
-    int whole_len;               /* with seg_len: tokens up to which a sequence is not cut, 0: seg_len */
+    int whole_len;               /* with seg_len: tokens up to which a sequence is not cut (up to seg_len it never is) */
 } mi355_ssm_args;
 int mi355_ssm_prefill(const mi355_ssm_args* args, int scan, void* stream);
 int mi355_ssm_decode(const mi355_ssm_args* args, void* stream);

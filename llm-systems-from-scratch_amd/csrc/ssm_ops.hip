@@ -832,7 +832,7 @@ extern "C" int mi355_ssm_prefill(const mi355_ssm_args* args, int scan, void* str
     if (!args->xbc) return set_error(MI355_EINVAL, "ssm_prefill: null xbc buffer");
     if (!args->cu_seqlens && args->n_rows != args->batch) return set_error(MI355_EINVAL, "ssm_prefill: one row per sequence without cu_seqlens");
     if (scan < MI355_SCAN_AUTO || scan > MI355_SCAN_CHUNKED) return set_error(MI355_EINVAL, "ssm_prefill: unknown scan");
-    if (args->seg_len < 0 || args->seg_len % 64 || args->whole_len < 0 ||
+    if (args->seg_len < 0 || args->seg_len % 64 ||
         (args->seg_len > 0 && (!args->seg_state || !args->seg_decay || (reinterpret_cast<uintptr_t>(args->seg_state) & 15))))
         return set_error(MI355_EINVAL, "ssm_prefill: segments are multiples of 64 tokens and need their buffers");
     if (args->n_rows == 0) return MI355_OK;

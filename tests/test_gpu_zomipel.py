@@ -393,6 +393,40 @@ def test_scan_of_unequal_sequences(ops, longest):
     assert float((state[1].cpu() - S).pow(2).mean().sqrt() / S.pow(2).mean().sqrt()) <= 1.5e-3
 
 
+@pytest.mark.parametrize("segment", [64, 192])
+def test_segments_of_more_sequences_than_lanes(ops, segment):
+    """150 sequences, some empty, long ones in each walk of 64 (the last of all among them): segments are numbered across the walks, their rows
+    against whole sequences (bit for bit where a sequence is one segment) and the long ones' against the oracle."""
+    print(f"case: ssm 150 sequences, segments of {segment}", flush=True)
+    m = dict(heads=3, vdim=16, state=32, groups=1, taps=2)
+    kw = {k: m[k] for k in ("heads", "vdim", "state", "groups")}
+    lens = [(7 * i) % 90 for i in range(150)]
+    lens[3], lens[63], lens[64], lens[100], lens[149] = 500, 193, 64, 1000, 321
+    assert lens.count(0) > 1
+    case, params, xbc_at, dt_at = ssm_case(m, 2, 4, torch.bfloat16)
+    params["neg_a"] = params["neg_a"] * 0.1
+    projs = [rnd(n, case.shape[1], seed=i, dtype=torch.bfloat16) for i, n in enumerate(lens)]
+    pc, sl = {k: v.cuda() for k, v in params.items()}, torch.randperm(150, generator=gen(1)).int().cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    pos = torch.cat([torch.arange(n) for n in lens]).int().cuda()
+    runs = []
+    for seg in (segment, 0):
+        conv, state = ssm_pools(m, 151, torch.bfloat16)
+        got = ops.ssm_mix(torch.cat(projs).cuda(), xbc_at, dt_at, pc, conv, state, sl, pos, cu, segment=seg, **kw)
+        runs.append((torch.split(got, lens), state))
+        assert bool((state[150] == 1e6).all())
+    for i, n in enumerate(lens):
+        (a, sa), (b, sb) = ((g[i], s[int(sl[i])]) for g, s in runs)
+        if n <= segment:
+            assert torch.equal(a, b) and torch.equal(sa, sb), i
+        elif n > 300:
+            want, S = ssm_oracle(m, projs[i], params, xbc_at, dt_at, True)
+            rows_close(a, want, torch.bfloat16, what=f"sequence {i}")
+            assert float((sa.cpu()[..., :m["vdim"]] - S).pow(2).mean().sqrt() / S.pow(2).mean().sqrt()) <= 1.5e-3
+        else:
+            rows_close(a, b.float().cpu(), torch.bfloat16, what=f"sequence {i}")
+
+
 def test_chunked_scan_forgets_and_remembers(ops):
     """Decays from almost none to complete within a token: chunks agree with the token-by-token form."""
     m = SSM[2]
@@ -453,7 +487,7 @@ def test_experts(ops, T, E, top, k, ff, n, tiling, dtype):
 @pytest.mark.parametrize("tiling,T,E,top,k,ff,n", [
     ("direct", 1, 8, 2, 64, 64, 40), ("direct", 33, 4, 1, 192, 128, 72), ("direct", 50, 8, 3, 1088, 192, 130), ("direct", 512, 8, 4, 64, 64, 8),
     ("wide", 1, 2, 1, 64, 64, 40), ("wide", 257, 3, 1, 192, 192, 264), ("wide", 300, 5, 2, 128, 320, 130), ("wide", 1024, 2, 2, 64, 128, 520),
-    ("wide", 300, 70, 3, 64, 64, 40),
+    ("wide", 300, 70, 3, 64, 64, 40), ("wide", 700, 130, 4, 64, 64, 520),
     ("auto", 1024, 2, 2, 1024, 3072, 200)])
 def test_expert_tilings(ops, tiling, T, E, top, k, ff, n):
     """The decode form that finds its pairs itself: one row, edges of 16 and 32 rows, the most pairs it takes, k of one step and of a remainder
