@@ -43,21 +43,24 @@ constexpr int kDsBlock = 4096, kDsKeys = 32, kDqWaves = 4;
 constexpr int kFuPairs = 4;               // pairs of wavefronts of the dK/dV kernel, 32 keys each
 constexpr int kFuCols = 32 * kFuPairs;
 
-struct DsLayout {
-    int n_kb, first, lo, hi;      // key blocks; row tile r has clamp(first + 2 r, 0, n_kb) of them, none up to lo, all from hi on
-    __host__ __device__ __forceinline__ DsLayout(int sq, int sk, bool causal) {
+// (T: int64_t where the number of blocks is asked for, int where it is known to fit)
+template <typename T>
+struct DsLayoutOf {
+    T n_kb, first, lo, hi;        // key blocks; row tile r has clamp(first + 2 r, 0, n_kb) of them, none up to lo, all from hi on
+    __host__ __device__ __forceinline__ DsLayoutOf(T sq, T sk, bool causal) {
         n_kb = (sk + kDsKeys - 1) / kDsKeys;
         first = causal ? ((sk - sq + kBwRows - 1) >> 5) + 1 : n_kb;
         lo = first > 0 ? 0 : (-first >> 1) + 1;
         hi = n_kb > first ? (n_kb - first + 1) >> 1 : 0;
         hi = hi > lo ? hi : lo;
     }
-    __host__ __device__ __forceinline__ int count(int r) const { return r < lo ? 0 : r < hi ? first + 2 * r : n_kb; }
-    __host__ __device__ __forceinline__ int before(int r) const {                  // blocks of the row tiles in front of r
-        const int m = r < lo ? lo : r < hi ? r : hi;
+    __host__ __device__ __forceinline__ T count(T r) const { return r < lo ? 0 : r < hi ? first + 2 * r : n_kb; }
+    __host__ __device__ __forceinline__ T before(T r) const {                      // blocks of the row tiles in front of r
+        const T m = r < lo ? lo : r < hi ? r : hi;
         return (m - lo) * first + m * (m - 1) - lo * (lo - 1) + (r > hi ? (r - hi) * n_kb : 0);
     }
 };
+using DsLayout = DsLayoutOf<int>;
 
 // Loader of a 64-row tile (rows of D bf16, row stride `stride` elements) into swizzled LDS:
 // wavefront w, instruction j covers LDS chunks (w*NI + j)*64 .. +63; rows past `last` re-read row `last`.
@@ -1272,7 +1275,7 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
         out.plan_bytes = round_up(16 + 4 * (int64_t)B, 16) + 8 * (out.k_room + out.q_room);
         out.n_units = Hkv;
     } else {
-        out.ds_room = DsLayout(Sq, Sk, causal).before((int)n_rt);
+        out.ds_room = DsLayoutOf<int64_t>(Sq, Sk, causal).before(n_rt);
         out.n_units = B * Hkv;
     }
     if (out.ds_room * G > 0x7fffffffLL || out.k_room > 0x7fffffffLL || out.q_room > 0x7fffffffLL) return false;

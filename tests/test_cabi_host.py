@@ -307,3 +307,21 @@ def test_workspace_of_the_backward_with_ds():
     assert ws(5000, 4, 4, 200, 200, 128, causal, 1, 1, 500000, 500000) == 0      # more sequences than the plan holds
     assert 3 << 30 < ws(8, 32, 8, 8192, 8192, 128, causal, 0, 1, 0, 0) <= 4 << 30   # in passes
     assert ws(1, 64, 1, 1 << 18, 1 << 18, 128, causal, 0, 1, 0, 0) == 0          # a kv head alone does not fit
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_workspace_of_the_backward_with_ds_at_lengths_beyond_32_bits_of_blocks(causal):
+    """Lengths up to 2^24, with the causal diagonal in the middle and at either end: the blocks of one head counted in Python's integers, or 0
+    where they do not fit."""
+    ws, mode = _lib.load().mi355_prefill_bwd_ds_workspace, _lib.MASK_CAUSAL if causal else _lib.MASK_NONE
+    lengths = [40000, 1 << 18, 1 << 20, 2097152, 2965824, 4194304, 4194368, 1 << 23, 1 << 24]
+    for sq in lengths:
+        for sk in {sq, 200, 1 << 20}:
+            rows, n_kb = -(-sq // 64), -(-sk // 32)
+            first = ((sk - sq + 63) >> 5) + 1 if causal else n_kb
+            blocks = int((first + 2 * torch.arange(rows, dtype=torch.int64)).clamp(0, n_kb).sum())
+            got = ws(1, 1, 1, sq, sk, 128, mode, 0, 1, 0, 0)
+            # (behind the blocks: fp32 shares of dk and dv, 16 at most)
+            assert got == 0 or 0 <= got - blocks * 4096 <= 2 * 16 * sk * 128 * 4 + 4096, (sq, sk, got, blocks)
+            assert got == 0 or blocks * 4096 <= 4 << 30, (sq, sk, got, blocks)
+    assert ws(1, 1, 1, 16384, 16384, 128, mode, 0, 1, 0, 0) > 0
