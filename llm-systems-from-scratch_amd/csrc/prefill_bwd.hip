@@ -1266,7 +1266,7 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
     const bool causal = mask_mode == MI355_MASK_CAUSAL;
     const int64_t G = Hq / Hkv, n_rt = (Sq + kBwRows - 1) / kBwRows, n_kb = (Sk + kDsKeys - 1) / kDsKeys;
     if (packed) {
-        if (B > kPlanSeqs) return false;
+        if (B > kPlanSeqs || total_q <= 0 || total_k <= 0 || total_q > 0x7fffffffLL || total_k > 0x7fffffffLL) return false;
         // row tiles of all sequences, times the most blocks a row tile can have; causal over the same bounds, row tile r has 2 r + 2
         const int64_t tiles = std::max<int64_t>(total_q, Sq) / kBwRows + B;
         out.ds_room = causal && same_bounds ? tiles * (n_rt + 1) : tiles * n_kb;
@@ -1464,13 +1464,11 @@ static int prefill_bwd_common(const void* q, const void* k, const void* v, const
     if (workspace) {
         DsPasses d;
         if (!ds_passes(B, Hq, Hkv, Sq_max, Sk_max, D, mask_mode, cu_seqlens_q != nullptr, cu_seqlens_q == cu_seqlens_k, total_q, total_k, d))
-            return set_error(MI355_EINVAL, "prefill_bwd: no form with a workspace for this call");
+            return set_error(MI355_EINVAL, "prefill_bwd: no form with a workspace for this call (packed: total_q and total_k are the tensors' rows)");
         // (a smaller workspace takes more passes)
         if (d.unit_bytes > 0) d.units_per_pass = (int)std::min<int64_t>(d.units_per_pass, (workspace_bytes - d.plan_bytes - d.part_bytes) / d.unit_bytes);
         if (((uintptr_t)workspace & 255) || workspace_bytes < d.bytes() || d.units_per_pass < 1)
             return set_error(MI355_EINVAL, "prefill_bwd: the workspace is too small or not 256-byte aligned");
-        if (cu_seqlens_q && (total_q <= 0 || total_q > 0x7fffffffLL))
-            return set_error(MI355_EINVAL, "prefill_bwd: total_q must be the rows of the packed queries");
         unsigned char* ws = (unsigned char*)workspace;
         const int rc = D == 128 ? launch_bwd_ds_mode<128>(p, d, mask_mode, total_q, ws, s)
                                 : (D == 64 ? launch_bwd_ds_mode<64>(p, d, mask_mode, total_q, ws, s) : launch_bwd_ds_mode<32>(p, d, mask_mode, total_q, ws, s));

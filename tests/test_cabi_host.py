@@ -305,6 +305,8 @@ def test_workspace_of_the_backward_with_ds():
     assert ws(8, 64, 64, 256, 256, 128, boolean, 0, 1, 0, 0) == 0
     assert ws(1, 4, 4, 128, 128, 128, causal, 0, 1, 0, 0) == 0                   # too little to gain
     assert ws(5000, 4, 4, 200, 200, 128, causal, 1, 1, 500000, 500000) == 0      # more sequences than the plan holds
+    for totals in ((0, 4096), (4096, 0), (-1, 4096), (4096, -1), (1 << 31, 4096), (4096, 1 << 31)):        # rows that no packed tensor has
+        assert ws(4, 8, 8, 1024, 1024, 128, causal, 1, 1, *totals) == 0, totals
     assert 3 << 30 < ws(8, 32, 8, 8192, 8192, 128, causal, 0, 1, 0, 0) <= 4 << 30   # in passes
     assert ws(1, 64, 1, 1 << 18, 1 << 18, 128, causal, 0, 1, 0, 0) == 0          # a kv head alone does not fit
 
