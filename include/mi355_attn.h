@@ -242,7 +242,9 @@ int mi355_prefill_bwd_typed(const void* q, const void* k, const void* v, const v
  * most (several passes where dS of the whole call is larger; any smaller workspace that holds one kv head's takes more passes); 0 where
  * the call has no such form or it is not the faster one.
  * total_q, total_k: rows of the packed tensors (unused in the dense layout); same_bounds: cu_seqlens_q and cu_seqlens_k are one array;
- * packed: cu_seqlens are given.  The workspace must be 256-byte aligned; nothing in it outlives the call. */
+ * packed: cu_seqlens are given.  The workspace must be 256-byte aligned; nothing in it outlives the call.
+ * Packed sequences longer than Sq_max or Sk_max: up to the next multiple of 256 their gradients are computed like all others; longer ones where
+ * the workspace still has room for their dS (it counts with the longest everywhere), else their gradients are zero. */
 int64_t mi355_prefill_bwd_ds_workspace(int B, int Hq, int Hkv, int Sq_max, int Sk_max, int D, int mask_mode, int packed, int same_bounds,
                                        int64_t total_q, int64_t total_k);
 int mi355_prefill_bwd_ds(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, float* delta,

@@ -373,15 +373,17 @@ __global__ __launch_bounds__(2 * kFuPairs * 64, 1) void bwd_dkv_kernel(BwdParams
     }
     const int G = p.Hq / p.Hkv;
     int sq, sk, q_start = 0;
+    int ds_base = 0;                                                    // (DS, packed: negative: no room for the sequence, its gradients are zero)
     int64_t k_base, v_base, dk_base, dv_base;
     if (p.cu_q) {
         q_start = p.cu_q[b];
         const int k_start = p.cu_k[b];
         sq = p.cu_q[b + 1] - q_start;
         sk = p.cu_k[b + 1] - k_start;
-        if constexpr (DS) {                                             // (as the plan counts them: what it leaves room for is never left)
-            sq = min(max(sq, 0), p.Sq);
-            sk = min(max(sk, 0), p.Sk);
+        if constexpr (DS) {                                             // (as the plan counts them)
+            sq = max(sq, 0);
+            sk = max(sk, 0);
+            ds_base = p.ds_base[b];
         }
         k_base = (int64_t)k_start * p.ks[2] + (int64_t)hk * p.ks[1];
         v_base = (int64_t)k_start * p.vs[2] + (int64_t)hk * p.vs[1];
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(2 * kFuPairs * 64, 1) void bwd_dkv_kernel(BwdParams
         // Steps: (query head of the group, row tile), heads innermost; the first key tile of the pair walks
         // its row tiles from the last one down, the second from its first one up, which keeps all workgroups
         // of a (batch, kv head) on the same Q/dO tiles at the same time (they share them through the L2).
-        const int n_steps = G * (DS ? max(0, n_tiles - first_tile - share + p.shares - 1) / p.shares : max(0, n_tiles - first_tile));
+        const int n_steps = DS && ds_base < 0 ? 0 : G * (DS ? max(0, n_tiles - first_tile - share + p.shares - 1) / p.shares : max(0, n_tiles - first_tile));
         // position of a step: first row of its tile and query head within the group; advanced incrementally
         // (steps i, i+1 and i+2 are in flight at any time; no division per step)
         struct Pos {
@@ -586,7 +588,7 @@ __global__ __launch_bounds__(2 * kFuPairs * 64, 1) void bwd_dkv_kernel(BwdParams
         int ds_blocks = 0;                                             // of one query head
         if constexpr (DS) {
             ds_blocks = dsl.before((sq + kBwRows - 1) / kBwRows);
-            const int64_t first = p.cu_q ? (int64_t)p.ds_base[b] * p.n_units * G + (int64_t)(hk - p.unit0) * G * ds_blocks
+            const int64_t first = p.cu_q ? (int64_t)ds_base * p.n_units * G + (int64_t)(hk - p.unit0) * G * ds_blocks
                                          : (int64_t)(b * p.Hkv + hk - p.unit0) * G * ds_blocks;
             ds_head = p.ds + first * kDsBlock;
         }
@@ -715,6 +717,7 @@ struct PlanParams {
     int2* k_jobs;
     int2* q_jobs;
     int k_room, q_room, ds_room;  // entries and blocks (of one head) there is room for
+    int most_q, most_k;           // lengths up to which every sequence has its blocks
     int shift, n_bins;            // costs in steps are binned by cost >> shift
     int total_q;
 };
@@ -762,8 +765,8 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
             __shared__ int bins[kPlanBins], sums[kPlanThreads / 64], lens_q[kPlanSeqs], lens_k[kPlanSeqs];
             const int G = p.Hq / p.Hkv;
             for (int b = tid; b < p.B; b += kPlanThreads) {
-                lens_q[b] = min(max(p.cu_q[b + 1] - p.cu_q[b], 0), p.Sq);
-                lens_k[b] = min(max(p.cu_k[b + 1] - p.cu_k[b], 0), p.Sk);
+                lens_q[b] = max(p.cu_q[b + 1] - p.cu_q[b], 0);
+                lens_k[b] = max(p.cu_k[b + 1] - p.cu_k[b], 0);
             }
             __syncthreads();
             const auto row_tiles = [&](int b) { return (lens_q[b] + kBwRows - 1) / kBwRows; };
@@ -777,15 +780,28 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
                 if (tid == 0) plan.n_jobs[0] = n;
                 return;
             }
-            // dS blocks in front of every sequence; one that would not fit (bounds that do not rise) begins at 0, in room that exists
+            // dS blocks in front of every sequence: first of those of the promised lengths, then, one by one, of longer ones that still fit
+            // (the room counts with the longest everywhere).  What does not fit (and, with bounds that do not rise, anything) has none: -1.
             if (tid < 64) {
                 int before = 0;
+                const auto promised = [&](int b) { return lens_q[b] <= plan.most_q && lens_k[b] <= plan.most_k; };
                 for (int b0 = 0; b0 < p.B; b0 += 64) {
                     const int b = b0 + tid;
-                    const int n = b < p.B ? DsLayout(lens_q[b], lens_k[b], CAUSAL).before(row_tiles(b)) : 0;
-                    const int upto = running_sum(n);
-                    if (b < p.B) plan.ds_base[b] = before + upto <= plan.ds_room ? before + upto - n : 0;
+                    const int n = b < p.B && promised(b) ? DsLayout(lens_q[b], lens_k[b], CAUSAL).before(row_tiles(b)) : 0;
+                    const int upto = running_sum(n), first = before + upto - n;
+                    if (b < p.B) plan.ds_base[b] = promised(b) && first >= 0 && n <= plan.ds_room - first ? first : -1;
                     before += __shfl(upto, 63, 64);
+                }
+                if (before < 0) before = plan.ds_room;
+                for (int b0 = 0; b0 < p.B; b0 += 64) {
+                    uint64_t more = __builtin_amdgcn_ballot_w64(b0 + tid < p.B && !promised(min(b0 + tid, p.B - 1)));
+                    for (; more != 0; more &= more - 1) {
+                        const int b = b0 + __builtin_ctzll(more);
+                        const int64_t n = DsLayoutOf<int64_t>(lens_q[b], lens_k[b], CAUSAL).before((int64_t)row_tiles(b));
+                        if (n > plan.ds_room - before) continue;
+                        if (tid == 0) plan.ds_base[b] = before;
+                        before += (int)n;
+                    }
                 }
             }
             const int n = plan_list(bins, sums, plan.n_bins, p.B, plan.shift, plan.q_jobs, plan.q_room,
@@ -846,6 +862,7 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
     const int id = (int)blockIdx.x / p.n_units, unit = p.unit0 + (int)blockIdx.x % p.n_units;
     int b, set, hk;
     int sq, sk;
+    int ds_base = 0;
     int64_t k_base, dq_base, first;
     if (p.cu_q) {
         if (id >= p.n_jobs[1]) return;
@@ -854,8 +871,9 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
         set = job.y;
         hk = unit;
         const int q_start = p.cu_q[b], k_start = p.cu_k[b];
-        sq = min(max(p.cu_q[b + 1] - q_start, 0), p.Sq);
-        sk = min(max(p.cu_k[b + 1] - k_start, 0), p.Sk);
+        sq = max(p.cu_q[b + 1] - q_start, 0);
+        sk = max(p.cu_k[b + 1] - k_start, 0);
+        ds_base = p.ds_base[b];
         k_base = (int64_t)k_start * p.ks[2] + (int64_t)hk * p.ks[1];
         dq_base = (int64_t)q_start * p.dqs[2];
     } else {
@@ -869,7 +887,7 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
     }
     const DsLayout dsl(sq, sk, CAUSAL);
     const int n_rt = (sq + kBwRows - 1) / kBwRows, ds_blocks = dsl.before(n_rt);
-    first = p.cu_q ? (int64_t)p.ds_base[b] * p.n_units * G + (int64_t)(hk - p.unit0) * G * ds_blocks
+    first = p.cu_q ? (int64_t)ds_base * p.n_units * G + (int64_t)(hk - p.unit0) * G * ds_blocks
                    : (int64_t)(b * p.Hkv + hk - p.unit0) * G * ds_blocks;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -879,7 +897,7 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
     const int mine = min(kDqWaves * set + wave, last_of_set);
     const bool busy = kDqWaves * set + wave <= last_of_set;
     const int rt = mine / G, h = hk * G + mine % G;
-    const int n_steps = dsl.count(last_of_set / G), my_steps = dsl.count(rt);
+    const int n_steps = ds_base < 0 ? 0 : dsl.count(last_of_set / G), my_steps = dsl.count(rt);
     const unsigned char* ds = p.ds + (first + (int64_t)(mine % G) * ds_blocks + dsl.before(rt)) * kDsBlock;
 
     R rd;
@@ -1254,7 +1272,7 @@ struct DsPasses {
     int n_units = 0, units_per_pass = 0;
     int shares = 1;
     int64_t part_rows = 0, part_bytes = 0;       // fp32 shares of dk and dv, behind the lists
-    int64_t ds_room = 0, k_room = 0, q_room = 0;
+    int64_t ds_room = 0, k_room = 0, q_room = 0, most_q = 0, most_k = 0;
     int64_t bytes() const { return plan_bytes + part_bytes + unit_bytes * units_per_pass; }
 };
 
@@ -1264,12 +1282,15 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
                       DsPasses& out) {
     if (mask_mode != MI355_MASK_NONE && mask_mode != MI355_MASK_CAUSAL) return false;
     const bool causal = mask_mode == MI355_MASK_CAUSAL;
-    const int64_t G = Hq / Hkv, n_rt = (Sq + kBwRows - 1) / kBwRows, n_kb = (Sk + kDsKeys - 1) / kDsKeys;
+    const int64_t G = Hq / Hkv, n_rt = (Sq + kBwRows - 1) / kBwRows;
     if (packed) {
         if (B > kPlanSeqs || total_q <= 0 || total_k <= 0 || total_q > 0x7fffffffLL || total_k > 0x7fffffffLL) return false;
-        // row tiles of all sequences, times the most blocks a row tile can have; causal over the same bounds, row tile r has 2 r + 2
-        const int64_t tiles = std::max<int64_t>(total_q, Sq) / kBwRows + B;
-        out.ds_room = causal && same_bounds ? tiles * (n_rt + 1) : tiles * n_kb;
+        // row tiles of all sequences, times the most blocks a row tile can have; causal over the same bounds, row tile r has 2 r + 2.
+        // (Lengths up to the next multiple of 256: as far as the form without a workspace reaches behind a promise that is too small.)
+        out.most_q = round_up(Sq, kBwCols);
+        out.most_k = round_up(Sk, kBwCols);
+        const int64_t tiles = std::max(total_q, out.most_q) / kBwRows + B;
+        out.ds_room = tiles * (causal && same_bounds ? out.most_q / kBwRows + 1 : out.most_k / kDsKeys);
         out.k_room = std::max<int64_t>(total_k, Sk) / kFuCols + B;
         out.q_room = (tiles * G + kDqWaves - 1) / kDqWaves + B;
         out.plan_bytes = round_up(16 + 4 * (int64_t)B, 16) + 8 * (out.k_room + out.q_room);
@@ -1321,6 +1342,8 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
         plan.k_room = (int)d.k_room;
         plan.q_room = (int)d.q_room;
         plan.ds_room = (int)d.ds_room;
+        plan.most_q = (int)std::min<int64_t>(d.most_q, 0x7fffffff);
+        plan.most_k = (int)std::min<int64_t>(d.most_k, 0x7fffffff);
         const int most = std::max(p.Sq, p.Sk) / kBwRows + 1;                      // (costs count row tiles, or pairs of dS blocks)
         while (most >> plan.shift >= kPlanBins) ++plan.shift;
         plan.n_bins = (most >> plan.shift) + 1;

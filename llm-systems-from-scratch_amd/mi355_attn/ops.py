@@ -513,7 +513,8 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, cau
     B = cu_seqlens_q.numel() - 1
     # max_seqlen_* are the caller's promise about the longest sequence (they are on the host, the lengths are not).
     # What can be checked without reading device memory is checked here; a sequence longer than the promise is
-    # still computed in full by the kernel (its workgroups walk on through the remaining query tiles).
+    # still computed in full by the kernel (its workgroups walk on through the remaining query tiles).  The gradients count on it: they are
+    # right up to the promise's next multiple of 256.
     max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
     if (Tq and max_seqlen_q < 1) or (Tk and max_seqlen_k < 1):
         raise ValueError("max_seqlen_q and max_seqlen_k must be at least 1 when there are tokens")

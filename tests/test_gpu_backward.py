@@ -518,6 +518,38 @@ def test_backward_with_ds_in_memory_in_passes(ops, monkeypatch, packed):
     _same_gradients(*_both_forms(ops, monkeypatch, [420] * 3, [420] * 3, 28, 14, True, packed, workspace_part=0.45))
 
 
+def _packed_gradients(ops, lens_q, lens_k, max_q, max_k, causal):
+    cu_q = torch.tensor([0] + torch.tensor(lens_q).cumsum(0).tolist(), dtype=torch.int32).cuda()
+    cu_k = cu_q if lens_k is None else torch.tensor([0] + torch.tensor(lens_k).cumsum(0).tolist(), dtype=torch.int32).cuda()
+    Tq, Tk = sum(lens_q), sum(lens_k or lens_q)
+    leaves = [rnd(T, H, 128, seed=430 + i, scale=0.5).cuda().requires_grad_() for i, (T, H) in enumerate(((Tq, 4), (Tk, 2), (Tk, 2)))]
+    out = ops.flash_attn_varlen_prefill(*leaves, cu_q, cu_k, max_q, max_k, causal=causal)
+    return torch.autograd.grad(out, leaves, rnd(Tq, 4, 128, seed=433, scale=0.5).cuda())
+
+
+@pytest.mark.parametrize("lens_q,lens_k,max_q,max_k,causal", [
+    ([420, 100], None, 320, 420, True), ([420, 100], None, 420, 300, True), ([420, 100], None, 260, 257, False), ([512, 512, 512], None, 257, 257, True),
+    ([300, 200], [500, 333], 260, 500, True), ([300, 200], [500, 333], 300, 460, False)])
+def test_backward_with_ds_in_memory_promises_that_are_too_small(ops, lens_q, lens_k, max_q, max_k, causal):
+    """Sequences longer than max_seqlen_*, up to its next multiple of 256: the gradients of the right promise, all rows of them."""
+    print(f"case: short promises {lens_q} {lens_k} {max_q} {max_k} {causal}", flush=True)
+    torch.full((1 << 26,), float("nan"), device="cuda")              # (what is not written shows)
+    short = _packed_gradients(ops, lens_q, lens_k, max_q, max_k, causal)
+    _same_gradients(short, _packed_gradients(ops, lens_q, lens_k, max(lens_q), max(lens_k or lens_q), causal))
+
+
+def test_backward_with_ds_in_memory_of_sequences_far_beyond_the_promise(ops):
+    """A sequence that dS has no room for gets gradients of zero; one beyond the promise that fits, and those that keep it, get theirs."""
+    lens = [700, 30, 500, 200]
+    torch.full((1 << 26,), float("nan"), device="cuda")
+    got = _packed_gradients(ops, lens, None, 256, 256, True)
+    want = [t.clone() for t in _packed_gradients(ops, lens, None, 700, 700, True)]
+    for t in want:
+        t[:700] = 0
+    _same_gradients(got, want)
+    assert all(bool((t[:700] == 0).all()) for t in got)
+
+
 @pytest.mark.parametrize("Sq,Sk", [(1, 1), (31, 33), (64, 64), (65, 40), (128, 129), (129, 256), (256, 255), (256, 256)])
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("causal", [True, False])
