@@ -943,6 +943,10 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
         for (int i = 0; i < NDT; ++i)
 #pragma unroll
             for (int j = 0; j < 16; ++j) dq[t][i][j] = 0.f;
+    // Column n of half t is row 32 t + my_row of the sequence.  From step `diagonal` on some row does not see all keys of the step: dS is zero there
+    // unless its dP overflowed (0 * inf), so it is set to zero here, where there is time (the dK/dV kernel takes 5 % longer with it).
+    const int my_row = kBwRows * rt + 16 * (n >> 4) + 8 * ((n >> 2) & 1) + 4 * ((n >> 3) & 1) + (n & 3);
+    const int diagonal = (kBwRows * rt + sk - sq + 1) >> 5;
     if (n_steps > 0) {
         issue(0, 0);
         issue(1, 1);
@@ -960,6 +964,19 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
 #pragma unroll
                     for (int t = 0; t < 2; ++t)
                         w[t] = join_bf16x8(lds_read_tr16(d_lds + 2048 * t + ds_off[c][0]), lds_read_tr16(d_lds + 2048 * t + ds_off[c][1]));
+                    if (CAUSAL && step >= diagonal) {
+                        const int lim = my_row + sk - sq - 32 * step - 16 * c - 4 * kg;         // the last of these 16 keys (less 4 kg) that this lane's row of half 0 sees
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            u32x4 x = __builtin_bit_cast(u32x4, w[t]);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {                // elements 2 i and 2 i + 1: keys 8 (i / 2) + 2 (i % 2) and the next one
+                                const int key = 8 * (i >> 1) + 2 * (i & 1) - 32 * t;
+                                x[i] &= (key <= lim ? 0xffffu : 0u) | (key + 1 <= lim ? 0xffff0000u : 0u);
+                            }
+                            w[t] = as_bf16x8(x);
+                        }
+                    }
 #pragma unroll
                     for (int dt = 0; dt < NDT; ++dt) {
                         const bf16x8 a = join_bf16x8(lds_read_tr16(k_lds + 16 * c * kRow + rd.tr_off[0][dt]), lds_read_tr16(k_lds + 16 * c * kRow + rd.tr_off[1][dt]));
@@ -973,10 +990,10 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
         wait_vmcnt<0>();
     }
     if (!busy) return;
-    // store: column n of half t is row 32 t + 16 (n / 16) + 8 (n / 4 % 2) + 4 (n / 8 % 2) + n % 4 of the tile, d = 32 dt + 8 (i / 4) + 4 kg + i % 4
+    // store: d = 32 dt + 8 (i / 4) + 4 kg + i % 4
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int qi = kBwRows * rt + 32 * t + 16 * (n >> 4) + 8 * ((n >> 2) & 1) + 4 * ((n >> 3) & 1) + (n & 3);
+        const int qi = my_row + 32 * t;
         if (qi >= sq) continue;
         const int64_t row = dq_base + (int64_t)qi * p.dqs[2] + (int64_t)h * p.dqs[1];
 #pragma unroll

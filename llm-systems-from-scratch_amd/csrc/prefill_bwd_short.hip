@@ -130,9 +130,9 @@ __global__ __launch_bounds__(NWV * 64, D == 32 ? 4 : 2) void bwd_short_kernel(Bw
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     const int i = 2 * j + e;
-                    float x = fast_exp2(fmaf(s_acc[i], p.scale_log2, -my_lse));
-                    if constexpr (decltype(masked_c)::value) x = 8 * (i >> 2) + (i & 3) <= lim ? x : 0.f;
-                    ds[e] = x * dp[i];
+                    ds[e] = fast_exp2(fmaf(s_acc[i], p.scale_log2, -my_lse)) * dp[i];
+                    // (behind the product: dP of a key that the row does not see may have overflowed)
+                    if constexpr (decltype(masked_c)::value) ds[e] = 8 * (i >> 2) + (i & 3) <= lim ? ds[e] : 0.f;
                 }
                 dsw[j >> 2][j & 3] = pack_bf16(ds[0], ds[1]);
             }
@@ -167,16 +167,21 @@ __global__ __launch_bounds__(NWV * 64, D == 32 ? 4 : 2) void bwd_short_kernel(Bw
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4*>(lse_l + 32 * t + 8 * j + 4 * kg);
-                float x[4];
+                float x[4], ds[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     x[e] = fast_exp2(fmaf(s_acc[4 * j + e], p.scale_log2, -l4[e]));
-                    if constexpr (decltype(masked_c)::value) x[e] = 8 * j + e >= lim ? x[e] : 0.f;
+                    ds[e] = x[e] * dp[4 * j + e];
+                    if constexpr (decltype(masked_c)::value) {
+                        const bool keep = 8 * j + e >= lim;
+                        x[e] = keep ? x[e] : 0.f;
+                        ds[e] = keep ? ds[e] : 0.f;
+                    }
                 }
                 pw[j >> 1][2 * (j & 1)] = pack_bf16(x[0], x[1]);
                 pw[j >> 1][2 * (j & 1) + 1] = pack_bf16(x[2], x[3]);
-                dsw[j >> 1][2 * (j & 1)] = pack_bf16(x[0] * dp[4 * j], x[1] * dp[4 * j + 1]);
-                dsw[j >> 1][2 * (j & 1) + 1] = pack_bf16(x[2] * dp[4 * j + 2], x[3] * dp[4 * j + 3]);
+                dsw[j >> 1][2 * (j & 1)] = pack_bf16(ds[0], ds[1]);
+                dsw[j >> 1][2 * (j & 1) + 1] = pack_bf16(ds[2], ds[3]);
             }
             update(dv, do_l + 32 * t * kRow, pw);
             update(dk, q_l + 32 * t * kRow, dsw);

@@ -518,6 +518,30 @@ def test_backward_with_ds_in_memory_in_passes(ops, monkeypatch, packed):
     _same_gradients(*_both_forms(ops, monkeypatch, [420] * 3, [420] * 3, 28, 14, True, packed, workspace_part=0.45))
 
 
+@pytest.mark.parametrize("D,B,H", [(128, 2, 3), (64, 2, 3), (32, 2, 3), (64, 26, 16), (32, 13, 16)])
+def test_backward_of_a_key_whose_dp_overflows_in_rows_that_do_not_see_it(ops, D, B, H):
+    """dO . v of a key behind the diagonal is beyond fp32 (1e15 * 1e25 * D): nothing that a row's dQ adds.  With dS in memory (few heads) and in
+    the kernel of short heads (many), where dK has nothing of it either."""
+    print(f"case: unseen overflow D={D} {B}x{H}", flush=True)
+    S, at = 200, 150
+    q, k, v, dout = (rnd(B, H, S, D, seed=440 + i) for i in range(4))
+    v[:, :, at] *= 1e25
+    dout[:, :, :at] *= 1e15
+    dout[:, :, at:] *= 1e-25
+    leaves = [t.cuda().requires_grad_() for t in (q, k, v)]
+    grads = torch.autograd.grad(ops.flash_attn_prefill(*leaves, causal=True), leaves, dout.cuda())
+    wide = [t[:1].double().requires_grad_() for t in (q, k, v)]
+    scores = (wide[0] @ wide[1].transpose(-1, -2) / D ** 0.5).masked_fill(~torch.ones(S, S, dtype=torch.bool).tril(), -float("inf"))
+    want = torch.autograd.grad(torch.softmax(scores, -1) @ wide[2], wide, dout[:1].double())
+    for name, got, ref in zip(("dq", "dk", "dv"), grads, want):
+        if name == "dk" and B * H < 200:                            # (there dK has such a key: NaN)
+            continue
+        assert bool(torch.isfinite(got).all()), name
+        for part in (slice(0, at), slice(at, at + 1), slice(at + 1, S)):                    # (sizes of their own)
+            size = ref[:, :, part].abs().max()
+            check_grad(name, got[:1, :, part].double().cpu() / size, ref[:, :, part] / size)
+
+
 def _packed_gradients(ops, lens_q, lens_k, max_q, max_k, causal):
     cu_q = torch.tensor([0] + torch.tensor(lens_q).cumsum(0).tolist(), dtype=torch.int32).cuda()
     cu_k = cu_q if lens_k is None else torch.tensor([0] + torch.tensor(lens_k).cumsum(0).tolist(), dtype=torch.int32).cuda()
