@@ -63,10 +63,23 @@ class CachedLM:
     def _token_list(self, tokens) -> list[int]:
         """_token_ids as a list; a list of ints is looked at as it is."""
         if type(tokens) is not list or not all(type(t) is int for t in tokens):
-            return self._token_ids(tokens).tolist()
+            tokens = self._token_ids(tokens).tolist()
         if tokens and not 0 <= min(tokens) <= max(tokens) < self.vocab_size:
             raise ValueError(f"token ids must be in 0..{self.vocab_size - 1}")
         return tokens
+
+    @staticmethod
+    def _row_ids(rows, n):
+        """Positions among n rows as torch indexes them: int64, negative ones count from the end.  Those on the host are checked; those on the GPU are
+        not looked at (the step would wait for them): what is out of range comes out as some row that is there."""
+        rows = torch.as_tensor(rows, dtype=torch.int64).reshape(-1)
+        if rows.numel() == 0 or n == 0:
+            return rows
+        if rows.is_cuda:
+            return rows.remainder(n)
+        if not -n <= int(rows.min()) <= int(rows.max()) < n:
+            raise IndexError(f"rows must be in {-n}..{n - 1}")
+        return torch.where(rows < 0, rows + n, rows)
 
     # ---- sequence-level API ---------------------------------------------------------------------
     def new_sequence(self) -> int:
@@ -83,10 +96,14 @@ class CachedLM:
         next portions of running ones.  Returns next-token logits (n_seq, vocab) fp32, the logits of every packed
         position (sum(len), vocab) with all_logits=True, or those of the packed positions `rows`."""
         toks = [self._token_ids(p) for p in prompts]
-        plan = self.engine.plan_prefill(list(seq_ids), [int(t.numel()) for t in toks])
-        ids = torch.cat(toks).to(self.device)
+        lens = [int(t.numel()) for t in toks]
         if rows is not None:
-            out_rows = torch.as_tensor(rows, dtype=torch.int64).reshape(-1).to(self.device)
+            rows = self._row_ids(rows, sum(lens))
+        plan = self.engine.plan_prefill(list(seq_ids), lens)
+        ids = torch.cat(toks)
+        ids = (ids.remainder(self.vocab_size) if ids.is_cuda else ids).to(self.device)
+        if rows is not None:
+            out_rows = rows.to(self.device)
         else:
             out_rows = None if all_logits else plan.last_rows
         return self._forward(ids, plan, self.engine.attend_prefill, out_rows)
@@ -96,7 +113,9 @@ class CachedLM:
         seq_ids = list(seq_ids)
         if self.decode_graphs:
             return self._decode_graphed(seq_ids, self._token_list(tokens))
-        ids = self._token_ids(tokens).to(self.device)
+        ids = self._token_ids(tokens)
+        # (up to MAX_LINEAR_ROWS of them rows_linear cuts to the vocabulary)
+        ids = (ids.remainder(self.vocab_size) if ids.is_cuda and ids.numel() > ops.MAX_LINEAR_ROWS else ids).to(self.device)
         if ids.numel() != len(seq_ids):
             raise ValueError("one token per sequence expected")
         plan = self.engine.plan_decode(seq_ids)
@@ -108,8 +127,10 @@ class CachedLM:
         sequence's last).  A step of one token for each of a few running sequences goes through `decode`."""
         seq_ids = list(seq_ids)
         if all(len(t) == 1 and self.engine.lengths[s] > 0 for s, t in zip(seq_ids, tokens)) and len(seq_ids) <= self.engine.max_batch:
+            if rows is not None:
+                rows = self._row_ids(rows, len(seq_ids))
             logits = self.decode(seq_ids, [int(t[0]) for t in tokens])
-            return logits if rows is None else logits[torch.as_tensor(rows, dtype=torch.int64).to(self.device)]
+            return logits if rows is None else logits[rows.to(self.device)]
         return self.prefill(seq_ids, tokens, rows=rows)
 
     def _decode_graphed(self, seq_ids, tokens):

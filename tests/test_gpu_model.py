@@ -357,6 +357,48 @@ def test_decode_across_the_row_limit_of_the_fused_layers(ops, d_ff, graphs):
         model.free_sequence(s)
 
 
+@pytest.mark.parametrize("n_tokens", [20, 50, 200, 1100])
+def test_rows_of_a_prompt_are_indexed_like_torch_indexes(ops, n_tokens):
+    """On either side of the sizes whose linear layers take row numbers: negative positions count from the end, none are few enough, rows that
+    are not there are refused before anything is reserved; ids and rows may be on the GPU."""
+    print(f"case: rows of {n_tokens} tokens", flush=True)
+    cfg = dict(CFG, context_length=1200)
+    model = ops.CachedTransformerLM(cfg, _bf16_params(cfg, seed=41), max_batch=4)
+    ids = torch.randint(0, cfg["vocab_size"], (n_tokens,), generator=torch.Generator().manual_seed(42))
+    parts = [ids[:n_tokens // 3], ids[n_tokens // 3:]]
+
+    def logits(rows=None, parts=parts):
+        sids = [model.new_sequence() for _ in parts]
+        try:
+            return model.prefill(sids, parts, **(dict(all_logits=True) if rows is None else dict(rows=rows)))
+        finally:
+            for s in sids:
+                model.free_sequence(s)
+
+    every = logits()
+    assert every.shape[0] == n_tokens
+    for rows in ([-1], [0, -n_tokens, n_tokens - 1, -2], list(range(-min(n_tokens, 90), 0)), torch.tensor([3, -3])):
+        picked = torch.as_tensor(rows)
+        _logit_close(logits(rows)[None], every[picked.cuda()][None].cpu())
+        _logit_close(logits(picked.cuda())[None], every[picked.cuda()][None].cpu())
+        _logit_close(logits(rows, [p.cuda() - cfg["vocab_size"] for p in parts])[None], every[picked.cuda()][None].cpu())      # (the same ids)
+    assert logits([]).shape == (0, cfg["vocab_size"])
+    free = model.engine.allocator.num_free
+    for rows in ([n_tokens], [0, -n_tokens - 1]):
+        with pytest.raises(IndexError):
+            logits(rows)
+    sids = [model.new_sequence() for _ in range(2)]
+    model.prefill(sids, [[1, 2], [3]])
+    one = model.step(sids, [[4], [5]], rows=[-1, 0])
+    assert one.shape == (2, cfg["vocab_size"])
+    with pytest.raises(IndexError):
+        model.step(sids, [[4], [5]], rows=[2])
+    assert model.engine.lengths[sids[0]] == 3                         # (nothing was appended)
+    for s in sids:
+        model.free_sequence(s)
+    assert model.engine.allocator.num_free == free
+
+
 def test_from_pretrained_reads_reference_files(ops, tmp_path):
     print("case: from_pretrained", flush=True)
     params = mo.random_lm_params(CFG, seed=22)
