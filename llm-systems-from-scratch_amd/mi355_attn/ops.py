@@ -8,6 +8,8 @@ arbitrary batch/head/seq strides (the reference's V is a strided view of the
 from __future__ import annotations
 
 import math
+import os
+import warnings
 
 import torch
 
@@ -15,8 +17,10 @@ from . import _lib
 
 try:
     from . import _calls as _native       # the calls in their plain form (csrc/calls.cpp); each gives None where it is not that
-except ImportError:                        # (the serving library is built without it)
+except ImportError as _error:              # (the serving library is built without it)
     _native = None
+    if os.path.exists(_lib.LIB_PATH):
+        warnings.warn(f"the native calls are not there, every call goes through Python ({_error})", RuntimeWarning)
 
 _BLOCK = 16
 

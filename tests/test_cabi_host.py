@@ -3,6 +3,8 @@ bad arguments before touching a GPU; host-side operator validation; workload gen
 import ctypes as C
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -327,3 +329,21 @@ def test_workspace_of_the_backward_with_ds_at_lengths_beyond_32_bits_of_blocks(c
             assert got == 0 or 0 <= got - blocks * 4096 <= 2 * 16 * sk * 128 * 4 + 4096, (sq, sk, got, blocks)
             assert got == 0 or blocks * 4096 <= 4 << 30, (sq, sk, got, blocks)
     assert ws(1, 1, 1, 16384, 16384, 128, mode, 0, 1, 0, 0) > 0
+
+
+@pytest.mark.parametrize("library,calls,warns", [(True, b"not a library", True), (True, None, True), (False, None, False)])
+def test_native_calls_that_do_not_load_are_reported(tmp_path, library, calls, warns):
+    """A module of native calls that is broken or missing beside the full library is said once; the serving library comes without one."""
+    package = os.path.dirname(mi355_attn.__file__)
+    copy = tmp_path / "mi355_attn"
+    copy.mkdir()
+    for name in os.listdir(package):
+        if name.endswith(".py") or (library and name == "libmi355attn.so"):
+            (copy / name).symlink_to(os.path.join(package, name))
+    if calls is not None:
+        (copy / "_calls.so").write_bytes(calls)
+    # (symlinks: the package's own folder is the one it was found in)
+    run = subprocess.run([sys.executable, "-c", "import mi355_attn; print(mi355_attn.ops._native)"], env=dict(os.environ, PYTHONPATH=str(tmp_path)),
+                         cwd=tmp_path, capture_output=True, text=True, timeout=110)
+    assert run.returncode == 0 and run.stdout.strip() == "None", run.stderr
+    assert ("native calls are not there" in run.stderr) == warns, run.stderr
