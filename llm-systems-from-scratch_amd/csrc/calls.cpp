@@ -232,10 +232,11 @@ Tensor bf16(const Tensor& t) { return t.scalar_type() == kBF16 ? t : t.to(kBF16)
 bool forward_rounded(Tensor& q, Tensor& k, Tensor& v, const Shape& s, Tensor& out, Tensor& lse) {
     Tensor* t[3] = {&q, &k, &v};
     const int f32 = f32_bits(q, k, v);
-    if (f32 == 0 || !(s.scale > 0) || !mi355_prefill_fwd_rounds(s.Hq, s.Hkv, s.Sq, s.Sk, s.D, s.mode())) return false;
+    if (f32 == 0 || !((float)s.scale > 0.f) || !mi355_prefill_fwd_rounds(s.Hq, s.Hkv, s.Sq, s.Sk, s.D, s.mode())) return false;
     Tensor r[3];
     for (int i = 0; i < 3; ++i) {
-        if (!whole_rows(*t[i])) return false;
+        const int64_t row = t[i]->stride(2);               // (a conversion in front brings rows together that are further apart)
+        if (!whole_rows(*t[i]) || row <= 0 || row >= (1 << 24)) return false;
         if (t[i]->scalar_type() != kF32) continue;
         r[i] = at::empty_like(*t[i], t[i]->options().dtype(kBF16));
         if (!whole_rows(r[i])) return false;

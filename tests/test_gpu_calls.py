@@ -80,6 +80,24 @@ def test_dense(ma, monkeypatch, B, Hq, Hkv, Sq, Sk, D, types, grad, causal):
         both(monkeypatch, call, types != (F32,) * 3 and not (form == "broadcast" and types[1] == F32 and Hkv > 1), f"{form} {B} {Hq} {Sq} {Sk} {D} {types}")
 
 
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_dense_float32_rows_far_apart(ma, which):
+    """Rows of 2^24 elements and more: the rounding forward does not take them, the conversion in front of the general one brings them together."""
+    t = [rnd(1, 2, 3, 32, seed=50 + i, dtype=F32 if i == which else BF) for i in range(3)]
+    far = torch.empty_strided((1, 2, 3, 32), (64, 32, 1 << 24, 1), dtype=F32, device="cuda")
+    far.copy_(t[which])
+    g = rnd(1, 2, 3, 32, seed=54)
+
+    def run(x):
+        leaves = [t[i] if i != which else x for i in range(3)]
+        leaves = [y.detach().requires_grad_() for y in leaves]
+        out = ma.flash_attn_prefill(*leaves, causal=True)
+        return [out, *torch.autograd.grad(out, leaves, g)]
+
+    for a, b in zip(run(far), run(t[which])):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("lens,Hq,Hkv,D,grad,causal,window", [
     ([1, 64, 0, 200], 4, 2, 64, False, True, 0), ([300, 31, 1], 4, 4, 128, True, True, 0), ([130, 40], 2, 1, 32, True, False, 0), ([70, 900], 2, 1, 128, False, True, 64)])
 def test_packed(ma, monkeypatch, lens, Hq, Hkv, D, grad, causal, window):
