@@ -1075,13 +1075,16 @@ extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max,
             const double wgs = (double)n_pairs * Hq * B * n;
             return rounds(wgs) * (keys_pair / n / kBN * (wgs >= 0.75 * n_cu ? 1.45 : 1.25) + 5.0 * halves);
         };
-        // Partial rows of launches that leave compute units without work stay in the caches: 6 TB/s each way and 4 us for the merge.  Against the
-        // best of 1 to 32 shares over 54 calls of few heads this costs 3 % on average, the 8-wavefront kernel's figures cost 8.  Us unsplit,
-        // with what those chose and with what these choose: 2 x 3247 tokens, 4 heads 73, 73, 52; one of 4096, 8 heads 82, 82, 65; one of 8192, 2
-        // heads 153, 69, 60; 3 x 3860, one head 81, 48, 43; 9 portions of 3931 rows, one head 95, 95, 80.
-        const auto merged = [&](int n) { return 4.0 + 2.0 * ((double)total_q_rows * Hq * (D + 1) * 4.0 * n) / 6.0e6; };
+        // Partial rows of launches that leave compute units without work stay in the caches: 6 TB/s each way and 4 us for the merge.  Us unsplit,
+        // with what the 8-wavefront kernel's figures chose and with what these choose: one of 4096 tokens, 8 heads 87, 87, 72; one of 8192, 2 heads
+        // 153, 71, 64.  These are for whole prompts of one length that is a multiple of 64.  Others end in tiles that run in ordinary code, about 5
+        // us each one behind the other whatever the share, so that short ones gain nothing (722 tokens, one head, unmasked 35 us, in four shares 44;
+        // 2 x 2044, one head, six shares 33, eight 40); and that take the largest scores for their references, which a share of one or two
+        // tiles at the end does for fewer of them (2 x 510 tokens unmasked, error against 64 bits 0.00226, in three shares 0.00228).
+        const bool whole = Sk_max % kBN == 0 && Sq_max == Sk_max && total_q_rows == (int64_t)B * Sq_max;
+        const auto merged = [&](int n) { return whole ? 4.0 + 2.0 * ((double)total_q_rows * Hq * (D + 1) * 4.0 * n) / 6.0e6 : partials(n); };
         plain = time_of(1);
-        double best = plain * 0.9;                    // a split must win clearly
+        double best = plain * (whole ? 0.9 : 0.85);   // a split must win clearly
         for (int n : kCandidates) {
             if (keys_single / kBN / n < 2.0) break;   // at least two tiles per share and query tile
             const double t = time_of(n) + merged(n);
