@@ -510,7 +510,8 @@ __device__ __forceinline__ bool find_wide_tile(const MoeParams& p, const WideTil
 // NF 2: a quarter of such a tile, 128 x 128, in the same way.
 // 32768 pairs, 16 equal experts, us for k 1024 / 2048 / 4096, two buffers that change hands at three quarters of a step before, the ring now:
 // gate and up (1024 columns) 133 / 209 / 438 -> 135 / 210 / 403, down (2048 columns) 136 / 256 / 484 -> 128 / 232 / 418 (1.3 PFLOP/s).  With no
-// request in the loop k 4096 takes 346 of them: that is the MFMAs at the clock they are held at.
+// request in the loop k 4096 takes 346 of them: that is the MFMAs at the clock they are held at.  (So the ring gives something to gate and up only for a
+// long k; with unequal experts, k 2048, what they gain is the order of the tiles and the last round's quarters: 1.04 PFLOP/s, down with k 1024 0.83.)
 // (One workgroup per compute unit that goes on to its next tile, its first steps requested in front of this one's results: all
 // workgroups end their tiles at the same time then, and nobody's MFMAs run beside the stores; gate and up 254, down 236.)
 __device__ __forceinline__ int wide_swz(int row) { return (((row >> 1) & 3) << 1) | ((row >> 3) & 1); }       // (banks repeat every 256 bytes)

@@ -94,7 +94,7 @@ class CachedLM:
     def prefill(self, seq_ids, prompts, *, all_logits: bool = False, rows=None):
         """Runs the prompts (lists / 1-D tensors of token ids, each 1..context_length long) of new sequences, or the
         next portions of running ones.  Returns next-token logits (n_seq, vocab) fp32, the logits of every packed
-        position (sum(len), vocab) with all_logits=True, or those of the packed positions `rows`."""
+        position (sum(len), vocab) with all_logits=True, or those of the packed positions `rows` (negative: from the end)."""
         toks = [self._token_ids(p) for p in prompts]
         lens = [int(t.numel()) for t in toks]
         if rows is not None:
