@@ -1298,6 +1298,9 @@ static int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mode, bool packed, bool same_bounds, int64_t total_q, int64_t total_k,
                       DsPasses& out) {
     if (mask_mode != MI355_MASK_NONE && mask_mode != MI355_MASK_CAUSAL) return false;
+    // Heads that the short kernel takes are one launch there, whatever their number.  256 tokens, head size 32, 8 / 64 / 128 heads: 9, 9, 10 us, here
+    // 20, 21, 22; head size 64, 8 / 64 / 192 heads: 13, 14, 19 / 24, 25, 37 (the form without a workspace, before: 28, 29, 33).
+    if (!packed && prefill_bwd_short_takes(Hq, Hkv, Sq, Sk, D, mask_mode)) return false;
     const bool causal = mask_mode == MI355_MASK_CAUSAL;
     const int64_t G = Hq / Hkv, n_rt = (Sq + kBwRows - 1) / kBwRows;
     if (packed) {
@@ -1514,7 +1517,7 @@ static int prefill_bwd_common(const void* q, const void* k, const void* v, const
                                 : (D == 64 ? launch_bwd_ds_mode<64>(p, d, mask_mode, total_q, ws, s) : launch_bwd_ds_mode<32>(p, d, mask_mode, total_q, ws, s));
         return rc == 0 ? MI355_OK : set_error(rc, hipGetErrorString((hipError_t)rc));
     }
-    if (prefill_bwd_short_takes(p, D, mask_mode)) {
+    if (!p.cu_q && prefill_bwd_short_takes(Hq, Hkv, Sq_max, Sk_max, D, mask_mode)) {
         const int rc = launch_prefill_bwd_short(p, D, mask_mode, s);
         return rc == 0 ? MI355_OK : set_error(rc, hipGetErrorString((hipError_t)rc));
     }

@@ -53,7 +53,7 @@ __device__ __forceinline__ void store_grad4(void* grad, bool f32, int64_t at, fl
 }
 
 // Up to 256 queries and keys at head sizes 32 and 64, dense layout, as many key heads as query heads: prefill_bwd_short.hip.
-bool prefill_bwd_short_takes(const BwdParams& p, int D, int mask_mode);
+bool prefill_bwd_short_takes(int Hq, int Hkv, int Sq, int Sk, int D, int mask_mode);
 int launch_prefill_bwd_short(const BwdParams& p, int D, int mask_mode, hipStream_t stream);
 
 }  // namespace mi355

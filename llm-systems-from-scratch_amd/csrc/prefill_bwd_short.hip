@@ -198,8 +198,8 @@ __global__ __launch_bounds__(NWV * 64, D == 32 ? 4 : 2) void bwd_short_kernel(Bw
     }
 }
 
-bool prefill_bwd_short_takes(const BwdParams& p, int D, int mask_mode) {
-    return (D == 32 || D == 64) && !p.cu_q && p.Hq == p.Hkv && p.Sq <= 256 && p.Sk <= 256 && (mask_mode == MI355_MASK_NONE || mask_mode == MI355_MASK_CAUSAL);
+bool prefill_bwd_short_takes(int Hq, int Hkv, int Sq, int Sk, int D, int mask_mode) {
+    return (D == 32 || D == 64) && Hq == Hkv && Sq <= 256 && Sk <= 256 && (mask_mode == MI355_MASK_NONE || mask_mode == MI355_MASK_CAUSAL);
 }
 
 template <int D, bool CAUSAL>

@@ -301,10 +301,13 @@ def test_workspace_of_the_backward_with_ds():
     assert ws(8, 64, 64, 256, 256, 128, causal, 0, 1, 0, 0) == 8 * 64 * (2 + 4 + 6 + 8) * 4096
     assert ws(8, 64, 64, 256, 256, 128, none, 0, 1, 0, 0) == 8 * 64 * 4 * 8 * 4096
     assert ws(8, 64, 64, 256, 256, 64, causal, 0, 1, 0, 0) == 0                  # head size 64: many key tiles,
-    assert ws(2, 64, 64, 256, 256, 64, causal, 0, 1, 0, 0) == 2 * 64 * 20 * 4096  # few of them,
+    assert ws(2, 64, 32, 256, 256, 64, causal, 0, 1, 0, 0) == 2 * 64 * 20 * 4096  # few of them,
     assert ws(8, 64, 64, 256, 256, 64, causal, 1, 1, 1023, 1023) > 0              # or lengths far apart
     assert ws(8, 64, 64, 256, 256, 64, causal, 1, 1, 1024, 1024) == 0
-    assert ws(2, 64, 64, 256, 256, 32, causal, 0, 1, 0, 0) == 2 * 64 * 20 * 4096
+    assert ws(2, 64, 32, 256, 256, 32, causal, 0, 1, 0, 0) == 2 * 64 * 20 * 4096
+    for D in (32, 64):                                                            # (a head per key head is the short kernel's up to 256 tokens)
+        assert ws(2, 64, 64, 256, 256, D, causal, 0, 1, 0, 0) == ws(1, 4, 4, 200, 256, D, none, 0, 1, 0, 0) == 0
+        assert ws(1, 4, 4, 200, 257, D, none, 0, 1, 0, 0) > 0 and ws(1, 4, 4, 257, 200, D, causal, 0, 1, 0, 0) > 0
     assert ws(3, 64, 64, 256, 256, 32, causal, 0, 1, 0, 0) == 0
     assert ws(8, 64, 64, 256, 256, 128, boolean, 0, 1, 0, 0) == 0
     assert ws(1, 4, 4, 128, 128, 128, causal, 0, 1, 0, 0) == 0                   # too little to gain
