@@ -171,6 +171,10 @@ size_t mi355_prefill_splitkv_workspace_bytes(int64_t total_q_rows, int Hq, int D
  */
 int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows,
                                     int causal, int n_compute_units);
+/* The same for keys and values that are packed or dense: 1 also where the unsplit call deals the keys to the wavefronts of its workgroups and
+ * is the faster one for it. */
+int mi355_prefill_suggest_prompt_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows,
+                                           int causal, int n_compute_units);
 int mi355_prefill_fwd_splitkv(const void* q, const void* k, const void* v, void* out,
                               const int64_t q_strides[3], const int64_t k_strides[3],
                               const int64_t v_strides[3], const int64_t o_strides[3],

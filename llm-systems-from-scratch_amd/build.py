@@ -22,7 +22,7 @@ LIB_NAME = "libmi355attn.so"
 SERVING_LIB_NAME = "libmi355attn_serving.so"      # without the kernels that only training needs
 CALLS_NAME = "_calls.so"                          # ... nor these
 TRAINING_ONLY = ("prefill_bwd.hip", "prefill_bwd_short.hip")
-SOURCES = ["api.hip", "paged_decode.hip", "prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "kv_cache_ops.hip",
+SOURCES = ["api.hip", "paged_decode.hip", "prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_keys.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "kv_cache_ops.hip",
            "layer_ops.hip", "paged_attn_any.hip", "ssm_ops.hip", "moe_ops.hip", "rows_linear.hip"]
 # prefill_fwd_w64.hip keeps its output accumulators in AGPRs that only its assembly statements touch: its builtin MFMAs
 # must therefore be selected in VGPR form, so that the compiler allocates no AGPR for them.
@@ -214,7 +214,7 @@ def build_library(verbose: bool = True) -> str:
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
 
     # sources whose kernels issue memory instructions from inline assembly
-    asm_dma = [s for s in ("prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "moe_ops.hip", "rows_linear.hip") if s in srcs]
+    asm_dma = [s for s in ("prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_keys.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "moe_ops.hip", "rows_linear.hip") if s in srcs]
     with ThreadPoolExecutor(max_workers=5) as ex:
         calls = ex.submit(compile_calls)
         check = ex.submit(check_w64_registers)

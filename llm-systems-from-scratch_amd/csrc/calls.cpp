@@ -343,7 +343,7 @@ Tensor forward_only(const Tensor& q, const Tensor& k, const Tensor& v, const int
               "mi355_prefill_fwd_window");
         return out;
     }
-    const int splits = mi355_prefill_suggest_kv_splits(s.B, s.Hq, s.D, s.Sq, s.Sk, rows, s.causal, compute_units(dev));
+    const int splits = mi355_prefill_suggest_prompt_kv_splits(s.B, s.Hq, s.D, s.Sq, s.Sk, rows, s.causal, compute_units(dev));
     if (splits > 1) {
         const Tensor ws = make({std::max<int64_t>((int64_t)mi355_prefill_splitkv_workspace_bytes(rows, s.Hq, s.D, splits), 16)}, at::kByte, dev);
         check(mi355_prefill_fwd_splitkv(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), Strides(q), Strides(k), Strides(v), Strides(out), cu_q, cu_k,

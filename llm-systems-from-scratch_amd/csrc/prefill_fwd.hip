@@ -22,6 +22,9 @@
 // Such a load writes 1 KiB of consecutive LDS per wavefront, so rows cannot be
 // padded; bank conflicts are avoided by an XOR swizzle instead: the 16-byte chunk
 // c of row r is stored in slot c ^ swz(r), applied on the global-address side.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -730,6 +733,51 @@ static int set_split(PrefillParams& p, int D, int n_split, int64_t total_q_rows,
     return 0;
 }
 
+static int device_compute_units() {
+    static std::atomic<int> known[64];                // (asked of the runtime once per device)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
+// Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; lengths of a packed batch are
+// judged by the longest).
+static double other_us(const PrefillParams& p, int D, int n_cu) {
+    const bool causal = p.mask_mode == MI355_MASK_CAUSAL;
+    const int Sk = p.block_table ? 16 * p.max_blocks : p.Sk;
+    const double over = causal && Sk > p.Sq ? Sk - p.Sq : 0, most = causal ? std::min<double>(Sk, over + p.Sq) : Sk;
+    const double heads = (double)p.Hq * p.B, kt = std::ceil(most / kBN);
+    if (prefill_short_takes(p, D)) {
+        // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
+        return (D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu;
+    }
+    // query tiles of a launch, dearest and mean number of key tiles; per key tile, per query tile, and what is the same for every call
+    const bool wide = D == 128 && prefill_w64_takes(p), by_head = wide && causal && p.Hq / p.Hkv % 4 == 0;
+    const int bm = by_head ? 64 : kBM;
+    const double qt = (p.Sq + bm - 1) / bm, jobs = qt * heads / (by_head ? 4 : 1), mean = causal ? std::min(kt, (over + 0.5 * p.Sq + 0.5 * bm) / kBN) : kt;
+    if (wide) {
+        // the last three key tiles of a length that is no multiple of 64 run in ordinary code, some 4 us each more
+        const double tail = Sk % kBN ? 12.0 : 0.0;
+        return 9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * mean + 4.0 + tail / (causal ? qt : 1.0)));
+    }
+    const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75;
+    return 5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * mean + 2.0));
+}
+
+// Wavefronts of prefill_keys.hip's kernel for p, 0: another kernel is the faster one.  One 183-token prompt, 16 heads, D 128: 64-query kernel 26.4 us, keys dealt to
+// the wavefronts 7.6; 4 of 700: 37.4, 33.0; of 1000: 44.9, 49.8; D 64, one of 1000: 21.9, 12.1; 4 of 1000: 24.6, 26.8.  Eight per cent are left to the fit.
+// (Training calls of short heads stay with the kernel that rounds fp32 operands on their way in: the same bits whichever type the inputs have.)
+static int keys_wavefronts(const PrefillParams& p, int D) {
+    if (p.lse && prefill_short_takes(p, D)) return 0;
+    const int n_cu = prefill_keys_takes(p, D) ? device_compute_units() : 0;
+    if (n_cu <= 0) return 0;
+    const PrefillKeysPlan plan = prefill_keys_plan(p.B, p.Hq, D, p.Sq, p.block_table ? 16 * p.max_blocks : p.Sk, p.mask_mode == MI355_MASK_CAUSAL, n_cu);
+    return plan.us < 0.92 * other_us(p, D, n_cu) ? plan.wavefronts : 0;
+}
+
 static int prefill_common(const void* q, const void* k, const void* v, void* out, const int64_t q_strides[3],
                           const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
                           const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const uint8_t* mask,
@@ -813,7 +861,9 @@ static int prefill_common(const void* q, const void* k, const void* v, void* out
         return MI355_OK;
     }
     // head_dim 128 without an explicit mask: the kernel with 64 queries per wavefront and a hand-scheduled tile loop
-    if (prefill_short_takes(p, D)) rc = launch_prefill_short(p, D, s);
+    const int keys = keys_wavefronts(p, D);
+    if (keys) rc = launch_prefill_keys(p, D, keys, s);
+    else if (prefill_short_takes(p, D)) rc = launch_prefill_short(p, D, s);
     else if (D == 128 && mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
     else rc = D == 128 ? launch_prefill<128>(p, s) : (D == 64 ? launch_prefill<64>(p, s) : launch_prefill<32>(p, s));
     if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
@@ -975,7 +1025,9 @@ static int prefill_paged_common(const void* q, const void* k_cache, const void* 
     hipStream_t s = (hipStream_t)stream;
     // head_dim 128: the kernel with 64 queries per wavefront, which reads the block table too
     int rc;
-    if (D == 128 && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
+    const int keys = keys_wavefronts(p, D);
+    if (keys) rc = launch_prefill_keys(p, D, keys, s);
+    else if (D == 128 && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
     else rc = D == 128 ? launch_prefill_paged<128>(p, s) : (D == 64 ? launch_prefill_paged<64>(p, s) : launch_prefill_paged<32>(p, s));
     if (rc == 0 && p.n_split > 1) rc = launch_merge(p, D, s);
     if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
@@ -1038,16 +1090,8 @@ extern "C" size_t mi355_prefill_splitkv_workspace_bytes(int64_t total_q_rows, in
 // keys (1.6 us in the split kernel) and 5 us per query tile outside the tile loop; the partial rows cost their bytes
 // twice (written, then read by the merge) at about 2.5 TB/s, plus 8 us for the second launch.  Head_dim 128 runs on
 // the persistent 64-query kernel, split or not, and has figures of its own (below).
-extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows,
-                                               int causal, int n_compute_units) {
-    if (B <= 0 || Hq <= 0 || D <= 0 || Sq_max <= 0 || Sk_max <= 0 || total_q_rows <= 0) return 1;
-    int n_cu = n_compute_units;
-    if (n_cu <= 0) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n_cu <= 0)
-            return 1;
-    }
+// (us: of the best split, where that is more than one)
+static int best_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows, int causal, int n_cu, double& us) {
     const int nq = (Sq_max + kBM - 1) / kBM, n_pairs = (nq + 1) / 2;
     const double over = causal && Sk_max > Sq_max ? Sk_max - Sq_max : 0;            // keys every query sees (causal)
     // K/V tiles of the heaviest single query tile and of the heaviest pair (causal: bottom-right diagonal)
@@ -1084,7 +1128,8 @@ extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max,
         const bool whole = Sk_max % kBN == 0 && Sq_max == Sk_max && total_q_rows == (int64_t)B * Sq_max;
         const auto merged = [&](int n) { return whole ? 4.0 + 2.0 * ((double)total_q_rows * Hq * (D + 1) * 4.0 * n) / 6.0e6 : partials(n); };
         plain = time_of(1);
-        double best = plain * (whole ? 0.9 : 0.85);   // a split must win clearly
+        double& best = us;
+        best = plain * (whole ? 0.9 : 0.85);   // a split must win clearly
         for (int n : kCandidates) {
             if (keys_single / kBN / n < 2.0) break;   // at least two tiles per share and query tile
             const double t = time_of(n) + merged(n);
@@ -1101,7 +1146,8 @@ extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max,
     const double jobs = (double)n_pairs * Hq * B;
     const double tiles = keys_pair / kBN;
     plain = rounds(jobs) * (tiles * tile_us + 5.0 * halves);
-    double best = plain * 0.85;                       // a split must win clearly
+    double& best = us;
+    best = plain * 0.85;                       // a split must win clearly
     for (int n : kCandidates) {
         if (tiles / n < 2.0 * halves) break;          // at least two tiles per share and query tile
         const double t = rounds(jobs * n) * (tiles / n * tile_us * 1.07 + 5.0 * halves) + partials(n);
@@ -1111,6 +1157,24 @@ extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max,
         }
     }
     return best_n;
+}
+
+extern "C" int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows,
+                                               int causal, int n_compute_units) {
+    if (B <= 0 || Hq <= 0 || D <= 0 || Sq_max <= 0 || Sk_max <= 0 || total_q_rows <= 0) return 1;
+    const int n_cu = n_compute_units > 0 ? n_compute_units : device_compute_units();
+    double us;
+    return n_cu > 0 ? best_kv_splits(B, Hq, D, Sq_max, Sk_max, total_q_rows, causal, n_cu, us) : 1;
+}
+
+// Whole prompts only: a chunk over keys that are there already keeps its splits.  Causal, D 128, us with splits / keys dealt to the wavefronts: one head, 1000
+// tokens 22.2 / 12.0, 4000 43.4 / 26.0; four heads, 4000 56.6 / 44.7.
+extern "C" int mi355_prefill_suggest_prompt_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows, int causal, int n_compute_units) {
+    if (B <= 0 || Hq <= 0 || D <= 0 || Sq_max <= 0 || Sk_max <= 0 || total_q_rows <= 0) return 1;
+    const int n_cu = n_compute_units > 0 ? n_compute_units : device_compute_units();
+    double us;
+    const int n = n_cu > 0 ? best_kv_splits(B, Hq, D, Sq_max, Sk_max, total_q_rows, causal, n_cu, us) : 1;
+    return n > 1 && Sq_max == Sk_max && prefill_keys_plan(B, Hq, D, Sq_max, Sk_max, causal != 0, n_cu).us < 0.92 * us ? 1 : n;
 }
 
 extern "C" int mi355_prefill_fwd_splitkv(const void* q, const void* k, const void* v, void* out,

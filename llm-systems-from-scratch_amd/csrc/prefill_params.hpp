@@ -63,4 +63,13 @@ struct RoundedInputs {
 };
 int launch_prefill_short_rounded(const PrefillParams& p, const RoundedInputs& r, int D, hipStream_t stream);
 
+// Small query tiles whose keys are dealt to a workgroup's wavefronts: prefill_keys.hip.  The plan: how many wavefronts, and about how long it takes.
+struct PrefillKeysPlan {
+    int wavefronts;
+    double us;
+};
+bool prefill_keys_takes(const PrefillParams& p, int D);
+PrefillKeysPlan prefill_keys_plan(int B, int Hq, int D, int Sq, int Sk, bool causal, int n_cu);
+int launch_prefill_keys(const PrefillParams& p, int D, int wavefronts, hipStream_t stream);
+
 }  // namespace mi355

@@ -107,14 +107,16 @@ def _packed_or_dense_strides(t, packed):
 _N_CU = {}
 
 
-def suggest_kv_splits(B, Hq, D, sq_max, sk_max, total_rows, causal, device):
+def suggest_kv_splits(B, Hq, D, sq_max, sk_max, total_rows, causal, device, prompt=False):
     """The library's suggestion for this shape (mi355_prefill_suggest_kv_splits: a cost model of tile-loop time
-    saved against the traffic of the partial rows); 1 = do not split."""
+    saved against the traffic of the partial rows); 1 = do not split.  prompt: keys and values packed or dense, without
+    per-head terms (mi355_prefill_suggest_prompt_kv_splits)."""
     idx = device.index if device.index is not None else torch.cuda.current_device()
     if idx not in _N_CU:
         _N_CU[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return _lib.load().mi355_prefill_suggest_kv_splits(int(B), int(Hq), int(D), int(sq_max), int(sk_max),
-                                                       int(total_rows), 1 if causal else 0, _N_CU[idx])
+    lib = _lib.load()
+    suggest = lib.mi355_prefill_suggest_prompt_kv_splits if prompt else lib.mi355_prefill_suggest_kv_splits
+    return suggest(int(B), int(Hq), int(D), int(sq_max), int(sk_max), int(total_rows), 1 if causal else 0, _N_CU[idx])
 
 
 def prefill_splitkv_workspace(total_q_rows, n_q_heads, head_dim, kv_splits, device):
@@ -123,9 +125,9 @@ def prefill_splitkv_workspace(total_q_rows, n_q_heads, head_dim, kv_splits, devi
     return torch.empty(max(int(n), 16), dtype=torch.uint8, device=device)
 
 
-def _split_args(kv_splits, workspace, B, Hq, D, sq_max, sk_max, total_rows, causal, device):
+def _split_args(kv_splits, workspace, B, Hq, D, sq_max, sk_max, total_rows, causal, device, prompt=False):
     """(n_split, workspace) for a forward-only prefill call; kv_splits None = choose."""
-    n = suggest_kv_splits(B, Hq, D, sq_max, sk_max, total_rows, causal, device) if kv_splits is None else int(kv_splits)
+    n = suggest_kv_splits(B, Hq, D, sq_max, sk_max, total_rows, causal, device, prompt) if kv_splits is None else int(kv_splits)
     if n < 1 or n > 64:
         raise ValueError("kv_splits must be in 1..64")
     if n == 1:
@@ -242,7 +244,7 @@ def _dense(q, k, v, mask, mode, softmax_scale, want_lse=False, kv_splits=1, work
     if Sk == 0:
         raise ValueError("attention over zero keys is undefined")
     n_split, workspace = (1, None) if (want_lse or mask is not None) else _split_args(
-        kv_splits, workspace, B, Hq, D, Sq, Sk, B * Sq, mode == _lib.MASK_CAUSAL, q.device)
+        kv_splits, workspace, B, Hq, D, Sq, Sk, B * Sq, mode == _lib.MASK_CAUSAL, q.device, prompt=True)
     _prefill(q, k, v, out, None, None, mask, B, Hq, Hkv, Sq, Sk, D, scale, mode, lse, n_split, workspace, B * Sq)
     return (out, lse) if want_lse else out
 
@@ -527,7 +529,7 @@ def _varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, cau
     lse = torch.empty(Hq, Tq, dtype=torch.float32, device=q.device) if want_lse else None
     if Tq and max_seqlen_q:
         n_split, workspace = (1, None) if want_lse or window else _split_args(
-            kv_splits, workspace, B, Hq, D, max_seqlen_q, max_seqlen_k, Tq, causal, q.device)
+            kv_splits, workspace, B, Hq, D, max_seqlen_q, max_seqlen_k, Tq, causal, q.device, prompt=head_scale is None and sinks is None)
         _prefill(q, k, v, out, cu_seqlens_q, cu_seqlens_k, None, B, Hq, Hkv, int(max_seqlen_q), int(max_seqlen_k),
                  D, scale, _lib.MASK_CAUSAL if causal else _lib.MASK_NONE, lse, n_split, workspace, Tq, head_scale, sinks,
                  window, keep_first)
