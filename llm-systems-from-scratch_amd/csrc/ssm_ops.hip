@@ -10,13 +10,15 @@
 //   ssm_state  (slots, heads, state, vdim_pad)    S in fp32 (vdim_pad: vdim rounded up to 4)
 // A sequence's first token is at position 0: its history is zero whatever the slot holds, so slots are never cleared.
 //
-// Three kernels besides the convolution:
+// Kernels besides the convolution:
 //   ssd_chunk_kernel   bf16 prompts: chunks of 64 tokens on MFMA, the state in accumulators from chunk to chunk; where
 //                      that walk leaves the chip idle, segments of a sequence side by side (ssd_carry_kernel between them)
+//   ssd_walk_kernel    the same in chunks of 128, outputs and state on different wavefronts: states of 64 or 128 rows
 //   ssm_scan_kernel    any sizes and fp32: token by token, the state in registers
 //   ... the same kernel with the convolution inside: one decode step of every sequence
 #include "common.hpp"
 #include "launch.hpp"
+#include "prefill_tile.hpp"
 
 #include <type_traits>
 
@@ -653,6 +655,416 @@ __global__ __launch_bounds__(256, NT == 8 ? 1 : 2) void ssd_chunk_kernel(SsmPara
         }
 }
 
+// The same recurrence in chunks of 128 tokens, outputs and state on different wavefronts: a workgroup of eight walks the chunks of a sequence or segment for
+// one head and 64 columns of vdim.  v_mfma_f32_32x32x16_bf16 throughout; what is computed in fp32 enters as a bf16 pair, as above.
+//   wavefronts 0-3, 32 tokens t each (column = lane = t; c: running sums from the chunk's start):
+//     G^T (s x t)  = B C^T           B's rows from LDS, C's in registers, tile by tile of 32 tokens s
+//     Y^T (p x t)  = S^T C^T + X^T F^T     F^T is G^T weighted in its registers: the accumulator is the operand
+//     A tile in front of the wavefront's own 32 tokens, which start behind c_r, is weighted by exp(c_r - c_s) dt_s, 32 factors for 1024 weights, and the sum
+//     over these and the state by exp(c_t - c_r): no exponent is above zero.  The tile on the diagonal has its exponentials one by one.
+//   wavefronts 4-7, half of the state's rows and 32 columns each: S <- exp(c_last) S + B^T (w x), w_s = exp(c_last - c_s) dt_s, in registers; S in front of the
+//     next chunk goes to LDS, column by column, so that the others read it as rows.  They also request the next chunk's B and x; wavefront 0 works out its decays.
+// Two barriers a chunk: everything that a chunk reads is there; S has been read and may change.
+//
+// Bound by the instructions of the fourth block of tokens, with its four tiles, and of the state wavefront on the same SIMD: some 8000 cycles a chunk, 5200 of
+// them vector instructions issued, 3300 MFMAs.  What keeps it there: fragments read one step ahead behind scheduling barriers (left alone, the compiler
+// holds all at once and spills), a body per block of tokens without branches, addresses it cannot hoist, rows that leave behind the next chunk's first product (a
+// wait for C in front of which stores stand waits for these too: 9 us of 82), decays on the wavefront with the least to do.  4 sequences of 2048
+// tokens, 64 heads, state 128: segments of 512, three launches of the kernels around this one 148 us; whole sequences on ssd_chunk_kernel 138; like this 78.
+constexpr int kWalkChunk = 128, kWalkAhead = 3;      // (steps of 16 tokens that the state takes while the outputs read it)
+template <int N, int MODE>
+__global__ __launch_bounds__(512, 2) void ssd_walk_kernel(SsmParams<__bf16> p) {
+    using RX = TileReads<64>;
+    constexpr int Q = kWalkChunk, NS = N / 16, kB = Q * N * 2, kX = Q * 128, kS = 64 * N * 2, NT = N / 64;      // NT: 32-row tiles of the state per wavefront
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kB + 2 * kX + 2 * kS];
+    __shared__ __attribute__((aligned(16))) float cum_lds[2][Q], dt_lds[2][Q], left_lds[2][Q], col_lds[4][Q];
+    unsigned char *const x_lds = lds + 2 * kB, *const s_lds = lds + 2 * kB + 2 * kX;
+    const int h = blockIdx.x / p.slices % p.H, col0 = blockIdx.x % p.slices * 64, unit = blockIdx.x / (p.slices * p.H);
+    int b = unit, first, len, place = 0, seg = 0;
+    bool last = true, alone = true;                      // the sequence's last segment, its only one
+    if constexpr (MODE == kWhole) {
+        seq_rows(p, b, first, len);
+        if (len <= 0) return;
+    } else {
+        if (!find_segment<0>(p, unit, b, first, len, place, seg) || seg >= p.n_segs) return;
+        alone = len <= max(p.seg_len, p.whole_len);
+        last = alone || (place + 1) * p.seg_len >= len;
+        first += place * p.seg_len;
+        len = last ? len - place * p.seg_len : p.seg_len;
+    }
+    const bool resumed = !alone || p.positions[first] > 0;
+    const int g = h / (p.H / p.G), inner = p.H * p.P;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 31, kg = lane >> 5;
+    const bool state_wave = wave >= 4;
+    const __bf16* xsrc = p.xbc + (int64_t)first * p.channels + h * p.P + col0;
+    const __bf16* bsrc = p.xbc + (int64_t)first * p.channels + inner + g * N;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
+    const int row_bytes = p.channels * 2;
+
+    // ---- wavefronts 4-7 ----
+    const int sw = wave & 3, pt = sw & 1, nt0 = (sw >> 1) * NT;
+    f32x16 S[NT];                                        // lane: column 32 pt + n, rows 32 (nt0 + i) + 8 (j / 4) + 4 kg + j % 4
+    float* const slot = p.ssm_state + ((int64_t)state_slot(p, b) * p.H + h) * N * p.Pp + col0 + 32 * pt + n;
+    // B and x of chunk c (rows past the end: the last one again, weighted by zero); offsets from a chunk's first row
+    const auto b_place = [&](int j, int last_row) {
+        const int at = 64 * (sw * (kB / 4096) + j) + lane, row = at / (N / 8);
+        return (uint32_t)(min(row, last_row) * row_bytes + (((at % (N / 8)) ^ swz<N>(row)) << 4));
+    };
+    const auto x_place = [&](int j, int last_row) {
+        const int row = 8 * (sw * (kX / 4096) + j) + lane / 8;
+        return (uint32_t)(min(row, last_row) * row_bytes + (((lane % 8) ^ swz<64>(row)) << 4));
+    };
+    uint32_t b_voff[kB / 4096], x_voff[kX / 4096];
+    const auto issue = [&](int c) {
+        const int last_row = len - 1 - c * Q;
+        const unsigned char* bs = reinterpret_cast<const unsigned char*>(bsrc) + (int64_t)(c * Q) * row_bytes;
+        const unsigned char* xs = reinterpret_cast<const unsigned char*>(xsrc) + (int64_t)(c * Q) * row_bytes;
+        const uint32_t b_dst = lds0 + (c & 1) * kB + sw * (kB / 4), x_dst = lds0 + 2 * kB + (c & 1) * kX + sw * (kX / 4);
+        if (last_row >= Q - 1) {
+#pragma unroll
+            for (int j = 0; j < kB / 4096; ++j) dma_to_lds_16(bs, b_voff[j], b_dst + j * 1024);
+#pragma unroll
+            for (int j = 0; j < kX / 4096; ++j) dma_to_lds_16(xs, x_voff[j], x_dst + j * 1024);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kB / 4096; ++j) dma_to_lds_16(bs, b_place(j, last_row), b_dst + j * 1024);
+#pragma unroll
+            for (int j = 0; j < kX / 4096; ++j) dma_to_lds_16(xs, x_place(j, last_row), x_dst + j * 1024);
+        }
+    };
+    const auto publish = [&]() {                         // S as rows of columns, leading parts and remainders
+        const int col = 32 * pt + n;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                u32x2 hi, lo;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    uint32_t a, c;
+                    split_bf16(S[i][4 * q + 2 * e], S[i][4 * q + 2 * e + 1], a, c);
+                    hi[e] = a;
+                    lo[e] = c;
+                }
+                unsigned char* to = s_lds + col * (N * 2) + (((4 * (nt0 + i) + q) ^ swz<N>(col)) << 4) + 8 * kg;
+                *reinterpret_cast<u32x2*>(to) = hi;
+                *reinterpret_cast<u32x2*>(to + kS) = lo;
+            }
+    };
+    const float bias = p.dt_bias[h], na2 = p.neg_a[h] * kLog2e;
+    const __bf16* dtsrc = p.proj + (int64_t)first * p.proj_stride + p.dt_at + h;
+    __bf16 raw[2] = {(__bf16)0.f, (__bf16)0.f};          // wavefront 0: dt of tokens 2 lane, 2 lane + 1 of the chunk whose decays come next
+    const auto fetch_dt = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) raw[i] = dtsrc[(int64_t)min(c * Q + 2 * lane + i, len - 1) * p.proj_stride];
+    };
+    const auto decays = [&](int c) {
+        float dt[2], sum = 0.f, cum[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            dt[i] = c * Q + 2 * lane + i < len ? softplus((float)raw[i] + bias) : 0.f;
+            sum += na2 * dt[i];
+            cum[i] = sum;
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const float up = __shfl_up(sum, off, 64);
+            sum += lane >= off ? up : 0.f;
+        }
+        const float all = __shfl(sum, 63, 64);
+        float before = __shfl_up(sum, 1, 64);
+        before = lane > 0 ? before : 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int t = 2 * lane + i;
+            cum_lds[c & 1][t] = before + cum[i];
+            dt_lds[c & 1][t] = dt[i];
+            left_lds[c & 1][t] = fast_exp2(all - (before + cum[i])) * dt[i];
+        }
+    };
+    int sb_off[2][NT], sx_off[2];                        // transposed fragments: tokens 8 kg + .. of a step of 16
+    {
+        const int g16 = lane >> 4, s16 = lane & 15;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int row = 8 * (g16 >> 1) + (s16 >> 2) + 4 * e, d = 16 * (g16 & 1) + 4 * (s16 & 3);
+            sx_off[e] = row * 128 + (((4 * pt + (d >> 3)) ^ swz<64>(row)) << 4) + (d & 7) * 2;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) sb_off[e][i] = row * (N * 2) + (((4 * (nt0 + i) + (d >> 3)) ^ swz<N>(row)) << 4) + (d & 7) * 2;
+        }
+    }
+    const int n_chunks = (len + Q - 1) / Q;
+    if (state_wave) {
+#pragma unroll
+        for (int j = 0; j < kB / 4096; ++j) b_voff[j] = b_place(j, Q);
+#pragma unroll
+        for (int j = 0; j < kX / 4096; ++j) x_voff[j] = x_place(j, Q);
+        issue(0);
+        const float* from = alone ? slot : p.seg_state + ((int64_t)seg * p.H + h) * N * p.Pp + col0 + 32 * pt + n;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) S[i][j] = 0.f;
+        if (resumed) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) S[i][j] = from[(int64_t)(32 * (nt0 + i) + 8 * (j >> 2) + 4 * kg + (j & 3)) * p.Pp];
+            publish();
+        }
+        for (int c = 0; c < n_chunks; ++c) {
+            const int buf = c & 1;
+            wait_vmcnt<0>();
+            __syncthreads();                             // B, x, decays and S of this chunk are there
+            if (c + 1 < n_chunks) issue(c + 1);
+            const bool wanted = MODE == kWhole || last || c + 1 < n_chunks;
+            const float decay = fast_exp2(cum_lds[buf][Q - 1]);
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) S[i][j] *= decay;
+            // (addresses that the compiler cannot trace: it then adds constants in the reads instead of holding every sum in a register of its own)
+            uint32_t x_at[2], b_at[2][NT];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                x_at[e] = lds0 + 2 * kB + buf * kX + sx_off[e];
+                asm volatile("" : "+v"(x_at[e]));
+#pragma unroll
+                for (int i = 0; i < NT; ++i) {
+                    b_at[e][i] = lds0 + buf * kB + sb_off[e][i];
+                    asm volatile("" : "+v"(b_at[e][i]));
+                }
+            }
+            // steps of 16 tokens, their fragments read one step ahead
+            bf16x8 xf[2], bf[2][NT];
+            f32x4 w[2][2];
+            const auto fragments = [&](int u) {
+                xf[u & 1] = join_bf16x8(lds_read_tr16_at(x_at[0] + 16 * u * 128), lds_read_tr16_at(x_at[1] + 16 * u * 128));
+#pragma unroll
+                for (int e = 0; e < 2; ++e) w[u & 1][e] = *reinterpret_cast<const f32x4*>(left_lds[buf] + 16 * u + 8 * kg + 4 * e);
+#pragma unroll
+                for (int i = 0; i < NT; ++i) bf[u & 1][i] = join_bf16x8(lds_read_tr16_at(b_at[0][i] + 16 * u * N * 2), lds_read_tr16_at(b_at[1][i] + 16 * u * N * 2));
+            };
+            const auto gather = [&](auto from_c, auto to_c) {
+                constexpr int from = decltype(from_c)::value, to = decltype(to_c)::value;
+                if constexpr (from == 0) fragments(0);
+#pragma unroll
+                for (int u = from; u < to; ++u) {
+                    if (u + 1 < Q / 16) fragments(u + 1);
+                    u32x4 hi, lo;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        uint32_t a, v;
+                        split_bf16((float)xf[u & 1][2 * e] * w[u & 1][e / 2][2 * e % 4], (float)xf[u & 1][2 * e + 1] * w[u & 1][e / 2][2 * e % 4 + 1], a, v);
+                        hi[e] = a;
+                        lo[e] = v;
+                    }
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) S[i] = mfma32(bf[u & 1][i], as_bf16x8(hi), S[i]);
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) S[i] = mfma32(bf[u & 1][i], as_bf16x8(lo), S[i]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            if (wanted) gather(std::integral_constant<int, 0>{}, std::integral_constant<int, kWalkAhead>{});
+            __syncthreads();                             // S has been read
+            if (wanted) gather(std::integral_constant<int, kWalkAhead>{}, std::integral_constant<int, Q / 16>{});
+            if (c + 1 < n_chunks) publish();
+        }
+        if (last)
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) slot[(int64_t)(32 * (nt0 + i) + 8 * (j >> 2) + 4 * kg + (j & 3)) * p.Pp] = S[i][j];
+        return;
+    }
+
+    // ---- wavefronts 0-3 ----
+    const int tb = wave, tq = 32 * tb + n;               // 32-token block, this lane's token of a chunk
+    RX rx;
+    rx.init(lane);
+    // rows of B and of S (column n): rows 16 s + 8 kg .. at this ^ s << 5
+    const uint32_t row0 = n * (N * 2) + ((kg ^ swz<N>(n)) << 4);
+    bf16x8 cf[NS];
+    const __bf16* csrc = p.xbc + (int64_t)first * p.channels + inner + (p.G + g) * N + 8 * kg;
+    const auto fetch_c = [&](int c) {
+        const __bf16* row = csrc + (int64_t)min(c * Q + tq, len - 1) * p.channels;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) cf[s] = as_bf16x8(*reinterpret_cast<const u32x4*>(row + 16 * s));
+    };
+    const float skip = p.d_skip[h];
+    // A chunk's rows leave behind the next one's first product: in front of it, the wait for C would be one for the stores too
+    u32x2 out[2][4];
+    const auto store = [&](int c) {
+        if (c * Q + tq >= len) return;
+        __bf16* row = p.y + (int64_t)(first + c * Q + tq) * p.y_stride + h * p.P + col0 + 4 * kg;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x2*>(row + 32 * dt + 8 * q) = out[dt][q];
+    };
+    if (tb == 0) {
+        fetch_dt(0);
+        decays(0);
+        fetch_dt(1);
+    }
+    fetch_c(0);
+    // a loop for every block, without branches inside a chunk: the products of one tile stand among the weights of another
+    const auto walk = [&](auto tb_c) {
+        constexpr int TB = decltype(tb_c)::value;
+        for (int c = 0; c < n_chunks; ++c) {
+            const int t0 = c * Q, buf = c & 1;
+            const bool busy = t0 + 32 * TB < len;
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(cf[s]));       // (the wait for C: further down it would be one for the stores as well)
+            const float* cum = cum_lds[buf];
+            const float* dts = dt_lds[buf];
+            f32x16 acc[2];
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) acc[dt][j] = 0.f;
+            if (busy && (resumed || c > 0)) {
+                uint32_t s_at = lds0 + 2 * kB + 2 * kX + row0;
+                asm volatile("" : "+v"(s_at));
+                u32x4 sf[2][4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sf[0][i] = lds_load_at<u32x4>(s_at + (i >> 1) * kS + 32 * (i & 1) * N * 2);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (s + 1 < NS) sf[(s + 1) & 1][i] = lds_load_at<u32x4>((s_at ^ ((s + 1) << 5)) + (i >> 1) * kS + 32 * (i & 1) * N * 2);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[i & 1] = mfma32(as_bf16x8(sf[s & 1][i]), cf[s], acc[i & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __syncthreads();
+            if (c > 0) store(c - 1);
+            if (!busy) continue;
+            const float ct = cum[tq], cref = TB > 0 ? cum[32 * TB - 1] : 0.f;
+            uint32_t b_at = lds0 + buf * kB + row0, x_at[2][2];
+            asm volatile("" : "+v"(b_at));
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    x_at[e][dt] = lds0 + 2 * kB + buf * kX + rx.tr_off[e][dt];
+                    asm volatile("" : "+v"(x_at[e][dt]));
+                }
+            for (int s = lane; s < 32 * TB; s += 64) col_lds[TB][s] = fast_exp2(cref - cum[s]) * dts[s];
+            // X^T F^T of the tile of tokens 32 st .. , F^T in accumulator order
+            const auto add = [&](int st, const float (&f)[16]) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    u32x4 hi, lo;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        uint32_t a, v;
+                        split_bf16(f[8 * u + 2 * w], f[8 * u + 2 * w + 1], a, v);
+                        hi[w] = a;
+                        lo[w] = v;
+                    }
+                    bf16x8 xf[2];
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt)
+                        xf[dt] = join_bf16x8(lds_read_tr16_at(x_at[0][dt] + (32 * st + 16 * u) * 128), lds_read_tr16_at(x_at[1][dt] + (32 * st + 16 * u) * 128));
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt) acc[dt] = mfma32(xf[dt], as_bf16x8(hi), acc[dt]);
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt) acc[dt] = mfma32(xf[dt], as_bf16x8(lo), acc[dt]);
+                }
+            };
+            {
+                f32x16 G[TB + 1];
+#pragma unroll
+                for (int st = 0; st <= TB; ++st)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) G[st][j] = 0.f;
+                // (fragments one step ahead, in program order: left alone, the compiler holds all of them at once, and spills)
+                u32x4 bfr[2][TB + 1];
+#pragma unroll
+                for (int st = 0; st <= TB; ++st) bfr[0][st] = lds_load_at<u32x4>(b_at + 32 * st * N * 2);
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+#pragma unroll
+                    for (int st = 0; st <= TB; ++st)
+                        if (s + 1 < NS) bfr[(s + 1) & 1][st] = lds_load_at<u32x4>((b_at ^ ((s + 1) << 5)) + 32 * st * N * 2);
+#pragma unroll
+                    for (int st = 0; st <= TB; ++st) G[st] = mfma32(as_bf16x8(bfr[s & 1][st]), cf[s], G[st]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const float head = fast_exp2(cref), rowf = fast_exp2(ct - cref);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) acc[dt][j] *= head;
+                float f[2][16];
+                const auto weigh = [&](int st, float (&to)[16]) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(col_lds[TB] + 32 * st + 8 * q + 4 * kg);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) to[4 * q + e] = G[st][4 * q + e] * w[e];
+                    }
+                };
+                const auto weigh_diagonal = [&](float (&to)[16]) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int s = 8 * q + 4 * kg;
+                        const f32x4 cs = *reinterpret_cast<const f32x4*>(cum + 32 * TB + s), ds = *reinterpret_cast<const f32x4*>(dts + 32 * TB + s);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = G[TB][4 * q + e] * (fast_exp2(ct - cs[e]) * ds[e]);
+                            to[4 * q + e] = s + e <= n ? v : 0.f;
+                        }
+                    }
+                };
+                if constexpr (TB > 0) weigh(0, f[0]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int st = 0; st < TB; ++st) {
+                    if (st + 1 < TB) weigh(st + 1, f[(st + 1) & 1]);
+                    else weigh_diagonal(f[TB & 1]);
+                    add(st, f[st & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if constexpr (TB == 0) weigh_diagonal(f[0]);
+                if (c + 1 < n_chunks) fetch_c(c + 1);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) acc[dt][j] *= rowf;
+                add(TB, f[TB & 1]);
+            }
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const u32x2 xw = *reinterpret_cast<const u32x2*>(x_lds + buf * kX + tq * 128 + (((4 * dt + q) ^ swz<64>(tq)) << 4) + 8 * kg);
+                    const uint32_t x01 = xw[0], x23 = xw[1];
+                    const bf16x2 xa = __builtin_bit_cast(bf16x2, x01), xb = __builtin_bit_cast(bf16x2, x23);
+                    out[dt][q][0] = pack_bf16(fmaf(skip, (float)xa[0], acc[dt][4 * q]), fmaf(skip, (float)xa[1], acc[dt][4 * q + 1]));
+                    out[dt][q][1] = pack_bf16(fmaf(skip, (float)xb[0], acc[dt][4 * q + 2]), fmaf(skip, (float)xb[1], acc[dt][4 * q + 3]));
+                }
+            if constexpr (TB == 0) {                         // (the block with the least to do)
+                if (c + 1 < n_chunks) {
+                    decays(c + 1);
+                    fetch_dt(c + 2);
+                }
+            }
+        }
+    };
+    if (tb == 0) walk(std::integral_constant<int, 0>{});
+    else if (tb == 1) walk(std::integral_constant<int, 1>{});
+    else if (tb == 2) walk(std::integral_constant<int, 2>{});
+    else walk(std::integral_constant<int, 3>{});
+    store(n_chunks - 1);
+}
+
 // What the segments of a sequence add -> the states in front of them, in place: a thread owns four columns of one row.
 __global__ __launch_bounds__(256) void ssd_carry_kernel(SsmParams<__bf16> p) {
     constexpr int kAhead = 4;
@@ -741,11 +1153,33 @@ static bool chunked_takes(const SsmParams<__bf16>& p) {
            (reinterpret_cast<uintptr_t>(p.y) & 7) == 0;
 }
 
+// Sizes that ssd_walk_kernel takes: a state of 64 or 128 rows, whole slices of vdim, rows in 16-byte pieces
+static bool walk_takes(const SsmParams<__bf16>& p) { return (p.N == 64 || p.N == 128) && p.P % 64 == 0 && p.channels % 8 == 0 && p.channels < (1 << 23); }
+
+// ... and where it is the faster one.  Its workgroup has a compute unit to itself and needs some 4.6 us per 128 tokens, the other kernel's needs half of one and
+// 3.3 us per 64 when it has company (less with a state of 64 rows): launches that give no compute unit a second workgroup, and whole sequences unless they
+// are short.  Us, this / the other, 64 heads, state 128: 4 x 2048 tokens whole 143 / 186, 9 x 961 172 / 200, 1 x 64 18 / 21, 16 x 64 45 / 42; 8000 tokens in
+// segments of 512 198 / 190; 16 heads, 4000 in segments of 256 57 / 64; state 64, 64 heads: 5 of 122 to 1965 75 / 97, 5 x 111 31 / 30, 14 of 56 to 911 88 / 86.
+// (A call that cuts only long sequences has most of them whole.)
+static bool walk_pays(const SsmParams<__bf16>& p, int64_t wgs, bool whole) {
+    int dev = 0, n_cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+    const bool longer = whole && p.n_rows >= 192LL * p.B;
+    return wgs <= (p.N == 128 || longer ? n_cu + n_cu / 4 : n_cu) || (longer && p.N == 128);
+}
+
 template <int MODE>
 static int launch_chunks(const SsmParams<__bf16>& p, int64_t units, hipStream_t s) {
     const int64_t wgs = units * p.H * p.slices;
     if (wgs > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)wgs), block(256);
+    if constexpr (MODE != kSegState) {
+        if (walk_takes(p) && walk_pays(p, wgs, MODE == kWhole || p.whole_len > 0)) {
+            if (p.N == 64) hipLaunchKernelGGL((ssd_walk_kernel<64, MODE>), grid, dim3(512), 0, s, p);
+            else hipLaunchKernelGGL((ssd_walk_kernel<128, MODE>), grid, dim3(512), 0, s, p);
+            return (int)hipGetLastError();
+        }
+    }
     if (p.N <= 32) hipLaunchKernelGGL((ssd_chunk_kernel<1, MODE>), grid, block, 0, s, p);
     else if (p.N <= 64) hipLaunchKernelGGL((ssd_chunk_kernel<2, MODE>), grid, block, 0, s, p);
     else if (p.N <= 128) hipLaunchKernelGGL((ssd_chunk_kernel<4, MODE>), grid, block, 0, s, p);

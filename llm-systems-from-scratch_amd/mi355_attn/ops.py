@@ -1479,6 +1479,19 @@ def ssm_segments(n_tokens: int, n_sequences: int, heads: int, vdim: int, state: 
     return 512, whole
 
 
+def _ssm_plan(n_tokens, n_sequences, heads, vdim, state, longest):
+    """ssm_segments for the kernels that a call of this size runs on: with states of 128 rows and whole slices of vdim, sequences stay whole from 192
+    workgroups on (4 x 2048 tokens, 64 heads: 143 us; in segments of 512 195; 2 x 3000: 143, 152; 1 x 8000: 299, 198) but for those of more than twice the
+    mean, as there (64 rows: 3 x 4087 tokens whole 268, in segments of 512 220)."""
+    workgroups = n_sequences * heads * (vdim // 64)
+    if state != 128 or vdim % 64 or workgroups < 192:
+        return ssm_segments(n_tokens, n_sequences, heads, vdim, state, longest)
+    whole = 2 * n_tokens // n_sequences
+    if n_sequences == 1 or n_tokens < 768 * n_sequences or workgroups >= 1024 or (longest is not None and longest <= whole):
+        return 0, 0
+    return 512, whole
+
+
 def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positions, cu_seqlens=None, *, heads, vdim, state, groups,
             out=None, scan="auto", segment: int | None = None, longest: int | None = None):
     """Mamba-2 mixer between its projections: causal convolution + silu of the channels (x | B | C) at column xbc_col of proj's
@@ -1493,7 +1506,7 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
     if _native is not None and cu_seqlens is not None and out is None and scan == "auto" and segment is None and proj.dim() == 2:
         T, B = proj.shape[0], slots.numel()
         fits = T and B and state % 8 == 0 and vdim % 8 == 0 and state <= 256
-        seg_len, whole_len = ssm_segments(T, B, heads, vdim, state, longest) if fits else (0, 0)
+        seg_len, whole_len = _ssm_plan(T, B, heads, vdim, state, longest) if fits else (0, 0)
         got = _native.ssm_prefill(proj, *(params[n] for n in ("conv", "conv_b", "dt_bias", "neg_a", "d_skip")), conv_state, ssm_state, slots, positions,
                                   cu_seqlens, xbc_col, dt_col, heads, vdim, state, groups, seg_len, whole_len)
         if got is not None:
@@ -1525,7 +1538,7 @@ def ssm_mix(proj, xbc_col, dt_col, params, conv_state, ssm_state, slots, positio
     xbc = None if cu_seqlens is None else torch.empty(T, channels, dtype=proj.dtype, device=proj.device)
     seg_len, whole_len, seg_state, seg_decay = 0, 0, None, None
     if cu_seqlens is not None and scan != "serial" and proj.dtype == torch.bfloat16 and state % 8 == 0 and vdim % 8 == 0 and state <= 256:
-        seg_len, whole_len = ssm_segments(T, B, heads, vdim, state, longest) if segment is None else (int(segment), 0)
+        seg_len, whole_len = _ssm_plan(T, B, heads, vdim, state, longest) if segment is None else (int(segment), 0)
     if seg_len:
         units = T // seg_len + B
         seg_state = torch.empty(units, heads, state, vdim, dtype=torch.float32, device=proj.device)

@@ -322,6 +322,18 @@ def test_no_sequence_of_a_scan_is_waited_for_alone(heads, lens):
         assert walks == lens and seg == 0
 
 
+@pytest.mark.parametrize("heads,lens", [(64, [8192] + [64] * 7), (24, [3000] + [500] * 7), (64, [2048] * 4), (64, [900] * 3), (32, [2000, 1000] * 3)])
+def test_sequences_that_stay_whole_are_not_waited_for_alone(heads, lens):
+    """The same of the plan for states of 128 rows, which keeps sequences whole from 192 workgroups on; equal lengths stay whole also where it cannot know."""
+    mean = sum(lens) / len(lens)
+    for longest in (None, max(lens)):
+        seg, whole = mi355_attn.ops._ssm_plan(sum(lens), len(lens), heads, 64, 128, longest)
+        walks = [n if not seg or n <= max(seg, whole) else seg for n in lens]
+        assert max(walks) <= max(512, 2 * mean) and (len(set(lens)) > 1 or walks == lens)
+    for state, vdim in ((64, 64), (128, 72), (256, 64)):
+        assert mi355_attn.ops._ssm_plan(sum(lens), len(lens), heads, vdim, state, None) == mi355_attn.ops.ssm_segments(sum(lens), len(lens), heads, vdim, state, None)
+
+
 @pytest.mark.parametrize("heads,n,lens,seg", [(16, 1, 500, 64), (16, 1, 2000, 128), (64, 1, 500, 128), (64, 1, 320, 0), (16, 6, 700, 192), (16, 6, 500, 0),
                                               (16, 1, 4100, 256), (64, 1, 1133, 256), (64, 8, 600, 0), (15, 1, 900, 256), (15, 1, 700, 0)])
 def test_little_work_takes_short_segments(heads, n, lens, seg):
