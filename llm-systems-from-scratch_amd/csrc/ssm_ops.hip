@@ -24,7 +24,6 @@
 
 namespace mi355 {
 
-constexpr int kConvTile = 16;        // tokens per thread of the convolution
 constexpr int kMaxTaps = 16;
 constexpr int kScanVecs = 16;        // most 4-wide state pieces per thread of the scan
 
@@ -108,22 +107,59 @@ __device__ __forceinline__ void store_ch(T* p, const float (&v)[V]) {
     }
 }
 
-// Causal convolution + silu of packed prompts.  A thread owns V adjacent channels of kConvTile tokens of one sequence; the
-// inputs it has read slide through registers when the number of taps is known at compile time (TAPS > 0).  The thread of a
-// sequence's first tile is the only one that touches the sequence's ring for its channels: it reads the history first and
-// writes the last taps - 1 inputs of the portion at its end.
-template <typename T, int V, int TAPS>
+// Causal convolution + silu of packed prompts.  A thread owns V adjacent channels of TILE tokens of one sequence; the inputs it has read
+// slide through registers when the number of taps is known at compile time (TAPS > 0).  The thread of a sequence's first tile is the only
+// one that touches the sequence's ring for its channels: it reads the history first and writes the last taps - 1 inputs of the portion at its end.
+//
+// Bound by its bytes where a call is large (8192 tokens, 4352 channels: 142 MB in 30 us) and by one load's latency where it is small, so all rows of a batch of
+// eight, and those that go to the ring, are requested before the first is used: a load in front of every token's sum took 11 to 13 us for 600 to 1700 tokens,
+// 4 tokens per thread in one batch take 7.  Tiles of 4 read 7 rows for 4, tiles of 16 19 for 16.
+template <typename T, int V>
+struct ChannelRow {                                      // V adjacent channels as they are in memory
+    static constexpr int kWords = V * sizeof(T) < 4 ? 1 : V * sizeof(T) / 4;
+    uint32_t w[kWords];
+    __device__ __forceinline__ void load(const T* p) {
+        if constexpr (V == 1) {
+            w[0] = 0u;
+            __builtin_memcpy(w, p, sizeof(T));
+        } else {
+#pragma unroll
+            for (int i = 0; i < kWords / 4; ++i) {
+                const u32x4 x = reinterpret_cast<const u32x4*>(p)[i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[4 * i + e] = x[e];
+            }
+        }
+    }
+    __device__ __forceinline__ void store(T* p) const {
+        if constexpr (V == 1) {
+            __builtin_memcpy(p, w, sizeof(T));
+        } else {
+#pragma unroll
+            for (int i = 0; i < kWords / 4; ++i) reinterpret_cast<u32x4*>(p)[i] = u32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]};
+        }
+    }
+    __device__ __forceinline__ void get(float (&v)[V]) const {
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            if constexpr (sizeof(T) == 2) v[e] = __builtin_bit_cast(float, e % 2 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
+            else v[e] = __builtin_bit_cast(float, w[e]);
+        }
+    }
+};
+
+template <typename T, int V, int TAPS, int TILE>
 __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
     constexpr bool FAST = sizeof(T) == 2;
     const int taps = TAPS > 0 ? TAPS : p.taps;
     const int ch_groups = p.channels / V;
-    const int g_blocks = (ch_groups + 255) / 256;
+    const int g_blocks = (ch_groups + (int)blockDim.x - 1) / (int)blockDim.x;
     const int tile = blockIdx.x / g_blocks;
-    const int cg = (blockIdx.x % g_blocks) * 256 + threadIdx.x;
-    const int b = seq_of_unit(p, tile, kConvTile);
+    const int cg = (blockIdx.x % g_blocks) * blockDim.x + threadIdx.x;
+    const int b = seq_of_unit(p, tile, TILE);
     int first, len;
     seq_rows(p, b, first, len);
-    const int t0 = (tile - (first / kConvTile + b)) * kConvTile;
+    const int t0 = (tile - (first / TILE + b)) * TILE;
     if (t0 < 0 || t0 >= len || cg >= ch_groups) return;
     const int c = cg * V;
     const int pos0 = p.positions[first];
@@ -140,19 +176,34 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
         }
     };
     float bias[V];
-    load_ch<float, V>(p.conv_b + c, bias);
-    const int n = min(kConvTile, len - t0);
+    const int n = min(TILE, len - t0);
     T* out = p.xbc + (int64_t)(first + t0) * p.channels + c;
     if constexpr (TAPS > 0) {
+        constexpr int BATCH = TILE < 8 ? TILE : 8, KEEP = TAPS > 1 ? TAPS - 1 : 1;
+        ChannelRow<T, V> row[BATCH], keep[KEEP];
+        const auto request = [&](int t1) {                       // (a tile's rows past the end: the last one again)
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i) row[i].load(in + (int64_t)(t0 + min(t1 + i, n - 1)) * p.proj_stride);
+        };
         float w[TAPS][V], x[TAPS][V];
+        request(0);
+#pragma unroll
+        for (int j = 0; j + 1 < TAPS; ++j) input(t0 - (TAPS - 1) + j, x[j]);
+        if (t0 == 0)
+#pragma unroll
+            for (int j = 0; j + 1 < TAPS; ++j) keep[j].load(in + (int64_t)max(0, len - (TAPS - 1) + j) * p.proj_stride);
+        load_ch<float, V>(p.conv_b + c, bias);
 #pragma unroll
         for (int j = 0; j < TAPS; ++j) load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w[j]);
 #pragma unroll
-        for (int j = 0; j + 1 < TAPS; ++j) input(t0 - (TAPS - 1) + j, x[j]);
+        for (int t1 = 0; t1 < TILE; t1 += BATCH) {
+            if (t1 > 0) {
+                if (t1 >= n) break;
+                request(t1);
+            }
 #pragma unroll
-        for (int t = 0; t < kConvTile; ++t) {
-            if (t < n) {
-                load_ch<T, V>(in + (int64_t)(t0 + t) * p.proj_stride, x[TAPS - 1]);
+            for (int i = 0; i < BATCH; ++i) {
+                row[i].get(x[TAPS - 1]);
                 float a[V];
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
@@ -161,29 +212,37 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
                     for (int j = 0; j < TAPS; ++j) a[e] = fmaf(w[j][e], x[j][e], a[e]);
                     a[e] = silu_of<FAST>(a[e]);
                 }
-                store_ch<T, V>(out + (int64_t)t * p.channels, a);
+                if (t1 + i < n) store_ch<T, V>(out + (int64_t)(t1 + i) * p.channels, a);
 #pragma unroll
                 for (int j = 0; j + 1 < TAPS; ++j)
 #pragma unroll
                     for (int e = 0; e < V; ++e) x[j][e] = x[j + 1][e];
             }
         }
-    } else {
-        for (int t = 0; t < n; ++t) {
-            float a[V];
+        if (t0 == 0) {
 #pragma unroll
-            for (int e = 0; e < V; ++e) a[e] = bias[e];
-            for (int j = 0; j < taps; ++j) {
-                float w[V], x[V];
-                load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w);
-                input(t0 + t - (taps - 1) + j, x);
-#pragma unroll
-                for (int e = 0; e < V; ++e) a[e] = fmaf(w[e], x[e], a[e]);
+            for (int j = 0; j + 1 < TAPS; ++j) {
+                const int t = len - (TAPS - 1) + j;
+                if (t >= 0) keep[j].store(ring + (int64_t)((pos0 + t) % TAPS) * p.channels);
             }
-#pragma unroll
-            for (int e = 0; e < V; ++e) a[e] = silu_of<FAST>(a[e]);
-            store_ch<T, V>(out + (int64_t)t * p.channels, a);
         }
+        return;
+    }
+    load_ch<float, V>(p.conv_b + c, bias);
+    for (int t = 0; t < n; ++t) {
+        float a[V];
+#pragma unroll
+        for (int e = 0; e < V; ++e) a[e] = bias[e];
+        for (int j = 0; j < taps; ++j) {
+            float w[V], x[V];
+            load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w);
+            input(t0 + t - (taps - 1) + j, x);
+#pragma unroll
+            for (int e = 0; e < V; ++e) a[e] = fmaf(w[e], x[e], a[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) a[e] = silu_of<FAST>(a[e]);
+        store_ch<T, V>(out + (int64_t)t * p.channels, a);
     }
     if (t0 == 0) {
         for (int t = max(0, len - (taps - 1)); t < len; ++t) {
@@ -1110,21 +1169,31 @@ __global__ __launch_bounds__(256) void ssd_carry_kernel(SsmParams<__bf16> p) {
     }
 }
 
+template <typename T, int TILE>
+static int launch_conv_tiles(const SsmParams<T>& p, bool vec, hipStream_t s) {
+    const int64_t groups = vec ? p.channels / 8 : p.channels;
+    const int threads = (groups + 255) / 256 * 256 <= (groups + 191) / 192 * 192 ? 256 : 192;      // (fewer without channels)
+    const int64_t wgs = (p.n_rows / TILE + p.B) * ((groups + threads - 1) / threads);
+    if (wgs > 0x7fffffffLL) return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)wgs), block(threads);
+    if (!vec) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 1, 0, TILE>), grid, block, 0, s, p);
+    else if (p.taps == 2) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 2, TILE>), grid, block, 0, s, p);
+    else if (p.taps == 3) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 3, TILE>), grid, block, 0, s, p);
+    else if (p.taps == 4) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 4, TILE>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 0, TILE>), grid, block, 0, s, p);
+    return (int)hipGetLastError();
+}
+
 template <typename T>
 static int launch_conv(const SsmParams<T>& p, hipStream_t s) {
     bool vec = p.channels % 8 == 0 && p.xbc_at % 8 == 0 && p.proj_stride % 8 == 0;
     for (const void* ptr : {(const void*)p.proj, (const void*)p.conv_w, (const void*)p.conv_b, (const void*)p.conv_state, (const void*)p.xbc})
         vec = vec && (reinterpret_cast<uintptr_t>(ptr) & 15) == 0;
-    const int64_t groups = vec ? p.channels / 8 : p.channels;
-    const int64_t wgs = (p.n_rows / kConvTile + p.B) * ((groups + 255) / 256);
-    if (wgs > 0x7fffffffLL) return (int)hipErrorInvalidValue;
-    const dim3 grid((unsigned)wgs), block(256);
-    if (!vec) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 1, 0>), grid, block, 0, s, p);
-    else if (p.taps == 2) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 2>), grid, block, 0, s, p);
-    else if (p.taps == 3) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 3>), grid, block, 0, s, p);
-    else if (p.taps == 4) hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 4>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((causal_conv_silu_kernel<T, 8, 0>), grid, block, 0, s, p);
-    return (int)hipGetLastError();
+    // us with 4 / 8 / 16 tokens per thread: 64 tokens of 4352 channels 5.1, 5.0, 6.7; 577 of 4352 7.4, 7.4, 9.0; 1024 9.1, 10.1, 10.1; 4000 of 1280
+    // 10.3, 10.7, 10.9; 8000 16.5, 14.1, 15.2 (7200 of 2240: 16 is 2 faster than 8); 8192 of 4352 40.9, 34.2, 29.5
+    const int64_t inputs = p.n_rows * p.channels;
+    const int tile = inputs <= 6 << 20 ? 4 : inputs <= 12 << 20 ? 8 : 16;
+    return tile == 4 ? launch_conv_tiles<T, 4>(p, vec, s) : tile == 8 ? launch_conv_tiles<T, 8>(p, vec, s) : launch_conv_tiles<T, 16>(p, vec, s);
 }
 
 template <typename T, bool DECODE>

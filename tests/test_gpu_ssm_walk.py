@@ -55,3 +55,26 @@ def test_walk_of_whole_and_cut_sequences(ops):  # noqa: F811
         outs.append((y.float().cpu(), state.cpu()))
     for a, b in zip(*outs):                               # fp32 sums in another order; y then rounded to 8 bits
         assert float((a - b).norm() / b.norm()) <= 1e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_convolution_tiles(ops, dtype):  # noqa: F811
+    """4, 8 and 16 tokens per thread, by the size of a call: 4203 tokens of two sequences at once, in halves and in quarters with tokens left over; what is
+    left in the ring is the same, the outputs but for the order of the scan's fp32 sums."""
+    m = dict(heads=64, vdim=64, state=128, groups=1, taps=4)
+    kw = {k: m[k] for k in ("heads", "vdim", "state", "groups")}
+    print(f"case: convolution tiles {dtype}", flush=True)
+    n = 2101 if dtype == torch.bfloat16 else 701                          # (fp32 goes token by token behind the convolution)
+    proj, params, xbc_at, dt_at = ssm_case(m, 2 * n, 32, dtype)
+    proj, pc = proj.view(2, n, -1).cuda(), {k: v.cuda() for k, v in params.items()}
+    outs = []
+    for parts in (1, 2, 4):
+        conv, state = ssm_pools(m, 2, dtype)
+        cuts = [n * i // parts for i in range(parts + 1)]
+        ys = [ops.ssm_mix(proj[:, a:b].reshape(2 * (b - a), -1), xbc_at, dt_at, pc, conv, state, torch.tensor([1, 0]).int().cuda(),
+                          torch.arange(a, b).repeat(2).int().cuda(), torch.tensor([0, b - a, 2 * (b - a)]).int().cuda(), **kw).view(2, b - a, -1)
+              for a, b in zip(cuts, cuts[1:])]
+        outs.append((torch.cat(ys, 1).float().cpu(), conv.cpu()[:, [t % 4 for t in range(n - 3, n)]]))       # (the rows that a next token reads)
+    for y, conv in outs[1:]:
+        assert torch.equal(conv, outs[0][1])
+        assert float((y - outs[0][0]).norm() / outs[0][0].norm()) <= 1e-3
