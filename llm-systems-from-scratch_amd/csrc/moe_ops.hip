@@ -87,7 +87,8 @@ __device__ __forceinline__ void choose_experts(const RouteParams& p, float* z, i
 // Up to 64 logits: GROUP lanes per token, a lane owns one logit and counts those in front of it (larger, or as large with a
 // lower index), which is its place; 64 / GROUP tokens at a time.  The general form above walks the maxima one after the other,
 // six exchanges each: 16 of 23 us for 8192 tokens of 16 logits, four chosen, were spent there.  What is no number counts as
-// -inf, and a choice without a logit above -inf is expert E - 1, as there.
+// -inf, and a choice without a logit above -inf is expert E - 1, as there.  (Router of 32 logits with 64 / 32 lanes per token: 81 tokens 7.7 / 6.1 us,
+// 3588 8.4 / 6.5.)
 template <int GROUP>
 __device__ __forceinline__ void choose_by_rank(const RouteParams& p, const float* z, int64_t t0, int lane, int wave, int n_waves) {
     const int e = lane % GROUP;
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(64 * kRouteWaves) void moe_route_kernel(RouteParams
     __syncthreads();
     if (p.extra_logit && tid < 16 && t0 + tid < p.T) p.extra_logit[t0 + tid] = z[tid * p.n_logits + p.E];
     if (p.E <= 16) return choose_by_rank<16>(p, z, t0, lane, wave, kRouteWaves);
+    if (p.E <= 32) return choose_by_rank<32>(p, z, t0, lane, wave, kRouteWaves);
     if (p.E <= 64) return choose_by_rank<64>(p, z, t0, lane, wave, kRouteWaves);
     for (int t = wave; t < 16; t += kRouteWaves) {
         if (t0 + t >= p.T) break;

@@ -602,6 +602,11 @@ def test_router_places_choices(ops, E, top):
     assert torch.equal(ids.cpu(), torch.arange(top).repeat(2, 1).int()) and torch.allclose(wt.cpu(), torch.full((2, top), 1.0 / top))
 
 
+@pytest.mark.parametrize("E,top", [(17, 3), (31, 31), (32, 4)])
+def test_router_with_two_tokens_per_wavefront(ops, E, top):
+    test_router_places_choices(ops, E, top)
+
+
 # ---- the model ---------------------------------------------------------------------------------------------------------
 def attn(window, keep, **kw):
     return {"type": "attention", "mixer": dict(dict(heads=4, kv_heads=2, dim=24, vdim=24, rot={"base": 300.0, "dims": 24}, scale=0.25,
