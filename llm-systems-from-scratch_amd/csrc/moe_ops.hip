@@ -351,13 +351,20 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
     }
 }
 
-// 128 rows x 128 rows of w per workgroup (gate_up: 64 gates and the 64 ups of the same columns), k in steps of 64 through two
-// LDS buffers filled by direct loads.  A 128-byte LDS row holds its eight 16-byte pieces in the order piece ^ (row % 8).
+// 128 rows x 128 rows of w per workgroup (gate_up: 64 gates and the 64 ups of the same columns), k in steps of 64 through LDS,
+// filled by direct loads.  A 128-byte LDS row holds its eight 16-byte pieces in the order piece ^ (row % 8).
 // Wavefront (wm, wn) computes 64 x 64; weights are the MFMA's first operand, so that a lane ends with adjacent columns.
+// Bound by the latency of its weights where there are few rows: they come from HBM, the rows from an L2.  So weights have three buffers
+// and are requested two steps ahead, rows two and one: all that two workgroups per compute unit leave of its 160 KB.  us of router and both
+// products, two buffers of each / this / rows two and weights five steps ahead with one workgroup per compute unit:
+//   tokens x hidden, experts of width, top k    334 x 2048, 8 of 2048, 1    320 x 2048, 16 of 1024, 4    550 x 2048, 32 of 2048, 4
+//                                               86 / 75 / 78                78 / 72 / 73                 222 / 215 / 222
+//                                               2640 x 1024, 32 of 512, 4   4108 x 1024, 16 of 1024, 4   2609 x 2048, 8 of 1024, 1
+//                                               97 / 90 / 88                173 / 167 / 188              84 / 82 / 104
 template <bool GATE_UP>
 __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int chunk) {
-    constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];          // [buffer][rows | w]
+    constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2, NA = 2, NW = 3;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[(NA + NW) * kTile];          // rows, then w
     int n_tile, e, first, end;
     if (!find_dense_tile<BM>(p, blockIdx.x, n_tiles, chunk, n_tile, e, first, end)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -375,12 +382,13 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
         w_off[j] = (uint32_t)((wr * p.k + piece * 8) * 2);
     }
     const uint32_t lds0 = lds_address(lds);
-    const auto issue = [&](int k0, int buf) {
+    const auto issue_a = [&](int step, int slot) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            dma_to_lds_16(a_base + k0, a_off[j], lds0 + (2 * buf) * kTile + (32 * wave + 8 * j) * 128);
-            dma_to_lds_16(w_base + k0, w_off[j], lds0 + (2 * buf + 1) * kTile + (32 * wave + 8 * j) * 128);
-        }
+        for (int j = 0; j < 4; ++j) dma_to_lds_16(a_base + step * BK, a_off[j], lds0 + slot * kTile + (32 * wave + 8 * j) * 128);
+    };
+    const auto issue_w = [&](int step, int slot) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dma_to_lds_16(w_base + step * BK, w_off[j], lds0 + (NA + slot) * kTile + (32 * wave + 8 * j) * 128);
     };
     f32x4 acc[4][4];                              // [16 rows of w][16 rows]
 #pragma unroll
@@ -389,13 +397,21 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     // 16-row groups of w of this wavefront: gate_up: gates 32 wn, 32 wn + 16, then the ups of these columns
     const auto w_group = [&](int i) { return GATE_UP ? (i >> 1) * 64 + 32 * wn + (i & 1) * 16 : 64 * wn + 16 * i; };
-    issue(0, 0);
-    for (int k0 = 0, buf = 0; k0 < p.k; k0 += BK, buf ^= 1) {
-        wait_vmcnt<0>();
-        __syncthreads();                          // the tile has landed, and everybody has read the other buffer
-        if (k0 + BK < p.k) issue(k0 + BK, buf ^ 1);
-        const unsigned char* at = lds + (2 * buf) * kTile;
-        const unsigned char* wt = at + kTile;
+    // in the order of the loop: w of a step, its rows, w of the next
+    const int n_steps = p.k / BK;
+    issue_w(0, 0);
+    issue_a(0, 0);
+    if (n_steps > 1) issue_w(1, 1);
+    for (int t = 0, sa = 0, sw = 0; t < n_steps; ++t) {
+        if (t + 1 < n_steps) wait_vmcnt<4>();     // all but w of step t + 1 has landed
+        else wait_vmcnt<0>();
+        __syncthreads();                          // ... everybody's, and everybody has read the step before
+        if (t + 1 < n_steps) issue_a(t + 1, sa ^ 1);
+        if (t + 2 < n_steps) issue_w(t + 2, sw == 0 ? 2 : sw - 1);
+        const unsigned char* at = lds + sa * kTile;
+        const unsigned char* wt = lds + (NA + sw) * kTile;
+        sa ^= 1;
+        sw = sw == 2 ? 0 : sw + 1;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int piece = ((4 * s + kg) ^ (r & 7)) * 16;

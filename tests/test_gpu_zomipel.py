@@ -584,6 +584,22 @@ def test_expert_tile_rounds(ops, idle, k, ff, n):
         assert float((got[mine].float() - ref[mine]).norm()) <= 2 ** -7 * float(ref[mine].norm())
 
 
+@pytest.mark.parametrize("k,ff", [(64, 64), (128, 192), (192, 128), (256, 320), (448, 512)])
+def test_expert_rings(ops, k, ff):
+    """128 x 128 tiles whose k has one step, as many as there are buffers and fewer, and turns of both rings.  Bound as in test_expert_tilings."""
+    T, E, n, bf = 300, 3, 136, torch.bfloat16
+    print(f"case: expert rings {k} {ff}", flush=True)
+    h, wg = rnd(T, k, seed=1, dtype=bf).cuda(), rnd(E, 2 * ff, k, seed=2, std=k ** -0.5, dtype=bf).cuda()
+    wd, wt = rnd(E, n, ff, seed=3, std=ff ** -0.5, dtype=bf).cuda(), torch.rand(T, 1, generator=gen(4)).cuda()
+    ids = torch.randint(0, E, (T, 1), generator=gen(5)).int().cuda()
+    got = ops.moe_experts(h, ids, wt, wg, wd, tiling="large")
+    for e in range(E):
+        mine = (ids == e)[:, 0]
+        z = h[mine].float() @ wg[e].float().T
+        ref = wt[mine] * ((zo.silu(z[:, :ff]) * z[:, ff:]) @ wd[e].float().T)
+        assert bool(torch.isfinite(got).all()) and float((got[mine].float() - ref).norm()) <= 2 ** -8 * float(ref.norm())
+
+
 @pytest.mark.parametrize("E,top", [(5, 5), (16, 4), (33, 7), (64, 64)])
 def test_router_places_choices(ops, E, top):
     """Experts that are switched off by a bias of -inf, ties, and infinities that leave too few choices."""
