@@ -1,9 +1,9 @@
 // FlashAttention-style prefill forward for gfx950 (bf16, MFMA 32x32x16).
 //
-// One workgroup = 8 wavefronts (two per SIMD, one workgroup per CU) = one tile of 256 queries
-// of one (batch, head); each wavefront owns 32 query rows.  K/V tiles of 64 keys are double-buffered in
-// LDS and shared by the eight wavefronts (256 queries per loaded tile: half the L2->LDS
-// traffic per MFMA of a 128-query workgroup, worth +1.5 %).  Per wavefront and KV tile:
+// One workgroup = NW wavefronts = one tile of 32 NW queries of one (batch, head); each wavefront owns 32 query rows.
+// K/V tiles of 64 keys are double-buffered in LDS and shared by the wavefronts.  NW 8 (head_dim 128: two wavefronts per SIMD, one workgroup
+// per CU): 256 queries per loaded tile, half the L2->LDS traffic per MFMA of a 128-query workgroup, worth +1.5 %.  NW 4 (head_dim 32 and 64):
+// see below.  Per wavefront and KV tile:
 //
 //   S^T (64 keys x 32 queries) = K . Q^T     K fragments: ds_read_b128 from LDS,
 //                                            Q^T fragments live in registers
@@ -31,10 +31,10 @@
 #include "launch.hpp"
 #include "prefill_params.hpp"
 #include "prefill_tile.hpp"
+#include "xcd_order.hpp"
 
 namespace mi355 {
 
-constexpr int kPfWaves = 8;
 constexpr int kBM = 256;   // queries per workgroup
 constexpr int kBN = 64;    // keys per LDS tile
 
@@ -42,22 +42,30 @@ constexpr int kBN = 64;    // keys per LDS tile
 // PAGED: keys and values are read from a paged cache through a block table (16 rows per block, so
 // every direct-to-LDS instruction -- 4, 8 or 16 whole rows -- stays inside one block and needs one
 // table entry, a scalar load); queries and outputs are packed.
-// Occupancy: at head_dim 64 the kernel is held to the registers of four wavefronts per SIMD (128; left alone the
-// compiler takes 163 and a compute unit then holds ONE workgroup, whose barriers and waits nobody fills): two
-// workgroups per compute unit, 7-8 % faster at throughput shapes and 14 % on short sequences, a handful of spilled
-// registers outside the tile loop.  Head_dim 32 has two workgroups per compute unit as it is (117 registers; a third
-// would need 85 and spills by the hundred: three to four times slower), head_dim 128 needs its 250.
+// Occupancy: at head_dim 64 and 32 the kernel is held to the registers of four wavefronts per SIMD (128; left alone the
+// compiler takes 163 at head_dim 64), a handful of spilled registers outside the tile loop.  Head_dim 128 needs its 250.
+// NW 4, head_dim 32 and 64: four workgroups per compute unit, whose output rows are staged in the place of the last K/V tiles and whose query rows
+// come in without staging (34 and 17 KB of LDS; 70 and 37 with eight wavefronts, two workgroups).  On the diagonal and at the ragged end the
+// wavefronts of a workgroup wait for the one with the most keys, so that smaller workgroups leave less idle, and the launch is dealt finer; the
+// tiles that are loaded twice as often come out of the L2.  Causal, heads of 64 / 32, us with eight wavefronts and pairs of query tiles / with four and the
+// tiles as with_units deals them: 64 heads of 1456 tokens 43 / 36 and 32 / 25, 64 of 3000 125 / 95 and 89 / 64, 136 of 1456 75 / 60 and 54 / 45, 1024 of 300
+// 65 / 60 and 40 / 30, 1024 of 700 152 / 140 and 102 / 79, 8 of 8192 138 / 105 and 99 / 68, 64 of 8192 549 / 568 and 352 / 364; 22 packed sequences
+// of 1334, 8 heads of 64, 92 / 65; 14 of 111 to 1172, 32 heads, 80 / 60.
+// With keys split and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
+// 9000 tokens, 32 heads of 64, 290 us, with four 325; 16 of 333 over 1500, heads of 32, 40 and 34.
 // WINDOW (causal): a query tile walks the K/V tiles that hold the kept first tokens, then those from its window's first
 // key on, as one sequence of tiles (tile_of); keys outside are masked in the tiles at the window's lower edge.
-template <int D, int MODE, bool PAGED = false, bool WINDOW = false>
-__global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_kernel(PrefillParams p) {
+template <int D, int MODE, bool PAGED, bool WINDOW, int NW>
+__global__ __launch_bounds__(NW * 64, D == 64 || NW == 4 ? 4 : 1) void prefill_fwd_kernel(PrefillParams p) {
+    constexpr int BM = 32 * NW;                   // queries per workgroup
+    constexpr bool kOwnSlab = NW == 8;            // staging of rows has LDS of its own
     constexpr int NS = D / 16;                    // MFMA k-steps of K.Q^T
     constexpr int NDT = D / 32;                   // 32-row tiles of O^T
     constexpr int CPR = D / 8;                    // 16-byte chunks per row
     constexpr int kRow = D * 2;                   // bytes per LDS row
     constexpr int kTile = kBN * kRow;             // bytes per K (or V) tile
     constexpr int NT = kBN * CPR / 64;            // direct-to-LDS instructions per tile and tensor
-    constexpr int NI = (NT + kPfWaves - 1) / kPfWaves;   // ... per wavefront (the last wavefronts may have none)
+    constexpr int NI = (NT + NW - 1) / NW;   // ... per wavefront (the last wavefronts may have none)
 
     // K/V tile buffers: tile t lives in buffer t % NB, and while tile t is computed tile t+1 is landing.  (Four buffers
     // with three tiles in flight were tried for head_dim 64 and 32, where a tile is only a few hundred cycles of work:
@@ -68,23 +76,37 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
     constexpr float kBias = 32.0f;             // first attempt: the weight of a score x (log2 domain) is 2^(x - kBias)
     constexpr float kUnderflow = 0x1p-92f;     // a final row sum below this may have lost terms
     constexpr float kOverflow = 0x1p40f;       // ... above this (or NaN) may have overflowed somewhere
-    __shared__ __attribute__((aligned(1024))) unsigned char k_lds[NB * kTile];
-    __shared__ __attribute__((aligned(1024))) unsigned char v_lds[NB * kTile];
+    __shared__ __attribute__((aligned(1024))) unsigned char kv_lds[2 * NB * kTile];
+    unsigned char* const k_lds = kv_lds;
+    unsigned char* const v_lds = kv_lds + NB * kTile;
     // Staging of the query rows on their way in and of the output rows on their way out, one private slab per
     // wavefront (32 rows of D bf16, rows padded by 16 bytes): fragments and accumulators hold a query per lane,
     // so direct accesses would touch 16- or 8-byte pieces of 32 different rows per instruction; through the
     // slab every global instruction moves whole 2*D-byte rows (+2.4 % for the stores alone at D = 128).
     constexpr int kORow = D * 2 + 16;
-    __shared__ __attribute__((aligned(16))) unsigned char o_lds[kPfWaves * 32 * kORow];
+    static_assert(kOwnSlab || NW * 32 * kORow <= 2 * NB * kTile, "rows in the place of the tiles");
+    __shared__ __attribute__((aligned(16))) unsigned char o_own[kOwnSlab ? NW * 32 * kORow : 16];
+    unsigned char* const o_lds = kOwnSlab ? o_own : kv_lds;
 
-    // Logical order: pair fastest, then the query heads of one kv head, then kv head, then batch.  The workgroups
-    // that stream the same K/V -- the pairs and query heads of one kv head -- form a chunk of that order and run on
-    // one XCD.
-    const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, p.n_pairs * (p.Hq / p.Hkv));
+    // The workgroups that stream the same K/V -- the units and query heads of one kv head -- run on one XCD.
+    // Pairs: pair fastest, then the query heads of one kv head, then kv head, then batch.
+    // Single tiles: by falling number, so that the dearest begin first and what is left for the end is small (xcd_unit).
     const int split = blockIdx.y;                    // share of the keys this workgroup serves (gridDim.y = n_split)
-    const int pair0 = lid % p.n_pairs;
-    const int h = (lid / p.n_pairs) % p.Hq;
-    const int b = lid / (p.n_pairs * p.Hq);
+    const bool singles = p.single_tiles != 0;
+    int pair0, head;
+    if (singles) {
+        const HeadUnit at = xcd_unit(blockIdx.x, p.n_pairs, p.Hq / p.Hkv, p.Hkv * p.B, p.chunk_heads, p.round);
+        if (at.unit < 0) return;
+        pair0 = p.n_pairs - 1 - at.unit;
+        head = at.head;
+    } else {
+        const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, p.n_pairs * (p.Hq / p.Hkv));
+        pair0 = lid % p.n_pairs;
+        head = lid / p.n_pairs;
+    }
+    pair0 = __builtin_amdgcn_readfirstlane(pair0);
+    const int b = __builtin_amdgcn_readfirstlane(head / p.Hq);
+    const int h = __builtin_amdgcn_readfirstlane(head - b * p.Hq);
     const int hk = h / (p.Hq / p.Hkv);
     const float scale_log2 = p.head_scale ? p.scale_log2 * p.head_scale[h] : p.scale_log2;
 
@@ -120,12 +142,9 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
         ob = p.out + (int64_t)b * p.os[0] + (int64_t)h * p.os[1];
         lb = p.lse ? p.lse + (int64_t)b * p.ls[0] + (int64_t)h * p.ls[1] : nullptr;
     }
-    // Causal work grows with the query-tile index, so a workgroup takes the tiles
+    // Causal work grows with the query-tile index, so a workgroup of pairs takes the tiles
     // (nq-1-pair) and (pair): every workgroup of a sequence then carries the same load.
-    // (A launch that would leave compute units without a workgroup deals single query tiles instead, heaviest first:
-    // p.n_pairs then counts tiles.)
-    const int nq = (sq + kBM - 1) / kBM;
-    const bool singles = p.single_tiles != 0;
+    const int nq = (sq + BM - 1) / BM;
     if ((singles ? pair0 : 2 * pair0) >= nq) return;         // (a sequence without keys still gets its rows written: no key kept -> NaN)
 
     const int tid = threadIdx.x;
@@ -228,15 +247,15 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
     // (with a correct Sq_max this loop runs once).
     for (int pair = pair0; (singles ? pair : 2 * pair) < nq; pair += p.n_pairs)
     for (int half = 0; half < (singles ? 1 : 2); ++half) {
-        const int qtile = half == 0 ? nq - 1 - pair : pair;
+        const int qtile = half == 0 && !singles ? nq - 1 - pair : pair;
         if (half == 1 && qtile == nq - 1 - pair) break;         // odd tile count: the middle tile has no partner
-        const int q0 = qtile * kBM;
+        const int q0 = qtile * BM;
         const int qw0 = q0 + 32 * wave;                    // first query of this wavefront
         const int qi = qw0 + n;                            // this lane's query
         const bool q_ok = qi < sq;
 
         int kv_end = sk;
-        if (causal) kv_end = max(0, min(sk, min(sq, q0 + kBM) + coff));
+        if (causal) kv_end = max(0, min(sk, min(sq, q0 + BM) + coff));
         int n_tiles = (kv_end + kBN - 1) / kBN;
         int kept_tiles = 0, skip = 0;              // WINDOW: tiles with kept tokens, and tiles left out behind them
         if constexpr (WINDOW) {
@@ -262,7 +281,13 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
         // rows come in whole (CPR lanes per row) and go through the wavefront's slab (private, and LDS operations
         // of a wavefront execute in order: no barrier); rows past the end of the sequence are zero
         bf16x8 qf[NS];
-        {
+        if constexpr (!kOwnSlab) {                           // (rows past the end repeat the last one and are not stored)
+            const __bf16* qrow = qb + (int64_t)min(qi, sq - 1) * p.qs[2] + 8 * kg;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) qf[s] = as_bf16x8(*reinterpret_cast<const u32x4*>(qrow + 16 * s));
+#pragma unroll
+            for (int s = 0; s < NS; ++s) asm volatile("" : "+v"(qf[s]));
+        } else {
             unsigned char* slab = o_lds + wave * (32 * kORow);
             constexpr int kRowsPerPass = 64 / CPR;
             const int c = lane % CPR, r0 = lane / CPR;
@@ -556,6 +581,7 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
             lb[qi] = l_run > 0.f ? 0.69314718056f * (__log2f(l_run) - neg_ref) : -INFINITY;
         {
             // (the slab is private to the wavefront and LDS operations of a wavefront execute in order: no barrier)
+            if constexpr (!kOwnSlab) __syncthreads();        // everybody is done with the tiles
             unsigned char* slab = o_lds + wave * (32 * kORow);
             unsigned char* mine = slab + n * kORow + 8 * kg;
 #pragma unroll
@@ -580,39 +606,62 @@ __global__ __launch_bounds__(kPfWaves * 64, D == 64 ? 4 : 1) void prefill_fwd_ke
     }
 }
 
-// Pairs of query tiles carry equal causal work, but a launch with fewer pairs than the GPU can hold at once (two
-// workgroups per compute unit) leaves compute units idle and makes every workgroup walk two tiles: such a launch
-// deals single tiles instead.
-static PrefillParams with_units(const PrefillParams& p0) {
-    PrefillParams p = p0;
-    p.single_tiles = 0;
-    int dev = 0, n_cu = 0;
-    if (p.n_qtiles > 1 && hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) {
-        const int64_t wgs = (int64_t)p.n_pairs * p.Hq * p.B * (p.n_split > 1 ? p.n_split : 1);
-        if (wgs < 2 * (int64_t)n_cu) {
-            p.single_tiles = 1;
-            p.n_pairs = p.n_qtiles;
-        }
-    }
-    return p;
+static int device_compute_units() {
+    static std::atomic<int> known[64];                // (asked of the runtime once per device)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
+    return n;
 }
 
-template <int D>
-static int launch_prefill(const PrefillParams& p0, hipStream_t stream) {
-    const PrefillParams p = with_units(p0);
-    // one workgroup per PAIR of query tiles (or per tile), 1-D in x (see the id remap); y = share of the keys
-    dim3 grid((unsigned)(p.n_pairs * p.Hq * p.B), (unsigned)(p.n_split > 1 ? p.n_split : 1));
-    dim3 block(kPfWaves * 64);
+// Query tiles in pairs, which carry equal causal work, or one by one, the dearest first (see the kernel).
+// One by one fills the chip better: the launch ends with small pieces, and sequences of different lengths, windows and launches without a mask have no equal
+// pairs.  A pair's two tiles and its neighbours read the same keys at about the same time, which counts where the launch goes over the chip many
+// times: NW 4, causal, heads of 64, singles / pairs: 136 heads of 1456 tokens 60 / 68 us, 64 of 8192 (four rounds) 568 / 581, 1024 of 700 (six) 150 /
+// 140, 256 of 3000 (six) 370 / 354.  So pairs from more than four rounds on, and with eight wavefronts from two workgroups per compute unit on.
+// (Packed: 35 sequences of 386 to 2835 tokens, 32 heads of 32, 434 / 480; 18 of 319 to 2850, 32 heads of 128, window of 512, NW 8, 471 / 517.)
+// An XCD takes as many kv heads at a time as have 8 MB of keys and values, twice its L2: with more, 512 heads of 1024 tokens take 126 us instead of 120.
+static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
+    PrefillParams p = p0;
+    p.n_qtiles = (p.Sq + 32 * waves - 1) / (32 * waves);
+    p.n_pairs = (p.n_qtiles + 1) / 2;
+    const int64_t n_cu = std::max(1, device_compute_units()), heads = (int64_t)p.Hq * p.B * std::max(1, p.n_split), tiles = p.n_qtiles * heads;
+    const int64_t resident = n_cu * (waves == 4 ? 4 : (D == 128 ? 1 : 2));                     // workgroups
+    const bool equal = p.mask_mode == MI355_MASK_CAUSAL && !(p.window > 0 && p.window < p.Sq) && (!p.cu_q || p.B == 1 || p.n_split > 1);
+    const bool pairs = equal && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
+    p.single_tiles = !pairs && tiles < 1 << 24;                                                // (a grid's threads are counted in 32 bits)
+    if (p.single_tiles) p.n_pairs = p.n_qtiles;
+    const int64_t keys = p.block_table ? 16 * (int64_t)p.max_blocks : p.Sk, kv_heads = (8 << 20) / (std::max<int64_t>(1, keys) * D * 4);
+    p.chunk_heads = p.Hq / p.Hkv * (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)p.Hkv * p.B / 8, kv_heads));
+    p.round = p.n_split <= 1 && tiles <= resident ? (int)(n_cu / 8) : 0;
+    return p;
+}
+static unsigned units_grid(const PrefillParams& p) {
+    return p.single_tiles ? (unsigned)xcd_units_grid(p.n_pairs, p.Hq / p.Hkv, p.Hkv * p.B) : (unsigned)(p.n_pairs * p.Hq * p.B);
+}
+template <int D, int NW>
+static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {
+    const PrefillParams p = with_units(p0, NW, D);
+    // 1-D in x (see the kernel's order); y = share of the keys
+    const dim3 grid(units_grid(p), (unsigned)(p.n_split > 1 ? p.n_split : 1)), block(NW * 64);
     if (p.mask_mode == MI355_MASK_CAUSAL && p.window > 0)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, true>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, true, NW>), grid, block, 0, stream, p);
     else if (p.mask_mode == MI355_MASK_CAUSAL)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, false, NW>), grid, block, 0, stream, p);
     else if (p.mask_mode == MI355_MASK_BOOL)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_BOOL>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_BOOL, false, false, NW>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE, false, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
+}
+// (the lines between four and eight wavefronts: see the kernel)
+template <int D>
+static int launch_prefill(const PrefillParams& p, hipStream_t stream) {
+    if constexpr (D != 128)
+        if (p.n_split <= 1) return launch_prefill_of<D, 4>(p, stream);
+    return launch_prefill_of<D, 8>(p, stream);
 }
 
 // Merge of the split-key partials: one wavefront per (query row, head).
@@ -692,15 +741,20 @@ static int launch_merge(const PrefillParams& p, int D, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
-template <int D>
-static int launch_prefill_paged(const PrefillParams& p0, hipStream_t stream) {
-    const PrefillParams p = with_units(p0);
-    dim3 grid((unsigned)(p.n_pairs * p.Hq * p.B), (unsigned)(p.n_split > 1 ? p.n_split : 1));
-    if (p.window > 0)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, true, true>), grid, dim3(kPfWaves * 64), 0, stream, p);
-    else
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, true>), grid, dim3(kPfWaves * 64), 0, stream, p);
+template <int D, int NW>
+static int launch_prefill_paged_of(const PrefillParams& p0, hipStream_t stream) {
+    const PrefillParams p = with_units(p0, NW, D);
+    const dim3 grid(units_grid(p), (unsigned)(p.n_split > 1 ? p.n_split : 1)), block(NW * 64);
+    if (p.window > 0) hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, true, true, NW>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, true, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
+}
+constexpr int kSmallPaged = 128;                  // blocks: paged contexts that four wavefronts take
+template <int D>
+static int launch_prefill_paged(const PrefillParams& p, hipStream_t stream) {
+    if constexpr (D != 128)
+        if (p.n_split <= 1 && p.max_blocks <= kSmallPaged) return launch_prefill_paged_of<D, 4>(p, stream);
+    return launch_prefill_paged_of<D, 8>(p, stream);
 }
 
 }  // namespace mi355
@@ -733,18 +787,8 @@ static int set_split(PrefillParams& p, int D, int n_split, int64_t total_q_rows,
     return 0;
 }
 
-static int device_compute_units() {
-    static std::atomic<int> known[64];                // (asked of the runtime once per device)
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    if (dev >= 0 && dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
-    return n;
-}
-
 // Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; lengths of a packed batch are
-// judged by the longest).
+// judged by the longest; of the rougher fits eight per cent are taken off).
 static double other_us(const PrefillParams& p, int D, int n_cu) {
     const bool causal = p.mask_mode == MI355_MASK_CAUSAL;
     const int Sk = p.block_table ? 16 * p.max_blocks : p.Sk;
@@ -752,7 +796,7 @@ static double other_us(const PrefillParams& p, int D, int n_cu) {
     const double heads = (double)p.Hq * p.B, kt = std::ceil(most / kBN);
     if (prefill_short_takes(p, D)) {
         // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
-        return (D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu;
+        return 0.92 * ((D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu);
     }
     // query tiles of a launch, dearest and mean number of key tiles; per key tile, per query tile, and what is the same for every call
     const bool wide = D == 128 && prefill_w64_takes(p), by_head = wide && causal && p.Hq / p.Hkv % 4 == 0;
@@ -761,21 +805,28 @@ static double other_us(const PrefillParams& p, int D, int n_cu) {
     if (wide) {
         // the last three key tiles of a length that is no multiple of 64 run in ordinary code, some 4 us each more
         const double tail = Sk % kBN ? 12.0 : 0.0;
-        return 9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * mean + 4.0 + tail / (causal ? qt : 1.0)));
+        return 0.92 * (9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * mean + 4.0 + tail / (causal ? qt : 1.0))));
+    }
+    if (D != 128 && (!p.block_table || p.max_blocks <= kSmallPaged)) {
+        // four wavefronts: the chain of the dearest tile and what a compute unit has to do, of which the longer one counts, and more where they are alike
+        // (150 calls of 1 to 1024 heads of 64 to 3000 tokens: 4 % off)
+        const double qt4 = std::ceil(p.Sq / 128.0), mean4 = causal ? std::min(kt, (over + 0.5 * p.Sq + 64.0) / kBN) : kt;
+        const double chain = (D == 64 ? 0.79 : 0.53) * kt, all = qt4 * heads / n_cu * (D == 64 ? 0.57 * mean4 + 2.33 : 0.354 * mean4 + 1.08);
+        return (D == 64 ? 6.5 : 4.9) + std::cbrt(chain * chain * chain + all * all * all);
     }
     const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75;
-    return 5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * mean + 2.0));
+    return 0.92 * (5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * mean + 2.0)));
 }
 
 // Wavefronts of prefill_keys.hip's kernel for p, 0: another kernel is the faster one.  One 183-token prompt, 16 heads, D 128: 64-query kernel 26.4 us, keys dealt to
-// the wavefronts 7.6; 4 of 700: 37.4, 33.0; of 1000: 44.9, 49.8; D 64, one of 1000: 21.9, 12.1; 4 of 1000: 24.6, 26.8.  Eight per cent are left to the fit.
+// the wavefronts 7.6; 4 of 700: 37.4, 33.0; of 1000: 44.9, 49.8; D 64, one of 1000: 18.7, 12.1; 8 sequences of 666, 8 heads: 18.1, 17.7; of 750: 20.4, 20.6.
 // (Training calls of short heads stay with the kernel that rounds fp32 operands on their way in: the same bits whichever type the inputs have.)
 static int keys_wavefronts(const PrefillParams& p, int D) {
     if (p.lse && prefill_short_takes(p, D)) return 0;
     const int n_cu = prefill_keys_takes(p, D) ? device_compute_units() : 0;
     if (n_cu <= 0) return 0;
     const PrefillKeysPlan plan = prefill_keys_plan(p.B, p.Hq, D, p.Sq, p.block_table ? 16 * p.max_blocks : p.Sk, p.mask_mode == MI355_MASK_CAUSAL, n_cu);
-    return plan.us < 0.92 * other_us(p, D, n_cu) ? plan.wavefronts : 0;
+    return plan.us < other_us(p, D, n_cu) ? plan.wavefronts : 0;
 }
 
 static int prefill_common(const void* q, const void* k, const void* v, void* out, const int64_t q_strides[3],

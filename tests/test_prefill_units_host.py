@@ -1,0 +1,51 @@
+"""The order of a launch's query tiles over the eight XCDs, checked on the CPU."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+import mi355_attn
+
+
+@pytest.fixture(scope="module")
+def order(tmp_path_factory):
+    d = tmp_path_factory.mktemp("units")
+    src, lib = d / "units.cpp", d / "units.so"
+    src.write_text('#include "xcd_order.hpp"\n'
+                   'extern "C" int units(int u, int group, int groups, int chunk, int round, int* out) {\n'
+                   '  const int n = mi355::xcd_units_grid(u, group, groups);\n'
+                   '  for (int i = 0; out && i < n; ++i) { const auto x = mi355::xcd_unit(i, u, group, groups, chunk, round); out[2 * i] = x.unit; out[2 * i + 1] = x.head; }\n'
+                   '  return n; }\n')
+    csrc = os.path.join(os.path.dirname(os.path.dirname(mi355_attn.__file__)), "csrc")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
+    fn = ctypes.CDLL(str(lib)).units
+
+    def units(u, group, groups, chunk, rnd):
+        n = fn(u, group, groups, chunk, rnd, None)
+        out = (ctypes.c_int * (2 * n))()
+        fn(u, group, groups, chunk, rnd, out)
+        return [(out[2 * i], out[2 * i + 1]) for i in range(n)]
+    return units
+
+
+@pytest.mark.parametrize("rnd", [0, 32])
+@pytest.mark.parametrize("group", [1, 4, 5])
+@pytest.mark.parametrize("u,groups", [(1, 1), (1, 8), (3, 7), (2, 9), (11, 16), (6, 37), (64, 8), (5, 129)])
+def test_every_unit_once(order, u, groups, group, rnd):
+    """Every unit of every head has one workgroup, and at most seven more have none; an XCD (workgroup modulo 8) keeps to its own kv heads beyond the first
+    groups % 8 of them, takes whole chunks, and begins a chunk's units in order."""
+    for chunk in {group, group * max(1, groups // 16), group * max(1, groups // 8)}:
+        got = order(u, group, groups, chunk, rnd)
+        work = [x for x in got if x[0] >= 0]
+        assert len(got) - len(work) <= 7
+        assert sorted(work) == sorted((i, h) for i in range(u) for h in range(group * groups))
+        front = -(-(groups % 8 * group * u) // 8) * 8
+        assert all(h >= groups // 8 * 8 * group for i, h in got[:front] if i >= 0)
+        for xcd in range(8):
+            mine = got[front + xcd::8]
+            assert {h // group % 8 for _, h in mine} <= {xcd}
+            if rnd == 0:
+                for c in range(0, len(mine), chunk * u):
+                    units = [i for i, _ in mine[c:c + chunk * u]]
+                    assert units == sorted(units) and len({h for _, h in mine[c:c + chunk * u]}) <= chunk
