@@ -29,6 +29,7 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "prefill_bwd_params.hpp"
+#include "xcd_order.hpp"
 #include "prefill_tile.hpp"
 
 namespace mi355 {
@@ -89,27 +90,41 @@ struct TileLoader {
 };
 
 // ---------------------------------------------------------------------------------------------
-// dQ: one workgroup per tile of 128 queries of one (batch, query head); K/V stream through LDS.
+// dQ: one workgroup of NWV wavefronts per 32 NWV queries of one (batch, query head); K/V stream through LDS.
 // Per wavefront: Q and dO fragments of its 32 query columns in registers (64), dQ^T accumulators (64).
-template <int D, int MODE>
-__global__ __launch_bounds__(kBwWaves * 64, 1) void bwd_dq_kernel(BwdParams p) {
+// NWV 4 at head sizes 64 and 32: three and four workgroups per compute unit (165 and 120 registers), where of eight wavefronts one is all that 161
+// registers leave at 64.  They wait less for the wavefront with the most keys and a launch is dealt finer (as in prefill_fwd_kernel).
+// us, eight wavefronts and pairs of tiles / four and single tiles, causal: heads of 64: 136 of 700 tokens 57 / 27, 136 of 1456 100 / 72, 64 of 3000 168 /
+// 119, 64 of 8192 869 / 774; 35 packed of 269 to 2871, 32 heads, 1136 / 805; heads of 32: 136 of 700 31 / 18, 64 of 3000 98 / 76, 256 of 1456 86 / 78.
+constexpr int dq_resident(int D) { return D == 32 ? 4 : 3; }                        // workgroups of four wavefronts per compute unit
+template <int D, int MODE, int NWV>
+__global__ __launch_bounds__(NWV * 64, NWV == 4 ? dq_resident(D) : 1) void bwd_dq_kernel(BwdParams p) {
     constexpr bool CAUSAL = MODE == MI355_MASK_CAUSAL, BOOLM = MODE == MI355_MASK_BOOL;
-    constexpr int NWV = kBwWaves;
+    constexpr int BM = 32 * NWV;                  // queries per workgroup
     using R = TileReads<D>;
     constexpr int NS = R::NS, NDT = R::NDT, kRow = R::kRow, kTile = kBwRows * kRow;
     // [K buffer 0][K buffer 1][V buffer 0][V buffer 1]
     __shared__ __attribute__((aligned(1024))) unsigned char lds[4 * kTile];
 
     // Workgroup ids are dealt round-robin to the 8 XCDs (private L2s) and, in order, to their shader
-    // engines: workgroups must carry EQUAL work (a periodic heavy/light pattern starves the engines that
-    // always draw the light ones), and the workgroups that stream the same K/V should share an XCD.  So a
-    // workgroup takes the query-tile PAIR (nq-1-i, i), and the pairs and query heads of one kv head -- a chunk
-    // of the logical order (pair, query head, batch) -- run on one XCD.
-    const int n_pairs = (p.n_qtiles + 1) / 2;
-    const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, n_pairs * (p.Hq / p.Hkv));
-    const int pair = lid % n_pairs;
-    const int h = (lid / n_pairs) % p.Hq;
-    const int b = lid / (n_pairs * p.Hq);
+    // engines: a periodic heavy/light pattern starves the engines that always draw the light ones, and the workgroups that stream
+    // the same K/V should share an XCD.  So a workgroup takes the query-tile PAIR (nq-1-i, i), and the pairs and query heads of
+    // one kv head -- a chunk of the logical order (pair, query head, batch) -- run on one XCD; or one tile, the dearest of the
+    // launch first.
+    const bool singles = p.deal.singles;
+    int pair, head;
+    if (singles) {
+        const HeadUnit at = xcd_unit(blockIdx.x, p.deal.units, p.Hq / p.Hkv, p.Hkv * p.B, p.deal.chunk_heads, p.deal.round);
+        if (at.unit < 0) return;
+        pair = p.deal.units - 1 - at.unit;
+        head = at.head;
+    } else {
+        const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, p.deal.units * (p.Hq / p.Hkv));
+        pair = lid % p.deal.units;
+        head = lid / p.deal.units;
+    }
+    pair = __builtin_amdgcn_readfirstlane(pair);
+    const int b = __builtin_amdgcn_readfirstlane(head / p.Hq), h = __builtin_amdgcn_readfirstlane(head - b * p.Hq);
     const int hk = h / (p.Hq / p.Hkv);
     int sq, sk;
     int64_t q_base, k_base, v_base, do_base, dq_base, l_base, o_base;
@@ -135,8 +150,8 @@ __global__ __launch_bounds__(kBwWaves * 64, 1) void bwd_dq_kernel(BwdParams p) {
         v_base = (int64_t)b * p.vs[0] + (int64_t)hk * p.vs[1];
         l_base = (int64_t)b * p.ls[0] + (int64_t)h * p.ls[1];
     }
-    const int nq = (sq + kBwCols - 1) / kBwCols;
-    if (2 * pair >= nq) return;                                         // (a sequence without keys still gets dq = 0 written)
+    const int nq = (sq + BM - 1) / BM;
+    if ((singles ? pair : 2 * pair) >= nq) return;                                         // (a sequence without keys still gets dq = 0 written)
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -149,10 +164,10 @@ __global__ __launch_bounds__(kBwWaves * 64, 1) void bwd_dq_kernel(BwdParams p) {
     rd.init(lane);
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_address(lds) + wave * TileLoader<D, NWV>::NI * 1024);
 
-    for (int half = 0; half < 2; ++half) {
-        const int qtile = half == 0 ? nq - 1 - pair : pair;
-        if (half == 1 && qtile == nq - 1 - pair) break;                 // odd tile count: the middle tile has no partner
-        const int q0 = qtile * kBwCols;
+    // single tiles: one, unless a packed sequence is longer than the caller said
+    for (int half = 0, qtile = singles ? pair : nq - 1 - pair; singles ? qtile < nq : half < 2; ++half, qtile = singles ? qtile + p.deal.units : pair) {
+        if (!singles && half == 1 && pair == nq - 1 - pair) break;                 // odd tile count: the middle tile has no partner
+        const int q0 = qtile * BM;
         const int qw0 = q0 + 32 * wave;
         const int qi = qw0 + n;
         const bool q_ok = qi < sq;
@@ -198,7 +213,7 @@ __global__ __launch_bounds__(kBwWaves * 64, 1) void bwd_dq_kernel(BwdParams p) {
         for (int j = 0; j < 16; ++j) neg_delta16[j] = -delta;
 
         int kv_end = sk;
-        if (CAUSAL) kv_end = max(0, min(sk, min(sq, q0 + kBwCols) + coff));
+        if (CAUSAL) kv_end = max(0, min(sk, min(sq, q0 + BM) + coff));
         const int n_tiles = (kv_end + kBwRows - 1) / kBwRows;
         const int last_key = CAUSAL ? min(sk - 1, qi + coff) : sk - 1;      // last key this lane's query sees
         const int wave_last_key = CAUSAL ? min(sk - 1, qw0 + coff) : sk - 1;   // ... and the last one ALL queries of the wavefront see
@@ -1038,13 +1053,22 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
     __shared__ __attribute__((aligned(16))) float lse_lds2[2 * kBwRows];
     __shared__ __attribute__((aligned(16))) float delta_lds2[2 * kBwRows];       // -delta
 
-    // (key-tile pairs as in the kernel with two roles: equal work, and one (batch, kv head) on one XCD.  Single tiles, the dearest
-    // first, for launches of up to one round: 4 x 32 / 8 heads x 4096 1218 us against 1001)
-    const int n_pairs = (p.n_ktiles + 1) / 2;
-    const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, n_pairs);
-    const int pair = lid % n_pairs;
-    const int hk = (lid / n_pairs) % p.Hkv;
-    const int b = lid / (n_pairs * p.Hkv);
+    // (key-tile pairs as in the kernel with two roles: equal work, and one (batch, kv head) on one XCD; or single tiles, the first and
+    // dearest ones first, all walking their rows downwards)
+    const bool singles = p.deal.singles;
+    int pair, head;
+    if (singles) {
+        const HeadUnit at = xcd_unit(blockIdx.x, p.deal.units, 1, p.Hkv * p.B, p.deal.chunk_heads, p.deal.round);
+        if (at.unit < 0) return;
+        pair = at.unit;
+        head = at.head;
+    } else {
+        const int lid = xcd_chunked_id(blockIdx.x, gridDim.x, p.deal.units);
+        pair = lid % p.deal.units;
+        head = lid / p.deal.units;
+    }
+    pair = __builtin_amdgcn_readfirstlane(pair);
+    const int b = __builtin_amdgcn_readfirstlane(head / p.Hkv), hk = __builtin_amdgcn_readfirstlane(head - b * p.Hkv);
     const int G = p.Hq / p.Hkv;
     int sq, sk;
     int64_t q_base, do_base, l_base, k_base, v_base, dk_base, dv_base;           // (q, dO, lse, delta: of the batch; heads are added)
@@ -1071,7 +1095,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
         dv_base = (int64_t)b * p.dvs[0] + (int64_t)hk * p.dvs[1];
     }
     const int nk = (sk + kFuCols - 1) / kFuCols;
-    if (2 * pair >= nk) return;                                         // (a sequence without queries still gets dk = dv = 0 written)
+    if ((singles ? pair : 2 * pair) >= nk) return;                                         // (a sequence without queries still gets dk = dv = 0 written)
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1085,9 +1109,9 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_address(lds) + wave * TileLoader<D, NWV>::NI * 1024);
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-    for (int half = 0; half < 2; ++half) {
-        const int ktile = half == 0 ? pair : nk - 1 - pair;
-        if (half == 1 && ktile == pair) break;                          // odd tile count: the middle tile has no partner
+    // single tiles: one, unless a packed sequence is longer than the caller said
+    for (int half = 0, ktile = pair; singles ? ktile < nk : half < 2; ++half, ktile = singles ? ktile + p.deal.units : nk - 1 - pair) {
+        if (!singles && half == 1 && ktile == pair) break;              // odd tile count: the middle tile has no partner
         const int k0 = ktile * kFuCols;
         const int kw0 = k0 + 32 * wave;
         const int kj = kw0 + n;
@@ -1117,7 +1141,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
         struct Pos {
             int r0, hq;
         };
-        const int r_step = half == 0 ? -kBwRows : kBwRows;
+        const int r_step = singles || half == 0 ? -kBwRows : kBwRows;
         const auto advance = [&](Pos ps) {
             ++ps.hq;
             if (ps.hq == G) {
@@ -1229,7 +1253,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
             }
         };
 
-        Pos ps = {(half == 0 ? n_tiles - 1 : first_tile) * kBwRows, 0};
+        Pos ps = {(singles || half == 0 ? n_tiles - 1 : first_tile) * kBwRows, 0};
         if (n_steps > 0) {
             issue(0, ps);
             publish(0, ps);
@@ -1261,21 +1285,58 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
     }
 }
 
+// How the units of a launch are dealt (see xcd_unit): tiles of equal and of falling cost in pairs or one by one.  An XCD takes as many heads at a time as
+// have 8 MB of streamed rows.  (With 4 MB and less launches of one and two rounds lose up to a quarter: 136 heads of 32, 2048 tokens, dK and dV
+// 106 us with 8, 135 with 4.)
+constexpr int64_t kCus = 256;
+static void deal_units(BwdDeal& d, bool pairs, int64_t n_tiles, int64_t n_heads, int64_t resident, int64_t head_bytes, int64_t kv_heads) {
+    d.singles = !pairs && n_tiles * n_heads < 1 << 24;                       // (a grid's threads are counted in 32 bits)
+    // (an even number of tiles: lengths beyond the promised one are covered as far as pairs cover them)
+    d.units = (int)((n_tiles + 1) / 2 * (d.singles ? 2 : 1));
+    d.chunk_heads = (int)(n_heads / kv_heads * std::max<int64_t>(1, std::min<int64_t>(kv_heads / 8, (8 << 20) / head_bytes)));
+    d.round = n_tiles * n_heads <= resident ? (int)(kCus / 8) : 0;
+}
+static unsigned deal_grid(const BwdDeal& d, int64_t n_heads, int64_t kv_heads) {
+    return d.singles ? (unsigned)xcd_units_grid(d.units, (int)(n_heads / kv_heads), (int)kv_heads) : (unsigned)(d.units * n_heads);
+}
+
+template <int D, int MODE>
+static void launch_dq(BwdParams p, hipStream_t stream) {
+    constexpr bool kSmall = D <= 64 && MODE != MI355_MASK_BOOL;             // (explicit masks: their words and bounds leave no registers for more)
+    constexpr int NW = kSmall ? 4 : kBwWaves;
+    const int64_t heads = (int64_t)p.Hq * p.B, kv_heads = (int64_t)p.Hkv * p.B, tiles = p.n_qtiles * (kBwWaves / NW), resident = kCus * dq_resident(D);
+    // one length and the causal triangle: pairs where the launch goes over the chip more than four times (256 heads of 64, 2048 tokens: 231 us either way)
+    const bool equal = MODE == MI355_MASK_CAUSAL && (!p.cu_q || p.B == 1);
+    deal_units(p.deal, !kSmall || (equal && tiles * heads > 4 * resident), tiles, heads, resident, (int64_t)p.Sk * D * 4, kv_heads);
+    hipLaunchKernelGGL((bwd_dq_kernel<D, MODE, NW>), dim3(deal_grid(p.deal, heads, kv_heads)), dim3(NW * 64), 0, stream, p);
+}
+template <int D, int MODE>
+static void launch_dkv_one(BwdParams p, hipStream_t stream) {
+    const int64_t heads = (int64_t)p.Hkv * p.B, tiles = p.n_ktiles, resident = kCus * (D == 32 ? 4 : 2), pairs = (tiles + 1) / 2 * heads;
+    // One length and the causal triangle: pairs at head size 32 beyond four rounds of the chip; at 64, where two workgroups per compute unit wait longer
+    // for rows that another head has pushed out of the L2, wherever pairs fill their rounds.  us, pairs / singles, heads of 64: 256 of 512 tokens
+    // (512 pairs, 1.0 rounds) 35 / 38, of 1024 (2.0) 102 / 107, 136 of 1456 (1.6) 124 / 104, 136 of 1024 (1.1) 81 / 58; of 32: 256 of 1024 59 / 56,
+    // 136 of 2048 131 / 106, 64 of 8192 (4 rounds) 791 / 740; 14 packed of 111 to 1172, 32 / 16 heads, 85 / 72.
+    const bool equal = MODE == MI355_MASK_CAUSAL && (!p.cu_q || p.B == 1);
+    const bool filled = D == 32 ? tiles * heads > 4 * resident : (pairs + resident - 1) / resident * resident * 10 <= 11 * pairs;
+    deal_units(p.deal, equal && filled, tiles, heads, resident, (int64_t)p.Sq * (p.Hq / p.Hkv) * D * 4, heads);
+    hipLaunchKernelGGL((bwd_dkv_one_kernel<D, MODE>), dim3(deal_grid(p.deal, heads, heads)), dim3(kFuPairs * 64), 0, stream, p);
+}
+
 template <int D, int MODE>
 static void launch_bwd_mode(const BwdParams& p, hipStream_t stream) {
-    const dim3 grid_q((unsigned)((p.n_qtiles + 1) / 2 * p.Hq * p.B)), grid_k((unsigned)((p.n_ktiles + 1) / 2 * p.Hkv * p.B));
-    hipLaunchKernelGGL((bwd_dq_kernel<D, MODE>), grid_q, dim3(kBwWaves * 64), 0, stream, p);             // dQ, writes delta
-    // dK and dV, reads delta.  Head sizes 32 and 64: one role per wavefront up to a workgroup per compute unit, where a workgroup's
-    // own chain is what counts (one sequence of 8192 tokens, 8 / 1 heads of 64: 1.56 ms against 1.75; 8 x 1024, 32 / 8 heads 192
-    // us against 199), both roles in each wavefront beyond (4 x 4096, 32 / 8 heads of 64 1.14 -> 1.00 ms, of 32 0.89 -> 0.69;
-    // 64 x 256, 16 heads of 64 129 -> 110 us, of 32 the kernel alone 56 -> 34)
+    launch_dq<D, MODE>(p, stream);                                           // dQ, writes delta
+    // dK and dV, reads delta.  Head sizes 32 and 64: both roles in each wavefront, but for few pairs of key tiles with many steps, where a workgroup's own
+    // chain is what counts.  us with dQ, roles apart / together: one of 8160 tokens, 64 / 8 heads of 32 2067 / 2100 (with the forward); 16 heads of 32,
+    // 3000 tokens 105 / 103; 64 of 32, 300 tokens 20 / 19, 64 of 64, 2048 tokens 192 / 157.
+    const dim3 grid((unsigned)((p.n_ktiles + 1) / 2 * p.Hkv * p.B));
     if constexpr (D <= 64) {
-        if (grid_k.x > 256) {
-            hipLaunchKernelGGL((bwd_dkv_one_kernel<D, MODE>), grid_k, dim3(kFuPairs * 64), 0, stream, p);
+        if (grid.x > kCus || (int64_t)(p.Sq + kBwRows - 1) / kBwRows * (p.Hq / p.Hkv) < 64) {
+            launch_dkv_one<D, MODE>(p, stream);
             return;
         }
     }
-    hipLaunchKernelGGL((bwd_dkv_kernel<D, MODE, false>), grid_k, dim3(2 * kFuPairs * 64), 0, stream, p);
+    hipLaunchKernelGGL((bwd_dkv_kernel<D, MODE, false>), grid, dim3(2 * kFuPairs * 64), 0, stream, p);
 }
 
 // ---- with dS in memory ----
@@ -1332,12 +1393,20 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
     // Up to 128 tokens that do not fill the chip either way: one launch more costs what dS saves (4 x 128, 8 / 2 heads 33 us against
     // 37; 64 x 128, 16 / 4 heads 83 against 73), and up to 64 it is most of what runs (16 x 64, 8 heads 17 against 20).
     if (std::max(Sq, Sk) <= (tiles_k < 256 ? 128 : 64)) return false;
-    // At head sizes 64 and 32 the products that dS saves are worth less than its bytes, and what this form has over the other is that
-    // its workgroups are smaller and come in order of cost.  So it is for launches of few key tiles, and at 64 for lengths far apart
-    // (their mean below half the longest).  Head size 64 and 32, us: 16 x 512, 16 / 4 heads (256 tiles) 101 -> 87, 79 -> 73; 3 x 2048,
-    // 32 / 8 heads (384) 330 -> 299, 251 -> 258; 32 x 256, 8 heads (512) 39 -> 46, 29 -> 38; 4 x 2048, 32 / 8 heads (512) 365 -> 370, 268 ->
-    // 314; 16 of 256 to 4096 on a log scale 1226 -> 1096, 772 -> 893; of uniform lengths 1953 -> 2054, 1203 -> 1759.
-    if (D < 128 && (std::max(Sq, Sk) <= 160 || tiles_k > (D == 64 ? 384 : 256)) && !(D == 64 && packed && 2 * total_k < (int64_t)B * Sk)) return false;
+    // At head sizes 64 and 32 the products that dS saves are worth less than its bytes, and what this form has over the other is that the rows of a key
+    // tile can be dealt out and workgroups come in order of cost.  So it is for launches whose longest chain -- the steps of the first key tile of the
+    // longest sequence -- is several times what a workgroup's place on the chip has to do on average, and at 64 for lengths far apart (their mean below half
+    // the longest).  us with dS / without (chain in steps, over the average): heads of 64: 8 of 3000 tokens (47, 5.4) 99 / 120, 16 of 3000 (47, 2.7) 129 /
+    // 133, 32 of 1456 (23, 2.7) 74 / 71, 16 of 6000 (94, 1.4) 413 / 315; heads of 32: 16 of 2048 (32, 8) 83 / 69, 8 of 3000 (47, 11) 91 / 95; packed, 8 / 1
+    // heads: 12 of 490 to 5500 tokens, of 32 (688, 13) 630 / 1041, of 64 (688, 6.7) 834 / 1340, 36 of 112 to 1802 262 / 357 and 281 / 456.
+    // (Few key tiles of short sequences: 3 to 7 us fewer without in calls that the host's side of a gradient, some 70 us, outlasts either way.)
+    if (D < 128) {
+        const int64_t steps = n_rt * G, places = kCus * (D == 32 ? 4 : 2);
+        const double longest = packed ? (double)B * Sk / total_k : 1.0, over = 2.0 * places / tiles_k * longest;
+        const bool chain = D == 64 ? over >= 2.69 && steps >= (out.shares > 1 ? 20 : 40) : over >= 10.0 && steps >= 32;
+        const bool few = std::max(Sq, Sk) > 160 && tiles_k <= (D == 64 ? 384 : 256) && steps < 24;
+        if (!chain && !few && !(D == 64 && packed && 2 * total_k < (int64_t)B * Sk)) return false;
+    }
     if (out.shares > 1) {
         out.part_rows = rows_k;
         out.part_bytes = round_up(2 * out.shares * rows_k * Hkv * D * 4, kDsBlock);

@@ -4,6 +4,13 @@
 
 namespace mi355 {
 
+// Units of a head in a launch's grid: pairs of tiles, or single ones; then also heads that an XCD takes at a time, and its compute units if all
+// workgroups are resident at once (else 0)
+struct BwdDeal {
+    int units, chunk_heads, round;
+    bool singles;
+};
+
 struct BwdParams {
     const __bf16* q;
     const __bf16* k;
@@ -25,6 +32,7 @@ struct BwdParams {
     int B, Hq, Hkv, Sq, Sk;
     float scale, scale_log2;
     int n_qtiles, n_ktiles;
+    BwdDeal deal;                         // of bwd_dq_kernel and bwd_dkv_one_kernel
     // with dS in memory (see DsLayout): units of one pass over it, and for packed sequences the lists that the plan wrote
     unsigned char* ds;
     int unit0, n_units;           // dense: (sequence, kv head) pairs; packed: kv heads

@@ -61,3 +61,41 @@ def test_dense_launches_of_every_size(ma, D, B, H, S, causal):
             s = s.masked_fill(torch.ones(S, S, device="cuda", dtype=torch.bool).triu(1), float("-inf"))
         ref = torch.softmax(s, -1) @ v[b, h].double()
         assert float((out[b, h].double() - ref).abs().max()) <= 3.1 * 2 ** -9 * float(v[b, h].float().abs().max()), (b, h)
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("H,Hkv,lens,promised", [
+    (9, 9, [127, 300, 129, 1, 513, 64] * 5, 513),   # more than one round of single tiles, some in front
+    (2, 1, [700, 31] * 9, 700),
+    (6, 3, [385, 1030, 255, 257, 1500] * 8, 1500),
+    (40, 40, [640], 640), (600, 600, [512], 512),   # equal pairs
+    (12, 12, [900, 200, 130, 600] * 4, 700)])       # longer than promised
+def test_gradients_of_dealt_tiles(ma, monkeypatch, D, H, Hkv, lens, promised):
+    """Without dS in memory.  Rounding of P, dS and the results to bf16 moves each gradient by up to 2^-9 of its terms three times; over a tensor these average, and
+    2^-7 of its norm leaves room for sums that cancel."""
+    from mi355_attn import _lib, ops
+    print(f"case: dealt gradients {D} {H} {Hkv} {lens[:6]} x{len(lens)}", flush=True)
+    monkeypatch.setattr(_lib.load(), "mi355_prefill_bwd_ds_workspace", lambda *a: 0)
+    g = torch.Generator(device="cuda").manual_seed(D + H)
+    T = sum(lens)
+    q, k, v, dout = (torch.randn(T, h, D, generator=g, device="cuda", dtype=torch.bfloat16) * 0.5 for h in (H, Hkv, Hkv, H))
+    cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+    out, lse = ops._varlen(q, k, v, cu, cu, promised, promised, True, None, want_lse=True)
+    got = ops._prefill_backward(q, k, v, out, dout, lse, cu, cu, promised, promised, D ** -0.5, _lib.MASK_CAUSAL)
+    torch.cuda.synchronize()
+    a = 0
+    for n in lens[:6]:
+        for h in {0, H // 2, H - 1} if H == Hkv else {0, H - H // Hkv}:
+            hk, G = h // (H // Hkv), H // Hkv
+            heads = range(hk * G, hk * G + G)
+            leaves = [t[a:a + n, i].double().cpu().requires_grad_() for t, i in [(q, j) for j in heads] + [(k, hk), (v, hk)]]
+            loss = 0.0
+            for qh, i in zip(leaves[:-2], heads):
+                sc = (qh @ leaves[-2].T * D ** -0.5).masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+                loss = loss + (torch.softmax(sc, -1) @ leaves[-1] * dout[a:a + n, i].double().cpu()).sum()
+            want = torch.autograd.grad(loss, leaves)
+            mine = [got[0][a:a + n, i] for i in heads] + [got[1][a:a + n, hk], got[2][a:a + n, hk]]
+            for x, y in zip(mine, want):
+                # (a single key has no gradient but what rounding leaves)
+                assert float((x.double().cpu() - y).norm()) <= 2 ** -7 * float(y.norm()) + (1e-2 if n == 1 else 0.0), (a, n, h)
+        a += n
