@@ -1,9 +1,7 @@
 // FlashAttention-style prefill forward for gfx950 (bf16, MFMA 32x32x16).
 //
 // One workgroup = NW wavefronts = one tile of 32 NW queries of one (batch, head); each wavefront owns 32 query rows.
-// K/V tiles of 64 keys are double-buffered in LDS and shared by the wavefronts.  NW 8 (head_dim 128: two wavefronts per SIMD, one workgroup
-// per CU): 256 queries per loaded tile, half the L2->LDS traffic per MFMA of a 128-query workgroup, worth +1.5 %.  NW 4 (head_dim 32 and 64):
-// see below.  Per wavefront and KV tile:
+// K/V tiles of 64 keys are double-buffered in LDS and shared by the wavefronts.  NW 4 or 8: see below.  Per wavefront and KV tile:
 //
 //   S^T (64 keys x 32 queries) = K . Q^T     K fragments: ds_read_b128 from LDS,
 //                                            Q^T fragments live in registers
@@ -44,21 +42,23 @@ constexpr int kBN = 64;    // keys per LDS tile
 // table entry, a scalar load); queries and outputs are packed.
 // Occupancy: at head_dim 64 and 32 the kernel is held to the registers of four wavefronts per SIMD (128; left alone the
 // compiler takes 163 at head_dim 64), a handful of spilled registers outside the tile loop.  Head_dim 128 needs its 250.
-// NW 4, head_dim 32 and 64: four workgroups per compute unit, whose output rows are staged in the place of the last K/V tiles and whose query rows
-// come in without staging (34 and 17 KB of LDS; 70 and 37 with eight wavefronts, two workgroups).  On the diagonal and at the ragged end the
+// NW 4: four workgroups per compute unit, two at head_dim 128, whose output rows are staged in the place of the last K/V tiles and whose query rows
+// come in without staging (64, 33 and 17 KB of LDS; 132, 70 and 37 with eight wavefronts, for one, two and two workgroups).  On the diagonal and at the ragged end the
 // wavefronts of a workgroup wait for the one with the most keys, so that smaller workgroups leave less idle, and the launch is dealt finer; the
 // tiles that are loaded twice as often come out of the L2.  Causal, heads of 64 / 32, us with eight wavefronts and pairs of query tiles / with four and the
 // tiles as with_units deals them: 64 heads of 1456 tokens 43 / 36 and 32 / 25, 64 of 3000 125 / 95 and 89 / 64, 136 of 1456 75 / 60 and 54 / 45, 1024 of 300
 // 65 / 60 and 40 / 30, 1024 of 700 152 / 140 and 102 / 79, 8 of 8192 138 / 105 and 99 / 68, 64 of 8192 549 / 568 and 352 / 364; 22 packed sequences
-// of 1334, 8 heads of 64, 92 / 65; 14 of 111 to 1172, 32 heads, 80 / 60.
+// of 1334, 8 heads of 64, 92 / 65; 14 of 111 to 1172, 32 heads, 80 / 60; head_dim 128, window of 512, 14 of 111 to 1172, 32 heads, 127 / 99, one of 2000,
+// 16 heads, 32 / 24; boolean mask, 4 x 16 heads of 512 75 / 49.
 // With keys split and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
 // 9000 tokens, 32 heads of 64, 290 us, with four 325; 16 of 333 over 1500, heads of 32, 40 and 34.
 // WINDOW (causal): a query tile walks the K/V tiles that hold the kept first tokens, then those from its window's first
 // key on, as one sequence of tiles (tile_of); keys outside are masked in the tiles at the window's lower edge.
 template <int D, int MODE, bool PAGED, bool WINDOW, int NW>
-__global__ __launch_bounds__(NW * 64, D == 64 || NW == 4 ? 4 : 1) void prefill_fwd_kernel(PrefillParams p) {
+__global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1)) void prefill_fwd_kernel(PrefillParams p) {
     constexpr int BM = 32 * NW;                   // queries per workgroup
     constexpr bool kOwnSlab = NW == 8;            // staging of rows has LDS of its own
+    constexpr bool kFollows = D == 128 && NW == 4 && MODE != MI355_MASK_BOOL;       // references that follow the scores at the end (below)
     constexpr int NS = D / 16;                    // MFMA k-steps of K.Q^T
     constexpr int NDT = D / 32;                   // 32-row tiles of O^T
     constexpr int CPR = D / 8;                    // 16-byte chunks per row
@@ -446,11 +446,11 @@ __global__ __launch_bounds__(NW * 64, D == 64 || NW == 4 ? 4 : 1) void prefill_f
         };
 
         // Lazy rescaling: the exponent reference m_ref only moves when some row's maximum
-        // outgrows it by more than 2^kSlack; until then weights are at most 2^kSlack (exact in
+        // outgrows it by more than 2^slack; until then weights are at most 2^slack (exact in
         // the fp32 sums, harmless in bf16) and the O accumulators need no per-tile multiply.
         // The fast loop below therefore only accumulates in place; a tile that needs the
         // reference moved leaves it, rescales, and re-enters.
-        constexpr float kSlack = 8.0f;
+        float slack = 8.0f;
         // The first attempt at a query tile does not look at row maxima at all (MODE NONE / CAUSAL): the reference is
         // preset to 0 (weights 2^(x - kBias), x the score in the log2 domain), and what is watched is the row SUM: a
         // partial sum that reaches 2 moves the row's reference up by the exponent of its sum, an exact rescaling by a
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 || NW == 4 ? 4 : 1) void prefill_f
                 bool pending = false;
                 while (tile < tile_end) {
                     if (head(masked_c, std::true_type{}, tile)) {
-                        const bool grow = !((mx - m_ref) * scale_log2 <= kSlack);   // also true while m_ref = -inf
+                        const bool grow = !((mx - m_ref) * scale_log2 <= slack);   // also true while m_ref = -inf
                         if (__builtin_amdgcn_ballot_w64(grow) != 0) {
                             pending = true;
                             break;
@@ -513,40 +513,75 @@ __global__ __launch_bounds__(NW * 64, D == 64 || NW == 4 ? 4 : 1) void prefill_f
         };
 
         bool tracked = boolmask;             // explicit masks: tracked from the start
-        if constexpr (!boolmask) {
+        // (a query that sees none of this share's keys -- causal with fewer keys than queries, or a share of split
+        // keys that lies past its diagonal, or a padded lane behind the last query's window -- has a sum of zero by right)
+        const int k_first = t0 * kBN;
+        const bool sees = t0 < t1 && k_first < sk && (!causal || k_first <= qi + coff) && (!WINDOW || q_ok);
+        const auto begin_tracked = [&]() {
+            tracked = true;
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i)
+                if (t0 + i < t1) issue_tile(tile_of(t0 + i), (t0 + i) & (NB - 1));
+#pragma unroll
+            for (int i = 0; i < NDT; ++i)
+#pragma unroll
+                for (int j = 0; j < 16; ++j) o[i][j] = 0.f;
+            m_ref = -INFINITY;
+            neg_ref = 0.f;
+            l_run = 0.f;
+        };
+        set_buf(t0 & (NB - 1));              // the offsets start at the first tile's buffer
+        cur_tile = t0;
+        if constexpr (kFollows) {
+            // the last three tiles that this wavefront sees, with references that begin at 0 and follow the scores: a row's largest weight there is 1 and
+            // is not rounded.  (With the preset ones the error of short sequences is a tenth larger.)
+            const int seen = causal ? min(t1, max(t0, WINDOW ? t1 : (qw0 + 31 + coff + kBN) / kBN)) : t1;
+            int from = scale_log2 > 0.f ? max(t0, seen - 3) : t1;        // (a maximum of scores is none of their negatives)
             neg_ref = -kBias;
-            set_buf(t0 & (NB - 1));          // the offsets start at the first tile's buffer
-            cur_tile = t0;
-            if constexpr (WINDOW) run_tiles_preset(std::true_type{}, t0, n_low);
-            run_tiles_preset(std::false_type{}, max(n_low, t0), min(n_plain, t1));
-            run_tiles_preset(std::true_type{}, max(n_plain, t0), t1);
-            const float l = xor32_sum(l_run);
-            // (a query that sees none of this share's keys -- causal with fewer keys than queries, or a share of split
-            // keys that lies past its diagonal, or a padded lane behind the last query's window -- has a sum of zero by right)
-            const int k_first = t0 * kBN;
-            const bool sees = t0 < t1 && k_first < sk && (!causal || k_first <= qi + coff) && (!WINDOW || q_ok);
-            const bool bad = redo || (sees && !(l >= kUnderflow)) || !(l <= kOverflow);
-            // the workgroup meets (everybody is done with the K/V buffers) and votes
-            if (__syncthreads_or(bad ? 1 : 0)) {
-                tracked = true;
+            if constexpr (WINDOW) run_tiles_preset(std::true_type{}, t0, min(n_low, from));
+            run_tiles_preset(std::false_type{}, max(n_low, t0), min(n_plain, from));
+            run_tiles_preset(std::true_type{}, max(n_plain, t0), from);
+            constexpr float kUp = 4294967296.0f;                         // 2^kBias
+            l_run *= kUp;
 #pragma unroll
-                for (int i = 0; i < kAhead; ++i)
-                    if (t0 + i < t1) issue_tile(tile_of(t0 + i), (t0 + i) & (NB - 1));
+            for (int i = 0; i < NDT; ++i)
 #pragma unroll
-                for (int i = 0; i < NDT; ++i)
-#pragma unroll
-                    for (int j = 0; j < 16; ++j) o[i][j] = 0.f;
-                m_ref = -INFINITY;
-                neg_ref = 0.f;
-                l_run = 0.f;
+                for (int j = 0; j < 16; ++j) o[i][j] *= kUp;
+            neg_ref += kBias;
+            m_ref = scale_log2 > 0.f ? -neg_ref / scale_log2 : 0.f;
+            slack = 0.0f;
+            for (;;) {
+                if constexpr (WINDOW) run_tiles(std::true_type{}, from, n_low);
+                run_tiles(std::false_type{}, max(n_low, from), min(n_plain, t1));
+                run_tiles(std::true_type{}, max(n_plain, from), t1);
+                if (tracked) break;
+                const float l = xor32_sum(l_run);
+                const bool bad = redo || (sees && !(l >= kUnderflow * kUp)) || !(l <= kOverflow * kUp);
+                if (!__syncthreads_or(bad ? 1 : 0)) break;
+                begin_tracked();
+                slack = 8.0f;
+                from = t0;
+                set_buf(t0 & (NB - 1));
+                cur_tile = t0;
             }
-        }
-        if (tracked) {
-            set_buf(t0 & (NB - 1));
-            cur_tile = t0;
-            if constexpr (WINDOW) run_tiles(std::true_type{}, t0, n_low);
-            run_tiles(std::false_type{}, max(n_low, t0), min(n_plain, t1));
-            run_tiles(std::true_type{}, max(n_plain, t0), t1);
+        } else {
+            if constexpr (!boolmask) {
+                neg_ref = -kBias;
+                if constexpr (WINDOW) run_tiles_preset(std::true_type{}, t0, n_low);
+                run_tiles_preset(std::false_type{}, max(n_low, t0), min(n_plain, t1));
+                run_tiles_preset(std::true_type{}, max(n_plain, t0), t1);
+                const float l = xor32_sum(l_run);
+                const bool bad = redo || (sees && !(l >= kUnderflow)) || !(l <= kOverflow);
+                // the workgroup meets (everybody is done with the K/V buffers) and votes
+                if (__syncthreads_or(bad ? 1 : 0)) begin_tracked();
+            }
+            if (tracked) {
+                set_buf(t0 & (NB - 1));
+                cur_tile = t0;
+                if constexpr (WINDOW) run_tiles(std::true_type{}, t0, n_low);
+                run_tiles(std::false_type{}, max(n_low, t0), min(n_plain, t1));
+                run_tiles(std::true_type{}, max(n_plain, t0), t1);
+            }
         }
 
         // ---- normalise and store: lane owns query qi, d = 32dt + 8(i/4) + 4kg + i%4 ---
@@ -628,7 +663,7 @@ static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
     p.n_qtiles = (p.Sq + 32 * waves - 1) / (32 * waves);
     p.n_pairs = (p.n_qtiles + 1) / 2;
     const int64_t n_cu = std::max(1, device_compute_units()), heads = (int64_t)p.Hq * p.B * std::max(1, p.n_split), tiles = p.n_qtiles * heads;
-    const int64_t resident = n_cu * (waves == 4 ? 4 : (D == 128 ? 1 : 2));                     // workgroups
+    const int64_t resident = n_cu * (waves == 4 ? 4 : 2) / (D == 128 ? 2 : 1);                     // workgroups
     const bool equal = p.mask_mode == MI355_MASK_CAUSAL && !(p.window > 0 && p.window < p.Sq) && (!p.cu_q || p.B == 1 || p.n_split > 1);
     const bool pairs = equal && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
     p.single_tiles = !pairs && tiles < 1 << 24;                                                // (a grid's threads are counted in 32 bits)
@@ -659,9 +694,7 @@ static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {
 // (the lines between four and eight wavefronts: see the kernel)
 template <int D>
 static int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-    if constexpr (D != 128)
-        if (p.n_split <= 1) return launch_prefill_of<D, 4>(p, stream);
-    return launch_prefill_of<D, 8>(p, stream);
+    return p.n_split <= 1 ? launch_prefill_of<D, 4>(p, stream) : launch_prefill_of<D, 8>(p, stream);
 }
 
 // Merge of the split-key partials: one wavefront per (query row, head).
@@ -752,9 +785,7 @@ static int launch_prefill_paged_of(const PrefillParams& p0, hipStream_t stream) 
 constexpr int kSmallPaged = 128;                  // blocks: paged contexts that four wavefronts take
 template <int D>
 static int launch_prefill_paged(const PrefillParams& p, hipStream_t stream) {
-    if constexpr (D != 128)
-        if (p.n_split <= 1 && p.max_blocks <= kSmallPaged) return launch_prefill_paged_of<D, 4>(p, stream);
-    return launch_prefill_paged_of<D, 8>(p, stream);
+    return p.n_split <= 1 && p.max_blocks <= kSmallPaged ? launch_prefill_paged_of<D, 4>(p, stream) : launch_prefill_paged_of<D, 8>(p, stream);
 }
 
 }  // namespace mi355
@@ -787,35 +818,63 @@ static int set_split(PrefillParams& p, int D, int n_split, int64_t total_q_rows,
     return 0;
 }
 
-// Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; lengths of a packed batch are
-// judged by the longest; of the rougher fits eight per cent are taken off).
-static double other_us(const PrefillParams& p, int D, int n_cu) {
-    const bool causal = p.mask_mode == MI355_MASK_CAUSAL;
-    const int Sk = p.block_table ? 16 * p.max_blocks : p.Sk;
-    const double over = causal && Sk > p.Sq ? Sk - p.Sq : 0, most = causal ? std::min<double>(Sk, over + p.Sq) : Sk;
-    const double heads = (double)p.Hq * p.B, kt = std::ceil(most / kBN);
-    if (prefill_short_takes(p, D)) {
-        // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
-        return 0.92 * ((D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu);
+// What the models below need of a call (lengths of a packed batch are judged by the longest)
+struct CallSize {
+    double heads, over, keys;                         // over: keys that every query sees (causal); keys: of the last query
+    bool causal;
+    explicit CallSize(const PrefillParams& p) : heads((double)p.Hq * p.B), causal(p.mask_mode == MI355_MASK_CAUSAL) {
+        const int Sk = p.block_table ? 16 * p.max_blocks : p.Sk;
+        over = causal && Sk > p.Sq ? Sk - p.Sq : 0;
+        keys = causal ? std::min<double>(Sk, over + p.Sq) : Sk;
     }
-    // query tiles of a launch, dearest and mean number of key tiles; per key tile, per query tile, and what is the same for every call
-    const bool wide = D == 128 && prefill_w64_takes(p), by_head = wide && causal && p.Hq / p.Hkv % 4 == 0;
+    // key tiles of a query tile of bm rows on average
+    double mean_tiles(const PrefillParams& p, int bm) const {
+        const double kt = std::ceil(keys / kBN);
+        return causal ? std::min(kt, (over + 0.5 * p.Sq + 0.5 * bm) / kBN) : kt;
+    }
+};
+// Microseconds of prefill_fwd_kernel with four wavefronts: the chain of the dearest tile and what a compute unit has to do, of which the longer one counts,
+// and more where they are alike; D 128, two workgroups per compute unit, loses to the L2 what the launch is longer than one round (150 calls of 1 to
+// 1024 heads of 64 to 3000 tokens at 32 and 64: 4 % off; 170 of 8 to 1024 heads of 64 to 5000 tokens at 128: 7 %).
+static double four_us(const PrefillParams& p, int D, int n_cu) {
+    const CallSize c(p);
+    const double tiles = std::ceil(p.Sq / 128.0) * c.heads, mean = c.mean_tiles(p, 128);
+    const double chain = (D == 128 ? 1.27 : D == 64 ? 0.79 : 0.53) * std::ceil(c.keys / kBN);
+    const double each = D == 128 ? 0.906 * mean + 2.98 : D == 64 ? 0.57 * mean + 2.33 : 0.354 * mean + 1.08;
+    const double all = tiles / n_cu * each * (D == 128 ? 1.0 + 0.077 * std::max(0.0, std::log2(tiles / (2.0 * n_cu))) : 1.0);
+    return (D == 128 ? 6.5 : D == 64 ? 6.5 : 4.9) + std::cbrt(chain * chain * chain + all * all * all);
+}
+// ... of the 64-query kernel
+static double wide_us(const PrefillParams& p, int n_cu) {
+    const CallSize c(p);
+    const bool by_head = c.causal && p.Hq / p.Hkv % 4 == 0;
     const int bm = by_head ? 64 : kBM;
-    const double qt = (p.Sq + bm - 1) / bm, jobs = qt * heads / (by_head ? 4 : 1), mean = causal ? std::min(kt, (over + 0.5 * p.Sq + 0.5 * bm) / kBN) : kt;
-    if (wide) {
-        // the last three key tiles of a length that is no multiple of 64 run in ordinary code, some 4 us each more
-        const double tail = Sk % kBN ? 12.0 : 0.0;
-        return 0.92 * (9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * mean + 4.0 + tail / (causal ? qt : 1.0))));
-    }
-    if (D != 128 && (!p.block_table || p.max_blocks <= kSmallPaged)) {
-        // four wavefronts: the chain of the dearest tile and what a compute unit has to do, of which the longer one counts, and more where they are alike
-        // (150 calls of 1 to 1024 heads of 64 to 3000 tokens: 4 % off)
-        const double qt4 = std::ceil(p.Sq / 128.0), mean4 = causal ? std::min(kt, (over + 0.5 * p.Sq + 64.0) / kBN) : kt;
-        const double chain = (D == 64 ? 0.79 : 0.53) * kt, all = qt4 * heads / n_cu * (D == 64 ? 0.57 * mean4 + 2.33 : 0.354 * mean4 + 1.08);
-        return (D == 64 ? 6.5 : 4.9) + std::cbrt(chain * chain * chain + all * all * all);
-    }
-    const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75;
-    return 0.92 * (5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * mean + 2.0)));
+    const double kt = std::ceil(c.keys / kBN), qt = (p.Sq + bm - 1) / bm, jobs = qt * c.heads / (by_head ? 4 : 1);
+    // the last three key tiles of a length that is no multiple of 64 run in ordinary code, some 4 us each more
+    const double tail = (p.block_table ? 16 * p.max_blocks : p.Sk) % kBN ? 12.0 : 0.0;
+    return 9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * c.mean_tiles(p, bm) + 4.0 + tail / (c.causal ? qt : 1.0)));
+}
+static bool four_takes(const PrefillParams& p) { return p.n_split <= 1 && (!p.block_table || p.max_blocks <= kSmallPaged); }
+// Whether the 64-query kernel is left to prefill_fwd_kernel: short and ragged lengths, whose last tiles it computes in ordinary code and whose rounds it does not
+// fill.  Heads of 128, causal, us 64-query kernel / this: 64 heads of 700 tokens 38 / 25, 136 of 300 30 / 17, 1024 of 300 161 / 103, 14 packed of 111 to 1172, 32
+// heads, 133 / 96, 60 of 20 to 300, 16 heads, 97 / 44; but 136 of 1024 57 / 74, 256 of 1024 91 / 106, 136 of 2000 166 / 204, 14 x 16 heads of 644 65 / 69.  Twelve per
+// cent are left to the wide model, with which none of 170 calls got slower.
+static bool four_beats_wide(const PrefillParams& p, int n_cu) { return n_cu > 0 && four_takes(p) && four_us(p, 128, n_cu) < 0.88 * wide_us(p, n_cu); }
+static bool wide_takes(const PrefillParams& p) {
+    return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p) && !four_beats_wide(p, device_compute_units());
+}
+
+// Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; of the rougher fits eight per cent are taken off).
+static double other_us(const PrefillParams& p, int D, int n_cu) {
+    const CallSize c(p);
+    const double kt = std::ceil(c.keys / kBN);
+    // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
+    if (prefill_short_takes(p, D))
+        return 0.92 * ((D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + c.heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu);
+    if (D == 128 && wide_takes(p)) return 0.92 * wide_us(p, n_cu);
+    if (four_takes(p)) return four_us(p, D, n_cu);
+    const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75, jobs = (p.Sq + kBM - 1) / kBM * c.heads;
+    return 0.92 * (5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * c.mean_tiles(p, kBM) + 2.0)));
 }
 
 // Wavefronts of prefill_keys.hip's kernel for p, 0: another kernel is the faster one.  One 183-token prompt, 16 heads, D 128: 64-query kernel 26.4 us, keys dealt to
@@ -905,7 +964,7 @@ static int prefill_common(const void* q, const void* k, const void* v, void* out
     hipStream_t s = (hipStream_t)stream;
     int rc;
     if (p.n_split > 1) {
-        if (D == 128 && mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
+        if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
         else rc = D == 128 ? launch_prefill<128>(p, s) : (D == 64 ? launch_prefill<64>(p, s) : launch_prefill<32>(p, s));
         if (rc == 0) rc = launch_merge(p, D, s);
         if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
@@ -915,7 +974,7 @@ static int prefill_common(const void* q, const void* k, const void* v, void* out
     const int keys = keys_wavefronts(p, D);
     if (keys) rc = launch_prefill_keys(p, D, keys, s);
     else if (prefill_short_takes(p, D)) rc = launch_prefill_short(p, D, s);
-    else if (D == 128 && mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
+    else if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
     else rc = D == 128 ? launch_prefill<128>(p, s) : (D == 64 ? launch_prefill<64>(p, s) : launch_prefill<32>(p, s));
     if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
     return MI355_OK;
@@ -1078,7 +1137,7 @@ static int prefill_paged_common(const void* q, const void* k_cache, const void* 
     int rc;
     const int keys = keys_wavefronts(p, D);
     if (keys) rc = launch_prefill_keys(p, D, keys, s);
-    else if (D == 128 && prefill_w64_takes(p)) rc = launch_prefill_w64(p, s);
+    else if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
     else rc = D == 128 ? launch_prefill_paged<128>(p, s) : (D == 64 ? launch_prefill_paged<64>(p, s) : launch_prefill_paged<32>(p, s));
     if (rc == 0 && p.n_split > 1) rc = launch_merge(p, D, s);
     if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
