@@ -1284,6 +1284,9 @@ extern "C" int mi355_prefill_suggest_prompt_kv_splits(int B, int Hq, int D, int 
     const int n_cu = n_compute_units > 0 ? n_compute_units : device_compute_units();
     double us;
     const int n = n_cu > 0 ? best_kv_splits(B, Hq, D, Sq_max, Sk_max, total_q_rows, causal, n_cu, us) : 1;
+    // Two shares at head sizes 32 and 64: four wavefronts and single tiles are faster by themselves.  Causal, one sequence, us with / without: heads of 64, 8 of 6000 tokens
+    // 89 / 66, 8 of 8192 139 / 109, 4 of 12000 153 / 140; of 32, 67 / 44, 100 / 74, 110 / 100.  (Four shares: 4 heads of 32, 8192 tokens 59 / 69; 2 of 64, 12000 89 / 80.)
+    if (n == 2 && D < 128 && causal && Sq_max == Sk_max) return 1;
     return n > 1 && Sq_max == Sk_max && prefill_keys_plan(B, Hq, D, Sq_max, Sk_max, causal != 0, n_cu).us < 0.92 * us ? 1 : n;
 }
 

@@ -49,3 +49,13 @@ def test_every_unit_once(order, u, groups, group, rnd):
                 for c in range(0, len(mine), chunk * u):
                     units = [i for i, _ in mine[c:c + chunk * u]]
                     assert units == sorted(units) and len({h for _, h in mine[c:c + chunk * u]}) <= chunk
+
+
+@pytest.mark.parametrize("D,prompt,chunk", [(32, 1, 2), (64, 1, 2), (128, 2, 2)])
+def test_two_shares_of_a_whole_prompt(D, prompt, chunk):
+    """Heads of 32 and 64: whole prompts are not cut in two, chunks and calls with per-head terms still are, and four shares stay."""
+    from mi355_attn import _lib
+    lib = _lib.load()
+    assert lib.mi355_prefill_suggest_prompt_kv_splits(1, 8, D, 8192, 8192, 8192, 1, 256) == prompt
+    assert lib.mi355_prefill_suggest_kv_splits(1, 8, D, 8192, 8192, 8192, 1, 256) == chunk
+    assert lib.mi355_prefill_suggest_prompt_kv_splits(1, 4, D, 8192, 8192, 8192, 1, 256) == 4
