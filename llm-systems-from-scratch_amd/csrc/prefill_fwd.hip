@@ -47,10 +47,10 @@ constexpr int kBN = 64;    // keys per LDS tile
 // wavefronts of a workgroup wait for the one with the most keys, so that smaller workgroups leave less idle, and the launch is dealt finer; the
 // tiles that are loaded twice as often come out of the L2.  Causal, heads of 64 / 32, us with eight wavefronts and pairs of query tiles / with four and the
 // tiles as with_units deals them: 64 heads of 1456 tokens 43 / 36 and 32 / 25, 64 of 3000 125 / 95 and 89 / 64, 136 of 1456 75 / 60 and 54 / 45, 1024 of 300
-// 65 / 60 and 40 / 30, 1024 of 700 152 / 140 and 102 / 79, 8 of 8192 138 / 105 and 99 / 68, 64 of 8192 549 / 568 and 352 / 364; 22 packed sequences
+// 65 / 60 and 40 / 30, 1024 of 700 152 / 140 and 102 / 79, 8 of 8192 138 / 105 and 99 / 68, 22 packed sequences
 // of 1334, 8 heads of 64, 92 / 65; 14 of 111 to 1172, 32 heads, 80 / 60; head_dim 128, window of 512, 14 of 111 to 1172, 32 heads, 127 / 99, one of 2000,
 // 16 heads, 32 / 24; boolean mask, 4 x 16 heads of 512 75 / 49.
-// With keys split and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
+// With keys split, in launches of many long sequences (launch_prefill) and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
 // 9000 tokens, 32 heads of 64, 290 us, with four 325; 16 of 333 over 1500, heads of 32, 40 and 34.
 // WINDOW (causal): a query tile walks the K/V tiles that hold the kept first tokens, then those from its window's first
 // key on, as one sequence of tiles (tile_of); keys outside are masked in the tiles at the window's lower edge.
@@ -651,6 +651,10 @@ static int device_compute_units() {
     return n;
 }
 
+// One length and the causal triangle: pairs of query tiles carry equal work.
+static bool equal_pairs(const PrefillParams& p) {
+    return p.mask_mode == MI355_MASK_CAUSAL && !(p.window > 0 && p.window < p.Sq) && (!p.cu_q || p.B == 1 || p.n_split > 1);
+}
 // Query tiles in pairs, which carry equal causal work, or one by one, the dearest first (see the kernel).
 // One by one fills the chip better: the launch ends with small pieces, and sequences of different lengths, windows and launches without a mask have no equal
 // pairs.  A pair's two tiles and its neighbours read the same keys at about the same time, which counts where the launch goes over the chip many
@@ -664,8 +668,7 @@ static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
     p.n_pairs = (p.n_qtiles + 1) / 2;
     const int64_t n_cu = std::max(1, device_compute_units()), heads = (int64_t)p.Hq * p.B * std::max(1, p.n_split), tiles = p.n_qtiles * heads;
     const int64_t resident = n_cu * (waves == 4 ? 4 : 2) / (D == 128 ? 2 : 1);                     // workgroups
-    const bool equal = p.mask_mode == MI355_MASK_CAUSAL && !(p.window > 0 && p.window < p.Sq) && (!p.cu_q || p.B == 1 || p.n_split > 1);
-    const bool pairs = equal && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
+    const bool pairs = equal_pairs(p) && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
     p.single_tiles = !pairs && tiles < 1 << 24;                                                // (a grid's threads are counted in 32 bits)
     if (p.single_tiles) p.n_pairs = p.n_qtiles;
     const int64_t keys = p.block_table ? 16 * (int64_t)p.max_blocks : p.Sk, kv_heads = (8 << 20) / (std::max<int64_t>(1, keys) * D * 4);
@@ -691,10 +694,13 @@ static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {
         hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE, false, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
 }
-// (the lines between four and eight wavefronts: see the kernel)
+// Eight wavefronts: split keys (see the kernel); and long sequences of one length that go over the chip more than four times, where the ends weigh little
+// and half as many loads of keys count.  us with four / eight, causal: heads of 64, 192 of 8132 tokens 1761 / 1709, 256 of 4096 620 / 603, 400 of 3000 563 / 570, 800 of
+// 2000 535 / 550; of 32, 192 of 8132 1142 / 1098, 256 of 4096 397 / 391, 400 of 3000 358 / 370.
 template <int D>
 static int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-    return p.n_split <= 1 ? launch_prefill_of<D, 4>(p, stream) : launch_prefill_of<D, 8>(p, stream);
+    const bool far = D != 128 && equal_pairs(p) && p.Sq >= 4000 && (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B > 16 * (int64_t)device_compute_units();
+    return p.n_split <= 1 && !far ? launch_prefill_of<D, 4>(p, stream) : launch_prefill_of<D, 8>(p, stream);
 }
 
 // Merge of the split-key partials: one wavefront per (query row, head).
