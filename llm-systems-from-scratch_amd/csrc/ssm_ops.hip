@@ -19,12 +19,12 @@
 #include "common.hpp"
 #include "launch.hpp"
 #include "prefill_tile.hpp"
+#include "ssm_conv.hpp"
 
 #include <type_traits>
 
 namespace mi355 {
 
-constexpr int kMaxTaps = 16;
 constexpr int kScanVecs = 16;        // most 4-wide state pieces per thread of the scan
 
 template <typename T>
@@ -110,6 +110,7 @@ __device__ __forceinline__ void store_ch(T* p, const float (&v)[V]) {
 // Causal convolution + silu of packed prompts.  A thread owns V adjacent channels of TILE tokens of one sequence; the inputs it has read
 // slide through registers when the number of taps is known at compile time (TAPS > 0).  The thread of a sequence's first tile is the only
 // one that touches the sequence's ring for its channels: it reads the history first and writes the last taps - 1 inputs of the portion at its end.
+// (So a tile has at least taps - 1 tokens: conv_tile.)
 //
 // Bound by its bytes where a call is large (8192 tokens, 4352 channels: 142 MB in 30 us) and by one load's latency where it is small, so all rows of a batch of
 // eight, and those that go to the ring, are requested before the first is used: a load in front of every token's sum took 11 to 13 us for 600 to 1700 tokens,
@@ -150,6 +151,7 @@ struct ChannelRow {                                      // V adjacent channels 
 
 template <typename T, int V, int TAPS, int TILE>
 __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
+    static_assert(TILE >= TAPS - 1, "only the first tile reads the ring");
     constexpr bool FAST = sizeof(T) == 2;
     const int taps = TAPS > 0 ? TAPS : p.taps;
     const int ch_groups = p.channels / V;
@@ -1189,10 +1191,7 @@ static int launch_conv(const SsmParams<T>& p, hipStream_t s) {
     bool vec = p.channels % 8 == 0 && p.xbc_at % 8 == 0 && p.proj_stride % 8 == 0;
     for (const void* ptr : {(const void*)p.proj, (const void*)p.conv_w, (const void*)p.conv_b, (const void*)p.conv_state, (const void*)p.xbc})
         vec = vec && (reinterpret_cast<uintptr_t>(ptr) & 15) == 0;
-    // us with 4 / 8 / 16 tokens per thread: 64 tokens of 4352 channels 5.1, 5.0, 6.7; 577 of 4352 7.4, 7.4, 9.0; 1024 9.1, 10.1, 10.1; 4000 of 1280
-    // 10.3, 10.7, 10.9; 8000 16.5, 14.1, 15.2 (7200 of 2240: 16 is 2 faster than 8); 8192 of 4352 40.9, 34.2, 29.5
-    const int64_t inputs = p.n_rows * p.channels;
-    const int tile = inputs <= 6 << 20 ? 4 : inputs <= 12 << 20 ? 8 : 16;
+    const int tile = conv_tile(p.n_rows, p.channels, p.taps);
     return tile == 4 ? launch_conv_tiles<T, 4>(p, vec, s) : tile == 8 ? launch_conv_tiles<T, 8>(p, vec, s) : launch_conv_tiles<T, 16>(p, vec, s);
 }
 

@@ -345,6 +345,31 @@ def test_little_work_takes_short_segments(heads, n, lens, seg):
         assert short % 64 == 0 and (short == 0 or short >= 256 or (tokens // short + n) * heads <= 1024 + n * heads)
 
 
+# ---- tiles of the causal convolution ------------------------------------------------------------------------------------
+def test_only_a_portions_first_tile_reads_the_ring(tmp_path):
+    """What the tiles of a resumed portion read of the ring of inputs against what the first of them writes there, for every number of taps and size
+    class: tiles run in any order, so no other tile may read a row of the ring at all."""
+    src, lib = tmp_path / "conv.cpp", tmp_path / "conv.so"
+    src.write_text('#include "ssm_conv.hpp"\n'
+                   'extern "C" int tile(long long rows, int channels, int taps) { return mi355::conv_tile(rows, channels, taps); }\n')
+    csrc = os.path.join(os.path.dirname(os.path.dirname(mi355_attn.__file__)), "csrc")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
+    tile = ctypes.CDLL(str(lib)).tile
+    tile.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
+    seen = set()
+    for taps in range(1, 17):
+        for rows, channels in ((64, 64), (1024, 4352), (2048, 4352), (8192, 4352)):
+            n = tile(rows, channels, taps)
+            assert n in (4, 8, 16)
+            seen.add(n)
+            for length in range(1, 50):
+                written = {(64 + t) % taps for t in range(max(0, length - (taps - 1)), length)}
+                for t0 in range(n, length, n):
+                    read = {(64 + t) % taps for t in range(t0 - (taps - 1), min(t0 + n, length)) if t < 0}
+                    assert not read, (taps, rows, length, t0, read & written)
+    assert seen == {4, 8, 16} and [tile(64, 64, taps) for taps in (1, 4, 5, 6, 9, 10, 16)] == [4, 4, 4, 8, 8, 16, 16]
+
+
 # ---- order of workgroups -------------------------------------------------------------------------------------------------
 def test_workgroups_with_work_are_dealt_evenly_to_the_xcds(tmp_path):
     """Every workgroup with work gets an id of its own, and no XCD (id modulo 8 of the launch) gets more than one of them more than another,
