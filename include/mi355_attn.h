@@ -175,6 +175,19 @@ int mi355_prefill_suggest_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max
  * is the faster one for it. */
 int mi355_prefill_suggest_prompt_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t total_q_rows,
                                            int causal, int n_compute_units);
+/*
+ * Which kernel a prefill call of these sizes runs on (strides within every kernel's range, softmax_scale > 0, no per-head terms), for tests and for reading
+ * profiles; 0: no such call.  packed, lse: non-zero where the call has cu_seqlens, an lse output.  max_blocks > 0: keys and values in a paged cache (Sk_max and
+ * mask_mode are not read).  n_split, window: as in the calls, 0 for none.  n_compute_units <= 0: ask the current device.  wavefronts (may be NULL): per workgroup.
+ */
+enum {
+    MI355_PREFILL_TILES = 1, /* 32 query rows per wavefront */
+    MI355_PREFILL_W64 = 2,   /* 64 query rows per wavefront, head_dim 128 */
+    MI355_PREFILL_SHORT = 3, /* heads of up to 256 keys */
+    MI355_PREFILL_KEYS = 4   /* keys dealt to the wavefronts of a workgroup */
+};
+int mi355_prefill_kernel(int B, int Hq, int Hkv, int D, int Sq_max, int Sk_max, int mask_mode, int packed, int max_blocks, int lse, int n_split, int window,
+                         int n_compute_units, int* wavefronts);
 int mi355_prefill_fwd_splitkv(const void* q, const void* k, const void* v, void* out,
                               const int64_t q_strides[3], const int64_t k_strides[3],
                               const int64_t v_strides[3], const int64_t o_strides[3],

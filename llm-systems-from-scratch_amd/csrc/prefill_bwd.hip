@@ -1290,9 +1290,10 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void bwd_dkv_one_kernel(BwdPa
 // 106 us with 8, 135 with 4.)
 constexpr int64_t kCus = 256;
 static void deal_units(BwdDeal& d, bool pairs, int64_t n_tiles, int64_t n_heads, int64_t resident, int64_t head_bytes, int64_t kv_heads) {
-    d.singles = !pairs && n_tiles * n_heads < 1 << 24;                       // (a grid's threads are counted in 32 bits)
     // (an even number of tiles: lengths beyond the promised one are covered as far as pairs cover them)
-    d.units = (int)((n_tiles + 1) / 2 * (d.singles ? 2 : 1));
+    const int64_t n_pairs = (n_tiles + 1) / 2;
+    d.singles = !pairs && xcd_units_fit(2 * n_pairs, n_heads / kv_heads, kv_heads, 256);
+    d.units = (int)(n_pairs * (d.singles ? 2 : 1));
     d.chunk_heads = (int)(n_heads / kv_heads * std::max<int64_t>(1, std::min<int64_t>(kv_heads / 8, (8 << 20) / head_bytes)));
     d.round = n_tiles * n_heads <= resident ? (int)(kCus / 8) : 0;
 }

@@ -669,7 +669,7 @@ static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
     const int64_t n_cu = std::max(1, device_compute_units()), heads = (int64_t)p.Hq * p.B * std::max(1, p.n_split), tiles = p.n_qtiles * heads;
     const int64_t resident = n_cu * (waves == 4 ? 4 : 2) / (D == 128 ? 2 : 1);                     // workgroups
     const bool pairs = equal_pairs(p) && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
-    p.single_tiles = !pairs && tiles < 1 << 24;                                                // (a grid's threads are counted in 32 bits)
+    p.single_tiles = !pairs && xcd_units_fit(p.n_qtiles, p.Hq / p.Hkv, (int64_t)p.Hkv * p.B, 64 * waves);
     if (p.single_tiles) p.n_pairs = p.n_qtiles;
     const int64_t keys = p.block_table ? 16 * (int64_t)p.max_blocks : p.Sk, kv_heads = (8 << 20) / (std::max<int64_t>(1, keys) * D * 4);
     p.chunk_heads = p.Hq / p.Hkv * (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)p.Hkv * p.B / 8, kv_heads));
@@ -694,13 +694,9 @@ static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {
         hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE, false, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
 }
-// Eight wavefronts: split keys (see the kernel); and long sequences of one length that go over the chip more than four times, where the ends weigh little
-// and half as many loads of keys count.  us with four / eight, causal: heads of 64, 192 of 8132 tokens 1761 / 1709, 256 of 4096 620 / 603, 400 of 3000 563 / 570, 800 of
-// 2000 535 / 550; of 32, 192 of 8132 1142 / 1098, 256 of 4096 397 / 391, 400 of 3000 358 / 370.
 template <int D>
-static int launch_prefill(const PrefillParams& p, hipStream_t stream) {
-    const bool far = D != 128 && equal_pairs(p) && p.Sq >= 4000 && (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B > 16 * (int64_t)device_compute_units();
-    return p.n_split <= 1 && !far ? launch_prefill_of<D, 4>(p, stream) : launch_prefill_of<D, 8>(p, stream);
+static int launch_prefill(const PrefillParams& p, int waves, hipStream_t stream) {
+    return waves == 4 ? launch_prefill_of<D, 4>(p, stream) : launch_prefill_of<D, 8>(p, stream);
 }
 
 // Merge of the split-key partials: one wavefront per (query row, head).
@@ -788,10 +784,9 @@ static int launch_prefill_paged_of(const PrefillParams& p0, hipStream_t stream) 
     else hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, true, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
 }
-constexpr int kSmallPaged = 128;                  // blocks: paged contexts that four wavefronts take
 template <int D>
-static int launch_prefill_paged(const PrefillParams& p, hipStream_t stream) {
-    return p.n_split <= 1 && p.max_blocks <= kSmallPaged ? launch_prefill_paged_of<D, 4>(p, stream) : launch_prefill_paged_of<D, 8>(p, stream);
+static int launch_prefill_paged(const PrefillParams& p, int waves, hipStream_t stream) {
+    return waves == 4 ? launch_prefill_paged_of<D, 4>(p, stream) : launch_prefill_paged_of<D, 8>(p, stream);
 }
 
 }  // namespace mi355
@@ -860,14 +855,24 @@ static double wide_us(const PrefillParams& p, int n_cu) {
     const double tail = (p.block_table ? 16 * p.max_blocks : p.Sk) % kBN ? 12.0 : 0.0;
     return 9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * c.mean_tiles(p, bm) + 4.0 + tail / (c.causal ? qt : 1.0)));
 }
-static bool four_takes(const PrefillParams& p) { return p.n_split <= 1 && (!p.block_table || p.max_blocks <= kSmallPaged); }
+// Whether prefill_fwd_kernel runs p with four wavefronts.  Eight: split keys and long paged contexts (see the kernel); and long sequences of one length that go over the
+// chip more than four times, where the ends weigh little and half as many loads of keys count.  us with four / eight, causal: heads of 64, 192 of 8132 tokens 1761 / 1709,
+// 256 of 4096 620 / 603, 400 of 3000 563 / 570, 800 of 2000 535 / 550; of 32, 192 of 8132 1142 / 1098, 256 of 4096 397 / 391, 400 of 3000 358 / 370.
+constexpr int kSmallPaged = 128;                  // blocks: paged contexts that four wavefronts take
+static bool four_takes(const PrefillParams& p, int D, int n_cu) {
+    if (p.n_split > 1) return false;
+    if (p.block_table) return p.max_blocks <= kSmallPaged;
+    return D == 128 || !equal_pairs(p) || p.Sq < 4000 || (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B <= 16 * (int64_t)n_cu;
+}
 // Whether the 64-query kernel is left to prefill_fwd_kernel: short and ragged lengths, whose last tiles it computes in ordinary code and whose rounds it does not
 // fill.  Heads of 128, causal, us 64-query kernel / this: 64 heads of 700 tokens 38 / 25, 136 of 300 30 / 17, 1024 of 300 161 / 103, 14 packed of 111 to 1172, 32
 // heads, 133 / 96, 60 of 20 to 300, 16 heads, 97 / 44; but 136 of 1024 57 / 74, 256 of 1024 91 / 106, 136 of 2000 166 / 204, 14 x 16 heads of 644 65 / 69.  Twelve per
-// cent are left to the wide model, with which none of 170 calls got slower.
-static bool four_beats_wide(const PrefillParams& p, int n_cu) { return n_cu > 0 && four_takes(p) && four_us(p, 128, n_cu) < 0.88 * wide_us(p, n_cu); }
-static bool wide_takes(const PrefillParams& p) {
-    return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p) && !four_beats_wide(p, device_compute_units());
+// cent are left to the wide model, with which none of 170 calls got slower.  (Its persistent launch takes any number of tiles, the other a grid's worth.)
+static bool four_beats_wide(const PrefillParams& p, int n_cu) {
+    return n_cu > 0 && four_takes(p, 128, n_cu) && grid_fits((int64_t)((p.Sq + 255) / 256) * p.Hq * p.B, 256) && four_us(p, 128, n_cu) < 0.88 * wide_us(p, n_cu);
+}
+static bool wide_takes(const PrefillParams& p, int n_cu) {
+    return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p) && !four_beats_wide(p, n_cu);
 }
 
 // Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; of the rougher fits eight per cent are taken off).
@@ -877,8 +882,8 @@ static double other_us(const PrefillParams& p, int D, int n_cu) {
     // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
     if (prefill_short_takes(p, D))
         return 0.92 * ((D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + c.heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu);
-    if (D == 128 && wide_takes(p)) return 0.92 * wide_us(p, n_cu);
-    if (four_takes(p)) return four_us(p, D, n_cu);
+    if (D == 128 && wide_takes(p, n_cu)) return 0.92 * wide_us(p, n_cu);
+    if (four_takes(p, D, n_cu)) return four_us(p, D, n_cu);
     const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75, jobs = (p.Sq + kBM - 1) / kBM * c.heads;
     return 0.92 * (5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * c.mean_tiles(p, kBM) + 2.0)));
 }
@@ -886,12 +891,59 @@ static double other_us(const PrefillParams& p, int D, int n_cu) {
 // Wavefronts of prefill_keys.hip's kernel for p, 0: another kernel is the faster one.  One 183-token prompt, 16 heads, D 128: 64-query kernel 26.4 us, keys dealt to
 // the wavefronts 7.6; 4 of 700: 37.4, 33.0; of 1000: 44.9, 49.8; D 64, one of 1000: 18.7, 12.1; 8 sequences of 666, 8 heads: 18.1, 17.7; of 750: 20.4, 20.6.
 // (Training calls of short heads stay with the kernel that rounds fp32 operands on their way in: the same bits whichever type the inputs have.)
-static int keys_wavefronts(const PrefillParams& p, int D) {
-    if (p.lse && prefill_short_takes(p, D)) return 0;
-    const int n_cu = prefill_keys_takes(p, D) ? device_compute_units() : 0;
-    if (n_cu <= 0) return 0;
+static int keys_wavefronts(const PrefillParams& p, int D, int n_cu) {
+    if ((p.lse && prefill_short_takes(p, D)) || n_cu <= 0 || !prefill_keys_takes(p, D)) return 0;
     const PrefillKeysPlan plan = prefill_keys_plan(p.B, p.Hq, D, p.Sq, p.block_table ? 16 * p.max_blocks : p.Sk, p.mask_mode == MI355_MASK_CAUSAL, n_cu);
     return plan.us < other_us(p, D, n_cu) ? plan.wavefronts : 0;
+}
+
+// The kernel that takes a call, and its wavefronts per workgroup
+struct PrefillChoice {
+    int kernel, waves;
+};
+static PrefillChoice choose_prefill(const PrefillParams& p, int D, int n_cu) {
+    if (const int waves = keys_wavefronts(p, D, n_cu)) return {MI355_PREFILL_KEYS, waves};
+    if (prefill_short_takes(p, D)) return {MI355_PREFILL_SHORT, 4};
+    // head_dim 128 without an explicit mask: the kernel with 64 queries per wavefront and a hand-scheduled tile loop
+    if (D == 128 && wide_takes(p, n_cu)) return {MI355_PREFILL_W64, 4};
+    return {MI355_PREFILL_TILES, four_takes(p, D, n_cu) ? 4 : 8};
+}
+static int run_prefill(const PrefillParams& p, int D, hipStream_t s) {
+    const PrefillChoice c = choose_prefill(p, D, device_compute_units());
+    int rc;
+    if (c.kernel == MI355_PREFILL_KEYS) rc = launch_prefill_keys(p, D, c.waves, s);
+    else if (c.kernel == MI355_PREFILL_SHORT) rc = launch_prefill_short(p, D, s);
+    else if (c.kernel == MI355_PREFILL_W64) rc = launch_prefill_w64(p, s);
+    else if (p.block_table)
+        rc = D == 128 ? launch_prefill_paged<128>(p, c.waves, s) : (D == 64 ? launch_prefill_paged<64>(p, c.waves, s) : launch_prefill_paged<32>(p, c.waves, s));
+    else rc = D == 128 ? launch_prefill<128>(p, c.waves, s) : (D == 64 ? launch_prefill<64>(p, c.waves, s) : launch_prefill<32>(p, c.waves, s));
+    if (rc == 0 && p.n_split > 1) rc = launch_merge(p, D, s);
+    return rc == 0 ? MI355_OK : set_error(rc, hipGetErrorString((hipError_t)rc));
+}
+
+extern "C" int mi355_prefill_kernel(int B, int Hq, int Hkv, int D, int Sq_max, int Sk_max, int mask_mode, int packed, int max_blocks, int lse, int n_split, int window,
+                                    int n_compute_units, int* wavefronts) {
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Sq_max <= 0 || (Sk_max <= 0 && max_blocks <= 0) || !(D == 128 || D == 64 || D == 32)) return 0;
+    PrefillParams p{};
+    const int32_t given = 0;
+    float row = 0.f;
+    p.cu_q = packed || max_blocks > 0 ? &given : nullptr;
+    p.cu_k = packed ? &given : nullptr;
+    p.block_table = max_blocks > 0 ? &given : nullptr;
+    p.max_blocks = max_blocks;
+    p.lse = lse ? &row : nullptr;
+    p.B = B;
+    p.Hq = Hq;
+    p.Hkv = Hkv;
+    p.Sq = Sq_max;
+    p.Sk = max_blocks > 0 ? 0 : Sk_max;
+    p.scale_log2 = 1.f;
+    p.mask_mode = max_blocks > 0 ? MI355_MASK_CAUSAL : mask_mode;
+    p.n_split = n_split;
+    p.window = window;
+    const PrefillChoice c = choose_prefill(p, D, n_compute_units > 0 ? n_compute_units : device_compute_units());
+    if (wavefronts) *wavefronts = c.waves;
+    return c.kernel;
 }
 
 static int prefill_common(const void* q, const void* k, const void* v, void* out, const int64_t q_strides[3],
@@ -967,23 +1019,7 @@ static int prefill_common(const void* q, const void* k, const void* v, void* out
         return e;
     if ((int64_t)p.n_pairs * Hq * B > 0x7fffffffLL) return set_error(MI355_EINVAL, "prefill: too many workgroups");
 
-    hipStream_t s = (hipStream_t)stream;
-    int rc;
-    if (p.n_split > 1) {
-        if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
-        else rc = D == 128 ? launch_prefill<128>(p, s) : (D == 64 ? launch_prefill<64>(p, s) : launch_prefill<32>(p, s));
-        if (rc == 0) rc = launch_merge(p, D, s);
-        if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
-        return MI355_OK;
-    }
-    // head_dim 128 without an explicit mask: the kernel with 64 queries per wavefront and a hand-scheduled tile loop
-    const int keys = keys_wavefronts(p, D);
-    if (keys) rc = launch_prefill_keys(p, D, keys, s);
-    else if (prefill_short_takes(p, D)) rc = launch_prefill_short(p, D, s);
-    else if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
-    else rc = D == 128 ? launch_prefill<128>(p, s) : (D == 64 ? launch_prefill<64>(p, s) : launch_prefill<32>(p, s));
-    if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
-    return MI355_OK;
+    return run_prefill(p, D, (hipStream_t)stream);
 }
 
 extern "C" int mi355_prefill_fwd(const void* q, const void* k, const void* v, void* out,
@@ -1138,16 +1174,7 @@ static int prefill_paged_common(const void* q, const void* k_cache, const void* 
     p.max_blocks = (int)max_blocks;
     if (int e = set_split(p, D, n_split, total_q_rows, workspace, workspace_bytes, -1)) return e;
     if ((int64_t)p.n_pairs * Hq * B > 0x7fffffffLL) return set_error(MI355_EINVAL, "prefill_paged: too many workgroups");
-    hipStream_t s = (hipStream_t)stream;
-    // head_dim 128: the kernel with 64 queries per wavefront, which reads the block table too
-    int rc;
-    const int keys = keys_wavefronts(p, D);
-    if (keys) rc = launch_prefill_keys(p, D, keys, s);
-    else if (D == 128 && wide_takes(p)) rc = launch_prefill_w64(p, s);
-    else rc = D == 128 ? launch_prefill_paged<128>(p, s) : (D == 64 ? launch_prefill_paged<64>(p, s) : launch_prefill_paged<32>(p, s));
-    if (rc == 0 && p.n_split > 1) rc = launch_merge(p, D, s);
-    if (rc != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
-    return MI355_OK;
+    return run_prefill(p, D, (hipStream_t)stream);
 }
 
 extern "C" int mi355_prefill_paged_fwd(const void* q, const void* k_cache, const void* v_cache, void* out,

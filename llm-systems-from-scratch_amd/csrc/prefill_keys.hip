@@ -270,7 +270,7 @@ PrefillKeysPlan prefill_keys_plan(int B, int Hq, int D, int Sq, int Sk, bool cau
     const double n = (double)((Sq + kKyRows - 1) / kKyRows) * Hq * B;
     PrefillKeysPlan r{4, base + std::max(chain4 * tiles / 4, n / n_cu * (each + per_tile * mean))};
     if (n <= n_cu && tiles >= 16) r = {8, base + chain8 * tiles / 8};
-    if (n > 0x7fffffff) r.us = INFINITY;
+    if (n >= 1LL << 31 || !grid_fits((int64_t)n, r.wavefronts * 64)) r.us = INFINITY;
     return r;
 }
 

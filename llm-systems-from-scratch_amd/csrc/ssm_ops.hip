@@ -1242,7 +1242,7 @@ static int launch_chunks(const SsmParams<__bf16>& p, int64_t units, hipStream_t 
     if (wgs > 0x7fffffffLL) return (int)hipErrorInvalidValue;
     const dim3 grid((unsigned)wgs), block(256);
     if constexpr (MODE != kSegState) {
-        if (walk_takes(p) && walk_pays(p, wgs, MODE == kWhole || p.whole_len > 0)) {
+        if (walk_takes(p) && grid_fits(wgs, 512) && walk_pays(p, wgs, MODE == kWhole || p.whole_len > 0)) {
             if (p.N == 64) hipLaunchKernelGGL((ssd_walk_kernel<64, MODE>), grid, dim3(512), 0, s, p);
             else hipLaunchKernelGGL((ssd_walk_kernel<128, MODE>), grid, dim3(512), 0, s, p);
             return (int)hipGetLastError();

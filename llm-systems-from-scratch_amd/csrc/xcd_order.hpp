@@ -34,6 +34,8 @@ MI355_ORDER int xcd_units_front(int n_units, int group, int n_groups) { return n
 MI355_ORDER int xcd_units_grid(int n_units, int group, int n_groups) {
     return (xcd_units_front(n_units, group, n_groups) + 7) / 8 * 8 + n_groups / 8 * 8 * group * n_units;
 }
+// Whether that grid can be launched: its threads are counted in 32 bits.
+MI355_ORDER bool xcd_units_fit(long long n_units, long long group, long long n_groups, int threads) { return (n_units * group * n_groups + 7) * threads < 1LL << 32; }
 MI355_ORDER int turned(int i, int n, int width) {
     const int start = width > 0 ? i / width * width : 0;
     return width > 0 && (i / width & 1) && start + width <= n ? 2 * start + width - 1 - i : i;

@@ -46,6 +46,7 @@ EXPORTS = (
     "mi355_prefill_splitkv_workspace_bytes",
     "mi355_prefill_suggest_kv_splits",
     "mi355_prefill_suggest_prompt_kv_splits",
+    "mi355_prefill_kernel",
     "mi355_rope_and_cache",
     "mi355_rope_and_cache_fp8",
     "mi355_quantize_kv_fp8",
@@ -182,6 +183,8 @@ def load():
     lib.mi355_prefill_suggest_kv_splits.argtypes = [i32, i32, i32, i32, i32, i64, i32, i32]
     lib.mi355_prefill_suggest_prompt_kv_splits.restype = i32
     lib.mi355_prefill_suggest_prompt_kv_splits.argtypes = [i32, i32, i32, i32, i32, i64, i32, i32]
+    lib.mi355_prefill_kernel.restype = i32
+    lib.mi355_prefill_kernel.argtypes = [i32] * 13 + [vp]
     lib.mi355_paged_decode_fwd.restype = i32
     lib.mi355_paged_decode_fwd.argtypes = [vp, vp, vp, vp, vp, i64, vp, vp, vp, vp, sz,
                                            i32, i32, i32, i32, i32, i64, i32, f32, i32, vp]

@@ -16,16 +16,21 @@ def order(tmp_path_factory):
                    'extern "C" int units(int u, int group, int groups, int chunk, int round, int* out) {\n'
                    '  const int n = mi355::xcd_units_grid(u, group, groups);\n'
                    '  for (int i = 0; out && i < n; ++i) { const auto x = mi355::xcd_unit(i, u, group, groups, chunk, round); out[2 * i] = x.unit; out[2 * i + 1] = x.head; }\n'
-                   '  return n; }\n')
+                   '  return n; }\n'
+                   'extern "C" int fits(long long u, long long group, long long groups, int threads) { return mi355::xcd_units_fit(u, group, groups, threads); }\n')
     csrc = os.path.join(os.path.dirname(os.path.dirname(mi355_attn.__file__)), "csrc")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
     fn = ctypes.CDLL(str(lib)).units
+    fits = ctypes.CDLL(str(lib)).fits
+    fits.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int]
 
     def units(u, group, groups, chunk, rnd):
         n = fn(u, group, groups, chunk, rnd, None)
         out = (ctypes.c_int * (2 * n))()
         fn(u, group, groups, chunk, rnd, out)
         return [(out[2 * i], out[2 * i + 1]) for i in range(n)]
+    units.grid = lambda u, group, groups: fn(u, group, groups, 1, 0, None)
+    units.fits = fits
     return units
 
 
@@ -59,3 +64,33 @@ def test_two_shares_of_a_whole_prompt(D, prompt, chunk):
     assert lib.mi355_prefill_suggest_prompt_kv_splits(1, 8, D, 8192, 8192, 8192, 1, 256) == prompt
     assert lib.mi355_prefill_suggest_kv_splits(1, 8, D, 8192, 8192, 8192, 1, 256) == chunk
     assert lib.mi355_prefill_suggest_prompt_kv_splits(1, 4, D, 8192, 8192, 8192, 1, 256) == 4
+
+
+@pytest.mark.parametrize("threads", [256, 512])
+def test_grids_of_single_units_stay_below_the_threads_of_a_launch(order, threads):
+    """A grid's threads are counted in 32 bits.  Where single units are said to fit, the grid with its empty workgroups has fewer; where they are not, it is within
+    seven workgroups of that, or beyond."""
+    most = (1 << 32) // threads
+    for u, group, groups in ((1, 1, most - 1), (1, 1, most - 9), (1, 1, most // 2), (2, 1, most // 2 - 1), (3, 4, most // 12 - 1), (3, 4, most // 12 + 1), (7, 1, 9)):
+        if order.fits(u, group, groups, threads):
+            assert order.grid(u, group, groups) * threads < 1 << 32
+        else:
+            assert (u * group * groups + 7) * threads >= 1 << 32
+    assert not order.fits(1 << 20, 64, 1 << 20, threads)
+
+
+def named(B, Hq, Hkv, D, Sq, Sk, mask=1, packed=0, blocks=0, lse=0, split=1, window=0):
+    from mi355_attn import _lib
+    waves = ctypes.c_int(0)
+    kernel = _lib.load().mi355_prefill_kernel(B, Hq, Hkv, D, Sq, Sk, mask, packed, blocks, lse, split, window, 256, ctypes.byref(waves))
+    return kernel, waves.value
+
+
+TILES, W64, SHORT, KEYS = 1, 2, 3, 4
+
+
+def test_launches_beyond_a_grid_stay_with_the_persistent_kernel():
+    """Dense calls of head size 128 with 2^24 workgroups of 32 rows and more: more threads than a launch counts, but for the kernel that takes any number of tiles."""
+    assert named(1 << 19, 31, 31, 128, 32, 32) == (KEYS, 4)
+    assert named(1 << 19, 32, 32, 128, 32, 32) == named(1 << 20, 16, 16, 128, 32, 32) == named(1 << 19, 64, 32, 128, 20, 20, mask=0) == named(1 << 17, 128, 128, 128, 1, 32, lse=1) == (W64, 4)
+    assert named(0, 1, 1, 128, 1, 1)[0] == named(1, 3, 2, 128, 1, 1)[0] == named(1, 1, 1, 96, 1, 1)[0] == 0
