@@ -4,7 +4,7 @@
 // A workgroup owns 32 query rows of one (sequence, head); each of its NW wavefronts takes every NW-th tile of 32 keys, with K and V in
 // LDS of its own, and keeps its own row maxima, row sums and accumulators.  There is no barrier until the end, where the partial rows meet
 // in LDS, so a query tile's chain of dependent key tiles is an NW-th as long, and a launch has a workgroup for every 32 rows.  The maxima are
-// exact: the largest weight of a share of a row is 1 and not rounded, and errors are a tenth smaller than with a reference set beforehand.
+// exact: the largest weight of a share of a row is a power of two and not rounded, and errors are a tenth smaller than with a reference set beforehand.
 //
 // Bound by that chain where a launch is small -- the ends of a workgroup some 4 us, then about 1 us per four tiles at head size 128, for loads
 // that go out when their place is free, LDS, eight products one behind the other, weights, eight products -- and by instructions issued where it
@@ -22,6 +22,8 @@
 namespace mi355 {
 
 constexpr int kKyRows = 32, kKyKeys = 32;
+// A row's largest weight is 2^-kKyDown: sums over a million of the largest bf16 values stay finite, and products with values down to 2^-106 normal.
+constexpr float kKyDown = 20.0f;
 
 // Workgroups by number, worked out on the host: query tiles of a sequence and head, those of all query heads of a key head, of all heads;
 // query heads of a key head; workgroups in whole rounds of eight chunks (as in xcd_chunked_id)
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_keys_kernel(PrefillParams 
                 const float m_new = fmaxf(m_ref, mx), m_use = m_new == -INFINITY ? 0.f : m_new;     // no key yet: weights 0, not NaN
                 const float alpha = fast_exp2((m_ref - m_use) * p.scale_log2);
                 m_ref = m_new;
-                neg_ref = -m_use * p.scale_log2;
+                neg_ref = -m_use * p.scale_log2 - kKyDown;
                 l *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt)
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(NW * 64, 2) void prefill_keys_kernel(PrefillParams 
 #pragma unroll
             for (int e = 0; e < 4; ++e) w8[e] = pack_bf16(x[2 * e] * inv, x[2 * e + 1] * inv);
             *reinterpret_cast<u32x4*>(p.out + o_at + h * p.os[1] + (int64_t)(qw0 + r) * p.os[2] + 8 * ch) = w8;
-            if (p.lse && ch == 0) p.lse[l_at + h * p.ls[1] + qw0 + r] = sum > 0.f ? 0.69314718056f * (__log2f(sum) + mr * p.scale_log2) : -INFINITY;
+            if (p.lse && ch == 0) p.lse[l_at + h * p.ls[1] + qw0 + r] = sum > 0.f ? 0.69314718056f * (__log2f(sum) + (mr * p.scale_log2 + kKyDown)) : -INFINITY;
         }
         __syncthreads();                                                   // (the next rows' keys land in the partial rows' place)
     }

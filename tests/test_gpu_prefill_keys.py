@@ -80,3 +80,19 @@ def test_scores_of_any_size_and_their_sums(ops, D):  # noqa: F811
     s = (want[0] @ want[1].transpose(-1, -2) / math.sqrt(D)).masked_fill(~torch.ones(200, 200).tril().bool(), -math.inf)
     for g, w in zip(got, torch.autograd.grad(torch.softmax(s, -1) @ want[2], want, dout.float())):
         check(g, w, atol=2e-2 * float(w.abs().max()), rtol=2e-2, what="gradient")
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("S", [40, 300])
+def test_means_of_the_largest_and_of_tiny_values(ops, D, S):  # noqa: F811
+    """Rows are means of values: finite for the largest finite ones, and of the values' own size for tiny ones (300 keys: eight wavefronts).  Within a column values
+    are equal, so a row is the column's value: rounding of the result to 8 bits."""
+    from mi355_attn import _lib
+    lib = _lib.load()
+    assert lib.mi355_prefill_kernel(1, 2, 2, D, S, S, 1, 1, 0, 0, 1, 0, 0, None) == 4
+    print(f"case: keys dealt, values D={D} {S}", flush=True)
+    q, k, cu = rnd(S, 2, D, seed=30), rnd(S, 2, D, seed=31), _cu([S])
+    for size in (torch.finfo(torch.bfloat16).max, 2.0 ** -100):
+        v = (torch.linspace(-1, 1, D) * size).to(torch.bfloat16).repeat(S, 2, 1)
+        got = ops.flash_attn_varlen_prefill(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), S, S, kv_splits=1).double().cpu()
+        assert bool(((got - v.double()).abs() <= 2.0 ** -8 * v.double().abs()).all()), size
