@@ -450,7 +450,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1
         // the fp32 sums, harmless in bf16) and the O accumulators need no per-tile multiply.
         // The fast loop below therefore only accumulates in place; a tile that needs the
         // reference moved leaves it, rescales, and re-enters.
-        float slack = 8.0f;
+        float slack = 8.0f, down = 0.0f;         // (down: a reference's own weight is 2^-down)
         // The first attempt at a query tile does not look at row maxima at all (MODE NONE / CAUSAL): the reference is
         // preset to 0 (weights 2^(x - kBias), x the score in the log2 domain), and what is watched is the row SUM: a
         // partial sum that reaches 2 moves the row's reference up by the exponent of its sum, an exact rescaling by a
@@ -500,7 +500,7 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1
                 const float m_use = (m_new == -INFINITY) ? 0.f : m_new;    // row with no key yet: keep p = 0, not NaN
                 const float alpha = fast_exp2((m_ref - m_use) * scale_log2);
                 m_ref = m_new;
-                neg_ref = -m_use * scale_log2;
+                neg_ref = -m_use * scale_log2 - down;
                 l_run *= alpha;
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt)
@@ -533,33 +533,28 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1
         set_buf(t0 & (NB - 1));              // the offsets start at the first tile's buffer
         cur_tile = t0;
         if constexpr (kFollows) {
-            // the last three tiles that this wavefront sees, with references that begin at 0 and follow the scores: a row's largest weight there is 1 and
-            // is not rounded.  (With the preset ones the error of short sequences is a tenth larger.)
+            // the last three tiles that this wavefront sees, with references that begin at 0 and follow the scores: a row's largest weight there is 2^-kBias
+            // and is not rounded.  (With the preset ones the error of short sequences is a tenth larger.)
             const int seen = causal ? min(t1, max(t0, WINDOW ? t1 : (qw0 + 31 + coff + kBN) / kBN)) : t1;
             int from = scale_log2 > 0.f ? max(t0, seen - 3) : t1;        // (a maximum of scores is none of their negatives)
             neg_ref = -kBias;
             if constexpr (WINDOW) run_tiles_preset(std::true_type{}, t0, min(n_low, from));
             run_tiles_preset(std::false_type{}, max(n_low, t0), min(n_plain, from));
             run_tiles_preset(std::true_type{}, max(n_plain, t0), from);
-            constexpr float kUp = 4294967296.0f;                         // 2^kBias
-            l_run *= kUp;
-#pragma unroll
-            for (int i = 0; i < NDT; ++i)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) o[i][j] *= kUp;
-            neg_ref += kBias;
-            m_ref = scale_log2 > 0.f ? -neg_ref / scale_log2 : 0.f;
+            m_ref = scale_log2 > 0.f ? -(neg_ref + kBias) / scale_log2 : 0.f;
             slack = 0.0f;
+            down = kBias;
             for (;;) {
                 if constexpr (WINDOW) run_tiles(std::true_type{}, from, n_low);
                 run_tiles(std::false_type{}, max(n_low, from), min(n_plain, t1));
                 run_tiles(std::true_type{}, max(n_plain, from), t1);
                 if (tracked) break;
                 const float l = xor32_sum(l_run);
-                const bool bad = redo || (sees && !(l >= kUnderflow * kUp)) || !(l <= kOverflow * kUp);
+                const bool bad = redo || (sees && !(l >= kUnderflow)) || !(l <= kOverflow);
                 if (!__syncthreads_or(bad ? 1 : 0)) break;
                 begin_tracked();
                 slack = 8.0f;
+                down = 0.0f;
                 from = t0;
                 set_buf(t0 & (NB - 1));
                 cur_tile = t0;

@@ -99,3 +99,25 @@ def test_gradients_of_dealt_tiles(ma, monkeypatch, D, H, Hkv, lens, promised):
                 # (a single key has no gradient but what rounding leaves)
                 assert float((x.double().cpu() - y).norm()) <= 2 ** -7 * float(y.norm()) + (1e-2 if n == 1 else 0.0), (a, n, h)
         a += n
+
+
+@pytest.mark.parametrize("window", [0, 150])
+@pytest.mark.parametrize("S", [64, 300, 700])
+def test_values_beyond_2_to_the_94_under_high_scores(ma, S, window):
+    """Heads of 128 on four wavefronts, every weight 2^24 times that of a score of 0: rows stay the means of their values, of which each column has equal
+    ones (S of 64: inside the last three key tiles, whose references follow the scores; 300 and 700: in front of them too)."""
+    import ctypes
+    from mi355_attn import _lib
+    D, H, B, waves = 128, 4, {64: 200, 300: 60, 700: 20}[S], ctypes.c_int(0)
+    kernel = _lib.load().mi355_prefill_kernel(B, H, H, D, S, S, 1, window, 0, 0, 1, window, 0, ctypes.byref(waves))
+    assert (kernel, waves.value) == (1, 4)
+    print(f"case: values of 2^120 {S} {window}", flush=True)
+    q = torch.zeros(B, H, S, D, device="cuda", dtype=torch.bfloat16)
+    k = torch.randn(B, H, S, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(S)).bfloat16()
+    q[..., 0], k[..., 0] = 13.75, 13.6875                 # 24 = 13.75 * 13.6875 / sqrt(128) * log2(e)
+    v = (torch.linspace(-1, 1, D, device="cuda") * 2.0 ** 120).bfloat16().expand(B, H, S, D).contiguous()
+    cu = (torch.arange(B + 1, device="cuda") * S).int()
+    rows = [x.transpose(1, 2).reshape(B * S, H, D) for x in (q, k, v)]
+    outs = [ma.flash_attn_varlen_prefill(*rows, cu, cu, S, S, window=window).view(B, S, H, D).transpose(1, 2)] if window else [ma.flash_attn_prefill(q, k, v, causal=True)]
+    for got in outs:
+        assert bool(((got.double() - v.double()).abs() <= 2.0 ** -8 * v.double().abs()).all())
