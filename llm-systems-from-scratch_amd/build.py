@@ -101,6 +101,16 @@ def _sregs(text):
     return out
 
 
+def issues_memory_from_assembly(src: str) -> bool:
+    """Whether kernels of `src` have inline-assembly memory instructions, of their own or through a header's."""
+    with open(os.path.join(CSRC, src)) as f:
+        text = f.read()
+    if re.search(r'\bdma_to_lds_\w+\(|"[^"\n]*\b(global|buffer|flat|scratch)_(load|store|atomic)', text):
+        return True
+    # (common.hpp defines the direct-to-LDS loads; who calls them is what counts)
+    return any(issues_memory_from_assembly(h) for h in re.findall(r'^#include "(\w+\.hpp)"', text, re.M) if h != "common.hpp")
+
+
 def check_scalar_address_hazards(src: str) -> str:
     """gfx9 wants five wait states between a VECTOR instruction that writes a scalar register (v_readlane restoring a
     spilled value, v_readfirstlane, a compare or a carry-out) and a vector-memory instruction that reads that register
@@ -213,12 +223,10 @@ def build_library(verbose: bool = True) -> str:
     _run([sys.executable, os.path.join(CSRC, "gen_prefill_w64_loop.py")])
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
 
-    # sources whose kernels issue memory instructions from inline assembly
-    asm_dma = [s for s in ("prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_keys.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "moe_ops.hip", "rows_linear.hip") if s in srcs]
     with ThreadPoolExecutor(max_workers=5) as ex:
         calls = ex.submit(compile_calls)
         check = ex.submit(check_w64_registers)
-        hazards = [ex.submit(check_scalar_address_hazards, s) for s in asm_dma]
+        hazards = [ex.submit(check_scalar_address_hazards, s) for s in srcs if issues_memory_from_assembly(s)]
         results = _compile_all(srcs)
         notes = [check.result()] + [h.result() for h in hazards]
     if verbose:

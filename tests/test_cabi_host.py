@@ -365,3 +365,16 @@ def test_native_calls_that_do_not_load_are_reported(tmp_path, library, calls, wa
                          cwd=tmp_path, capture_output=True, text=True, timeout=110)
     assert run.returncode == 0 and run.stdout.strip() == "None", run.stderr
     assert ("native calls are not there" in run.stderr) == warns, run.stderr
+
+
+def test_the_build_looks_at_every_source_with_memory_instructions_in_assembly():
+    """Those that issue direct-to-LDS loads or loads of their own from inline assembly, themselves or through a header, and no others."""
+    import importlib.util
+    import os
+    root = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llm-systems-from-scratch_amd")
+    spec = importlib.util.spec_from_file_location("mi355_build_sources", os.path.join(root, "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    looked_at = {s for s in build.SOURCES if build.issues_memory_from_assembly(s)}
+    assert looked_at == {"prefill_fwd.hip", "prefill_fwd_w64.hip", "prefill_short.hip", "prefill_keys.hip", "prefill_bwd.hip", "prefill_bwd_short.hip", "ssm_ops.hip",
+                         "moe_ops.hip", "rows_linear.hip"}
