@@ -2,6 +2,8 @@
 #include <hip/hip_runtime.h>
 #include <string.h>
 
+#include <atomic>
+
 #include "launch.hpp"
 
 static thread_local char g_last_error[256] = "";
@@ -10,6 +12,16 @@ int set_error(int code, const char* msg) {
     strncpy(g_last_error, msg ? msg : "", sizeof(g_last_error) - 1);
     g_last_error[sizeof(g_last_error) - 1] = '\0';
     return code;
+}
+
+int device_compute_units() {
+    static std::atomic<int> known[64];                // (asked of the runtime once per device)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
+    return n;
 }
 
 extern "C" const char* mi355_last_error(void) { return g_last_error; }

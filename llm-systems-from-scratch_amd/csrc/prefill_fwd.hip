@@ -21,7 +21,6 @@
 // padded; bank conflicts are avoided by an XOR swizzle instead: the 16-byte chunk
 // c of row r is stored in slot c ^ swz(r), applied on the global-address side.
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <type_traits>
 
@@ -636,16 +635,6 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1
     }
 }
 
-static int device_compute_units() {
-    static std::atomic<int> known[64];                // (asked of the runtime once per device)
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    if (dev >= 0 && dev < 64 && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (dev >= 0 && dev < 64) known[dev].store(n, std::memory_order_relaxed);
-    return n;
-}
-
 // One length and the causal triangle: pairs of query tiles carry equal work.
 static bool equal_pairs(const PrefillParams& p) {
     return p.mask_mode == MI355_MASK_CAUSAL && !(p.window > 0 && p.window < p.Sq) && (!p.cu_q || p.B == 1 || p.n_split > 1);
@@ -679,14 +668,18 @@ static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {
     const PrefillParams p = with_units(p0, NW, D);
     // 1-D in x (see the kernel's order); y = share of the keys
     const dim3 grid(units_grid(p), (unsigned)(p.n_split > 1 ? p.n_split : 1)), block(NW * 64);
-    if (p.mask_mode == MI355_MASK_CAUSAL && p.window > 0)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, true, NW>), grid, block, 0, stream, p);
-    else if (p.mask_mode == MI355_MASK_CAUSAL)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, false, NW>), grid, block, 0, stream, p);
-    else if (p.mask_mode == MI355_MASK_BOOL)
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_BOOL, false, false, NW>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE, false, false, NW>), grid, block, 0, stream, p);
+    if constexpr (NW == 4) {                                         // (see four_takes)
+        if (p.mask_mode == MI355_MASK_CAUSAL && p.window > 0) {
+            hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, true, NW>), grid, block, 0, stream, p);
+            return (int)hipGetLastError();
+        }
+        if (p.mask_mode == MI355_MASK_BOOL) {
+            hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_BOOL, false, false, NW>), grid, block, 0, stream, p);
+            return (int)hipGetLastError();
+        }
+    }
+    if (p.mask_mode == MI355_MASK_CAUSAL) hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_CAUSAL, false, false, NW>), grid, block, 0, stream, p);
+    else hipLaunchKernelGGL((prefill_fwd_kernel<D, MI355_MASK_NONE, false, false, NW>), grid, block, 0, stream, p);
     return (int)hipGetLastError();
 }
 template <int D>
@@ -857,7 +850,7 @@ constexpr int kSmallPaged = 128;                  // blocks: paged contexts that
 static bool four_takes(const PrefillParams& p, int D, int n_cu) {
     if (p.n_split > 1) return false;
     if (p.block_table) return p.max_blocks <= kSmallPaged;
-    return D == 128 || !equal_pairs(p) || p.Sq < 4000 || (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B <= 16 * (int64_t)n_cu;
+    return D == 128 || p.window > 0 || !equal_pairs(p) || p.Sq < 4000 || (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B <= 16 * (int64_t)n_cu;
 }
 // Whether the 64-query kernel is left to prefill_fwd_kernel: short and ragged lengths, whose last tiles it computes in ordinary code and whose rounds it does not
 // fill.  Heads of 128, causal, us 64-query kernel / this: 64 heads of 700 tokens 38 / 25, 136 of 300 30 / 17, 1024 of 300 161 / 103, 14 packed of 111 to 1172, 32

@@ -115,36 +115,23 @@ __device__ __forceinline__ void store_ch(T* p, const float (&v)[V]) {
 // Bound by its bytes where a call is large (8192 tokens, 4352 channels: 142 MB in 30 us) and by one load's latency where it is small, so all rows of a batch of
 // eight, and those that go to the ring, are requested before the first is used: a load in front of every token's sum took 11 to 13 us for 600 to 1700 tokens,
 // 4 tokens per thread in one batch take 7.  Tiles of 4 read 7 rows for 4, tiles of 16 19 for 16.
-template <typename T, int V>
-struct ChannelRow {                                      // V adjacent channels as they are in memory
-    static constexpr int kWords = V * sizeof(T) < 4 ? 1 : V * sizeof(T) / 4;
-    uint32_t w[kWords];
+template <typename T>
+struct ChannelRow {                                      // eight adjacent channels as they are in memory
+    static constexpr int kPieces = 8 * sizeof(T) / 16;
+    u32x4 w[kPieces];
     __device__ __forceinline__ void load(const T* p) {
-        if constexpr (V == 1) {
-            w[0] = 0u;
-            __builtin_memcpy(w, p, sizeof(T));
-        } else {
 #pragma unroll
-            for (int i = 0; i < kWords / 4; ++i) {
-                const u32x4 x = reinterpret_cast<const u32x4*>(p)[i];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) w[4 * i + e] = x[e];
-            }
-        }
+        for (int i = 0; i < kPieces; ++i) w[i] = reinterpret_cast<const u32x4*>(p)[i];
     }
     __device__ __forceinline__ void store(T* p) const {
-        if constexpr (V == 1) {
-            __builtin_memcpy(p, w, sizeof(T));
-        } else {
 #pragma unroll
-            for (int i = 0; i < kWords / 4; ++i) reinterpret_cast<u32x4*>(p)[i] = u32x4{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]};
-        }
+        for (int i = 0; i < kPieces; ++i) reinterpret_cast<u32x4*>(p)[i] = w[i];
     }
-    __device__ __forceinline__ void get(float (&v)[V]) const {
+    __device__ __forceinline__ void get(float (&v)[8]) const {
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            if constexpr (sizeof(T) == 2) v[e] = __builtin_bit_cast(float, e % 2 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
-            else v[e] = __builtin_bit_cast(float, w[e]);
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t x = sizeof(T) == 2 ? w[e / 8][e / 2] : w[e / 4][e % 4];
+            v[e] = __builtin_bit_cast(float, sizeof(T) == 2 ? (e % 2 ? x & 0xffff0000u : x << 16) : x);
         }
     }
 };
@@ -181,8 +168,9 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
     const int n = min(TILE, len - t0);
     T* out = p.xbc + (int64_t)(first + t0) * p.channels + c;
     if constexpr (TAPS > 0) {
-        constexpr int BATCH = TILE < 8 ? TILE : 8, KEEP = TAPS > 1 ? TAPS - 1 : 1;
-        ChannelRow<T, V> row[BATCH], keep[KEEP];
+        static_assert(V == 8 && TAPS > 1, "rows in whole pieces");
+        constexpr int BATCH = TILE < 8 ? TILE : 8;
+        ChannelRow<T> row[BATCH], keep[TAPS - 1];
         const auto request = [&](int t1) {                       // (a tile's rows past the end: the last one again)
 #pragma unroll
             for (int i = 0; i < BATCH; ++i) row[i].load(in + (int64_t)(t0 + min(t1 + i, n - 1)) * p.proj_stride);
@@ -1230,8 +1218,8 @@ static bool walk_takes(const SsmParams<__bf16>& p) { return (p.N == 64 || p.N ==
 // segments of 512 198 / 190; 16 heads, 4000 in segments of 256 57 / 64; state 64, 64 heads: 5 of 122 to 1965 75 / 97, 5 x 111 31 / 30, 14 of 56 to 911 88 / 86.
 // (A call that cuts only long sequences has most of them whole.)
 static bool walk_pays(const SsmParams<__bf16>& p, int64_t wgs, bool whole) {
-    int dev = 0, n_cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+    const int n_cu = device_compute_units();
+    if (n_cu <= 0) return false;
     const bool longer = whole && p.n_rows >= 192LL * p.B;
     return wgs <= (p.N == 128 || longer ? n_cu + n_cu / 4 : n_cu) || (longer && p.N == 128);
 }
