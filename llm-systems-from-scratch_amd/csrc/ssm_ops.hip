@@ -112,9 +112,11 @@ __device__ __forceinline__ void store_ch(T* p, const float (&v)[V]) {
 // one that touches the sequence's ring for its channels: it reads the history first and writes the last taps - 1 inputs of the portion at its end.
 // (So a tile has at least taps - 1 tokens: conv_tile.)
 //
-// Bound by its bytes where a call is large (8192 tokens, 4352 channels: 142 MB in 30 us) and by one load's latency where it is small, so all rows of a batch of
-// eight, and those that go to the ring, are requested before the first is used: a load in front of every token's sum took 11 to 13 us for 600 to 1700 tokens,
-// 4 tokens per thread in one batch take 7.  Tiles of 4 read 7 rows for 4, tiles of 16 19 for 16.
+// Bound by its bytes where a call is large (8192 tokens, 4352 channels: 142 MB in 26 us) and by one load's latency where it is small, so all rows of a tile of 4 or 8
+// tokens, and those that go to the ring, are requested before the first is used: a load in front of every token's sum took 11 to 13 us for 600 to 1700 tokens,
+// 4 tokens per thread take 7.  Tiles of 4 read 7 rows for 4, tiles of 16 19 for 16.  In those, whose calls have wavefronts enough, loads stand where
+// they are used: eight rows ahead hold registers that wavefronts would have.  us like this / eight ahead: 4000 tokens of 4352 channels 15.7 / 18.0, 64 x 100 26.4 / 29.6,
+// 2 x 7000 49.2 / 52.1, 4 x 8000 of 1792 47.7 / 51.0.
 template <typename T>
 struct ChannelRow {                                      // eight adjacent channels as they are in memory
     static constexpr int kPieces = 8 * sizeof(T) / 16;
@@ -169,70 +171,81 @@ __global__ __launch_bounds__(256) void causal_conv_silu_kernel(SsmParams<T> p) {
     T* out = p.xbc + (int64_t)(first + t0) * p.channels + c;
     if constexpr (TAPS > 0) {
         static_assert(V == 8 && TAPS > 1, "rows in whole pieces");
-        constexpr int BATCH = TILE < 8 ? TILE : 8;
-        ChannelRow<T> row[BATCH], keep[TAPS - 1];
-        const auto request = [&](int t1) {                       // (a tile's rows past the end: the last one again)
-#pragma unroll
-            for (int i = 0; i < BATCH; ++i) row[i].load(in + (int64_t)(t0 + min(t1 + i, n - 1)) * p.proj_stride);
-        };
         float w[TAPS][V], x[TAPS][V];
-        request(0);
+        const auto load_weights = [&]() {
+            load_ch<float, V>(p.conv_b + c, bias);
 #pragma unroll
-        for (int j = 0; j + 1 < TAPS; ++j) input(t0 - (TAPS - 1) + j, x[j]);
-        if (t0 == 0)
+            for (int j = 0; j < TAPS; ++j) load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w[j]);
+        };
+        const auto load_history = [&]() {
 #pragma unroll
-            for (int j = 0; j + 1 < TAPS; ++j) keep[j].load(in + (int64_t)max(0, len - (TAPS - 1) + j) * p.proj_stride);
-        load_ch<float, V>(p.conv_b + c, bias);
+            for (int j = 0; j + 1 < TAPS; ++j) input(t0 - (TAPS - 1) + j, x[j]);
+        };
+        const auto emit = [&](int t) {                           // token t of the tile, whose own input is in x[TAPS - 1]
+            float a[V];
 #pragma unroll
-        for (int j = 0; j < TAPS; ++j) load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w[j]);
+            for (int e = 0; e < V; ++e) {
+                a[e] = bias[e];
 #pragma unroll
-        for (int t1 = 0; t1 < TILE; t1 += BATCH) {
-            if (t1 > 0) {
-                if (t1 >= n) break;
-                request(t1);
+                for (int j = 0; j < TAPS; ++j) a[e] = fmaf(w[j][e], x[j][e], a[e]);
+                a[e] = silu_of<FAST>(a[e]);
             }
+            if (t < n) store_ch<T, V>(out + (int64_t)t * p.channels, a);
 #pragma unroll
-            for (int i = 0; i < BATCH; ++i) {
+            for (int j = 0; j + 1 < TAPS; ++j)
+#pragma unroll
+                for (int e = 0; e < V; ++e) x[j][e] = x[j + 1][e];
+        };
+        if constexpr (TILE < kMostConvTile) {
+            ChannelRow<T> row[TILE], keep[TAPS - 1];
+#pragma unroll
+            for (int i = 0; i < TILE; ++i) row[i].load(in + (int64_t)(t0 + min(i, n - 1)) * p.proj_stride);       // (rows past the end: the last one again)
+            load_history();
+            if (t0 == 0)
+#pragma unroll
+                for (int j = 0; j + 1 < TAPS; ++j) keep[j].load(in + (int64_t)max(0, len - (TAPS - 1) + j) * p.proj_stride);
+            load_weights();
+#pragma unroll
+            for (int i = 0; i < TILE; ++i) {
                 row[i].get(x[TAPS - 1]);
-                float a[V];
+                emit(i);
+            }
+            if (t0 == 0) {
 #pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    a[e] = bias[e];
-#pragma unroll
-                    for (int j = 0; j < TAPS; ++j) a[e] = fmaf(w[j][e], x[j][e], a[e]);
-                    a[e] = silu_of<FAST>(a[e]);
+                for (int j = 0; j + 1 < TAPS; ++j) {
+                    const int t = len - (TAPS - 1) + j;
+                    if (t >= 0) keep[j].store(ring + (int64_t)((pos0 + t) % TAPS) * p.channels);
                 }
-                if (t1 + i < n) store_ch<T, V>(out + (int64_t)(t1 + i) * p.channels, a);
+            }
+            return;
+        } else {
+            load_weights();
+            load_history();
 #pragma unroll
-                for (int j = 0; j + 1 < TAPS; ++j)
-#pragma unroll
-                    for (int e = 0; e < V; ++e) x[j][e] = x[j + 1][e];
+            for (int t = 0; t < TILE; ++t) {
+                if (t < n) {
+                    load_ch<T, V>(in + (int64_t)(t0 + t) * p.proj_stride, x[TAPS - 1]);
+                    emit(t);
+                }
             }
         }
-        if (t0 == 0) {
+    } else {
+        load_ch<float, V>(p.conv_b + c, bias);
+        for (int t = 0; t < n; ++t) {
+            float a[V];
 #pragma unroll
-            for (int j = 0; j + 1 < TAPS; ++j) {
-                const int t = len - (TAPS - 1) + j;
-                if (t >= 0) keep[j].store(ring + (int64_t)((pos0 + t) % TAPS) * p.channels);
+            for (int e = 0; e < V; ++e) a[e] = bias[e];
+            for (int j = 0; j < taps; ++j) {
+                float w[V], x[V];
+                load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w);
+                input(t0 + t - (taps - 1) + j, x);
+#pragma unroll
+                for (int e = 0; e < V; ++e) a[e] = fmaf(w[e], x[e], a[e]);
             }
+#pragma unroll
+            for (int e = 0; e < V; ++e) a[e] = silu_of<FAST>(a[e]);
+            store_ch<T, V>(out + (int64_t)t * p.channels, a);
         }
-        return;
-    }
-    load_ch<float, V>(p.conv_b + c, bias);
-    for (int t = 0; t < n; ++t) {
-        float a[V];
-#pragma unroll
-        for (int e = 0; e < V; ++e) a[e] = bias[e];
-        for (int j = 0; j < taps; ++j) {
-            float w[V], x[V];
-            load_ch<float, V>(p.conv_w + (int64_t)j * p.channels + c, w);
-            input(t0 + t - (taps - 1) + j, x);
-#pragma unroll
-            for (int e = 0; e < V; ++e) a[e] = fmaf(w[e], x[e], a[e]);
-        }
-#pragma unroll
-        for (int e = 0; e < V; ++e) a[e] = silu_of<FAST>(a[e]);
-        store_ch<T, V>(out + (int64_t)t * p.channels, a);
     }
     if (t0 == 0) {
         for (int t = max(0, len - (taps - 1)); t < len; ++t) {
