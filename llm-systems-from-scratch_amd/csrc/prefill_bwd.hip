@@ -24,6 +24,7 @@
 // of llm-core/llm_core/model.py:308-325, which its non-flash branch passes at model.py:384-385).  The explicit mask is
 // the general, slower path: every tile takes the per-element select and reads its mask bytes from global memory.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -1394,19 +1395,29 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
     // Up to 128 tokens that do not fill the chip either way: one launch more costs what dS saves (4 x 128, 8 / 2 heads 33 us against
     // 37; 64 x 128, 16 / 4 heads 83 against 73), and up to 64 it is most of what runs (16 x 64, 8 heads 17 against 20).
     if (std::max(Sq, Sk) <= (tiles_k < 256 ? 128 : 64)) return false;
-    // At head sizes 64 and 32 the products that dS saves are worth less than its bytes, and what this form has over the other is that the rows of a key
-    // tile can be dealt out and workgroups come in order of cost.  So it is for launches whose longest chain -- the steps of the first key tile of the
-    // longest sequence -- is several times what a workgroup's place on the chip has to do on average, and at 64 for lengths far apart (their mean below half
-    // the longest).  us with dS / without (chain in steps, over the average): heads of 64: 8 of 3000 tokens (47, 5.4) 99 / 120, 16 of 3000 (47, 2.7) 129 /
-    // 133, 32 of 1456 (23, 2.7) 74 / 71, 16 of 6000 (94, 1.4) 413 / 315; heads of 32: 16 of 2048 (32, 8) 83 / 69, 8 of 3000 (47, 11) 91 / 95; packed, 8 / 1
-    // heads: 12 of 490 to 5500 tokens, of 32 (688, 13) 630 / 1041, of 64 (688, 6.7) 834 / 1340, 36 of 112 to 1802 262 / 357 and 281 / 456.
-    // (Few key tiles of short sequences: 3 to 7 us fewer without in calls that the host's side of a gradient, some 70 us, outlasts either way.)
+    // At head sizes 64 and 32 the products that dS saves are worth less than its bytes.  What this form has over the other is that the row tiles of a key tile can be dealt
+    // out (shares) and that workgroups come in order of cost.  So it is for launches whose longest chain -- the steps of the first key tile of the longest
+    // sequence -- is many steps and many times what a workgroup's place on the chip has to do on average (`over`, for the causal triangle; longest: of the
+    // lengths, over their mean).  us with dS / without (steps, over):
+    //   heads of 32, causal: 16 of 2048 tokens (32, 8) 80 / 68, 8 of 4096 (64, 8) 122 / 128, 4 x 1024, 32 / 8 heads, (64, 8) 96 / 113, 2 x 3494, 32 / 4, (440, 9.3) 435 / 623,
+    //     16 / 4 heads, 512 (32, 128) 34 / 51, 6 x 326, 32 / 8, (24, 16) 42 / 45, 4 x 3900, 16 / 4, (244, 4.2) 562 / 450; not dealt out: 24 of 1456 (23, 7.1) 61 / 53;
+    //     packed, 32 of up to 339 tokens, 64 / 8, (48, 14, longest 2.2) 127 / 107, 12 of 490 to 5500, 8 / 1, (688, 13, 2) 630 / 1041
+    //   heads of 64, causal: 8 of 1456 (23, 11) 59 / 63, 16 of 1456 (23, 5.3) 64 / 64, 24 of 1024 (16, 5.3) 58 / 50, 32 / 16, 3 x 738 (24, 3.6) 70 / 64, 8 x 1589,
+    //     16 / 4, (100, 2.56) 268 / 260, 6315, 32 / 8, (396, 2.56) 933 / 840, 6 x 6166, 8 / 2, packed, (388, 2.9) 814 / 933, 8 of up to 764, 16 / 8, (24, 7.4, longest 1.7) 72 / 64; not dealt out: 16 of 3000 (47, 2.7) 126 / 133, 24 of 2048 (32, 2.7) 95 / 96
+    //   without a mask, of 32: 4223, 16 / 4, (264, 16) 349 / 622, 24 x 1234, 4 / 1, (80, 8.8) 160 / 209; of 64: 3796, 64 / 16, (240, 2.1) 1231 / 995; not dealt out: packed,
+    //     12 of up to 2001, 4 heads, (32, 8.4) 95 / 116
+    // Of 2619 drawn calls of 130 to 7000 tokens none is more than 8 % slower than by the number of key tiles alone, and 6 by more than 3 %.  (Short sequences with few key
+    // tiles, and at 64 lengths far apart, keep dS: up to 10 us of the GPU more, in calls that the host's side of a gradient, some 70 us, outlasts either way.)
     if (D < 128) {
         const int64_t steps = n_rt * G, places = kCus * (D == 32 ? 4 : 2);
         const double longest = packed ? (double)B * Sk / total_k : 1.0, over = 2.0 * places / tiles_k * longest;
-        const bool chain = D == 64 ? over >= 2.69 && steps >= (out.shares > 1 ? 20 : 40) : over >= 10.0 && steps >= 32;
-        const bool few = std::max(Sq, Sk) > 160 && tiles_k <= (D == 64 ? 384 : 256) && steps < 24;
-        if (!chain && !few && !(D == 64 && packed && 2 * total_k < (int64_t)B * Sk)) return false;
+        const bool short_ones = std::max(Sq, Sk) <= 160, few = !short_ones && tiles_k <= (D == 64 ? 384 : 256) && steps < 24;
+        const double line = D == 32 ? (causal ? 490.0 : 600.0) : causal ? 164.0 : 270.0;
+        const bool dealt = out.shares > 1 && (D == 64 || !short_ones) && over >= (D == 32 ? 8.0 : causal ? 2.69 : 3.5) && steps >= 24 &&
+                           steps * over >= line * std::sqrt(longest);
+        const bool ordered = D == 64 && ((packed && 2 * total_k < (int64_t)B * Sk) ||
+                                         (out.shares == 1 && !short_ones && (causal ? steps >= 36 && over >= 2.69 : steps >= 20 && over >= 5.0)));
+        if (!dealt && !ordered && !few) return false;
     }
     if (out.shares > 1) {
         out.part_rows = rows_k;

@@ -331,6 +331,24 @@ def test_workspace_of_the_backward_with_ds():
     assert ws(1, 64, 1, 1 << 18, 1 << 18, 128, causal, 0, 1, 0, 0) == 0          # a kv head alone does not fit
 
 
+def test_heads_of_32_and_64_keep_ds_where_it_is_the_faster_form():
+    """Both sides of each line, measured (us with dS / without): causal ones of many steps and of launches that fill the chip, none masked, packed of different lengths."""
+    ws = _lib.load().mi355_prefill_bwd_ds_workspace
+
+    def keeps(B, Hq, Hkv, S, D, causal=True, total=0):
+        return ws(B, Hq, Hkv, S, S, D, _lib.MASK_CAUSAL if causal else _lib.MASK_NONE, 1 if total else 0, 1, total, total) > 0
+
+    assert keeps(2, 32, 4, 3494, 32) and keeps(4, 32, 8, 1024, 32) and keeps(3, 16, 2, 4557, 32)               # 435 / 623, 96 / 113, 593 / 840
+    assert keeps(1, 8, 8, 4096, 32) and keeps(12, 8, 1, 5500, 32, total=33500)                                 # 122 / 128, 630 / 1041
+    assert not keeps(1, 16, 16, 2048, 32) and not keeps(4, 16, 4, 3900, 32)                                    # 80 / 68, 562 / 450
+    assert not keeps(32, 64, 8, 339, 32, total=4940) and not keeps(12, 16, 4, 681, 32, total=8172)             # 127 / 107, 93 / 85
+    assert keeps(1, 8, 8, 3000, 64) and keeps(4, 32, 8, 1024, 64) and keeps(1, 16, 16, 2814, 64)               # 100 / 121, 119 / 151, 123 / 128
+    assert not keeps(3, 32, 16, 738, 64) and not keeps(1, 24, 24, 3000, 64) and not keeps(1, 32, 32, 2048, 64)  # 70 / 64, 170 / 144, 106 / 101
+    assert keeps(6, 8, 2, 6166, 64, total=28887) and not keeps(1, 32, 8, 6315, 64)                             # 814 / 933, 933 / 840
+    assert keeps(1, 16, 4, 4223, 32, causal=False) and keeps(24, 4, 1, 1234, 32, causal=False)                 # 349 / 622, 160 / 209
+    assert not keeps(1, 64, 16, 3796, 64, causal=False) and not keeps(64, 4, 1, 1115, 32, causal=False)        # 1231 / 995, 392 / 218
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_workspace_of_the_backward_with_ds_at_lengths_beyond_32_bits_of_blocks(causal):
     """Lengths up to 2^24, with the causal diagonal in the middle and at either end: the blocks of one head counted in Python's integers, or 0
