@@ -809,29 +809,33 @@ static int set_split(PrefillParams& p, int D, int n_split, int64_t total_q_rows,
 
 // What the models below need of a call (lengths of a packed batch are judged by the longest)
 struct CallSize {
-    double heads, over, keys;                         // over: keys that every query sees (causal); keys: of the last query
+    double heads, over, keys, Sk;                     // over: keys that every query sees (causal); keys: of the last query
     bool causal;
-    explicit CallSize(const PrefillParams& p) : heads((double)p.Hq * p.B), causal(p.mask_mode == MI355_MASK_CAUSAL) {
-        const int Sk = p.block_table ? 16 * p.max_blocks : p.Sk;
+    explicit CallSize(const PrefillParams& p) : heads((double)p.Hq * p.B), Sk(p.block_table ? 16.0 * p.max_blocks : p.Sk), causal(p.mask_mode == MI355_MASK_CAUSAL) {
         over = causal && Sk > p.Sq ? Sk - p.Sq : 0;
         keys = causal ? std::min<double>(Sk, over + p.Sq) : Sk;
     }
     // key tiles of a query tile of bm rows on average
     double mean_tiles(const PrefillParams& p, int bm) const {
-        const double kt = std::ceil(keys / kBN);
-        return causal ? std::min(kt, (over + 0.5 * p.Sq + 0.5 * bm) / kBN) : kt;
+        const double kt = std::ceil(keys / kBN), seeing = std::min<double>(p.Sq, Sk);      // (rows in front of the first key: none)
+        return causal ? seeing / p.Sq * std::min(kt, (over + 0.5 * seeing + 0.5 * bm) / kBN) : kt;
     }
 };
-// Microseconds of prefill_fwd_kernel with four wavefronts: the chain of the dearest tile and what a compute unit has to do, of which the longer one counts,
-// and more where they are alike; D 128, two workgroups per compute unit, loses to the L2 what the launch is longer than one round (150 calls of 1 to
-// 1024 heads of 64 to 3000 tokens at 32 and 64: 4 % off; 170 of 8 to 1024 heads of 64 to 5000 tokens at 128: 7 %).
-static double four_us(const PrefillParams& p, int D, int n_cu) {
+// Microseconds of prefill_fwd_kernel with four or eight wavefronts and single tiles: the chain of the dearest tile and what a compute unit has to do (so much per query tile
+// and so much per key tile of it), of which the longer one counts, and more where they are alike (1500 calls of 1 to 4096 heads of 32 and 64, 16 to 8000 queries and 16 to
+// 12000 keys, with and without a mask: rms 6 and 8 %).  D 128, two workgroups per compute unit, loses to the L2 what the launch is longer than one round (170 calls of 8 to
+// 1024 heads of 64 to 5000 tokens: 7 %); with eight wavefronts it has keys split or far from the 64-query kernel's strides.
+static double tiles_us(const PrefillParams& p, int D, int waves, int n_cu) {
     const CallSize c(p);
-    const double tiles = std::ceil(p.Sq / 128.0) * c.heads, mean = c.mean_tiles(p, 128);
-    const double chain = (D == 128 ? 1.27 : D == 64 ? 0.79 : 0.53) * std::ceil(c.keys / kBN);
-    const double each = D == 128 ? 0.906 * mean + 2.98 : D == 64 ? 0.57 * mean + 2.33 : 0.354 * mean + 1.08;
-    const double all = tiles / n_cu * each * (D == 128 ? 1.0 + 0.077 * std::max(0.0, std::log2(tiles / (2.0 * n_cu))) : 1.0);
-    return (D == 128 ? 6.5 : D == 64 ? 6.5 : 4.9) + std::cbrt(chain * chain * chain + all * all * all);
+    const int bm = 32 * waves;
+    const double tiles = std::ceil(p.Sq / (double)bm) * c.heads, mean = c.mean_tiles(p, bm), kt = std::ceil(c.keys / kBN);
+    if (D == 128) {
+        if (waves == 8) return 0.92 * (5.3 + std::max(1.45 * kt, tiles / n_cu * (1.74 * mean + 2.0)));
+        const double all = tiles / n_cu * (0.906 * mean + 2.98) * (1.0 + 0.077 * std::max(0.0, std::log2(tiles / (2.0 * n_cu))));
+        return 6.5 + together(1.27 * kt, all, 3.0);
+    }
+    if (waves == 4) return D == 64 ? 6.742 + together(0.7534 * kt, tiles / n_cu * (0.5079 * mean + 1.926), 2.353) : 5.228 + together(0.5332 * kt, tiles / n_cu * (0.3352 * mean + 0.9081), 2.317);
+    return D == 64 ? 6.603 + together(0.9768 * kt, tiles / n_cu * (1.012 * mean + 2.973), 2.832) : 5.564 + together(0.7229 * kt, tiles / n_cu * (0.6442 * mean + 1.962), 2.574);
 }
 // ... of the 64-query kernel
 static double wide_us(const PrefillParams& p, int n_cu) {
@@ -843,37 +847,48 @@ static double wide_us(const PrefillParams& p, int n_cu) {
     const double tail = (p.block_table ? 16 * p.max_blocks : p.Sk) % kBN ? 12.0 : 0.0;
     return 9.0 + std::max(1.3 * kt + tail, std::ceil(jobs / n_cu) * (1.3 * c.mean_tiles(p, bm) + 4.0 + tail / (c.causal ? qt : 1.0)));
 }
-// Whether prefill_fwd_kernel runs p with four wavefronts.  Eight: split keys and long paged contexts (see the kernel); and long sequences of one length that go over the
-// chip more than four times, where the ends weigh little and half as many loads of keys count.  us with four / eight, causal: heads of 64, 192 of 8132 tokens 1761 / 1709,
-// 256 of 4096 620 / 603, 400 of 3000 563 / 570, 800 of 2000 535 / 550; of 32, 192 of 8132 1142 / 1098, 256 of 4096 397 / 391, 400 of 3000 358 / 370.
+// Whether prefill_fwd_kernel runs p with four wavefronts.  Eight: split keys and long paged contexts (see the kernel); long sequences of one length that go over the
+// chip more than four times, where the ends weigh little and half as many loads of keys count (us with four / eight, causal: heads of 64, 192 of 8132 tokens 1761 / 1709,
+// 256 of 4096 620 / 603, 400 of 3000 563 / 570, 800 of 2000 535 / 550; of 32, 192 of 8132 1142 / 1098, 256 of 4096 397 / 391, 400 of 3000 358 / 370);
+// and dense calls without a mask, whose tiles are all alike, so that what counts is the compute unit with the most workgroups.  us per key tile with 1, 2, 3, 4, 5, 6 of
+// them, heads of 64: four wavefronts 0.76, 1.11, 1.65, 2.26, 2.82, 3.28, eight 1.03, 1.96, 3.09; of 32: 0.56, 0.92, 1.23, 1.53, 1.87, 2.20 and 0.75, 1.41, 2.07.
+// So eight where twice their number is no more than that of four: 16 heads of 32, 7093 tokens (4 workgroups, 2) 164 / 151 us, 48 of 64, 933 tokens (2, 1)
+// 25.9 / 24.1; 128 of 64, 970 (4, 2) 46.4 / 43.8.
 constexpr int kSmallPaged = 128;                  // blocks: paged contexts that four wavefronts take
 static bool four_takes(const PrefillParams& p, int D, int n_cu) {
     if (p.n_split > 1) return false;
     if (p.block_table) return p.max_blocks <= kSmallPaged;
-    return D == 128 || p.window > 0 || !equal_pairs(p) || p.Sq < 4000 || (int64_t)((p.Sq + 127) / 128) * p.Hq * p.B <= 16 * (int64_t)n_cu;
+    if (D == 128) return true;
+    const int64_t heads = (int64_t)p.Hq * p.B, n4 = (p.Sq + 127) / 128 * heads, n8 = (p.Sq + 255) / 256 * heads;
+    if (p.mask_mode == MI355_MASK_NONE && !p.cu_q && p.Sk >= 256) return 2 * ((n8 + n_cu - 1) / n_cu) > (n4 + n_cu - 1) / n_cu;
+    return p.window > 0 || !equal_pairs(p) || p.Sq < 4000 || n4 <= 16 * (int64_t)n_cu;
 }
 // Whether the 64-query kernel is left to prefill_fwd_kernel: short and ragged lengths, whose last tiles it computes in ordinary code and whose rounds it does not
 // fill.  Heads of 128, causal, us 64-query kernel / this: 64 heads of 700 tokens 38 / 25, 136 of 300 30 / 17, 1024 of 300 161 / 103, 14 packed of 111 to 1172, 32
 // heads, 133 / 96, 60 of 20 to 300, 16 heads, 97 / 44; but 136 of 1024 57 / 74, 256 of 1024 91 / 106, 136 of 2000 166 / 204, 14 x 16 heads of 644 65 / 69.  Twelve per
 // cent are left to the wide model, with which none of 170 calls got slower.  (Its persistent launch takes any number of tiles, the other a grid's worth.)
 static bool four_beats_wide(const PrefillParams& p, int n_cu) {
-    return n_cu > 0 && four_takes(p, 128, n_cu) && grid_fits((int64_t)((p.Sq + 255) / 256) * p.Hq * p.B, 256) && four_us(p, 128, n_cu) < 0.88 * wide_us(p, n_cu);
+    return n_cu > 0 && four_takes(p, 128, n_cu) && grid_fits((int64_t)((p.Sq + 255) / 256) * p.Hq * p.B, 256) && tiles_us(p, 128, 4, n_cu) < 0.88 * wide_us(p, n_cu);
 }
 static bool wide_takes(const PrefillParams& p, int n_cu) {
     return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p) && !four_beats_wide(p, n_cu);
 }
 
-// Microseconds of the kernel that takes p where prefill_keys.hip's does not (fitted like prefill_keys_plan; of the rougher fits eight per cent are taken off).
-static double other_us(const PrefillParams& p, int D, int n_cu) {
+// Microseconds of prefill_short.hip's kernel: the chain of the most halves of a key tile, and what a compute unit has to do -- workgroups, pieces of 32 rows and 32 keys, rows
+// (650 calls: rms 8 %).  By key tiles and query tiles of 256 rows alone the model was 1.6 times too high for 68 to 74 tokens.
+static double short_us(const PrefillParams& p, int D, int n_cu) {
     const CallSize c(p);
-    const double kt = std::ceil(c.keys / kBN);
-    // four tiles of a head behind one wait, a chain per tile, all heads of a compute unit side by side
-    if (prefill_short_takes(p, D))
-        return 0.92 * ((D == 32 ? 4.5 : 4.0) + (D == 32 ? 0.55 : 1.1) * kt + c.heads * ((p.Sq + kBM - 1) / kBM) * kt * (D == 32 ? 0.69 : 1.48) / n_cu);
+    const double h = std::ceil(c.keys / 32), nb = std::ceil(p.Sq / 32.0), m = std::min(nb, h), pieces = c.causal ? m * h - 0.5 * m * (m - 1) : nb * h;
+    const double wgs = c.heads * ((p.Sq + 255) / 256), deep = nb > 4 ? (D == 32 ? 1.472 : 1.515) : 1.0;
+    if (D == 32) return 3.658 + together(0.3307 * h * deep, (0.3204 * wgs + 0.04208 * c.heads * pieces) / n_cu + 2.148e-5 * c.heads * p.Sq, 1.751);
+    return 4.019 + together(0.44 * h * deep, (0.5476 * wgs + 0.06277 * c.heads * pieces) / n_cu + 4.941e-5 * c.heads * p.Sq, 2.632);
+}
+
+// Microseconds of the kernel that takes p where prefill_keys.hip's does not (of the rougher fits at D 128 eight per cent are taken off).
+static double other_us(const PrefillParams& p, int D, int n_cu) {
+    if (prefill_short_takes(p, D)) return short_us(p, D, n_cu);
     if (D == 128 && wide_takes(p, n_cu)) return 0.92 * wide_us(p, n_cu);
-    if (four_takes(p, D, n_cu)) return four_us(p, D, n_cu);
-    const double tile = D == 128 ? 1.45 : D == 64 ? 1.0 : 0.75, jobs = (p.Sq + kBM - 1) / kBM * c.heads;
-    return 0.92 * (5.3 + std::max(tile * kt, jobs / n_cu * (1.2 * tile * c.mean_tiles(p, kBM) + 2.0)));
+    return tiles_us(p, D, four_takes(p, D, n_cu) ? 4 : 8, n_cu);
 }
 
 // Wavefronts of prefill_keys.hip's kernel for p, 0: another kernel is the faster one.  One 183-token prompt, 16 heads, D 128: 64-query kernel 26.4 us, keys dealt to
@@ -1308,7 +1323,7 @@ extern "C" int mi355_prefill_suggest_prompt_kv_splits(int B, int Hq, int D, int 
     // Two shares at head sizes 32 and 64: four wavefronts and single tiles are faster by themselves.  Causal, one sequence, us with / without: heads of 64, 8 of 6000 tokens
     // 89 / 66, 8 of 8192 139 / 109, 4 of 12000 153 / 140; of 32, 67 / 44, 100 / 74, 110 / 100.  (Four shares: 4 heads of 32, 8192 tokens 59 / 69; 2 of 64, 12000 89 / 80.)
     if (n == 2 && D < 128 && causal && Sq_max == Sk_max) return 1;
-    return n > 1 && Sq_max == Sk_max && prefill_keys_plan(B, Hq, D, Sq_max, Sk_max, causal != 0, n_cu).us < 0.92 * us ? 1 : n;
+    return n > 1 && Sq_max == Sk_max && prefill_keys_plan(B, Hq, D, Sq_max, Sk_max, causal != 0, n_cu).us < (D == 128 ? 0.92 : 0.95) * us ? 1 : n;
 }
 
 extern "C" int mi355_prefill_fwd_splitkv(const void* q, const void* k, const void* v, void* out,

@@ -258,20 +258,28 @@ bool prefill_keys_takes(const PrefillParams& p, int D) {
            p.scale_log2 > 0.f;
 }
 
-// Microseconds of this kernel, from timings on an MI355X (256 compute units; 1 to 32 heads, 1 to 64 sequences of 16 to 4096 tokens, each head size): a
-// launch and the ends of a workgroup, then the longer of a chain -- of the query tile with the most key tiles, an NW-th of them one behind the other --
-// and of what all workgroups need when they share the compute units: so much each, and so much per tile of 32 keys.
+// Microseconds of this kernel, from timings on an MI355X (256 compute units): a launch and the ends of a workgroup, then a chain -- of the query tile with the most
+// key tiles, an NW-th of them one behind the other -- and what all workgroups need when they share the compute units: so much each, and so much per tile of
+// 32 keys.  D 128: the longer of the two (1 to 32 heads, 1 to 64 sequences of 16 to 4096 tokens); D 32 and 64: of which the longer one counts, and more where they are alike
+// (1500 calls of 1 to 4096 heads, 16 to 8000 queries and 16 to 12000 keys: rms 6 to 8 % with four wavefronts, 9 to 12 with eight.  By the longer alone 512 heads of 73 tokens
+// at D 64 were 7.4 us, 9.8 as measured, and 256 of 312 17.0, 22.4).
 // With eight wavefronts instead of four a compute unit holds half as many workgroups (D 128) and each costs more to end, but the chain is half
 // as long: for launches that give no compute unit a second workgroup, from 16 tiles on (one head, 512 / 2000 / 4000 tokens, D 128: 9.2 / 20.1 / 33.8 us
 // with four, 9.4 / 16.9 / 26.0 with eight; D 64: 6.5 / 14.0 / 23.5, 6.8 / 11.4 / 17.7).
 PrefillKeysPlan prefill_keys_plan(int B, int Hq, int D, int Sq, int Sk, bool causal, int n_cu) {
-    const double base = D == 128 ? 5.0 : 4.3, chain4 = D == 128 ? 1.0 : D == 64 ? 0.61 : 0.45, chain8 = D == 128 ? 1.45 : D == 64 ? 0.86 : 0.61;
-    const double each = D == 128 ? 2.0 : D == 64 ? 0.82 : 0.55, per_tile = D == 128 ? 0.24 : D == 64 ? 0.13 : 0.085;      // per compute unit
-    const double over = causal && Sk > Sq ? Sk - Sq : 0, most = causal ? std::min<double>(Sk, over + Sq) : Sk;
-    const double tiles = std::ceil(most / kKyKeys), mean = causal ? std::min(tiles, (over + 0.5 * Sq) / kKyKeys + 0.5) : tiles;
+    const double over = causal && Sk > Sq ? Sk - Sq : 0, most = causal ? std::min<double>(Sk, over + Sq) : Sk, seeing = std::min(Sq, Sk);
+    const double tiles = std::ceil(most / kKyKeys), mean = causal ? seeing / Sq * std::min(tiles, (over + 0.5 * seeing) / kKyKeys + 0.5) : tiles;
     const double n = (double)((Sq + kKyRows - 1) / kKyRows) * Hq * B;
-    PrefillKeysPlan r{4, base + std::max(chain4 * tiles / 4, n / n_cu * (each + per_tile * mean))};
-    if (n <= n_cu && tiles >= 16) r = {8, base + chain8 * tiles / 8};
+    PrefillKeysPlan r{4, 0.0};
+    if (D == 128) r.us = 5.0 + std::max(tiles / 4, n / n_cu * (2.0 + 0.24 * mean));
+    else if (D == 64) r.us = 4.197 + together(0.6195 * tiles / 4, n / n_cu * (0.9588 + 0.09975 * mean), 1.504);
+    else r.us = 3.738 + together(0.4722 * tiles / 4, n / n_cu * (0.5321 + 0.05937 * mean), 1.223);
+    if (n <= n_cu && tiles >= 16) {
+        double us = 5.0 + 1.45 * tiles / 8;
+        if (D == 64) us = 4.221 + together(0.8226 * tiles / 8, n / n_cu * (2.805 + 0.1274 * mean), 1.649);
+        else if (D == 32) us = 3.903 + together(0.6298 * tiles / 8, n / n_cu * (1.18 + 0.06362 * mean), 1.254);
+        if (D == 128 || us < r.us) r = {8, us};
+    }
     if (n >= 1LL << 31 || !grid_fits((int64_t)n, r.wavefronts * 64)) r.us = INFINITY;
     return r;
 }

@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 #include "common.hpp"
 
 namespace mi355 {
@@ -69,6 +71,8 @@ struct PrefillKeysPlan {
     int wavefronts;
     double us;
 };
+// Two times of which the longer one counts, and more where they are alike (the larger the power, the less)
+inline double together(double a, double b, double power) { return std::pow(std::pow(a, power) + std::pow(b, power), 1.0 / power); }
 bool prefill_keys_takes(const PrefillParams& p, int D);
 PrefillKeysPlan prefill_keys_plan(int B, int Hq, int D, int Sq, int Sk, bool causal, int n_cu);
 int launch_prefill_keys(const PrefillParams& p, int D, int wavefronts, hipStream_t stream);

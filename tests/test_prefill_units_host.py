@@ -94,3 +94,18 @@ def test_launches_beyond_a_grid_stay_with_the_persistent_kernel():
     assert named(1 << 19, 31, 31, 128, 32, 32) == (KEYS, 4)
     assert named(1 << 19, 32, 32, 128, 32, 32) == named(1 << 20, 16, 16, 128, 32, 32) == named(1 << 19, 64, 32, 128, 20, 20, mask=0) == named(1 << 17, 128, 128, 128, 1, 32, lse=1) == (W64, 4)
     assert named(0, 1, 1, 128, 1, 1)[0] == named(1, 3, 2, 128, 1, 1)[0] == named(1, 1, 1, 96, 1, 1)[0] == 0
+
+
+def test_calls_of_heads_of_32_and_64_go_where_they_are_faster():
+    """Both sides of the lines between the kernels, as measured (us): short heads against keys dealt, keys dealt against query tiles, four wavefronts against eight."""
+    for B, Hq, Hkv, D, S in ((16, 64, 16, 64, 68), (64, 8, 8, 64, 73), (32, 8, 2, 64, 158), (8, 64, 16, 64, 74), (16, 16, 8, 32, 67)):
+        assert named(B, Hq, Hkv, D, S, S)[0] == SHORT          # 11.1 / 17.1, 6.9 / 10.5, 8.0 / 12.1, 6.6 / 10.0, 4.8 / 5.6
+    for B, Hq, Hkv, D, S, mask in ((1, 16, 16, 64, 165, 0), (2, 4, 1, 64, 238, 1), (8, 1, 1, 64, 195, 0), (2, 16, 16, 32, 208, 1), (1, 4, 1, 32, 199, 0)):
+        assert named(B, Hq, Hkv, D, S, S, mask) == (KEYS, 4)  # 6.0 / 9.8, 5.4 / 9.2, 6.0 / 10.4, 5.2 / 7.0, 4.9 / 7.7
+    for B, Hq, Hkv, S, lse in ((32, 8, 4, 312, 1), (64, 4, 2, 303, 1), (16, 16, 16, 305, 1)):
+        assert named(B, Hq, Hkv, 64, S, S, lse=lse) == (TILES, 4)                         # 17.6 / 22.4, 17.4 / 22.6, 18.1 / 22.0
+    assert named(64, 8, 1, 64, 191, 191, packed=1, lse=1) == (TILES, 4)                   # 18.0 / 23.7
+    for B, Hq, Hkv, D, S in ((1, 16, 16, 32, 7093), (3, 16, 4, 64, 933), (4, 32, 4, 64, 970), (8, 8, 4, 32, 2769)):
+        assert named(B, Hq, Hkv, D, S, S, 0, lse=1) == (TILES, 8)                         # 151 / 164, 24 / 26, 44 / 46, 94 / 99
+    for B, Hq, Hkv, D, S in ((24, 4, 4, 32, 1309), (1, 32, 4, 64, 2658), (3, 8, 8, 64, 5902)):
+        assert named(B, Hq, Hkv, D, S, S, 0, lse=1) == (TILES, 4)                         # 45.7 / 50.3, 79 / 89, 256 / 278
