@@ -807,11 +807,11 @@ static int set_split(PrefillParams& p, int D, int n_split, int64_t total_q_rows,
     return 0;
 }
 
-// What the models below need of a call (lengths of a packed batch are judged by the longest)
+// What the models below need of a call (lengths of a packed batch are judged by the longest; others: what each further sequence weighs against it)
 struct CallSize {
     double heads, over, keys, Sk;                     // over: keys that every query sees (causal); keys: of the last query
     bool causal;
-    explicit CallSize(const PrefillParams& p) : heads((double)p.Hq * p.B), Sk(p.block_table ? 16.0 * p.max_blocks : p.Sk), causal(p.mask_mode == MI355_MASK_CAUSAL) {
+    explicit CallSize(const PrefillParams& p, double others = 1.0) : heads(p.Hq * (1.0 + others * (p.B - 1))), Sk(p.block_table ? 16.0 * p.max_blocks : p.Sk), causal(p.mask_mode == MI355_MASK_CAUSAL) {
         over = causal && Sk > p.Sq ? Sk - p.Sq : 0;
         keys = causal ? std::min<double>(Sk, over + p.Sq) : Sk;
     }
@@ -838,8 +838,8 @@ static double tiles_us(const PrefillParams& p, int D, int waves, int n_cu) {
     return D == 64 ? 6.603 + together(0.9768 * kt, tiles / n_cu * (1.012 * mean + 2.973), 2.832) : 5.564 + together(0.7229 * kt, tiles / n_cu * (0.6442 * mean + 1.962), 2.574);
 }
 // ... of the 64-query kernel
-static double wide_us(const PrefillParams& p, int n_cu) {
-    const CallSize c(p);
+static double wide_us(const PrefillParams& p, int n_cu, double others = 1.0) {
+    const CallSize c(p, others);
     const bool by_head = c.causal && p.Hq / p.Hkv % 4 == 0;
     const int bm = by_head ? 64 : kBM;
     const double kt = std::ceil(c.keys / kBN), qt = (p.Sq + bm - 1) / bm, jobs = qt * c.heads / (by_head ? 4 : 1);
@@ -867,11 +867,19 @@ static bool four_takes(const PrefillParams& p, int D, int n_cu) {
 // fill.  Heads of 128, causal, us 64-query kernel / this: 64 heads of 700 tokens 38 / 25, 136 of 300 30 / 17, 1024 of 300 161 / 103, 14 packed of 111 to 1172, 32
 // heads, 133 / 96, 60 of 20 to 300, 16 heads, 97 / 44; but 136 of 1024 57 / 74, 256 of 1024 91 / 106, 136 of 2000 166 / 204, 14 x 16 heads of 644 65 / 69.  Twelve per
 // cent are left to the wide model, with which none of 170 calls got slower.  (Its persistent launch takes any number of tiles, the other a grid's worth.)
+// Where the lengths are the device's, the others may be far shorter than the longest: then the 64-query kernel, whose workgroups take the next tile when one ends, has far
+// less to do, and this one waits for the longest sequence's heads on their dies.  So over more than 768 keys the model has to find it the faster one also with each of the
+// other sequences at two fifths of the longest's work (us 64-query kernel / this: 2 sequences, 8 heads, of 4480 tokens and 576 without a mask 108 / 207, 8 x 4 heads, the
+// longest 2779 of 5958, 75 / 124, 6 x 16 heads of up to 708 rows over 1442 paged keys 63 / 91; of 687 drawn calls, with lengths alike and far apart, 4 of those given to
+// this kernel by the longest alone were up to 1.45 times slower, and now none is by more than 1 %).  Over fewer keys the other one's start and its last key tiles
+// weigh more than that: of 144 such calls none was slower here.
+constexpr double kShorter = 0.4, kFewKeys = 768;
 static bool four_beats_wide(const PrefillParams& p, int n_cu) {
     return n_cu > 0 && four_takes(p, 128, n_cu) && grid_fits((int64_t)((p.Sq + 255) / 256) * p.Hq * p.B, 256) && tiles_us(p, 128, 4, n_cu) < 0.88 * wide_us(p, n_cu);
 }
+static bool wide_could(const PrefillParams& p) { return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p); }
 static bool wide_takes(const PrefillParams& p, int n_cu) {
-    return p.mask_mode != MI355_MASK_BOOL && prefill_w64_takes(p) && !four_beats_wide(p, n_cu);
+    return wide_could(p) && !(four_beats_wide(p, n_cu) && (!p.cu_q || CallSize(p).keys <= kFewKeys || tiles_us(p, 128, 4, n_cu) < wide_us(p, n_cu, kShorter)));
 }
 
 // Microseconds of prefill_short.hip's kernel: the chain of the most halves of a key tile, and what a compute unit has to do -- workgroups, pieces of 32 rows and 32 keys, rows
@@ -884,10 +892,10 @@ static double short_us(const PrefillParams& p, int D, int n_cu) {
     return 4.019 + together(0.44 * h * deep, (0.5476 * wgs + 0.06277 * c.heads * pieces) / n_cu + 4.941e-5 * c.heads * p.Sq, 2.632);
 }
 
-// Microseconds of the kernel that takes p where prefill_keys.hip's does not (of the rougher fits at D 128 eight per cent are taken off).
+// Microseconds of the kernel that takes p where prefill_keys.hip's does not, with lengths alike (of the rougher fits at D 128 eight per cent are taken off).
 static double other_us(const PrefillParams& p, int D, int n_cu) {
     if (prefill_short_takes(p, D)) return short_us(p, D, n_cu);
-    if (D == 128 && wide_takes(p, n_cu)) return 0.92 * wide_us(p, n_cu);
+    if (D == 128 && wide_could(p) && !four_beats_wide(p, n_cu)) return 0.92 * wide_us(p, n_cu);
     return tiles_us(p, D, four_takes(p, D, n_cu) ? 4 : 8, n_cu);
 }
 

@@ -109,3 +109,12 @@ def test_calls_of_heads_of_32_and_64_go_where_they_are_faster():
         assert named(B, Hq, Hkv, D, S, S, 0, lse=1) == (TILES, 8)                         # 151 / 164, 24 / 26, 44 / 46, 94 / 99
     for B, Hq, Hkv, D, S in ((24, 4, 4, 32, 1309), (1, 32, 4, 64, 2658), (3, 8, 8, 64, 5902)):
         assert named(B, Hq, Hkv, D, S, S, 0, lse=1) == (TILES, 4)                         # 45.7 / 50.3, 79 / 89, 256 / 278
+
+
+def test_packed_heads_of_128_with_lengths_far_apart_stay_with_the_wide_kernel():
+    """Lengths on the device may be far shorter than the longest, which then waits for its heads on their dies: four wavefronts only where they win either way (us wide / tiles)."""
+    for B, Hq, Hkv, S, mask in ((2, 8, 4, 4480, 0), (8, 4, 1, 2779, 0), (2, 16, 16, 2448, 0), (12, 8, 2, 1119, 0), (3, 4, 1, 6731, 0)):
+        assert named(B, Hq, Hkv, 128, S, S, mask, packed=1) == (W64, 4)               # 108 / 207, 75 / 124, 75 / 108, 45 / 63, 156 / 172
+    assert named(6, 16, 16, 128, 708, 1442, blocks=91) == named(12, 8, 1, 128, 754, 1556, blocks=98) == (W64, 4)   # 63 / 91, 55 / 71
+    for B, Hq, Hkv, S, mask in ((60, 16, 16, 300, 1), (24, 4, 4, 248, 0), (32, 32, 16, 119, 0), (6, 8, 8, 981, 1), (2, 16, 16, 1286, 1)):
+        assert named(B, Hq, Hkv, 128, S, S, mask, packed=1) == (TILES, 4)             # 97 / 44, 27 / 13, 57 / 20, 41 / 31, 48 / 37
