@@ -148,8 +148,8 @@ def test_backward_packed_sequences_of_very_different_lengths(ops, D, seed):
 
 @pytest.mark.parametrize("D", [64, 128])
 def test_forward_lse_matches_oracle(ops, D):
-    """head_dim 64: the 8-wavefront kernel; 128: the 64-query kernel, whose log-sum-exp comes from its row sums and
-    the exponent reference that went into them -- also after that reference has moved (keys with runaway scores),
+    """The log-sum-exp that comes from row sums and the exponent reference that went into them (as the sizes choose; each
+    kernel by name in test_gpu_prefill_kernels.py) -- also after that reference has moved (keys with runaway scores),
     for ragged packed sequences, and for rows past the end of a partial query tile."""
     print(f"case: forward lse D={D}", flush=True)
     from mi355_attn import ops as raw

@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from oracle import attention_oracle as orc
+from test_gpu_prefill_kernels import TILES, W64, promise
 
 pytestmark = pytest.mark.gpu
 
@@ -312,9 +313,9 @@ def test_prefill_varlen_ragged(ops, lens):
 
 @pytest.mark.parametrize("Sq,Sk", [(256, 4096), (700, 1500), (64, 191), (513, 64), (300, 8192 + 37)])
 def test_prefill_unmasked_head_dim_128_long_and_ragged(ops, Sq, Sk):
-    """head_dim 128 without a mask runs on the kernel with 64 queries per wavefront, whose loop over whole K/V tiles
-    is hand-scheduled assembly: many tiles, ragged query and key ends (the assembly stops three tiles before a
-    partial last tile), GQA, fewer rows than a wavefront owns."""
+    """head_dim 128 without a mask: many tiles, ragged query and key ends, GQA, fewer rows than a wavefront owns; as the sizes
+    choose, and packed under a promise for which the kernel with 64 queries per wavefront takes them, whose loop over whole
+    K/V tiles is hand-scheduled assembly that stops three tiles before a partial last tile."""
     print(f"case: prefill unmasked D128 Sq={Sq} Sk={Sk}", flush=True)
     B, Hq, Hkv, D = 2, 4, 2, 128
     q, k, v = rnd(B, Hq, Sq, D, seed=81, scale=0.5), rnd(B, Hkv, Sk, D, seed=82, scale=0.5), rnd(B, Hkv, Sk, D, seed=83, scale=0.5)
@@ -322,6 +323,10 @@ def test_prefill_unmasked_head_dim_128_long_and_ragged(ops, Sq, Sk):
     got = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=False, kv_splits=1)
     torch.cuda.synchronize()
     check(got, ref, what=f"unmasked D128 {Sq}x{Sk}")
+    most = promise((W64, 4), B, Hq, Hkv, D, Sq, Sk, ops._lib.MASK_NONE)
+    packed = [x.transpose(1, 2).reshape(-1, x.shape[1], D).cuda() for x in (q, k, v)] + [(torch.arange(B + 1) * n).int().cuda() for n in (Sq, Sk)]
+    wide = ops.flash_attn_varlen_prefill(*packed, *most, causal=False, kv_splits=1).view(B, Sq, Hq, D).transpose(1, 2)
+    check(wide, ref, what=f"unmasked D128 {Sq}x{Sk}, 64-query kernel")
     # the default may split the keys of so small a launch over several workgroups (another kernel and a merge)
     check(ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=False), ref, what=f"unmasked D128 {Sq}x{Sk}, default")
     # the reference's own signature (no GQA there: first kv head only)
@@ -346,7 +351,7 @@ def test_prefill_unmasked_scores_that_outgrow_the_reference(ops):
     got = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=False)
     torch.cuda.synchronize()
     check(got, ref, what="reference moves")
-    # the same through the 8-wavefront kernel (an all-true explicit mask takes that path): both must agree with the oracle
+    # the same through the tile kernel (an all-true explicit mask takes that path): both must agree with the oracle
     keep = torch.ones(Sq, Sk, dtype=torch.bool, device="cuda")
     check(ops.scaled_dot_product_attention(q.cuda(), k.cuda(), v.cuda(), keep), ref, what="reference moves, masked path")
 
@@ -354,10 +359,10 @@ def test_prefill_unmasked_scores_that_outgrow_the_reference(ops):
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("seed", [0, 1, 2])
 def test_prefill_head_dim_64_32_preset_reference_against_tracked_maxima(ops, D, seed):
-    """The 8-wavefront kernel first runs a query tile with a preset exponent reference, watching row sums, and runs it
-    again with the reference tracked from the row maxima when a row's sum leaves the safe range.  An explicit
-    all-visible mask takes the tracked path from the start, so the two paths can be compared with each other and with
-    the oracle: drawn shapes (ragged, more keys than queries, GQA, causal or not), keys whose scores run away by
+    """Query tiles run with a preset exponent reference first, watching row sums, and again with the reference tracked
+    from the row maxima when a row's sum leaves the safe range.  An explicit all-visible mask takes the tracked path of
+    the tile kernel from the start, so the paths can be compared with each other and with the oracle (unsplit calls
+    of these sizes run where keys are dealt to wavefronts; test_gpu_prefill_kernels.py names each kernel): drawn shapes (ragged, more keys than queries, GQA, causal or not), keys whose scores run away by
     tens to thousands of binary orders in both directions (rescaling in the loop, second attempts), keys split over
     workgroups, and rows whose scores are all hugely negative."""
     g = torch.Generator().manual_seed(3000 + 10 * D + seed)
@@ -520,8 +525,9 @@ def test_prefill_split_keys_varlen_and_paged(ops, splits):
 
 @pytest.mark.parametrize("seed", [0, 1, 2, 3])
 def test_prefill_head_dim_128_two_kernels_agree_on_random_shapes(ops, seed):
-    """The 64-query kernel (hand-scheduled, pipelined tile loop) against the 8-wavefront kernel (reached through an
-    explicit boolean mask that says the same thing) and the oracle, on drawn shapes: ragged query and key counts,
+    """The kernel that the sizes choose, with keys split the 64-query kernel (hand-scheduled, pipelined tile loop), against the
+    tile kernel (reached through an explicit boolean mask that says the same thing) and the oracle, on drawn shapes
+    (unsplit calls of the 64-query kernel by name: test_gpu_prefill_kernels.py): ragged query and key counts,
     Sk >= Sq (bottom-right diagonal), GQA, several query tiles per workgroup, and keys whose scores run away in
     both directions at drawn places -- in unmasked tiles, on the diagonal, in the last partial tile -- so that the
     loop is left and re-entered at every kind of tile."""
@@ -552,15 +558,16 @@ def test_prefill_head_dim_128_two_kernels_agree_on_random_shapes(ops, seed):
         n_shares = 2 + (seed + case) % 3              # shares that start at odd and even tiles, some of them empty
         shared = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=causal, kv_splits=n_shares)
         torch.cuda.synchronize()
-        check(fast, ref, what=f"64-query kernel seed {seed} #{case}")
-        check(slow, ref, what=f"8-wavefront kernel seed {seed} #{case}")
+        check(fast, ref, what=f"chosen kernel seed {seed} #{case}")
+        check(slow, ref, what=f"tile kernel, boolean mask, seed {seed} #{case}")
         check(shared, ref, what=f"64-query kernel, keys split {n_shares} ways, seed {seed} #{case}")
 
 
 @pytest.mark.parametrize("seed", [0, 1, 2])
 def test_prefill_head_dim_128_four_heads_per_workgroup_on_random_shapes(ops, seed):
     """Causal prefill with a multiple of four query heads per K/V head: the 64-query kernel then gives the four wavefronts
-    of a workgroup the same 64 rows of four heads (one head each) instead of 4 x 64 rows of one head.  Drawn shapes --
+    of a workgroup the same 64 rows of four heads (one head each) instead of 4 x 64 rows of one head (here with the keys
+    split; unsplit by name in test_gpu_prefill_kernels.py, here as the sizes choose).  Drawn shapes --
     4, 8 or 12 query heads per K/V head, ragged query and key counts, more keys than queries, runaway keys -- against
     the oracle and against the other kernel; with the keys split (partial rows per head), with the log-sum-exp output,
     and the gradients that the training forward feeds."""
@@ -588,8 +595,8 @@ def test_prefill_head_dim_128_four_heads_per_workgroup_on_random_shapes(ops, see
         from mi355_attn import ops as raw
         out2, lse = raw._dense(q.cuda(), k.cuda(), v.cuda(), None, 1, None, want_lse=True)
         torch.cuda.synchronize()
-        check(fast, ref, what=f"four heads per workgroup seed {seed} #{case}")
-        check(slow, ref, what=f"8-wavefront kernel seed {seed} #{case}")
+        check(fast, ref, what=f"chosen kernel, four heads per K/V head, seed {seed} #{case}")
+        check(slow, ref, what=f"tile kernel, boolean mask, seed {seed} #{case}")
         check(shared, ref, what=f"four heads per workgroup, keys split, seed {seed} #{case}")
         assert torch.equal(out2, fast)
         s_ = torch.einsum("bhqd,bhkd->bhqk", q.float(), k.float().repeat_interleave(Hq // Hkv, 1)) / math.sqrt(128)
@@ -597,8 +604,8 @@ def test_prefill_head_dim_128_four_heads_per_workgroup_on_random_shapes(ops, see
 
 
 def test_prefill_head_dim_128_four_heads_per_workgroup_packed_and_trained(ops):
-    """The same job layout on a packed batch of drawn lengths (an empty sequence and a one-token one included), and
-    through autograd: the forward with the log-sum-exp runs on this layout, the backward kernels read what it wrote."""
+    """The same job layout (reached by a larger promise) on a packed batch of drawn lengths (an empty sequence and a one-token one
+    included), and through autograd: the forward with the log-sum-exp, the backward kernels read what it wrote."""
     print("case: four heads per workgroup, packed + backward", flush=True)
     Hq, Hkv, D = 8, 2, 128
     lens = [300, 0, 1, 129, 517, 64]
@@ -607,7 +614,8 @@ def test_prefill_head_dim_128_four_heads_per_workgroup_packed_and_trained(ops):
     q, k, v, dout = rnd(T, Hq, D, seed=7100), rnd(T, Hkv, D, seed=7101), rnd(T, Hkv, D, seed=7102), rnd(T, Hq, D, seed=7103)
     ref = orc.varlen_prefill_reference(q, k, v, cu, cu, causal=True)
     qg, kg, vg = (t.cuda().requires_grad_() for t in (q, k, v))
-    out = ops.flash_attn_varlen_prefill(qg, kg, vg, cu.cuda(), cu.cuda(), max(lens), max(lens), causal=True)
+    most = promise((W64, 4), len(lens), Hq, Hkv, D, max(lens), max(lens), ops._lib.MASK_CAUSAL)
+    out = ops.flash_attn_varlen_prefill(qg, kg, vg, cu.cuda(), cu.cuda(), *most, causal=True)
     out.backward(dout.cuda())
     torch.cuda.synchronize()
     check(out.detach(), ref, what="packed, four heads per workgroup")
@@ -624,9 +632,9 @@ def test_prefill_head_dim_128_four_heads_per_workgroup_packed_and_trained(ops):
 
 @pytest.mark.parametrize("seed", [0, 1, 2])
 def test_prefill_head_dim_128_packed_sequences_of_drawn_lengths(ops, seed):
-    """Packed sequences of drawn lengths (empty ones included) through the persistent 64-query kernel: a workgroup
-    walks from job to job across sequences of different lengths, prefetching the next job's rows and tiles; with
-    a promised maximum that is too small for one sequence; forward-only and with the log-sum-exp output."""
+    """Packed sequences of drawn lengths (empty ones included) as the sizes choose, and through the persistent 64-query kernel
+    (by a larger promise), where a workgroup walks from job to job across sequences of different lengths, prefetching the
+    next job's rows and tiles; with a promised maximum that is too small for one sequence; with the log-sum-exp output."""
     g = torch.Generator().manual_seed(2000 + seed)
     Hq, Hkv, D = 4, 2, 128
     n_seq = int(torch.randint(2, 9, (1,), generator=g))
@@ -642,6 +650,9 @@ def test_prefill_head_dim_128_packed_sequences_of_drawn_lengths(ops, seed):
     got = ops.flash_attn_varlen_prefill(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), max(lens), max(lens),
                                         causal=True, kv_splits=1)
     check(got, ref, what="packed drawn lengths")
+    most = promise((W64, 4), n_seq, Hq, Hkv, D, max(lens), max(lens), ops._lib.MASK_CAUSAL)
+    wide = ops.flash_attn_varlen_prefill(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), *most, causal=True, kv_splits=1)
+    check(wide, ref, what="packed drawn lengths, 64-query kernel")
     short = ops.flash_attn_varlen_prefill(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), max(1, max(lens) // 3),
                                           max(1, max(lens) // 3), causal=True, kv_splits=1)
     check(short, ref, what="packed drawn lengths, promised maximum too small")
@@ -680,9 +691,15 @@ def test_prefill_head_dim_128_rounds_no_weight_that_is_a_rows_largest(ops, S, Hq
     tops[..., :preset] = 0.0
     weights = (torch.exp2(halves - tops[..., None]).to(torch.bfloat16).double() * torch.exp2(tops)[..., None]).flatten(-2)[..., :S]
     same = ((weights @ vv) / weights.sum(-1, keepdim=True)).to(torch.bfloat16).double()
-    got = ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=False, kv_splits=1).double().cpu()
-    off, off_same = ((x - ref).norm() / ref.norm() for x in (got, same))
-    assert off <= 1.03 * off_same, (float(off), float(off_same))
+    off_same = (same - ref).norm() / ref.norm()
+    outs = {"as the sizes choose": ops.flash_attn_prefill(q.cuda(), k.cuda(), v.cuda(), causal=False, kv_splits=1)}
+    rows, cu = [x.transpose(1, 2).reshape(B * S, -1, D).cuda() for x in (q, k, v)], (torch.arange(B + 1) * S).int().cuda()
+    for kernel in (W64, TILES):                                                   # (the two whose references these are, by what they are promised)
+        most = promise((kernel, 4), B, Hq, Hkv, D, S, S, ops._lib.MASK_NONE)
+        outs[kernel] = ops.flash_attn_varlen_prefill(*rows, cu, cu, *most, causal=False, kv_splits=1).view(B, S, Hq, D).transpose(1, 2)
+    for what, got in outs.items():
+        off = (got.double().cpu() - ref).norm() / ref.norm()
+        assert off <= 1.03 * off_same, (what, float(off), float(off_same))
 
 
 @pytest.mark.parametrize("seed", [0, 1])
@@ -750,7 +767,7 @@ def test_prefill_head_dim_128_more_packed_sequences_than_the_64_query_kernel_kee
     ref = orc.varlen_prefill_reference(q, k, v, cu, cu, causal=True)
     got = ops.flash_attn_varlen_prefill(q.cuda(), k.cuda(), v.cuda(), cu.cuda(), cu.cuda(), 3, 3, causal=True, kv_splits=1)
     check(got, ref, what="4100 packed sequences")
-    # the same tokens as 4096 sequences (the last one takes what is left): the 64-query kernel at its limit
+    # the same tokens as 4096 sequences, the last one takes what is left (both kernels by name: test_gpu_prefill_kernels.py)
     cu2 = torch.cat([cu[:4096], cu[-1:]])
     ref2 = orc.varlen_prefill_reference(q, k, v, cu2, cu2, causal=True)
     longest = int((cu2[1:] - cu2[:-1]).max())
@@ -929,8 +946,8 @@ def test_paged_prefill_head_dim_128_random_shapes_with_runaway_keys(ops, seed):
 
 @pytest.mark.parametrize("B", [4096, 4097])
 def test_paged_prefill_head_dim_128_thousands_of_short_sequences(ops, B):
-    """As many sequences as the 64-query kernel keeps counts for in LDS (4096: 64 groups of 64), and one more (the
-    8-wavefront kernel then serves the launch): chunks of one to three tokens over contexts of a few blocks."""
+    """As many sequences as the 64-query kernel keeps counts for in LDS (4096: 64 groups of 64), and one more (which it
+    does not take): chunks of one to three tokens over contexts of a few blocks."""
     print(f"case: paged prefill D=128, {B} sequences", flush=True)
     g = torch.Generator().manual_seed(40)
     ctx = [int(x) for x in torch.randint(1, 40, (B,), generator=g)]

@@ -32,8 +32,8 @@ def reference(q, k, v, window, keep):
     (2, 2, [96] * 40 + [1030], 1030)])
 @pytest.mark.parametrize("window,keep", [(0, 0), (100, 3), (5000, 0)])
 def test_tiles_and_orders(ma, D, H, Hkv, lens, promised, window, keep):
-    """Each output is a convex mean of bf16 values: rounding of the weights (2^-9 each, both in the products and in their sum) and of the result 2^-9 of the largest value, so
-    3 * 2^-9 of it together, and a little for fp32 sums."""
+    """Each output is a convex mean of bf16 values: rounding of the weights, in the products and in their sum, and of the result, up to 2^-8 of themselves and half of it on
+    average.  As outputs are well below the largest value, 3 * 2^-9 of that holds, with a little for fp32 sums."""
     print(f"case: units {D} {H} {Hkv} {lens} {window}", flush=True)
     g = torch.Generator().manual_seed(D + H)
     T = sum(lens)
@@ -49,7 +49,8 @@ def test_tiles_and_orders(ma, D, H, Hkv, lens, promised, window, keep):
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("B,H,S,causal", [(1, 3, 700, False), (2, 9, 130, False), (1, 17, 1025, True), (260, 16, 384, True), (1, 1100, 640, True)])
 def test_dense_launches_of_every_size(ma, D, B, H, S, causal):
-    """All workgroups resident at once, more of them, and the pairs of launches beyond four rounds of the chip; a few heads are looked at."""
+    """All workgroups resident at once, more of them, and the pairs of launches beyond four rounds of the chip; a few heads are looked at (eight wavefronts and each kernel by
+    name: test_gpu_prefill_kernels.py)."""
     print(f"case: dense units {D} {B} {H} {S}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(S)
     q, k, v = (torch.randn(B, H, S, D, generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(3))

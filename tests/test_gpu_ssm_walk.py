@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from test_gpu_zomipel import ops, rnd, rows_close, ssm_case, ssm_oracle, ssm_pools  # noqa: F401
+from test_zomipel_host import conv_tile
 
 pytestmark = pytest.mark.gpu
 FORMS = [dict(heads=4, vdim=64, state=64, groups=2, taps=4), dict(heads=2, vdim=128, state=128, groups=1, taps=4), dict(heads=2, vdim=128, state=64, groups=2, taps=2)]
@@ -58,13 +59,15 @@ def test_walk_of_whole_and_cut_sequences(ops):  # noqa: F811
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_convolution_tiles(ops, dtype):  # noqa: F811
-    """4, 8 and 16 tokens per thread, by the size of a call: 4203 tokens of two sequences at once, in halves and in quarters with tokens left over; what is
-    left in the ring is the same, the outputs but for the order of the scan's fp32 sums."""
+def test_convolution_tiles(ops, tmp_path, dtype):  # noqa: F811
+    """4, 8 and 16 tokens per thread, by the size of a call: two sequences of 2101 (fp32: 1501) tokens at once, in halves and in quarters with tokens left over; what
+    is left in the ring is the same, the outputs but for the order of the scan's fp32 sums."""
     m = dict(heads=64, vdim=64, state=128, groups=1, taps=4)
     kw = {k: m[k] for k in ("heads", "vdim", "state", "groups")}
     print(f"case: convolution tiles {dtype}", flush=True)
-    n = 2101 if dtype == torch.bfloat16 else 701                          # (fp32 goes token by token behind the convolution)
+    n = 2101 if dtype == torch.bfloat16 else 1501                         # (fp32 goes token by token behind the convolution)
+    tile = conv_tile(tmp_path)
+    assert [tile(2 * (n // parts), 64 * 64 + 2 * 128, 4) for parts in (1, 2, 4)] == [16, 8, 4]
     proj, params, xbc_at, dt_at = ssm_case(m, 2 * n, 32, dtype)
     proj, pc = proj.view(2, n, -1).cuda(), {k: v.cuda() for k, v in params.items()}
     outs = []

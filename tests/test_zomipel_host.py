@@ -346,9 +346,7 @@ def test_little_work_takes_short_segments(heads, n, lens, seg):
 
 
 # ---- tiles of the causal convolution ------------------------------------------------------------------------------------
-def test_only_a_portions_first_tile_reads_the_ring(tmp_path):
-    """What the tiles of a resumed portion read of the ring of inputs against what the first of them writes there, for every number of taps and size
-    class: tiles run in any order, so no other tile may read a row of the ring at all."""
+def conv_tile(tmp_path):
     src, lib = tmp_path / "conv.cpp", tmp_path / "conv.so"
     src.write_text('#include "ssm_conv.hpp"\n'
                    'extern "C" int tile(long long rows, int channels, int taps) { return mi355::conv_tile(rows, channels, taps); }\n')
@@ -356,6 +354,13 @@ def test_only_a_portions_first_tile_reads_the_ring(tmp_path):
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
     tile = ctypes.CDLL(str(lib)).tile
     tile.argtypes = [ctypes.c_longlong, ctypes.c_int, ctypes.c_int]
+    return tile
+
+
+def test_only_a_portions_first_tile_reads_the_ring(tmp_path):
+    """What the tiles of a resumed portion read of the ring of inputs against what the first of them writes there, for every number of taps and size
+    class: tiles run in any order, so no other tile may read a row of the ring at all."""
+    tile = conv_tile(tmp_path)
     seen = set()
     for taps in range(1, 17):
         for rows, channels in ((64, 64), (1024, 4352), (2048, 4352), (8192, 4352)):
