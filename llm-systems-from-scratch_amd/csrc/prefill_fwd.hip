@@ -88,12 +88,12 @@ __global__ __launch_bounds__(NW * 64, D == 128 ? 2 : (D == 64 || NW == 4 ? 4 : 1
     unsigned char* const o_lds = kOwnSlab ? o_own : kv_lds;
 
     // The workgroups that stream the same K/V -- the units and query heads of one kv head -- run on one XCD.
-    // Pairs: pair fastest, then the query heads of one kv head, then kv head, then batch.
-    // Single tiles: by falling number, so that the dearest begin first and what is left for the end is small (xcd_unit).
+    // Pairs, and the single tiles of some launches with keys split: fastest, then the query heads of one kv head, then kv head, then batch.
+    // Other single tiles: by falling number, so that the dearest begin first and what is left for the end is small (xcd_unit).
     const int split = blockIdx.y;                    // share of the keys this workgroup serves (gridDim.y = n_split)
     const bool singles = p.single_tiles != 0;
     int pair0, head;
-    if (singles) {
+    if (p.single_tiles == 1) {
         const HeadUnit at = xcd_unit(blockIdx.x, p.n_pairs, p.Hq / p.Hkv, p.Hkv * p.B, p.chunk_heads, p.round);
         if (at.unit < 0) return;
         pair0 = p.n_pairs - 1 - at.unit;
@@ -645,6 +645,9 @@ static bool equal_pairs(const PrefillParams& p) {
 // times: NW 4, causal, heads of 64, singles / pairs: 136 heads of 1456 tokens 60 / 68 us, 64 of 8192 (four rounds) 568 / 581, 1024 of 700 (six) 150 /
 // 140, 256 of 3000 (six) 370 / 354.  So pairs from more than four rounds on, and with eight wavefronts from two workgroups per compute unit on.
 // (Packed: 35 sequences of 386 to 2835 tokens, 32 heads of 32, 434 / 480; 18 of 319 to 2850, 32 heads of 128, window of 512, NW 8, 471 / 517.)
+// With keys split, by falling number only where a share's workgroups all have work: in order of heads otherwise (us, by number / in order: 6 packed chunks of up to 1349
+// rows over 10854 tokens, 4 / 2 heads of 64, 115 / 83; one of 135 rows over 15239, 4 / 2 heads of 32, 54 / 50; 223 drawn calls of heads of 32 and 64, where all have work
+// 0.993, otherwise 1.012).
 // An XCD takes as many kv heads at a time as have 8 MB of keys and values, twice its L2: with more, 512 heads of 1024 tokens take 126 us instead of 120.
 static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
     PrefillParams p = p0;
@@ -655,13 +658,14 @@ static PrefillParams with_units(const PrefillParams& p0, int waves, int D) {
     const bool pairs = equal_pairs(p) && (waves == 4 ? tiles > 4 * resident : p.n_pairs * heads >= 2 * n_cu);
     p.single_tiles = !pairs && xcd_units_fit(p.n_qtiles, p.Hq / p.Hkv, (int64_t)p.Hkv * p.B, 64 * waves);
     if (p.single_tiles) p.n_pairs = p.n_qtiles;
+    if (p.single_tiles && !xcd_units_spread(p.Hkv * p.B, p.n_split)) p.single_tiles = 2;
     const int64_t keys = p.block_table ? 16 * (int64_t)p.max_blocks : p.Sk, kv_heads = (8 << 20) / (std::max<int64_t>(1, keys) * D * 4);
     p.chunk_heads = p.Hq / p.Hkv * (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)p.Hkv * p.B / 8, kv_heads));
     p.round = p.n_split <= 1 && tiles <= resident ? (int)(n_cu / 8) : 0;
     return p;
 }
 static unsigned units_grid(const PrefillParams& p) {
-    return p.single_tiles ? (unsigned)xcd_units_grid(p.n_pairs, p.Hq / p.Hkv, p.Hkv * p.B) : (unsigned)(p.n_pairs * p.Hq * p.B);
+    return p.single_tiles == 1 ? (unsigned)xcd_units_grid(p.n_pairs, p.Hq / p.Hkv, p.Hkv * p.B) : (unsigned)(p.n_pairs * p.Hq * p.B);
 }
 template <int D, int NW>
 static int launch_prefill_of(const PrefillParams& p0, hipStream_t stream) {

@@ -31,7 +31,7 @@ struct PrefillParams {
     int window, keep_first;               // causal only: query i sees key j when i - j < window or j < keep_first (window 0: every key j <= i)
     int n_qtiles;
     int n_pairs;                          // units per (batch, head) of prefill_fwd_kernel's grid: pairs of query tiles, or ...
-    int single_tiles;                     // ... single query tiles when this is set; then also ...
+    int single_tiles;                     // ... single query tiles when this is not 0; 1: by their number, and then also ...
     int chunk_heads, round;               // ... query heads that an XCD takes at a time, and its compute units if all workgroups are resident at once (else 0)
     // paged keys and values (prefill of a chunk on top of cached context): k, v are cache pools
     // (num_blocks, Hkv, 16, D); sequence b owns blocks block_table[b * table_stride + j] and ctx_lens[b] keys

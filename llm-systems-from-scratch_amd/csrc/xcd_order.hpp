@@ -36,6 +36,9 @@ MI355_ORDER int xcd_units_grid(int n_units, int group, int n_groups) {
 }
 // Whether that grid can be launched: its threads are counted in 32 bits.
 MI355_ORDER bool xcd_units_fit(long long n_units, long long group, long long n_groups, int threads) { return (n_units * group * n_groups + 7) * threads < 1LL << 32; }
+// Whether shares of split keys, each a whole grid of them, the ids running on from one to the next, are spread evenly over the XCDs: not where workgroups without
+// work fill up a share's grid, as then the few with work begin on the same XCDs in every share.
+MI355_ORDER bool xcd_units_spread(int n_groups, int n_split) { return n_split <= 1 || n_groups % 8 == 0; }
 MI355_ORDER int turned(int i, int n, int width) {
     const int start = width > 0 ? i / width * width : 0;
     return width > 0 && (i / width & 1) && start + width <= n ? 2 * start + width - 1 - i : i;

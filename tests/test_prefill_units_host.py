@@ -17,7 +17,8 @@ def order(tmp_path_factory):
                    '  const int n = mi355::xcd_units_grid(u, group, groups);\n'
                    '  for (int i = 0; out && i < n; ++i) { const auto x = mi355::xcd_unit(i, u, group, groups, chunk, round); out[2 * i] = x.unit; out[2 * i + 1] = x.head; }\n'
                    '  return n; }\n'
-                   'extern "C" int fits(long long u, long long group, long long groups, int threads) { return mi355::xcd_units_fit(u, group, groups, threads); }\n')
+                   'extern "C" int fits(long long u, long long group, long long groups, int threads) { return mi355::xcd_units_fit(u, group, groups, threads); }\n'
+                   'extern "C" int spread(int groups, int n_split) { return mi355::xcd_units_spread(groups, n_split); }\n')
     csrc = os.path.join(os.path.dirname(os.path.dirname(mi355_attn.__file__)), "csrc")
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", csrc, str(src), "-o", str(lib)], check=True)
     fn = ctypes.CDLL(str(lib)).units
@@ -30,7 +31,7 @@ def order(tmp_path_factory):
         fn(u, group, groups, chunk, rnd, out)
         return [(out[2 * i], out[2 * i + 1]) for i in range(n)]
     units.grid = lambda u, group, groups: fn(u, group, groups, 1, 0, None)
-    units.fits = fits
+    units.fits, units.spread = fits, ctypes.CDLL(str(lib)).spread
     return units
 
 
@@ -54,6 +55,16 @@ def test_every_unit_once(order, u, groups, group, rnd):
                 for c in range(0, len(mine), chunk * u):
                     units = [i for i, _ in mine[c:c + chunk * u]]
                     assert units == sorted(units) and len({h for _, h in mine[c:c + chunk * u]}) <= chunk
+
+
+@pytest.mark.parametrize("group", [1, 4, 5])
+@pytest.mark.parametrize("u,groups,n_split", [(1, 1, 30), (1, 2, 16), (6, 12, 5), (2, 3, 64), (3, 16, 4), (1, 8, 20), (5, 9, 1), (4, 37, 3)])
+def test_shares_of_split_keys_reach_every_xcd(order, u, groups, group, n_split):
+    """Workgroups of a launch whose shares follow each other, single tiles by number where the rule says so, else in order without a gap: no XCD (id modulo 8) gets
+    more than one of those with work more than another."""
+    ids = [i >= 0 for i, _ in order(u, group, groups, group, 0)] if order.spread(groups, n_split) else [True] * (u * group * groups)
+    with_work = [sum((ids * n_split)[xcd::8]) for xcd in range(8)]
+    assert sum(with_work) == u * group * groups * n_split and max(with_work) - min(with_work) <= 1
 
 
 @pytest.mark.parametrize("D,prompt,chunk", [(32, 1, 2), (64, 1, 2), (128, 2, 2)])
