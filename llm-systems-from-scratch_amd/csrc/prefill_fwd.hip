@@ -35,7 +35,6 @@ namespace mi355 {
 constexpr int kBM = 256;   // queries per workgroup
 constexpr int kBN = 64;    // keys per LDS tile
 
-
 // PAGED: keys and values are read from a paged cache through a block table (16 rows per block, so
 // every direct-to-LDS instruction -- 4, 8 or 16 whole rows -- stays inside one block and needs one
 // table entry, a scalar load); queries and outputs are packed.
@@ -49,7 +48,7 @@ constexpr int kBN = 64;    // keys per LDS tile
 // 65 / 60 and 40 / 30, 1024 of 700 152 / 140 and 102 / 79, 8 of 8192 138 / 105 and 99 / 68, 22 packed sequences
 // of 1334, 8 heads of 64, 92 / 65; 14 of 111 to 1172, 32 heads, 80 / 60; head_dim 128, window of 512, 14 of 111 to 1172, 32 heads, 127 / 99, one of 2000,
 // 16 heads, 32 / 24; boolean mask, 4 x 16 heads of 512 75 / 49.
-// With keys split, in launches of many long sequences (launch_prefill) and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
+// With keys split, in launches of many long sequences (four_takes) and on long paged contexts (a look-up in the block table in front of every request) eight remain: 8 chunks of 400 rows over
 // 9000 tokens, 32 heads of 64, 290 us, with four 325; 16 of 333 over 1500, heads of 32, 40 and 34.
 // WINDOW (causal): a query tile walks the K/V tiles that hold the kept first tokens, then those from its window's first
 // key on, as one sequence of tiles (tile_of); keys outside are masked in the tiles at the window's lower edge.
@@ -1278,7 +1277,7 @@ static int best_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t 
             return rounds(wgs) * (keys_pair / n / kBN * (wgs >= 0.75 * n_cu ? 1.45 : 1.25) + 5.0 * halves);
         };
         // Partial rows of launches that leave compute units without work stay in the caches: 6 TB/s each way and 4 us for the merge.  Us unsplit,
-        // with what the 8-wavefront kernel's figures chose and with what these choose: one of 4096 tokens, 8 heads 87, 87, 72; one of 8192, 2 heads
+        // with what the tile kernel's figures chose and with what these choose: one of 4096 tokens, 8 heads 87, 87, 72; one of 8192, 2 heads
         // 153, 71, 64.  These are for whole prompts of one length that is a multiple of 64.  Others end in tiles that run in ordinary code, about 5
         // us each one behind the other whatever the share, so that short ones gain nothing (722 tokens, one head, unmasked 35 us, in four shares 44;
         // 2 x 2044, one head, six shares 33, eight 40); and that take the largest scores for their references, which a share of one or two
@@ -1298,7 +1297,7 @@ static int best_kv_splits(int B, int Hq, int D, int Sq_max, int Sk_max, int64_t 
         }
         return best_n;
     }
-    // the 8-wavefront kernel: a K/V tile of 64 keys takes a workgroup about 1.5 / 0.9 / 0.6 us at head_dim 128 / 64 / 32
+    // the tile kernel: a K/V tile of 64 keys takes a workgroup about 1.5 / 0.9 / 0.6 us at head_dim 128 / 64 / 32
     // (one 4096-token prompt with 16 heads of 64: 72 us unsplit, 84 us with two shares)
     const double tile_us = D >= 128 ? 1.5 : (D >= 64 ? 0.9 : 0.6);
     const double jobs = (double)n_pairs * Hq * B;
