@@ -31,8 +31,9 @@ SOURCES = ["api.hip", "paged_decode.hip", "prefill_fwd.hip", "prefill_fwd_w64.hi
 # prefetched query rows into scratch memory, whose reloads wait for every load in flight.
 EXTRA_FLAGS = {"prefill_fwd_w64.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1", "-mllvm", "-disable-machine-licm"],
                # prefill_bwd.hip orders its LDS reads and MFMAs by hand (reads two MFMAs ahead, a scheduling barrier after
-               # every MFMA); the scheduler that runs after register allocation undoes part of that: 1.5 % (measured)
-               "prefill_bwd.hip": ["-mllvm", "-enable-post-misched=0"]}
+               # every MFMA); the scheduler that runs after register allocation undoes part of that: 1.5 % (measured).
+               # Its kernel on wavefronts of 64 keys has all AGPRs in inline assembly, so the compiler's own MFMAs are in VGPR form.
+               "prefill_bwd.hip": ["-mllvm", "-enable-post-misched=0", "-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -170,6 +171,53 @@ def check_scalar_address_hazards(src: str) -> str:
     return "%s: %d inline-assembly memory instructions, none reads a scalar register within five wait states of a vector write" % (src, n_checked)
 
 
+_VREG = re.compile(r"\b([va])(?:\[(\d+):(\d+)\]|(\d+)\b)")
+
+
+def _vregs(text):
+    out = set()
+    for m in _VREG.finditer(text):
+        first, last = (int(m.group(4)),) * 2 if m.group(4) else (int(m.group(2)), int(m.group(3)))
+        out.update(m.group(1) + str(i) for i in range(first, last + 1))
+    return out
+
+
+def check_mfma_hazards(src: str) -> str:
+    """An MFMA may read a register two wait states after a vector instruction wrote it, and its result is there eleven behind an MFMA of eight passes.  The compiler
+    sees to that for its own instructions, not for MFMAs in inline assembly: this fails the build if, on the straight-line path, such an MFMA reads what a
+    vector instruction has just written, or another instruction touches its result too early (an MFMA counts as one state here, and takes eight)."""
+    with tempfile.TemporaryDirectory() as tmp:
+        asm = os.path.join(tmp, "k.s")
+        _run([HIPCC, *FLAGS, *EXTRA_FLAGS.get(src, []), "-S", "--cuda-device-only", os.path.join(CSRC, src), "-o", asm])
+        lines = open(asm).read().splitlines()
+    code, inside, bad, n_checked = [], False, [], 0
+    for no, raw in enumerate(lines, 1):
+        if "#ASMSTART" in raw or "#ASMEND" in raw:
+            inside = "#ASMSTART" in raw
+            continue
+        text = raw.split(";")[0].strip()
+        if text and not text.startswith(".") and not text.endswith(":"):
+            ops = text.split(None, 1)[1].split(",") if " " in text or "\t" in text else []
+            code.append((no, text.split()[0], ops, inside))
+    for i, (no, op, ops, in_asm) in enumerate(code):
+        own = in_asm and op.startswith("v_mfma")
+        n_checked += own
+        reads = _vregs(",".join(ops[1:] if own else ops)) if own or not in_asm else set()
+        states, j = 0, i - 1
+        while reads and j >= 0 and states < (2 if own else 11):
+            _, prev, prev_ops, prev_asm = code[j]
+            written = _vregs(prev_ops[0]) if prev.startswith("v_") and prev_ops else set()
+            mfma = prev.startswith("v_mfma")
+            if written & reads and ((own and not mfma) or (not own and mfma and prev_asm and not op.startswith("v_mfma"))):
+                bad.append("%s:%d: %s reads or writes %s, written %d wait state(s) earlier by %s" % (src, no, op, sorted(written & reads)[:4], states, prev))
+                break
+            states += int(prev_ops[0], 0) + 1 if prev == "s_nop" else 1
+            j -= 1
+    if bad:
+        raise RuntimeError("MFMA hazard in inline assembly:\n" + "\n".join(bad[:20]))
+    return "%s: %d MFMAs in inline assembly, none reads a register that a vector instruction has just written" % (src, n_checked)
+
+
 def _compile_all(srcs, tag=""):
     """Objects of `srcs`, compiled in parallel: [(object, compiler messages)]."""
     obj_dir = os.path.join(HERE, "build")
@@ -227,6 +275,7 @@ def build_library(verbose: bool = True) -> str:
         calls = ex.submit(compile_calls)
         check = ex.submit(check_w64_registers)
         hazards = [ex.submit(check_scalar_address_hazards, s) for s in srcs if issues_memory_from_assembly(s)]
+        hazards.append(ex.submit(check_mfma_hazards, "prefill_bwd.hip"))
         results = _compile_all(srcs)
         notes = [check.result()] + [h.result() for h in hazards]
     if verbose:

@@ -144,6 +144,18 @@ __device__ __forceinline__ void dma_to_lds_16_once(const void* gbase, uint32_t v
                  : "v"(voff), "s"(gbase), "{m0}"(lds_addr)
                  : "memory");
 }
+// ... of 4 bytes a lane, 256 of the wavefront
+__device__ __forceinline__ void dma_to_lds_4(const void* gbase, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1" : : "v"(voff), "s"(gbase), "{m0}"(lds_addr) : "memory");
+}
+// The same for all lanes (-1) or none (0) of a wavefront that runs with all of them.  Without the five wait states: no vector instruction may have written gbase in front,
+// which the build checks.
+__device__ __forceinline__ void dma_to_lds_16_of(int lanes, const void* gbase, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" : : "v"(voff), "s"(gbase), "s"(lanes), "{m0}"(lds_addr) : "memory");
+}
+__device__ __forceinline__ void dma_to_lds_4_of(int lanes, const void* gbase, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dword %0, %1\n\ts_mov_b64 exec, -1" : : "v"(voff), "s"(gbase), "s"(lanes), "{m0}"(lds_addr) : "memory");
+}
 // Sum over the lanes up to this one: shifts inside rows of 16 lanes, then row ends into the rows behind them
 __device__ __forceinline__ int running_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);        // row_shr:1, 2, 4, 8

@@ -719,6 +719,10 @@ __global__ __launch_bounds__(2 * kFuPairs * 64, 1) void bwd_dkv_kernel(BwdParams
     }
 }
 
+}  // namespace mi355
+#include "prefill_bwd_wide.hpp"
+namespace mi355 {
+
 // ---------------------------------------------------------------------------------------------
 // delta, and for packed sequences the plan of the launches behind it.
 //
@@ -853,7 +857,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
         for (int e = 0; e < 8; ++e) sum += (float)o8[e] * (float)g8[e];
 #pragma unroll
         for (int m = kLanes / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
-        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = sum;
+        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = p.wide ? -sum : sum;
     }
 }
 
@@ -1464,10 +1468,19 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
     const int64_t q_jobs = p.cu_q ? d.q_room : ((int64_t)(p.Sq + kBwRows - 1) / kBwRows * G + kDqWaves - 1) / kDqWaves;
     if (delta_wgs > 0x7fffffffLL || k_jobs * d.units_per_pass * d.shares > 0x7fffffffLL || q_jobs * d.units_per_pass > 0x7fffffffLL)
         return (int)hipErrorInvalidValue;
+    // Key tiles with twelve steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
+    // 56 / 70; 4 x 602, 16 heads (5) 32 / 37; 16 x 920 (7) 231 / 243; 4 packed of 324 to 5199, 4 / 2 heads, 4 shares (11) 116 / 120; 2 x 2048, 32 heads (16) 186 / 175; 3000
+    // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
+    const double row_tiles = (double)(p.cu_q ? total_q : (int64_t)p.B * p.Sq) / kBwRows / p.B;
+    p.wide = D == 128 && row_tiles * G * (MODE == MI355_MASK_CAUSAL ? 0.5 : 1.0) >= 12.0 * p.shares;
     hipLaunchKernelGGL((bwd_delta_kernel<D, MODE>), dim3((unsigned)delta_wgs), dim3(kPlanThreads), 0, stream, p, plan);
     for (p.unit0 = 0; p.unit0 < d.n_units; p.unit0 += p.n_units) {
         p.n_units = std::min(d.units_per_pass, d.n_units - p.unit0);
-        hipLaunchKernelGGL((bwd_dkv_kernel<D, MODE, true>), dim3((unsigned)(k_jobs * p.n_units * p.shares)), dim3(2 * kFuPairs * 64), 0, stream, p);
+        const dim3 grid((unsigned)(k_jobs * p.n_units * p.shares));
+        if constexpr (D == 128) {
+            if (p.wide) hipLaunchKernelGGL((bwd_dkv_wide_kernel<MODE>), grid, dim3(kWdWaves * 64), 0, stream, p);
+        }
+        if (!p.wide) hipLaunchKernelGGL((bwd_dkv_kernel<D, MODE, true>), grid, dim3(2 * kFuPairs * 64), 0, stream, p);
         hipLaunchKernelGGL((bwd_dq_ds_kernel<D, MODE>), dim3((unsigned)(q_jobs * p.n_units)), dim3(kDqWaves * 64), 0, stream, p);
     }
     if (p.shares > 1)
@@ -1585,6 +1598,7 @@ static int prefill_bwd_common(const void* q, const void* k, const void* v, const
     p.shares = 1;
     p.part = nullptr;
     p.part_rows = 0;
+    p.wide = false;
     if (workspace) {
         DsPasses d;
         if (!ds_passes(B, Hq, Hkv, Sq_max, Sk_max, D, mask_mode, cu_seqlens_q != nullptr, cu_seqlens_q == cu_seqlens_k, total_q, total_k, d))

@@ -44,6 +44,7 @@ struct BwdParams {
     int shares;
     float* part;
     int64_t part_rows;
+    bool wide;                    // bwd_dkv_wide_kernel, which reads -delta
 };
 
 // Gradients leave in bf16, or in fp32 for an fp32 input: the sums as they are, where a conversion behind the kernel would
