@@ -12,9 +12,7 @@
 // see weight_stream.hpp.  GPU time of a whole step, this against library products and separate operators: 4 layers of width 512,
 // 8 rows 84 / 180 us, 32 rows 104 / 225; 4 layers of 2048, 8 rows 212 / 349, 32 rows 284 / 392; 2 layers of 4096, 16 rows
 // 265 / 375, 32 rows 335 / 340.  The line at 32 rows is not where it breaks even but what the ring and the accumulators are laid out
-// for, two tiles of 16 rows: a small model's step doubles behind it (width 512, 33 rows 227 us), a wide one's does not (4096: 350).  What
-// is slower than the library's product by itself is a long k at 17 rows and more, where the ring holds one step (ADD of 4096 x 14336,
-// 32 rows: 34 us against 22).  A workgroup takes 32 weight rows; its four wavefronts share k and meet in LDS.
+// for, two tiles of 16 rows: a small model's step doubles behind it (width 512, 33 rows 227 us), a wide one's does not (4096: 350).  A workgroup takes 32 weight rows; its four or eight wavefronts share k and meet in LDS.
 //
 // The rows of short prompts go the same way in tiles of 32 (blockIdx.y), each of which reads the weights again: out of the L2s, and what that
 // costs is less than the launches that it saves up to a few hundred rows.  GPU us of a layer's four products and what stands between them,
@@ -27,6 +25,7 @@
 namespace mi355 {
 
 constexpr int kMaxRows = 32, kMaxPromptRows = 1024, kMaxNormCols = 4096;
+constexpr int kWideStreamBytes = 16 * 1024;       // of eight wavefronts: two steps each, with a norm's columns one workgroup per compute unit
 
 struct RowsParams {
     const __bf16* x;
@@ -56,11 +55,12 @@ __device__ __forceinline__ void store_row4(__bf16* to, const float (&v)[4]) {
     *reinterpret_cast<u32x2*>(to) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
 }
 
-template <int MODE, int MT, bool NORM>
-__global__ __launch_bounds__(256) void rows_linear_kernel(RowsParams p) {
-    __shared__ __attribute__((aligned(1024))) unsigned char ring[4 * kStreamBytes];
+template <int MODE, int MT, bool NORM, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
+    constexpr int kRing = WAVES == 4 ? kStreamBytes : kWideStreamBytes;
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[WAVES * kRing];
     __shared__ __attribute__((aligned(16))) float norm_l[NORM ? kMaxNormCols : 4];
-    __shared__ float squares[4][16 * MT];
+    __shared__ float squares[WAVES][16 * MT];
     constexpr bool kGateUp = MODE == MI355_ROWS_GATE_UP;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kg = lane >> 4, piece = (lane & 7) ^ (lane >> 3);
@@ -102,9 +102,9 @@ __global__ __launch_bounds__(256) void rows_linear_kernel(RowsParams p) {
     float sq[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) sq[m] = 0.f;
-    weight_stream<MT>(p.w, w_off, p.x, x_off, p.k, wave, ring + wave * kStreamBytes, acc, [&] {
+    weight_stream<MT, WAVES, kRing>(p.w, w_off, p.x, x_off, p.k, wave, ring + wave * kRing, acc, [&] {
         if constexpr (NORM) {
-            for (int c = tid; c < (p.k + 63) / 64 * 64; c += 256) norm_l[c] = c < p.k ? p.norm[c] : 0.f;
+            for (int c = tid; c < (p.k + 63) / 64 * 64; c += 64 * WAVES) norm_l[c] = c < p.k ? p.norm[c] : 0.f;
             __syncthreads();
         }
     }, [&](int t, int s, int m, bf16x8& x) {
@@ -140,13 +140,13 @@ __global__ __launch_bounds__(256) void rows_linear_kernel(RowsParams p) {
     for (int i = 0; i < NW; ++i) {
         sum[i] = part[(m_sum * 2 + half + i) * 64 + lane];
 #pragma unroll
-        for (int w4 = 1; w4 < 4; ++w4) sum[i] += part[((w4 * MT + m_sum) * 2 + half + i) * 64 + lane];
+        for (int w4 = 1; w4 < WAVES; ++w4) sum[i] += part[((w4 * MT + m_sum) * 2 + half + i) * 64 + lane];
     }
     if (!writes) return;
     if constexpr (NORM) {
         float ssq = 0.f;
 #pragma unroll
-        for (int w4 = 0; w4 < 4; ++w4) ssq += squares[w4][row];
+        for (int w4 = 0; w4 < WAVES; ++w4) ssq += squares[w4][row];
         const float rstd = 1.0f / sqrtf(ssq / (float)p.k + p.eps);
 #pragma unroll
         for (int i = 0; i < NW; ++i) sum[i] *= rstd;
@@ -207,15 +207,26 @@ __global__ __launch_bounds__(256) void rows_linear_kernel(RowsParams p) {
     }
 }
 
+// Eight wavefronts with two steps each, one workgroup per compute unit, where every workgroup has one to itself and k is long: four have their steps one or
+// two at a time, a wait on memory each.  Us, four / eight (k x n): 2048 x 512, 8 rows 3.66 / 3.47, 17 rows 4.75 / 4.39, 100 rows 4.85 / 4.52; 4096 x 1024, 8 rows 5.3 /
+// 4.9, 32 rows 7.4 / 6.4; norm and 2048 x 6144, 8 rows 7.3 / 5.8; 14336 x 4096, 17 rows 33.7 / 20.4, 32 rows 33.4 / 24.1.  At k = 512 both are the launch (2.41 / 2.48,
+// with a norm 3.24 / 3.14 and 17 rows 3.73 / 3.76), at 256 eight lose 0.1 to 0.25; with more workgroups than units a second one hides the waits (300 rows,
+// 2688 x 1024 7.0 / 7.1).
+template <int MODE, int MT, bool NORM>
+static void launch_rows_as(const RowsParams& p, const dim3& grid, hipStream_t s) {
+    if (p.k >= 1024 && (int64_t)grid.x * grid.y <= 256) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 8>), grid, dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4>), grid, dim3(256), 0, s, p);
+}
+
 template <int MODE>
 static int launch_rows(const RowsParams& p, hipStream_t s) {
     const int bn = MODE == MI355_ROWS_GATE_UP ? 16 : 32;
     const int bm = p.T <= 16 ? 16 : 32;
-    const dim3 grid((unsigned)((p.n + bn - 1) / bn), (unsigned)((p.T + bm - 1) / bm)), block(256);
-    if (p.norm && p.T <= 16) hipLaunchKernelGGL((rows_linear_kernel<MODE, 1, true>), grid, block, 0, s, p);
-    else if (p.norm) hipLaunchKernelGGL((rows_linear_kernel<MODE, 2, true>), grid, block, 0, s, p);
-    else if (p.T <= 16) hipLaunchKernelGGL((rows_linear_kernel<MODE, 1, false>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((rows_linear_kernel<MODE, 2, false>), grid, block, 0, s, p);
+    const dim3 grid((unsigned)((p.n + bn - 1) / bn), (unsigned)((p.T + bm - 1) / bm));
+    if (p.norm && p.T <= 16) launch_rows_as<MODE, 1, true>(p, grid, s);
+    else if (p.norm) launch_rows_as<MODE, 2, true>(p, grid, s);
+    else if (p.T <= 16) launch_rows_as<MODE, 1, false>(p, grid, s);
+    else launch_rows_as<MODE, 2, false>(p, grid, s);
     return (int)hipGetLastError();
 }
 

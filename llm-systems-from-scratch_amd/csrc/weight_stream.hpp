@@ -3,7 +3,7 @@
 // Such a product reads every weight once, so what counts is how the weights come in.  16-byte loads straight into the
 // MFMA's operand layout touch 64 bytes of each of 16 rows per instruction, and the address unit takes four times as long for
 // one as for a load of whole lines; here a direct load to LDS brings 8 rows of 128 bytes.  Each wavefront has a ring of its own
-// (no barrier inside the stream) and takes every fourth 64-wide step of k; the caller adds the four up.
+// (no barrier inside the stream) and takes every fourth (of eight wavefronts every eighth) 64-wide step of k; the caller adds them up.
 #pragma once
 #include "common.hpp"
 
@@ -26,11 +26,11 @@ __device__ __forceinline__ void first_weights(const void* w, const uint32_t (&w_
     for (int j = 0; j < 4; ++j) dma_to_lds_16((const char*)w + 128 * (int64_t)wave, w_off[j], lds_address(ring) + j * 1024);
 }
 
-template <int MT, typename G, typename F>
+template <int MT, int WAVES = 4, int RING = kStreamBytes, typename G, typename F>
 __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],
                                               int k, int wave, unsigned char* ring, f32x4 (&acc)[MT][2], G&& meanwhile, F&& on_rows, bool sent = false) {
-    constexpr int kStep = (32 + 16 * MT) * 128, kDeep = MT == 1 ? 2 : 1, kLoads = 4 + 2 * MT;
-    static_assert(kDeep * kStep <= kStreamBytes, "ring");
+    constexpr int kStep = (32 + 16 * MT) * 128, kDeep = RING / kStep, kLoads = 4 + 2 * MT;
+    static_assert(kDeep >= 1 && (kDeep - 1) * kLoads < 64, "ring");
     const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
     const uint32_t ring0 = lds_address(ring);
     const int n_steps = (k + 63) / 64;
@@ -51,11 +51,11 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
         for (int i = 0; i < 2; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int d = 0; d < kDeep; ++d)
-        if (wave + 4 * d < n_steps) request(wave + 4 * d, d, d > 0 || !sent);
+        if (wave + WAVES * d < n_steps) request(wave + WAVES * d, d, d > 0 || !sent);
     meanwhile();
     int slot = 0;
-    for (int t = wave; t < n_steps; t += 4) {
-        if (t + 4 * (kDeep - 1) < n_steps) wait_vmcnt<(kDeep - 1) * kLoads>();
+    for (int t = wave; t < n_steps; t += WAVES) {
+        if (t + WAVES * (kDeep - 1) < n_steps) wait_vmcnt<(kDeep - 1) * kLoads>();
         else wait_vmcnt<0>();                     // (the last steps are all on their way already)
         const unsigned char* at = ring + slot * kStep;
         bf16x8 wf[2][2], af[MT][2];
@@ -77,9 +77,9 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
                     for (int i = 0; i < 2; ++i) wf[i][s] = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
                 }
         }
-        if (t + 4 * kDeep < n_steps) {
+        if (t + WAVES * kDeep < n_steps) {
             wait_lgkmcnt0();                      // the slot's bytes are in registers
-            request(t + 4 * kDeep, slot);
+            request(t + WAVES * kDeep, slot);
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s)
