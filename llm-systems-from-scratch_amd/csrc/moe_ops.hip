@@ -803,12 +803,13 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(MoeParams p, int n_tile
 // gates and their ups) looks through the ids for its expert's pairs itself, and row `pair` of the left and the output matrix
 // belongs to the pair.  The weights are read once for every 32 rows.  What it saves against group + skinny: a launch, and the
 // chain of dependent loads offsets -> order -> rows in front of the first weight.  Bound by the weights' stream (16 experts of
-// 2048 x 1024, 32 tokens: 134 + 67 MB in 31 + 13 us, 4.4 and 5.0 TB/s, where group + skinny took 3 + 34 + 21).
+// 2048 x 1024, 32 tokens: 134 + 67 MB in 39.5 us, 5.1 TB/s, 44 where all workgroups began with the same step of k, see turn_of; group + skinny took 58).
 constexpr int kDirectPairs = 2048;
-template <bool GATE_UP>
+constexpr int kDirectRing = 18 * 1024;            // three steps of 32 + 16 rows, two of 32 + 32; two workgroups per compute unit
+template <bool GATE_UP, int RING, bool TURN>
 __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int32_t* ids, int n_tiles) {
     constexpr int NW = GATE_UP ? 2 : 1;
-    __shared__ __attribute__((aligned(1024))) unsigned char ring[4 * kStreamBytes];
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[4 * RING];
     __shared__ uint16_t mine[kDirectPairs];
     __shared__ int counts[4];
     // (an expert's tiles go round the XCDs: a step of one token uses few experts)
@@ -828,8 +829,9 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
     // none would read weights for nothing (one in seven at two).  Us of router, experts and norm, without / with: 16 experts of 2048 x 1024, top
     // 4, 8 tokens 51.2 / 49.9, 16 57.4 / 55.7, 32 59.8 / 58.0; at 16 pairs an expert, where most take two row tiles and one step
     // at a time, 73.9 / 74.1.
+    const int turn = TURN ? turn_of(p.k, 4) : 0;
     const bool ahead = p.n_pairs >= 2 * p.E && p.n_pairs < 16 * p.E;
-    if (ahead) first_weights(w_base, w_off, p.k, wave, ring + wave * kStreamBytes);
+    if (ahead) first_weights(w_base, w_off, p.k, wave, ring + wave * RING, turn);
     // wavefront w looks through pairs 64 (w + 4 i) + lane, kLook of them at a time
     constexpr int kLook = kDirectPairs / 256;
     uint64_t hit[kLook];
@@ -868,7 +870,7 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
             a_off[j] = (uint32_t)(((int64_t)(GATE_UP ? pair / p.top : pair) * p.a_stride + piece * 8) * 2);
         }
         f32x4 acc[MT][2];
-        weight_stream<MT>(w_base, w_off, p.a, a_off, p.k, wave, ring + wave * kStreamBytes, acc, [] {}, [](int, int, int, bf16x8&) {}, ahead && r0 == 0);
+        weight_stream<MT, 4, RING, TURN>(w_base, w_off, p.a, a_off, p.k, turn, wave, ring + wave * RING, acc, [] {}, [](int, int, int, bf16x8&) {}, ahead && r0 == 0);
         __syncthreads();                          // (the sums travel through the ring)
         f32x4* part = reinterpret_cast<f32x4*>(ring);                           // [wave][row tile][16 rows of w][lane]
 #pragma unroll
@@ -904,6 +906,20 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
         if (n_rows - r0 <= 16) rows(r0, std::integral_constant<int, 1>{});
         else rows(r0, std::integral_constant<int, 2>{});
     }
+}
+
+// From twelve pairs an expert on most experts take two row tiles, of which the small ring holds one step: with the large one 8 experts of 2048 x 2048, top 2, 64 tokens
+// 46.5 -> 41.1 us, 16 of 2048 x 1024, top 4, 100 tokens 49.5 -> 45.8; below, three workgroups per compute unit are worth more (32 tokens 39.5 / 40.7), and so they are where a
+// wavefront has four steps (16 of 1024 x 1024, top 4, 64 tokens 25.3 / 25.8).  (24 of 1536 x 768, top 4, 96 tokens 42, in tiles of 128 rows 50.)
+template <bool GATE_UP>
+static void launch_direct(const MoeParams& p, const int32_t* ids, hipStream_t s) {
+    const int tiles = (p.n + (GATE_UP ? 15 : 31)) / (GATE_UP ? 16 : 32);
+    const dim3 grid((unsigned)(tiles * p.E)), block(256);
+    const bool large = p.k >= 1536 && p.n_pairs >= 12 * p.E, turn = turn_pays(p.k);
+    if (large && turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, true>), grid, block, 0, s, p, ids, tiles);
+    else if (large) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, false>), grid, block, 0, s, p, ids, tiles);
+    else if (turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, true>), grid, block, 0, s, p, ids, tiles);
+    else hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, false>), grid, block, 0, s, p, ids, tiles);
 }
 
 // fp32: 16 rows x 64 columns per workgroup, a thread owns four rows of one column
@@ -1120,10 +1136,9 @@ extern "C" int mi355_moe_direct(const void* h, const void* w_gate_up, const void
                        n_experts, top, ff, n, MI355_BF16, MI355_TILING_AUTO);
     if (rc != MI355_OK || n_tokens == 0) return rc;
     hipStream_t s = (hipStream_t)stream;
-    const int up_tiles = (ff + 15) / 16, down_tiles = (n + 31) / 32;
-    hipLaunchKernelGGL(moe_direct_kernel<true>, dim3((unsigned)(up_tiles * n_experts)), dim3(256), 0, s, up, ids, up_tiles);
+    launch_direct<true>(up, ids, s);
     if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
-    hipLaunchKernelGGL(moe_direct_kernel<false>, dim3((unsigned)(down_tiles * n_experts)), dim3(256), 0, s, down, ids, down_tiles);
+    launch_direct<false>(down, ids, s);
     if ((rc = (int)hipGetLastError()) != 0) return set_error(rc, hipGetErrorString((hipError_t)rc));
     return MI355_OK;
 }

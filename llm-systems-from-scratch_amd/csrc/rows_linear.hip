@@ -55,7 +55,7 @@ __device__ __forceinline__ void store_row4(__bf16* to, const float (&v)[4]) {
     *reinterpret_cast<u32x2*>(to) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
 }
 
-template <int MODE, int MT, bool NORM, int WAVES>
+template <int MODE, int MT, bool NORM, int WAVES, bool TURN>
 __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
     constexpr int kRing = WAVES == 4 ? kStreamBytes : kWideStreamBytes;
     __shared__ __attribute__((aligned(1024))) unsigned char ring[WAVES * kRing];
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
     float sq[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) sq[m] = 0.f;
-    weight_stream<MT, WAVES, kRing>(p.w, w_off, p.x, x_off, p.k, wave, ring + wave * kRing, acc, [&] {
+    weight_stream<MT, WAVES, kRing, TURN>(p.w, w_off, p.x, x_off, p.k, TURN ? turn_of(p.k, WAVES) : 0, wave, ring + wave * kRing, acc, [&] {
         if constexpr (NORM) {
             for (int c = tid; c < (p.k + 63) / 64 * 64; c += 64 * WAVES) norm_l[c] = c < p.k ? p.norm[c] : 0.f;
             __syncthreads();
@@ -211,11 +211,13 @@ __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
 // two at a time, a wait on memory each.  Us, four / eight (k x n): 2048 x 512, 8 rows 3.66 / 3.47, 17 rows 4.75 / 4.39, 100 rows 4.85 / 4.52; 4096 x 1024, 8 rows 5.3 /
 // 4.9, 32 rows 7.4 / 6.4; norm and 2048 x 6144, 8 rows 7.3 / 5.8; 14336 x 4096, 17 rows 33.7 / 20.4, 32 rows 33.4 / 24.1.  At k = 512 both are the launch (2.41 / 2.48,
 // with a norm 3.24 / 3.14 and 17 rows 3.73 / 3.76), at 256 eight lose 0.1 to 0.25; with more workgroups than units a second one hides the waits (300 rows,
-// 2688 x 1024 7.0 / 7.1).
+// 2688 x 1024 7.0 / 7.1).  More workgroups than units over rows of whole 4096 bytes begin with steps of their own (turn_of): norm and 4096 x 12288, 8 rows 26.7 -> 20.4, gate and
+// up of 4096 x 14336, 32 rows 45.0 -> 43.1, 2048 x 5632 11.5 -> 11.0; with fewer it costs 1 to 2 %.
 template <int MODE, int MT, bool NORM>
 static void launch_rows_as(const RowsParams& p, const dim3& grid, hipStream_t s) {
-    if (p.k >= 1024 && (int64_t)grid.x * grid.y <= 256) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 8>), grid, dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4>), grid, dim3(256), 0, s, p);
+    if (p.k >= 1024 && (int64_t)grid.x * grid.y <= 256) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 8, false>), grid, dim3(512), 0, s, p);
+    else if (turn_pays(p.k) && (int64_t)grid.x * grid.y > 256) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4, false>), grid, dim3(256), 0, s, p);
 }
 
 template <int MODE>

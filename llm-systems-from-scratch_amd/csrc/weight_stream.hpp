@@ -18,23 +18,33 @@ constexpr int kStreamBytes = 12 * 1024;
 // change a fragment of activations: lane holds row 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
 // sent: first_weights has been called (its requests are older than all of these, so the waits count the same).
 // acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
+// Workgroups that stream rows of whole 4096 bytes side by side, all from step 0 on, want the same few of an L2's sixteen channels (256 bytes each in turn) at any
+// time: 16 experts of 2048 x 1024, 32 tokens 44.0 us, 5.1 TB/s with the steps begun somewhere else by every one of an XCD's workgroups (every eighth of a launch) 39.5.  The same
+// beginning within an XCD and another on each other one gives nothing (45.0); nor does any with rows of 2048 bytes (24.3 / 25.1), which have two sets of channels.
+inline bool turn_pays(int k) { return k % 2048 == 0; }
+__device__ __forceinline__ int turn_of(int k, int waves) { return (int)(blockIdx.x / 8 * waves) % (k / 64); }
+
 // The weights of a wavefront's first step, requested while the rows are still being looked for (slot 0 begins with them, whatever MT);
 // k a multiple of 64.
-__device__ __forceinline__ void first_weights(const void* w, const uint32_t (&w_off)[4], int k, int wave, unsigned char* ring) {
+__device__ __forceinline__ void first_weights(const void* w, const uint32_t (&w_off)[4], int k, int wave, unsigned char* ring, int turn) {
     if (64 * wave >= k) return;
+    const int t = wave + turn >= k / 64 ? wave + turn - k / 64 : wave + turn;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dma_to_lds_16((const char*)w + 128 * (int64_t)wave, w_off[j], lds_address(ring) + j * 1024);
+    for (int j = 0; j < 4; ++j) dma_to_lds_16((const char*)w + 128 * (int64_t)t, w_off[j], lds_address(ring) + j * 1024);
 }
 
-template <int MT, int WAVES = 4, int RING = kStreamBytes, typename G, typename F>
+// turn: the step that the wavefronts begin with (TURN; else 0)
+template <int MT, int WAVES, int RING, bool TURN, typename G, typename F>
 __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],
-                                              int k, int wave, unsigned char* ring, f32x4 (&acc)[MT][2], G&& meanwhile, F&& on_rows, bool sent = false) {
+                                              int k, int turn, int wave, unsigned char* ring, f32x4 (&acc)[MT][2], G&& meanwhile, F&& on_rows, bool sent = false) {
     constexpr int kStep = (32 + 16 * MT) * 128, kDeep = RING / kStep, kLoads = 4 + 2 * MT;
-    static_assert(kDeep >= 1 && (kDeep - 1) * kLoads < 64, "ring");
+    static_assert(kDeep >= 1 && kDeep <= 3, "ring");
     const int lane = threadIdx.x & 63, r = lane & 15, kg = lane >> 4;
     const uint32_t ring0 = lds_address(ring);
     const int n_steps = (k + 63) / 64;
-    const auto request = [&](int t, int slot, bool weights = true) {
+    const auto turned = [&](int i) { return TURN && i + turn >= n_steps ? i + turn - n_steps : i + turn; };
+    const auto request = [&](int i, int slot, bool weights = true) {
+        const int t = turned(i);
         const char* wt = (const char*)w + 128 * (int64_t)t;
         const char* at = (const char*)a + 128 * (int64_t)t;
         // (pieces behind the end of a row: its first piece of this step once more)
@@ -54,9 +64,11 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
         if (wave + WAVES * d < n_steps) request(wave + WAVES * d, d, d > 0 || !sent);
     meanwhile();
     int slot = 0;
-    for (int t = wave; t < n_steps; t += WAVES) {
-        if (t + WAVES * (kDeep - 1) < n_steps) wait_vmcnt<(kDeep - 1) * kLoads>();
-        else wait_vmcnt<0>();                     // (the last steps are all on their way already)
+    for (int i0 = wave; i0 < n_steps; i0 += WAVES) {
+        const int t = turned(i0);
+        if (kDeep > 2 && i0 + 2 * WAVES < n_steps) wait_vmcnt<2 * kLoads>();
+        else if (kDeep > 1 && i0 + WAVES < n_steps) wait_vmcnt<kLoads>();
+        else wait_vmcnt<0>();
         const unsigned char* at = ring + slot * kStep;
         bf16x8 wf[2][2], af[MT][2];
 #pragma unroll
@@ -77,9 +89,9 @@ __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_
                     for (int i = 0; i < 2; ++i) wf[i][s] = as_bf16x8(u32x4{0u, 0u, 0u, 0u});
                 }
         }
-        if (t + WAVES * kDeep < n_steps) {
+        if (i0 + WAVES * kDeep < n_steps) {
             wait_lgkmcnt0();                      // the slot's bytes are in registers
-            request(t + WAVES * kDeep, slot);
+            request(i0 + WAVES * kDeep, slot);
         }
 #pragma unroll
         for (int s = 0; s < 2; ++s)

@@ -1,0 +1,34 @@
+"""Experts whose rows are whole 4096 bytes, products without an order: steps of k that begin elsewhere in every workgroup, few and many pairs per expert (the line between the
+two rings on either side, one and two row tiles, more than one pass over the weights), columns that are no whole tile, experts without pairs.  Against float64 products of
+the bf16 operands; one rounding of the activation and one of the result, 2^-8 of the norm each at most."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 8, 1, 2048, 64, 2048), (5, 8, 2, 2048, 1024, 72), (47, 4, 1, 2048, 192, 2048), (48, 4, 1, 2048, 192, 100), (50, 3, 3, 4096, 128, 36),
+                                            (96, 4, 1, 2048, 2048, 2048), (97, 4, 1, 2048, 2048, 40), (300, 6, 2, 2048, 64, 64), (33, 4, 2, 1536, 2048, 96)])
+def test_direct_products_of_whole_pages(T, E, top, k, ff, n):
+    import mi355_attn as ma
+    print(f"case: direct {T} {E} {top} {k} {ff} {n}", flush=True)
+    g = torch.Generator().manual_seed(T + E)
+
+    def t(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g) * std).to(torch.bfloat16).cuda()
+
+    h, up, down = t(T, k), t(E, 2 * ff, k, std=k ** -0.5), t(E, n, ff, std=ff ** -0.5)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).to(torch.int32).cuda()
+    if T > 40:
+        ids[:30] = torch.arange(top, dtype=torch.int32)                  # (more rows than one pass takes)
+    weights = torch.rand(T, top, generator=g).cuda()
+    got = ma.moe_experts(h, ids, weights, up, down, tiling="direct")
+    ref = torch.zeros(T, top, n, dtype=torch.float64, device="cuda")
+    for e in range(E):
+        t_at, c_at = (ids == e).nonzero(as_tuple=True)
+        x = h[t_at].double() @ up[e].double().T
+        act = torch.nn.functional.silu(x[:, :ff]) * x[:, ff:]
+        ref[t_at, c_at] = weights[t_at, c_at].double()[:, None] * (act @ down[e].double().T)
+    got = got.double().view(T, top, n)
+    assert bool(torch.isfinite(got).all())
+    assert float((got - ref).norm()) <= 2 * 2 ** -8 * float(ref.norm())
