@@ -1588,13 +1588,13 @@ _DIRECT_PAIRS = 2048        # the most pairs mi355_moe_direct takes
 def _direct_pairs(experts: int, k: int, ff: int, n: int) -> int:
     """Up to how many pairs the expert products run without an order.  That saves a launch and the padding of 128-row tiles, and costs
     what the pairs' rows take up: each 32 weight rows read those of their expert (k wide, then ff wide, and n out), and the weights once
-    more for every 32 of them.  So the line is drawn at 1.2 M elements in all pairs' rows, but not below 24 nor above 64 pairs per expert,
-    where one expert with more than its share would be waited for.  Us without and with an order, uniform ids: 8 experts of 1024 x 1024
-    (line at 48 pairs per expert) 32 pairs 20 / 30, 48 26 / 31, 64 31 / 32; 16 of 1024 x 1024 (24) 16 25 / 31, 24 28 / 31, 32 34 / 32; 32 of
-    512 x 512 (24) 16 20 / 22, 24 22 / 23, 32 24 / 23; 24 of 1536 x 768 16 42 / 50, 24 47 / 52, 29 51 / 52; 16 of 2048 x 1024 16 44 / 53, 24
-    48 / 53, 29 51 / 54; 32 of 2048 x 2048 16 146 / 195, 24 162 / 196, 32 196 / 198; 8 of 3072 x 1024 24 34 / 49; 16 of 1792 x 896, whose
-    tiles of 128 rows make one round, 13 35 / 37, 24 42 / 38; 8 of 1024 x 3072 (29) 24 34 / 51, 48 58 / 54."""
-    return min(_DIRECT_PAIRS, 64 * experts, max(24 * experts, (9 << 17) // (k + ff + n)))
+    more for every 32 of them.  So the line is drawn at 1.2 M elements in all pairs' rows, but not below 24 pairs per expert -- 16 where 128-row tiles of so
+    many experts fill the chip -- nor above 64, where one expert with more than its share would be waited for.  Us without and with an order, uniform ids: 8 experts of
+    1024 x 1024 (line at 48 pairs per expert) 32 pairs 20 / 30, 48 26 / 31, 64 31 / 32; 16 of 1024 x 1024 (24) 16 25 / 31, 24 28 / 31, 32 34 / 32; 32 of
+    512 x 512 (24) 16 20 / 22, 24 22 / 23, 32 24 / 23; 24 of 1536 x 768 16 42 / 50, 24 47 / 52; 16 of 2048 x 1024 16 42 / 44, 24 46 / 45; 8 of 2048 x 1024 24 28 / 40;
+    8 of 2048 x 2048 24 43 / 52; 32 of 2048 x 2048 12 142 / 144, 16 146 / 145, 24 168 / 147; 32 of 2048 x 1024 12 76 / 79, 16 81 / 79, 24 88 / 80; 8 of 3072 x 1024 24
+    34 / 49; 16 of 1792 x 896, whose tiles make one round, 13 35 / 37, 24 42 / 38; 8 of 1024 x 3072 (29) 24 34 / 51, 48 58 / 54."""
+    return min(_DIRECT_PAIRS, 64 * experts, max((24 if experts * ff <= 16384 else 16) * experts, (9 << 17) // (k + ff + n)))
 
 
 def moe_experts(h, ids, weights, w_gate_up, w_down, *, tiling="auto"):

@@ -10,8 +10,18 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 8, 1, 2048, 64, 2048), (5, 8, 2, 2048, 1024, 72), (47, 4, 1, 2048, 192, 2048), (48, 4, 1, 2048, 192, 100), (50, 3, 3, 4096, 128, 36),
                                             (96, 4, 1, 2048, 2048, 2048), (97, 4, 1, 2048, 2048, 40), (300, 6, 2, 2048, 64, 64), (33, 4, 2, 1536, 2048, 96)])
 def test_direct_products_of_whole_pages(T, E, top, k, ff, n):
+    _products(T, E, top, k, ff, n, "direct")
+
+
+@pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 2, 1, 2048, 64, 2048), (130, 3, 1, 2048, 2048, 136), (200, 8, 2, 4096, 192, 2048), (513, 2, 1, 2048, 128, 128), (512, 2, 1, 2048, 2048, 96)])
+def test_large_tiles_of_whole_pages(T, E, top, k, ff, n):
+    """(128 x 128 tiles, up to 256 pairs an expert and one more)"""
+    _products(T, E, top, k, ff, n, "large")
+
+
+def _products(T, E, top, k, ff, n, tiling):
     import mi355_attn as ma
-    print(f"case: direct {T} {E} {top} {k} {ff} {n}", flush=True)
+    print(f"case: {tiling} {T} {E} {top} {k} {ff} {n}", flush=True)
     g = torch.Generator().manual_seed(T + E)
 
     def t(*shape, std=1.0):
@@ -22,7 +32,7 @@ def test_direct_products_of_whole_pages(T, E, top, k, ff, n):
     if T > 40:
         ids[:30] = torch.arange(top, dtype=torch.int32)                  # (more rows than one pass takes)
     weights = torch.rand(T, top, generator=g).cuda()
-    got = ma.moe_experts(h, ids, weights, up, down, tiling="direct")
+    got = ma.moe_experts(h, ids, weights, up, down, tiling=tiling)
     ref = torch.zeros(T, top, n, dtype=torch.float64, device="cuda")
     for e in range(E):
         t_at, c_at = (ids == e).nonzero(as_tuple=True)
