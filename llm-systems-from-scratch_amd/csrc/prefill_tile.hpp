@@ -17,6 +17,12 @@ __device__ __forceinline__ int swz(int row) {
     else return (row >> 2) & 3;
 }
 
+// Heads that the kernels of short sequences keep on one XCD.  Rows of 32 elements are half a line: where a tensor's heads stand side by side (V, the output and its gradient are views of
+// (batch, seq, heads, d)), two heads share each line, and on two XCDs both fetch it.  us, heads dealt one by one / two together / eight: forward of 64 x 16 heads, 256 tokens 20.6 /
+// 18.2 / 18.2, with gradients (forward, backward) 21.1, 44.3 / 18.9, 40.4 / 19.0, 40.0; 200 x 16 heads, 100 tokens 28.1, 46.2 / 25.6, 42.1 / 23.2, 39.5.  Heads of 64
+// (64 x 16, 256 tokens 41.1, 81.8 / 40.3, 82.4 / 40.3, 80.6; 64 x 8, 128 tokens 9.55 / 9.57 / 9.92) have lines of their own.
+constexpr int short_heads(int D) { return D == 32 ? 8 : 1; }
+
 // Per-lane LDS offsets of the two read patterns of a swizzled 64 x D tile.
 template <int D>
 struct TileReads {
