@@ -1,4 +1,4 @@
-"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with twelve steps and more on average) against the form without dS in memory: rows and keys
+"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with fifteen steps and more on average) against the form without dS in memory: rows and keys
 around the tiles of 64 and 128 and their halves, a tile of rows that is the sequence's only one, wavefronts without keys or rows, more queries than keys
 and the other way round, one to many steps, shares, fp32 gradients, several passes.  Tolerance of test_gpu_backward.py: one rounding of the result over a tensor."""
 import pytest
