@@ -809,18 +809,30 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(MoeParams p, int n_tile
 // belongs to the pair.  The weights are read once for every 32 rows.  What it saves against group + skinny: a launch, and the
 // chain of dependent loads offsets -> order -> rows in front of the first weight.  Bound by the weights' stream (16 experts of
 // 2048 x 1024, 32 tokens: 134 + 67 MB in 39.5 us, 5.1 TB/s, 44 where all workgroups began with the same step of k, see turn_of; group + skinny took 58).
-constexpr int kDirectPairs = 2048;
+// FEW (fewer pairs than experts, up to a wavefront's lanes): workgroups per pair instead, of which those of an expert's first one go on.  Experts without pairs, most of
+// them then, have no workgroups that hold LDS while they find out, and one load tells a wavefront all it has to know.  Us of both products, workgroups per expert /
+// like this: 32 experts of 2048 x 1024, top 2, one token 13.9 / 10.1, 6 tokens 25.4 / 23.2, 15 tokens 45.2 / 42.8; 32 of 1024 x 512, top 2, 1 token 9.6 / 7.6; 8 of
+// 2048 x 1024, 7 tokens 19.5 / 19.1; 16 of 512 x 256, top 2, 4 tokens 7.8 / 7.0.  (Eight wavefronts with 18 KB each, one workgroup per compute unit: 10.2, 30.0, 51.6.)
+constexpr int kDirectPairs = 2048, kFewPairs = 64;
 constexpr int kDirectRing = 18 * 1024;            // three steps of 32 + 16 rows, two of 32 + 32; two workgroups per compute unit
-template <bool GATE_UP, int RING, bool TURN>
+template <bool GATE_UP, int RING, bool TURN, bool FEW>
 __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int32_t* ids, int n_tiles) {
     constexpr int NW = GATE_UP ? 2 : 1;
     __shared__ __attribute__((aligned(1024))) unsigned char ring[4 * RING];
-    __shared__ uint16_t mine[kDirectPairs];
+    __shared__ uint16_t mine[FEW ? kFewPairs : kDirectPairs];
     __shared__ int counts[4];
     // (an expert's tiles go round the XCDs: a step of one token uses few experts)
-    const int n0 = blockIdx.x % n_tiles * (GATE_UP ? 16 : 32), e = blockIdx.x / n_tiles;
+    const int n0 = blockIdx.x % n_tiles * (GATE_UP ? 16 : 32);
+    int e = blockIdx.x / n_tiles;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kg = lane >> 4;
+    uint64_t of_expert = 0;
+    if constexpr (FEW) {                          // workgroups of pair e: for its expert, if no pair in front has the same
+        const int id = lane < p.n_pairs ? ids[lane] : -1, pair = e;
+        e = __builtin_amdgcn_readlane(id, pair);
+        of_expert = __builtin_amdgcn_ballot_w64(id == e);
+        if ((unsigned)e >= (unsigned)p.E || (of_expert & ((1ull << pair) - 1)) != 0) return;
+    }
     const __bf16* w_base = (const __bf16*)p.w + (int64_t)e * (GATE_UP ? 2 : 1) * p.n * p.k;
     const int piece = (lane & 7) ^ (lane >> 3);   // what a lane requests of its row's 128 bytes: see weight_stream
     uint32_t w_off[4];
@@ -835,35 +847,41 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
     // 4, 8 tokens 51.2 / 49.9, 16 57.4 / 55.7, 32 59.8 / 58.0; at 16 pairs an expert, where most take two row tiles and one step
     // at a time, 73.9 / 74.1.
     const int turn = TURN ? turn_of(p.k, 4) : 0;
-    const bool ahead = p.n_pairs >= 2 * p.E && p.n_pairs < 16 * p.E;
-    if (ahead) first_weights(w_base, w_off, p.k, wave, ring + wave * RING, turn);
-    // wavefront w looks through pairs 64 (w + 4 i) + lane, kLook of them at a time
-    constexpr int kLook = kDirectPairs / 256;
-    uint64_t hit[kLook];
-    int found = 0;
+    const bool ahead = !FEW && p.n_pairs >= 2 * p.E && p.n_pairs < 16 * p.E;
+    int n_rows = 0;
+    if constexpr (FEW) {
+        n_rows = __popcll(of_expert);
+        if (wave == 0 && (of_expert >> lane & 1)) mine[__popcll(of_expert & ((1ull << lane) - 1))] = (uint16_t)lane;
+    } else {
+        if (ahead) first_weights(w_base, w_off, p.k, wave, ring + wave * RING, turn);
+        // wavefront w looks through pairs 64 (w + 4 i) + lane, kLook of them at a time
+        constexpr int kLook = kDirectPairs / 256;
+        uint64_t hit[kLook];
+        int found = 0;
 #pragma unroll
-    for (int i = 0; i < kLook; ++i) {
-        const int pair = 64 * (wave + 4 * i) + lane;
-        hit[i] = 0;
-        if (64 * (wave + 4 * i) < p.n_pairs) hit[i] = __builtin_amdgcn_ballot_w64(pair < p.n_pairs && ids[min(pair, p.n_pairs - 1)] == e);
-        found += __popcll(hit[i]);
-    }
-    if (lane == 0) counts[wave] = found;
-    __syncthreads();
-    int at = 0, n_rows = 0;
+        for (int i = 0; i < kLook; ++i) {
+            const int pair = 64 * (wave + 4 * i) + lane;
+            hit[i] = 0;
+            if (64 * (wave + 4 * i) < p.n_pairs) hit[i] = __builtin_amdgcn_ballot_w64(pair < p.n_pairs && ids[min(pair, p.n_pairs - 1)] == e);
+            found += __popcll(hit[i]);
+        }
+        if (lane == 0) counts[wave] = found;
+        __syncthreads();
+        int at = 0;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        at += w < wave ? counts[w] : 0;
-        n_rows += counts[w];
-    }
-    if (n_rows == 0) {
-        wait_vmcnt<0>();                          // (nothing lands in LDS that is somebody else's by then)
-        return;
-    }
+        for (int w = 0; w < 4; ++w) {
+            at += w < wave ? counts[w] : 0;
+            n_rows += counts[w];
+        }
+        if (n_rows == 0) {
+            wait_vmcnt<0>();                          // (nothing lands in LDS that is somebody else's by then)
+            return;
+        }
 #pragma unroll
-    for (int i = 0; i < kLook; ++i) {
-        if (hit[i] >> lane & 1) mine[at + __popcll(hit[i] & ((1ull << lane) - 1))] = (uint16_t)(64 * (wave + 4 * i) + lane);
-        at += __popcll(hit[i]);
+        for (int i = 0; i < kLook; ++i) {
+            if (hit[i] >> lane & 1) mine[at + __popcll(hit[i] & ((1ull << lane) - 1))] = (uint16_t)(64 * (wave + 4 * i) + lane);
+            at += __popcll(hit[i]);
+        }
     }
     __syncthreads();
     const auto rows = [&](int r0, auto tiles) {
@@ -921,10 +939,19 @@ static void launch_direct(const MoeParams& p, const int32_t* ids, hipStream_t s)
     const int tiles = (p.n + (GATE_UP ? 15 : 31)) / (GATE_UP ? 16 : 32);
     const dim3 grid((unsigned)(tiles * p.E)), block(256);
     const bool large = p.k >= 1536 && p.n_pairs >= 12 * p.E, turn = turn_pays(p.k);
-    if (large && turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, true>), grid, block, 0, s, p, ids, tiles);
-    else if (large) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, false>), grid, block, 0, s, p, ids, tiles);
-    else if (turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, true>), grid, block, 0, s, p, ids, tiles);
-    else hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, false>), grid, block, 0, s, p, ids, tiles);
+    if (p.n_pairs < p.E && p.n_pairs <= kFewPairs) {
+        const dim3 few((unsigned)(tiles * p.n_pairs));
+        if (turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, true, true>), few, block, 0, s, p, ids, tiles);
+        else hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, false, true>), few, block, 0, s, p, ids, tiles);
+    } else if (large && turn) {
+        hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, true, false>), grid, block, 0, s, p, ids, tiles);
+    } else if (large) {
+        hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kDirectRing, false, false>), grid, block, 0, s, p, ids, tiles);
+    } else if (turn) {
+        hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, true, false>), grid, block, 0, s, p, ids, tiles);
+    } else {
+        hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, false, false>), grid, block, 0, s, p, ids, tiles);
+    }
 }
 
 // fp32: 16 rows x 64 columns per workgroup, a thread owns four rows of one column

@@ -1,4 +1,4 @@
-"""Experts whose rows are whole 4096 bytes, products without an order: steps of k that begin elsewhere in every workgroup, few and many pairs per expert (the line between the
+"""Experts' products without an order, of few pairs and over rows of whole 4096 bytes: steps of k that begin elsewhere in every workgroup, few and many pairs per expert (the line between the
 two rings on either side, one and two row tiles, more than one pass over the weights), columns that are no whole tile, experts without pairs.  Against float64 products of
 the bf16 operands; one rounding of the activation and one of the result, 2^-8 of the norm each at most."""
 import pytest
@@ -10,6 +10,13 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 8, 1, 2048, 64, 2048), (5, 8, 2, 2048, 1024, 72), (47, 4, 1, 2048, 192, 2048), (48, 4, 1, 2048, 192, 100), (50, 3, 3, 4096, 128, 36),
                                             (96, 4, 1, 2048, 2048, 2048), (97, 4, 1, 2048, 2048, 40), (300, 6, 2, 2048, 64, 64), (33, 4, 2, 1536, 2048, 96)])
 def test_direct_products_of_whole_pages(T, E, top, k, ff, n):
+    _products(T, E, top, k, ff, n, "direct")
+
+
+@pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 2, 1, 64, 64, 40), (7, 32, 4, 2048, 128, 64), (16, 80, 4, 128, 64, 36), (21, 80, 3, 512, 192, 2048), (13, 80, 5, 128, 64, 64),
+                                            (63, 64, 1, 256, 64, 72), (64, 64, 1, 256, 64, 72)])
+def test_fewer_pairs_than_experts(T, E, top, k, ff, n):
+    """(workgroups per pair: experts that several pairs name, most of them, up to 64 pairs and fewer than experts, and one more of each)"""
     _products(T, E, top, k, ff, n, "direct")
 
 
