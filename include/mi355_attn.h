@@ -99,6 +99,12 @@ int mi355_prefill_fwd_lse_rounded(const void* q, const void* k, const void* v, v
                                   const int64_t v_strides[3], const int64_t o_strides[3], const int64_t lse_strides[2], int f32, void* q16, void* k16,
                                   void* v16, const int64_t q16_strides[3], const int64_t k16_strides[3], const int64_t v16_strides[3], int B, int Hq, int Hkv,
                                   int Sq, int Sk, int D, float softmax_scale, int mask_mode, void* stream);
+/* ... without a backward: nothing is left but out. */
+int mi355_prefill_fwd_rounded(const void* q, const void* k, const void* v, void* out, const int64_t q_strides[3], const int64_t k_strides[3],
+                              const int64_t v_strides[3], const int64_t o_strides[3], int f32, int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                              float softmax_scale, int mask_mode, void* stream);
+/* Up to three fp32 operands to bf16 in one launch: out[i][j] = bf16(in[i][j]), j < n[i] (up to 2^32); 16-byte aligned; in[i] null: none. */
+int mi355_round_operands(const float* const in[3], void* const out[3], const int64_t n[3], void* stream);
 
 /*
  * Causal prefill of a CHUNK of new tokens on top of context that is already in a paged bf16 cache

@@ -226,7 +226,29 @@ torch::autograd::variable_list backward_of(const Tensor& q0, const Tensor& k0, c
 int f32_bits(const Tensor& q, const Tensor& k, const Tensor& v) {
     return (q.scalar_type() == kF32 ? 1 : 0) | (k.scalar_type() == kF32 ? 2 : 0) | (v.scalar_type() == kF32 ? 4 : 0);
 }
-Tensor bf16(const Tensor& t) { return t.scalar_type() == kBF16 ? t : t.to(kBF16); }
+
+// q, k and v with what is fp32 among them rounded: in one launch where their elements fill their memory
+std::array<Tensor, 3> bf16(const Tensor& q, const Tensor& k, const Tensor& v) {
+    const Tensor* t[3] = {&q, &k, &v};
+    std::array<Tensor, 3> r;
+    const float* in[3] = {nullptr, nullptr, nullptr};
+    void* out[3] = {nullptr, nullptr, nullptr};
+    int64_t n[3] = {0, 0, 0};
+    for (int i = 0; i < 3; ++i) {
+        if (t[i]->scalar_type() == kBF16) {
+            r[i] = *t[i];
+        } else if (!t[i]->is_non_overlapping_and_dense() || !Args::aligned(*t[i]) || t[i]->numel() > 1LL << 32) {
+            r[i] = t[i]->to(kBF16);
+        } else {
+            r[i] = at::empty_like(*t[i], t[i]->options().dtype(kBF16));
+            in[i] = (const float*)t[i]->data_ptr();
+            out[i] = r[i].data_ptr();
+            n[i] = t[i]->numel();
+        }
+    }
+    if (in[0] || in[1] || in[2]) check(mi355_round_operands(in, out, n, stream_of(q.device())), "mi355_round_operands");
+    return r;
+}
 
 // forward_lse of short heads with fp32 among q, k and v, which it rounds: q, k, v become what the backward reads
 bool forward_rounded(Tensor& q, Tensor& k, Tensor& v, const Shape& s, Tensor& out, Tensor& lse) {
@@ -262,9 +284,7 @@ struct DenseFn : torch::autograd::Function<DenseFn> {
         Tensor q = q0, k = k0, v = v0, out, lse;
         const Shape s{false, causal, (int)q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2), (int)k.size(2), (int)q.size(3), scale};
         if (!forward_rounded(q, k, v, s, out, lse)) {
-            q = bf16(q0);
-            k = bf16(k0);
-            v = bf16(v0);
+            std::tie(q, k, v) = std::tuple_cat(bf16(q0, k0, v0));
             std::tie(out, lse) = forward_lse(rows16(q), rows16(k), rows16(v), nullptr, nullptr, s);
         }
         ctx->save_for_backward({q, k, v, out, lse});
@@ -286,7 +306,7 @@ struct DenseFn : torch::autograd::Function<DenseFn> {
 struct PackedFn : torch::autograd::Function<PackedFn> {
     static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q0, const Tensor& k0, const Tensor& v0, const Tensor& cu_q, const Tensor& cu_k,
                           int64_t max_q, int64_t max_k, bool causal, double scale) {
-        const Tensor q = bf16(q0), k = bf16(k0), v = bf16(v0);
+        const auto [q, k, v] = bf16(q0, k0, v0);
         const Shape s{true, causal, (int)cu_q.numel() - 1, (int)q.size(1), (int)k.size(1), (int)max_q, (int)max_k, (int)q.size(2), scale};
         auto [out, lse] = forward_lse(rows16(q), rows16(k), rows16(v), (const int32_t*)cu_q.data_ptr(), (const int32_t*)cu_k.data_ptr(), s);
         ctx->save_for_backward({q, k, v, out, lse, cu_q, cu_k});
@@ -359,6 +379,20 @@ Tensor forward_only(const Tensor& q, const Tensor& k, const Tensor& v, const int
     return out;
 }
 
+// forward_only of short heads with fp32 among q, k and v, which the kernel rounds on their way in; undefined: no such form of this call
+Tensor forward_mixed(const Tensor& q, const Tensor& k, const Tensor& v, const Shape& s) {
+    const int f32 = f32_bits(q, k, v);
+    if (f32 == 0 || !((float)s.scale > 0.f) || !mi355_prefill_fwd_rounds(s.Hq, s.Hkv, s.Sq, s.Sk, s.D, s.mode())) return {};
+    for (const Tensor* t : {&q, &k, &v})
+        if (!whole_rows(*t) || t->stride(2) <= 0 || t->stride(2) >= (1 << 24)) return {};
+    const auto dev = q.device();
+    const Tensor out = make({s.B, s.Sq, s.Hq, s.D}, kBF16, dev).permute({0, 2, 1, 3});
+    check(mi355_prefill_fwd_rounded(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), Strides(q), Strides(k), Strides(v), Strides(out), f32, s.B, s.Hq,
+                                    s.Hkv, s.Sq, s.Sk, s.D, (float)s.scale, s.mode(), stream_of(dev)),
+          "mi355_prefill_fwd_rounded");
+    return out;
+}
+
 // (q, k, v, causal, softmax_scale)
 PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -377,7 +411,11 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
             out = DenseFn::apply(*q, *k, *v, causal, scale);
         } else {
             const Shape s{false, causal, (int)q->size(0), (int)q->size(1), (int)k->size(1), (int)q->size(2), (int)k->size(2), (int)q->size(3), scale};
-            out = forward_only(rows16(bf16(*q)), rows16(bf16(*k)), rows16(bf16(*v)), nullptr, nullptr, s, 0, 0);
+            out = forward_mixed(*q, *k, *v, s);
+            if (!out.defined()) {
+                const auto [q16, k16, v16] = bf16(*q, *k, *v);
+                out = forward_only(rows16(q16), rows16(k16), rows16(v16), nullptr, nullptr, s, 0, 0);
+            }
         }
     }
     return THPVariable_Wrap(std::move(out));
@@ -412,7 +450,8 @@ PyObject* prefill_packed(PyObject*, PyObject* const* args, Py_ssize_t n) {
             out = PackedFn::apply(*q, *k, *v, *cu_q, *cu_k, max_q, max_k, causal, scale);
         } else {
             const Shape s{true, causal, (int)cu_q->numel() - 1, (int)q->size(1), (int)k->size(1), (int)max_q, (int)max_k, (int)q->size(2), scale};
-            out = forward_only(rows16(bf16(*q)), rows16(bf16(*k)), rows16(bf16(*v)), (const int32_t*)cu_q->data_ptr(), (const int32_t*)cu_k->data_ptr(), s,
+            const auto [q16, k16, v16] = bf16(*q, *k, *v);
+            out = forward_only(rows16(q16), rows16(k16), rows16(v16), (const int32_t*)cu_q->data_ptr(), (const int32_t*)cu_k->data_ptr(), s,
                                (int)window, (int)keep_first);
         }
     }

@@ -1070,45 +1070,46 @@ extern "C" int mi355_prefill_fwd_rounds(int Hq, int Hkv, int Sq, int Sk, int D, 
     return Hq == Hkv && Sq > 0 && Sk > 0 && Sq <= 256 && mask_mode != MI355_MASK_BOOL && prefill_short_takes(p, D);
 }
 
-extern "C" int mi355_prefill_fwd_lse_rounded(const void* q, const void* k, const void* v, void* out, float* lse, const int64_t q_strides[3],
-                                             const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
-                                             const int64_t lse_strides[2], int f32, void* q16, void* k16, void* v16, const int64_t q16_strides[3],
-                                             const int64_t k16_strides[3], const int64_t v16_strides[3], int B, int Hq, int Hkv, int Sq, int Sk, int D,
-                                             float softmax_scale, int mask_mode, void* stream) {
+// keep: for a backward, which reads the rounded operands and lse
+static int fwd_rounded(bool keep, const void* q, const void* k, const void* v, void* out, float* lse, const int64_t q_strides[3], const int64_t k_strides[3],
+                       const int64_t v_strides[3], const int64_t o_strides[3], const int64_t lse_strides[2], int f32, void* const rounded[3],
+                       const int64_t* const st16[3], int B, int Hq, int Hkv, int Sq, int Sk, int D, float softmax_scale, int mask_mode, void* stream) {
     const void* in[3] = {q, k, v};
-    void* rounded[3] = {q16, k16, v16};
-    const int64_t *st[3] = {q_strides, k_strides, v_strides}, *st16[3] = {q16_strides, k16_strides, v16_strides};
-    if (!q || !k || !v || !out || !lse || !q_strides || !k_strides || !v_strides || !o_strides || !lse_strides)
-        return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: null pointer argument");
+    const int64_t* st[3] = {q_strides, k_strides, v_strides};
+    if (!q || !k || !v || !out || !q_strides || !k_strides || !v_strides || !o_strides || (keep && (!lse || !lse_strides)))
+        return set_error(MI355_EINVAL, "prefill_fwd rounded: null pointer argument");
     if (f32 < 1 || f32 > 7 || B <= 0 || !(softmax_scale > 0.f) || !mi355_prefill_fwd_rounds(Hq, Hkv, Sq, Sk, D, mask_mode))
-        return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: no such form of this call (see mi355_prefill_fwd_rounds)");
+        return set_error(MI355_EINVAL, "prefill_fwd rounded: no such form of this call (see mi355_prefill_fwd_rounds)");
     PrefillParams p{};
     RoundedInputs r{};
     int64_t* own[3] = {p.qs, p.ks, p.vs};
     for (int i = 0; i < 3; ++i) {
         const bool wide = f32 >> i & 1;
-        if (wide && (!rounded[i] || !st16[i])) return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: nowhere to leave a rounded operand");
+        const bool leaves = wide && keep;
+        if (leaves && (!rounded[i] || !st16[i])) return set_error(MI355_EINVAL, "prefill_fwd rounded: nowhere to leave a rounded operand");
         for (int j = 0; j < 3; ++j) {
-            if (st[i][j] & 7 || (wide && st16[i][j] & 7) || o_strides[j] & 7)
-                return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: strides must be multiples of 8 elements");
+            if (st[i][j] & 7 || (leaves && st16[i][j] & 7) || o_strides[j] & 7)
+                return set_error(MI355_EINVAL, "prefill_fwd rounded: strides must be multiples of 8 elements");
             own[i][j] = st[i][j];
-            if (wide) r.strides[i][j] = st16[i][j];
+            if (leaves) r.strides[i][j] = st16[i][j];
             p.os[j] = o_strides[j];
         }
-        if (st[i][2] <= 0 || st[i][2] >= (1 << 24)) return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: row strides must be positive and below 2^24 elements");
-        if (((uintptr_t)in[i] | (uintptr_t)out | (wide ? (uintptr_t)rounded[i] : 0)) & 15)
-            return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: tensors must be 16-byte aligned");
+        if (st[i][2] <= 0 || st[i][2] >= (1 << 24)) return set_error(MI355_EINVAL, "prefill_fwd rounded: row strides must be positive and below 2^24 elements");
+        if (((uintptr_t)in[i] | (uintptr_t)out | (leaves ? (uintptr_t)rounded[i] : 0)) & 15)
+            return set_error(MI355_EINVAL, "prefill_fwd rounded: tensors must be 16-byte aligned");
         r.in[i] = wide ? (const float*)in[i] : nullptr;
-        r.out[i] = wide ? (__bf16*)rounded[i] : nullptr;
+        r.out[i] = leaves ? (__bf16*)rounded[i] : nullptr;
     }
-    if ((int64_t)B * Hq > 0x7fffffffLL) return set_error(MI355_EINVAL, "prefill_fwd_lse_rounded: too many workgroups");
+    if ((int64_t)B * Hq > 0x7fffffffLL) return set_error(MI355_EINVAL, "prefill_fwd rounded: too many workgroups");
     p.q = (const __bf16*)q;
     p.k = (const __bf16*)k;
     p.v = (const __bf16*)v;
     p.out = (__bf16*)out;
-    p.lse = lse;
-    p.ls[0] = lse_strides[0];
-    p.ls[1] = lse_strides[1];
+    if (keep) {
+        p.lse = lse;
+        p.ls[0] = lse_strides[0];
+        p.ls[1] = lse_strides[1];
+    }
     p.B = B;
     p.Hq = Hq;
     p.Hkv = Hkv;
@@ -1117,6 +1118,40 @@ extern "C" int mi355_prefill_fwd_lse_rounded(const void* q, const void* k, const
     p.scale_log2 = softmax_scale * kLog2e;
     p.mask_mode = mask_mode;
     const int rc = launch_prefill_short_rounded(p, r, D, (hipStream_t)stream);
+    return rc == 0 ? MI355_OK : set_error(rc, hipGetErrorString((hipError_t)rc));
+}
+
+extern "C" int mi355_prefill_fwd_lse_rounded(const void* q, const void* k, const void* v, void* out, float* lse, const int64_t q_strides[3],
+                                             const int64_t k_strides[3], const int64_t v_strides[3], const int64_t o_strides[3],
+                                             const int64_t lse_strides[2], int f32, void* q16, void* k16, void* v16, const int64_t q16_strides[3],
+                                             const int64_t k16_strides[3], const int64_t v16_strides[3], int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                                             float softmax_scale, int mask_mode, void* stream) {
+    void* const rounded[3] = {q16, k16, v16};
+    const int64_t* const st16[3] = {q16_strides, k16_strides, v16_strides};
+    return fwd_rounded(true, q, k, v, out, lse, q_strides, k_strides, v_strides, o_strides, lse_strides, f32, rounded, st16, B, Hq, Hkv, Sq, Sk, D, softmax_scale,
+                       mask_mode, stream);
+}
+
+extern "C" int mi355_prefill_fwd_rounded(const void* q, const void* k, const void* v, void* out, const int64_t q_strides[3], const int64_t k_strides[3],
+                                         const int64_t v_strides[3], const int64_t o_strides[3], int f32, int B, int Hq, int Hkv, int Sq, int Sk, int D,
+                                         float softmax_scale, int mask_mode, void* stream) {
+    return fwd_rounded(false, q, k, v, out, nullptr, q_strides, k_strides, v_strides, o_strides, nullptr, f32, nullptr, nullptr, B, Hq, Hkv, Sq, Sk, D,
+                       softmax_scale, mask_mode, stream);
+}
+
+extern "C" int mi355_round_operands(const float* const in[3], void* const out[3], const int64_t n[3], void* stream) {
+    if (!in || !out || !n) return set_error(MI355_EINVAL, "round_operands: null pointer argument");
+    __bf16* to[3];
+    int64_t total = 0;
+    for (int i = 0; i < 3; ++i) {
+        to[i] = (__bf16*)out[i];
+        if (!in[i]) continue;
+        if (!out[i] || n[i] < 0 || n[i] > 1LL << 32 || (((uintptr_t)in[i] | (uintptr_t)out[i]) & 15))
+            return set_error(MI355_EINVAL, "round_operands: an operand's elements, 16-byte aligned, and a place for them");
+        total += n[i];
+    }
+    if (total == 0) return MI355_OK;
+    const int rc = launch_round_operands(in, to, n, (hipStream_t)stream);
     return rc == 0 ? MI355_OK : set_error(rc, hipGetErrorString((hipError_t)rc));
 }
 

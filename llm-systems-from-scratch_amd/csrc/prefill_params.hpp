@@ -58,12 +58,19 @@ int launch_prefill_w64(const PrefillParams& p, hipStream_t stream);
 // Up to 256 keys at head sizes 32 and 64, dense layout: prefill_short.hip.
 bool prefill_short_takes(const PrefillParams& p, int D);
 int launch_prefill_short(const PrefillParams& p, int D, hipStream_t stream);
-// The same with fp32 among q, k and v: what is given here (else null) is read in place of p's and leaves rounded in bf16.
+// The same with fp32 among q, k and v: what is given here (else null) is read in place of p's and leaves rounded in bf16 where there is an out.
 struct RoundedInputs {
     const float* in[3];                   // with p's strides
     __bf16* out[3];
     int64_t strides[3][3];                // of out: batch, head, row
 };
+// Operands whose elements fill their memory
+struct RoundedOperands {
+    const float* in[3];
+    __bf16* out[3];
+    int64_t n[3], room[3];                // elements; rounded up to eight
+};
+int launch_round_operands(const float* const in[3], __bf16* const out[3], const int64_t n[3], hipStream_t stream);
 int launch_prefill_short_rounded(const PrefillParams& p, const RoundedInputs& r, int D, hipStream_t stream);
 
 // Small query tiles whose keys are dealt to a workgroup's wavefronts: prefill_keys.hip.  The plan: how many wavefronts, and about how long it takes.

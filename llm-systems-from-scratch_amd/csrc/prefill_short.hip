@@ -22,8 +22,8 @@ __device__ __forceinline__ u32x4 rounded8(const float* x) {
     return u32x4{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])};
 }
 
-// ROUND (a forward for training, one query tile, a key head per query head): fp32 operands are rounded on their way in, and what the backward
-// will read in bf16 leaves from here.  64 x 16 heads of 32, 256 tokens, fp32 Q and K: two conversions and this kernel without it 38 us, like this 29.
+// ROUND (one query tile, a key head per query head): fp32 operands are rounded on their way in, and what a backward will read in bf16 leaves from here.  64 x 16 heads of 32, 256 tokens, fp32 Q and K, without a backward: two conversions and this kernel without it 38.7 us, like
+// this 24.9; 8 x 32 heads, 128 tokens 15.3 / 5.7; 64 x 16 heads of 64, 256 tokens 69.7 / 49.2.
 template <int D, bool CAUSAL, bool ROUND>
 __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(PrefillParams p, int n_qtiles, int chunk, RoundedInputs r) {
     using R = TileReads<D>;
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(Pre
         };
         const auto bring_rounded = [&](int which, const int64_t (&st)[3], unsigned char* tile) {
             const float* in = r.in[which] + b * st[0] + hk * st[1] + (int64_t)(64 * wave) * st[2];
-            __bf16* out = r.out[which] + b * r.strides[which][0] + hk * r.strides[which][1] + (int64_t)(64 * wave) * r.strides[which][2];
+            __bf16* out = r.out[which] ? r.out[which] + b * r.strides[which][0] + hk * r.strides[which][1] + (int64_t)(64 * wave) * r.strides[which][2] : nullptr;
             u32x4 x[CPR];
 #pragma unroll
             for (int j = 0; j < CPR; ++j) {
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(Pre
             for (int j = 0; j < CPR; ++j) {
                 const int idx = 64 * j + lane, row = idx / CPR, c = idx % CPR;
                 *reinterpret_cast<u32x4*>(tile + row * kRow + ((c ^ swz<D>(row)) << 4)) = x[j];
-                if (row <= last) *reinterpret_cast<u32x4*>(out + row * r.strides[which][2] + c * 8) = x[j];
+                if (out && row <= last) *reinterpret_cast<u32x4*>(out + row * r.strides[which][2] + c * 8) = x[j];
             }
         };
         if (!ROUND || !r.in[2]) bring(vt, p.vs[2], v_dst);
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(Pre
                 const int64_t at = (int64_t)qi * p.qs[2] + 16 * s + 8 * kg;
                 if (ROUND && r.in[0]) {
                     a = rounded8(r.in[0] + b * p.qs[0] + h * p.qs[1] + at);
-                    *reinterpret_cast<u32x4*>(r.out[0] + b * r.strides[0][0] + h * r.strides[0][1] + qi * r.strides[0][2] + 16 * s + 8 * kg) = a;
+                    if (r.out[0]) *reinterpret_cast<u32x4*>(r.out[0] + b * r.strides[0][0] + h * r.strides[0][1] + qi * r.strides[0][2] + 16 * s + 8 * kg) = a;
                 } else {
                     a = *reinterpret_cast<const u32x4*>(qb + at);
                 }
@@ -203,6 +203,34 @@ __global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(Pre
                 }
         }
     }
+}
+
+// fp32 operands of a prefill as bf16, up to three in one launch, in their order in memory; 8 elements a thread.  Bound by bytes, and by the launch where they are few.  Whole call with
+// fp32 Q and K, us, a library conversion each / this: 2 x 4 heads of 128, 177 tokens 14.9 / 10.1, 22 x 8 heads, 221 tokens 28.7 / 26.5, 4 x 16 heads of 64, 600 tokens 25.1 / 22.3,
+// 8 x 16 heads of 128, 2000 tokens 203 / 201.
+__global__ __launch_bounds__(256) void round_operands_kernel(RoundedOperands r) {
+    int64_t at = 8 * (blockIdx.x * 256LL + threadIdx.x);
+    int i = 0;
+    while (i < 2 && at >= r.room[i]) at -= r.room[i++];
+    if (at + 8 <= r.n[i]) {
+        *reinterpret_cast<u32x4*>(r.out[i] + at) = rounded8(r.in[i] + at);
+    } else {
+        for (; at < r.n[i]; ++at) r.out[i][at] = (__bf16)r.in[i][at];
+    }
+}
+
+int launch_round_operands(const float* const in[3], __bf16* const out[3], const int64_t n[3], hipStream_t s) {
+    RoundedOperands r{};
+    int64_t total = 0;
+    for (int i = 0; i < 3; ++i) {
+        r.in[i] = in[i];
+        r.out[i] = out[i];
+        r.n[i] = in[i] ? n[i] : 0;
+        r.room[i] = (r.n[i] + 7) / 8 * 8;
+        total += r.room[i];
+    }
+    hipLaunchKernelGGL(round_operands_kernel, dim3((unsigned)((total / 8 + 255) / 256)), dim3(256), 0, s, r);
+    return (int)hipGetLastError();
 }
 
 // Without a mask every block sees every key, and what is saved around the tiles no longer pays for the row maxima at 256 keys (64 x

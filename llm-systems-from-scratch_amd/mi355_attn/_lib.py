@@ -30,6 +30,8 @@ EXPORTS = (
     "mi355_prefill_fwd_lse",
     "mi355_prefill_fwd_rounds",
     "mi355_prefill_fwd_lse_rounded",
+    "mi355_prefill_fwd_rounded",
+    "mi355_round_operands",
     "mi355_prefill_bwd",
     "mi355_prefill_fwd_mask_lse",
     "mi355_prefill_bwd_mask",
@@ -152,6 +154,10 @@ def load():
     lib.mi355_prefill_fwd_lse_rounded.restype = i32
     lib.mi355_prefill_fwd_lse_rounded.argtypes = [vp] * 5 + [_i64x3] * 4 + [_i64x2, i32, vp, vp, vp, _i64x3, _i64x3, _i64x3,
                                                                           i32, i32, i32, i32, i32, i32, f32, i32, vp]
+    lib.mi355_prefill_fwd_rounded.restype = i32
+    lib.mi355_prefill_fwd_rounded.argtypes = [vp] * 4 + [_i64x3] * 4 + [i32, i32, i32, i32, i32, i32, i32, f32, i32, vp]
+    lib.mi355_round_operands.restype = i32
+    lib.mi355_round_operands.argtypes = [vp * 3, vp * 3, _i64x3, vp]
     lib.mi355_prefill_bwd.restype = i32
     lib.mi355_prefill_bwd.argtypes = [vp] * 10 + [_i64x3] * 8 + [_i64x2, vp, vp,
                                                                  i32, i32, i32, i32, i32, i32, f32, i32, i32, vp]
