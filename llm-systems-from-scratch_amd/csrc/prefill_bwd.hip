@@ -739,17 +739,24 @@ struct PlanParams {
     int k_room, q_room, ds_room;  // entries and blocks (of one head) there is room for
     int most_q, most_k;           // lengths up to which every sequence has its blocks
     int shift, n_bins;            // costs in steps are binned by cost >> shift
+    int k_width, q_width;         // of plan_list
     int total_q;
 };
 
-// One list: entries (b, i), i < n(b), of cost(b, i) < n_bins << shift.  A wavefront per sequence, its lanes over the entries.
+// What the plan holds in LDS.  Every workgroup of the launch has that much, so it is what this batch takes, not what the largest would (41 KB, three workgroups per compute
+// unit): 46 sequences of 298 tokens 13.0 -> 12.3 us.
+inline size_t plan_lds_bytes(const PlanParams& plan, int B) { return 4 * ((size_t)plan.n_bins + kPlanThreads / 64 + 2 * (size_t)B); }
+
+// One list: entries (b, i), i < n(b), of cost(b, i) < n_bins << shift.  `width` lanes (a power of two up to 64) per sequence, over its entries: as many as the longest
+// promised sequence has, so that a batch of short ones is a few rounds of the workgroup (46 sequences of
+// 298 tokens, a wavefront each 12.3 us of the launch, like this 8.4).
 template <class N, class Cost>
-__device__ __forceinline__ int plan_list(int* bins, int* sums, int n_bins, int B, int shift, int2* out, int room, N n_of, Cost cost) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__device__ __forceinline__ int plan_list(int* bins, int* sums, int n_bins, int B, int shift, int width, int2* out, int room, N n_of, Cost cost) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, b0 = tid / width, i0 = tid % width, step = kPlanThreads / width;
     for (int i = tid; i < n_bins; i += kPlanThreads) bins[i] = 0;
     __syncthreads();
-    for (int b = wave; b < B; b += kPlanThreads / 64)
-        for (int i = lane, n = n_of(b); i < n; i += 64) atomicAdd(&bins[min(cost(b, i) >> shift, n_bins - 1)], 1);
+    for (int b = b0; b < B; b += step)
+        for (int i = i0, n = n_of(b); i < n; i += width) atomicAdd(&bins[min(cost(b, i) >> shift, n_bins - 1)], 1);
     __syncthreads();
     // where a bin's entries begin: the sum of the dearer bins
     int total = 0;
@@ -766,8 +773,8 @@ __device__ __forceinline__ int plan_list(int* bins, int* sums, int n_bins, int B
         if (bin >= 0) bins[bin] = at;
         __syncthreads();
     }
-    for (int b = wave; b < B; b += kPlanThreads / 64)
-        for (int i = lane, n = n_of(b); i < n; i += 64) {
+    for (int b = b0; b < B; b += step)
+        for (int i = i0, n = n_of(b); i < n; i += width) {
             const int pos = atomicAdd(&bins[min(cost(b, i) >> shift, n_bins - 1)], 1);
             if (pos < room) out[pos] = int2{b, i};
         }
@@ -782,7 +789,8 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
     int bid = blockIdx.x;
     if (p.cu_q) {
         if (bid < 2) {
-            __shared__ int bins[kPlanBins], sums[kPlanThreads / 64], lens_q[kPlanSeqs], lens_k[kPlanSeqs];
+            extern __shared__ int plan_lds[];     // plan_lds_bytes
+            int *bins = plan_lds, *sums = bins + plan.n_bins, *lens_q = sums + kPlanThreads / 64, *lens_k = lens_q + p.B;
             const int G = p.Hq / p.Hkv;
             for (int b = tid; b < p.B; b += kPlanThreads) {
                 lens_q[b] = max(p.cu_q[b + 1] - p.cu_q[b], 0);
@@ -791,7 +799,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
             __syncthreads();
             const auto row_tiles = [&](int b) { return (lens_q[b] + kBwRows - 1) / kBwRows; };
             if (bid == 0) {
-                const int n = plan_list(bins, sums, plan.n_bins, p.B, plan.shift, plan.k_jobs, plan.k_room,
+                const int n = plan_list(bins, sums, plan.n_bins, p.B, plan.shift, plan.k_width, plan.k_jobs, plan.k_room,
                                         [&](int b) { return (lens_k[b] + kFuCols - 1) / kFuCols; },
                                         [&](int b, int i) {
                                             const int skip = CAUSAL ? max(0, i * kFuCols - (lens_k[b] - lens_q[b])) / kBwRows : 0;
@@ -824,7 +832,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
                     }
                 }
             }
-            const int n = plan_list(bins, sums, plan.n_bins, p.B, plan.shift, plan.q_jobs, plan.q_room,
+            const int n = plan_list(bins, sums, plan.n_bins, p.B, plan.shift, plan.q_width, plan.q_jobs, plan.q_room,
                                     [&](int b) { return (row_tiles(b) * G + kDqWaves - 1) / kDqWaves; },
                                     [&](int b, int i) {
                                         return DsLayout(lens_q[b], lens_k[b], CAUSAL).count(min(row_tiles(b) * G - 1, kDqWaves * (i + 1) - 1) / G) >> 1;
@@ -842,6 +850,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
     const __bf16* o = p.out + (p.cu_q ? 0 : (int64_t)b * p.os[0]) + (int64_t)r * p.os[2] + 8 * part;
     const __bf16* g = p.dout + (p.cu_q ? 0 : (int64_t)b * p.dos[0]) + (int64_t)r * p.dos[2] + 8 * part;
     float* out = p.delta + (p.cu_q ? 0 : (int64_t)b * p.ls[0]) + r;
+    const uint32_t sign = p.wide ? 0x80000000u : 0u;
     u32x4 x[kHeads], y[kHeads];
 #pragma unroll
     for (int i = 0; i < kHeads; ++i) {
@@ -857,7 +866,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
         for (int e = 0; e < 8; ++e) sum += (float)o8[e] * (float)g8[e];
 #pragma unroll
         for (int m = kLanes / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
-        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = p.wide ? -sum : sum;
+        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ sign);
     }
 }
 
@@ -1452,6 +1461,13 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
         const int most = std::max(p.Sq, p.Sk) / kBwRows + 1;                      // (costs count row tiles, or pairs of dS blocks)
         while (most >> plan.shift >= kPlanBins) ++plan.shift;
         plan.n_bins = (most >> plan.shift) + 1;
+        const auto width = [](int64_t entries) {
+            int w = 1;
+            while (w < 64 && w < entries) w *= 2;
+            return w;
+        };
+        plan.k_width = width((p.Sk + kFuCols - 1) / kFuCols);
+        plan.q_width = width(((p.Sq + kBwRows - 1) / kBwRows * (int64_t)(p.Hq / p.Hkv) + kDqWaves - 1) / kDqWaves);
         plan.total_q = (int)total_q;
         p.n_jobs = plan.n_jobs;
         p.ds_base = plan.ds_base;
@@ -1474,7 +1490,7 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
     // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
     const double row_tiles = (double)(p.cu_q ? total_q : (int64_t)p.B * p.Sq) / kBwRows / p.B;
     p.wide = D == 128 && row_tiles * G * (MODE == MI355_MASK_CAUSAL ? 0.5 : 1.0) >= 15.0 * p.shares;
-    hipLaunchKernelGGL((bwd_delta_kernel<D, MODE>), dim3((unsigned)delta_wgs), dim3(kPlanThreads), 0, stream, p, plan);
+    hipLaunchKernelGGL((bwd_delta_kernel<D, MODE>), dim3((unsigned)delta_wgs), dim3(kPlanThreads), p.cu_q ? plan_lds_bytes(plan, p.B) : 0, stream, p, plan);
     for (p.unit0 = 0; p.unit0 < d.n_units; p.unit0 += p.n_units) {
         p.n_units = std::min(d.units_per_pass, d.n_units - p.unit0);
         const dim3 grid((unsigned)(k_jobs * p.n_units * p.shares));
