@@ -361,12 +361,12 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
 //                                               86 / 75 / 78                78 / 72 / 73                 222 / 215 / 222
 //                                               2640 x 1024, 32 of 512, 4   4108 x 1024, 16 of 1024, 4   2609 x 2048, 8 of 1024, 1
 //                                               97 / 90 / 88                173 / 167 / 188              84 / 82 / 104
-// apart: the workgroups of an XCD begin 0, 1, 2 or 3 times so many steps of k in.  Rows of whole 4096 bytes from step 0 on all want the same channels of its L2 (turn_of), and
+// TURN: the workgroups of an XCD begin 0, 8, 16 or 24 steps of k in.  Rows of whole 4096 bytes from step 0 on all want the same channels of its L2 (turn_of), and
 // weights that come from HBM wait for these: 32 experts of 2048 x 2048, 64 pairs an expert 200 -> 154 us, 16 of 2048 x 1024 32 pairs 54.5 -> 45.7, 128 pairs 78.1 -> 77.1,
 // 8 of 2048 x 2048 75 pairs 66 -> 56, 250 pairs 103.9 / 104.2.  Where an expert's row tiles share its weights in the L2 their steps had better go together, so
 // not behind 256 pairs an expert, and not in the 256 x 256 tiles (396 -> 399 to 409).
-template <bool GATE_UP>
-__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int chunk, int apart) {
+template <bool GATE_UP, bool TURN>
+__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int chunk) {
     constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2, NA = 2, NW = 3;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[(NA + NW) * kTile];          // rows, then w
     int n_tile, e, first, end;
@@ -386,8 +386,8 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
         w_off[j] = (uint32_t)((wr * p.k + piece * 8) * 2);
     }
     const uint32_t lds0 = lds_address(lds);
-    const int n_steps = p.k / BK, turn = blockIdx.x / 8 % 4 * apart;
-    const auto turned = [&](int step) { return (step + turn >= n_steps ? step + turn - n_steps : step + turn) * BK; };
+    const int n_steps = p.k / BK, turn = TURN ? blockIdx.x / 8 % 4 * 8 : 0;
+    const auto turned = [&](int step) { return (TURN && step + turn >= n_steps ? step + turn - n_steps : step + turn) * BK; };
     const auto issue_a = [&](int step, int slot) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) dma_to_lds_16(a_base + turned(step), a_off[j], lds0 + slot * kTile + (32 * wave + 8 * j) * 128);
@@ -1037,7 +1037,8 @@ static int launch_moe(const MoeParams& p, int dtype, int tiling, hipStream_t s) 
     const int chunk = n_tiles * std::max(1, (wide ? 32 : 64) / n_tiles);
     if (dtype == MI355_FP32) hipLaunchKernelGGL(moe_f32_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     else if (wide) hipLaunchKernelGGL(moe_wide_kernel<GATE_UP>, dim3((unsigned)(n_tiles * m_tiles + 384)), block, 0, s, p, n_tiles, chunk);
-    else if (large) hipLaunchKernelGGL(moe_gemm_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, chunk, turn_pays(p.k) && p.n_pairs <= 256LL * p.E ? 8 : 0);
+    else if (large && turn_pays(p.k) && p.n_pairs <= 256LL * p.E) hipLaunchKernelGGL((moe_gemm_kernel<GATE_UP, true>), grid, block, 0, s, p, n_tiles, chunk);
+    else if (large) hipLaunchKernelGGL((moe_gemm_kernel<GATE_UP, false>), grid, block, 0, s, p, n_tiles, chunk);
     else hipLaunchKernelGGL(moe_skinny_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     return (int)hipGetLastError();
 }

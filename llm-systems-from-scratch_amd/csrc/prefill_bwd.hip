@@ -1484,12 +1484,12 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
     const int64_t q_jobs = p.cu_q ? d.q_room : ((int64_t)(p.Sq + kBwRows - 1) / kBwRows * G + kDqWaves - 1) / kDqWaves;
     if (delta_wgs > 0x7fffffffLL || k_jobs * d.units_per_pass * d.shares > 0x7fffffffLL || q_jobs * d.units_per_pass > 0x7fffffffLL)
         return (int)hipErrorInvalidValue;
-    // Key tiles with fifteen steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
+    // Key tiles with sixteen steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
     // 56 / 70; 4 x 602, 16 heads (5) 32 / 37; 16 x 920 (7) 231 / 243; 4 packed of 324 to 5199, 4 / 2 heads, 4 shares (11) 116 / 120; 51 packed of 1701, one head (13) all kernels
-    // 258 / 262; 2 x 2048, 32 heads (16) 186 / 175; 3000
+    // 258 / 262; 21 packed of 995, 16 / 8 (15.5) all kernels 548 / 554; 2 x 2048, 32 heads (16) 186 / 175; 3000
     // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
     const double row_tiles = (double)(p.cu_q ? total_q : (int64_t)p.B * p.Sq) / kBwRows / p.B;
-    p.wide = D == 128 && row_tiles * G * (MODE == MI355_MASK_CAUSAL ? 0.5 : 1.0) >= 15.0 * p.shares;
+    p.wide = D == 128 && row_tiles * G * (MODE == MI355_MASK_CAUSAL ? 0.5 : 1.0) >= 16.0 * p.shares;
     hipLaunchKernelGGL((bwd_delta_kernel<D, MODE>), dim3((unsigned)delta_wgs), dim3(kPlanThreads), p.cu_q ? plan_lds_bytes(plan, p.B) : 0, stream, p, plan);
     for (p.unit0 = 0; p.unit0 < d.n_units; p.unit0 += p.n_units) {
         p.n_units = std::min(d.units_per_pass, d.n_units - p.unit0);

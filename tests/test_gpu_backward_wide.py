@@ -1,4 +1,4 @@
-"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with fifteen steps and more on average) against the form without dS in memory: rows and keys
+"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with sixteen steps and more on average) against the form without dS in memory: rows and keys
 around the tiles of 64 and 128 and their halves, a tile of rows that is the sequence's only one, wavefronts without keys or rows, more queries than keys
 and the other way round, one to many steps, shares, fp32 gradients, several passes.  Tolerance of test_gpu_backward.py: one rounding of the result over a tensor."""
 import pytest
@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("lens_q,lens_k,Hq,Hkv,causal", [
-    ([1, 900, 33, 0, 700, 64, 65], None, 8, 1, True), ([31, 32, 33, 1800, 97, 95, 96], None, 16, 2, True), ([1500, 1, 129, 1023], [1600, 300, 64, 900], 6, 2, True),
-    ([800, 1, 63, 900], [129, 64, 1, 127], 3, 1, False), ([1000, 2000], [40, 2100], 4, 4, True), ([700, 900, 64], [66, 193, 32], 4, 2, False),
+    ([1, 900, 33, 0, 830, 64, 65], None, 8, 1, True), ([31, 32, 33, 1800, 97, 95, 96], None, 16, 2, True), ([1700, 1, 129, 1023], [1800, 300, 64, 900], 6, 2, True),
+    ([800, 1, 63, 900], [129, 64, 1, 127], 3, 1, False), ([2100, 2000], [40, 2100], 4, 4, True), ([700, 900, 64], [66, 193, 32], 4, 2, False),
     ([2113] * 5, None, 12, 12, True)])
 def test_wide_packed(ops, monkeypatch, lens_q, lens_k, Hq, Hkv, causal):  # noqa: F811
     print(f"case: wide packed {lens_q} {lens_k} {Hq}/{Hkv} {causal}", flush=True)
