@@ -850,7 +850,6 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
     const __bf16* o = p.out + (p.cu_q ? 0 : (int64_t)b * p.os[0]) + (int64_t)r * p.os[2] + 8 * part;
     const __bf16* g = p.dout + (p.cu_q ? 0 : (int64_t)b * p.dos[0]) + (int64_t)r * p.dos[2] + 8 * part;
     float* out = p.delta + (p.cu_q ? 0 : (int64_t)b * p.ls[0]) + r;
-    const uint32_t sign = p.wide ? 0x80000000u : 0u;
     u32x4 x[kHeads], y[kHeads];
 #pragma unroll
     for (int i = 0; i < kHeads; ++i) {
@@ -866,7 +865,7 @@ __global__ __launch_bounds__(kPlanThreads) void bwd_delta_kernel(BwdParams p, Pl
         for (int e = 0; e < 8; ++e) sum += (float)o8[e] * (float)g8[e];
 #pragma unroll
         for (int m = kLanes / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
-        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) ^ sign);
+        if (part == 0 && h0 + i < p.Hq) out[(int64_t)(h0 + i) * p.ls[1]] = sum;
     }
 }
 

@@ -44,7 +44,7 @@ struct BwdParams {
     int shares;
     float* part;
     int64_t part_rows;
-    bool wide;                    // bwd_dkv_wide_kernel, which reads -delta
+    bool wide;                    // dK, dV and dS by bwd_dkv_wide_kernel
 };
 
 // Gradients leave in bf16, or in fp32 for an fp32 input: the sums as they are, where a conversion behind the kernel would

@@ -81,7 +81,9 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
     const int kw0 = k0 + 64 * keys;
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_address(lds));
 
-    bf16x8 kf[2][NS], vf[2][NS];                         // K and V of this lane's keys kw0 + 32 c + n: step s covers d = 16 s + 8 kg + j
+    // K and -V of this lane's keys kw0 + 32 c + n: step s covers d = 16 s + 8 kg + j.  (With -V the C operand of dP is delta as it is: the products give delta - dP, and the
+    // sign that dS needs is a modifier of its multiplication.)
+    bf16x8 kf[2][NS], vf[2][NS];
     f32x16 dk[2][NDT], dv[2][NDT];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
@@ -101,11 +103,13 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
     const int my_steps = __builtin_amdgcn_readfirstlane(steps_from(kw0, kWdRows * rows + kWdRows - 1));
 
     // ---- what a step is: worked out 32 steps at a time, a lane each, and kept in LDS ----
-    // (addresses of the tiles of Q and dO | of lse (keys 0) or -delta, and of this wavefront's dS blocks | its first row, whether rows or keys are masked, how
+    // (addresses of the tiles of Q and dO | of lse (keys 0) or delta, and of this wavefront's dS blocks | its first row, whether rows or keys are masked, how
     // many of its two blocks some row sees | the lanes that request it: none for steps past the end, so that a step is always as many instructions)
     const bool ragged = r_top + kBwRows > sq;
     const DsLayout dsl(sq, sk, CAUSAL);
     const auto describe = [&](int from) __attribute__((always_inline)) {
+        int G = p.Hq / p.Hkv;
+        asm volatile("" : "+s"(G));                  // (a reciprocal worked out here, not held in a register over the steps)
         const int lane = lane_here() & 31, t = min(from + lane, n_steps - 1), tile = t / G, head = t - tile * G, r = r_top - tile * apart, first = r + kWdRows * rows;
         const int ds_blocks = dsl.before(n_tiles), most = CAUSAL ? min(sk - 1, r + kBwRows - 1 + coff) : sk - 1;
         const __bf16* q = p.q + base_of(p.qs, q_start, hk * G) + head * p.qs[1] + r * p.qs[2];
@@ -130,7 +134,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
     };
 
     // ---- requests ----
-    // Requests 2 i and 2 i + 1 of this wavefront bring rows 16 wave + 4 i + lane / 16 of the tiles of Q and dO, the last one 64 of lse or -delta
+    // Requests 2 i and 2 i + 1 of this wavefront bring rows 16 wave + 4 i + lane / 16 of the tiles of Q and dO, the last one 64 of lse or delta
     uint64_t q_from = 0, do_from = 0, row_from = 0;      // of the step that is requested
     const auto aim = [&](const u32x4& tiles, const u32x2& row) {
         q_from = scalar64(tiles[0], tiles[1]);
@@ -231,9 +235,9 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
         // word w & 3 of rows u = w / 4 & 1 of keys c = w / 8
         const auto pack_p = [&](int w) { pw[w >> 3][(w >> 2) & 1][w & 3] = pack_bf16_here(s[w >> 3][2 * (w & 7)], s[w >> 3][2 * (w & 7) + 1]); };
         const auto make_ds = [&](int w) {
-            dsw[w >> 3][(w >> 2) & 1][w & 3] = pack_bf16_here(s[w >> 3][2 * (w & 7)] * dp[w >> 3][2 * (w & 7)], s[w >> 3][2 * (w & 7) + 1] * dp[w >> 3][2 * (w & 7) + 1]);
+            dsw[w >> 3][(w >> 2) & 1][w & 3] = pack_bf16_here(s[w >> 3][2 * (w & 7)] * -dp[w >> 3][2 * (w & 7)], s[w >> 3][2 * (w & 7) + 1] * -dp[w >> 3][2 * (w & 7) + 1]);
         };
-        const auto read_minus_delta = [&](int g) {
+        const auto read_delta = [&](int g) {
             const f32x4 d4 = lds_load_at<f32x4>(rows_at + 256 + 32 * g);
 #pragma unroll
             for (int r = 0; r < 4; ++r) c0[4 * g + r] = d4[r];
@@ -313,7 +317,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
 #pragma unroll
             for (int e = 0; e < 32; ++e) scale_s(e);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) read_minus_delta(g);
+            for (int g = 0; g < 4; ++g) read_delta(g);
         } else {
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
                         flags = read_flags(step);
                     }
                     if (m == 12) go_on(block_at, flags);
-                    if (m >= 8 && m < 12) read_minus_delta(m - 8);
+                    if (m >= 8 && m < 12) read_delta(m - 8);
                 }
                 fence();
             }
@@ -349,7 +353,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
         if constexpr (!LAST) {
             mask();
             fence();
-            // ---- dP - delta; P ----
+            // ---- delta - dP; P ----
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
                 const int i = m >> 1, c = m & 1;
@@ -432,7 +436,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
             for (int s = 0; s < NS; ++s) {
                 const uint32_t at = lds0 + (2 + keys) * kTile + c * (kTile / 2);
                 kf[c][s] = as_bf16x8(read_row(at, s));
-                vf[c][s] = as_bf16x8(read_row(at + kWdRing * kTile, s));
+                vf[c][s] = as_bf16x8(read_row(at + kWdRing * kTile, s) ^ 0x80008000u);
             }
         __syncthreads();
         if (my_steps > 0) {

@@ -2,7 +2,9 @@
 around the tiles of 64 and 128 and their halves, a tile of rows that is the sequence's only one, wavefronts without keys or rows, more queries than keys
 and the other way round, one to many steps, shares, fp32 gradients, several passes.  Tolerance of test_gpu_backward.py: one rounding of the result over a tensor."""
 import pytest
+import torch
 
+from mi355_attn import ops as inner
 from test_gpu_backward import _both_forms, _same_gradients, ops  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -29,3 +31,28 @@ def test_wide_dense(ops, monkeypatch, B, Hq, Hkv, Sq, Sk, causal, f32):  # noqa:
 def test_wide_in_passes(ops, monkeypatch, packed):  # noqa: F811
     print(f"case: wide in passes {packed}", flush=True)
     _same_gradients(*_both_forms(ops, monkeypatch, [1000] * 3, [1000] * 3, 28, 14, True, packed, workspace_part=0.45))
+
+
+@pytest.mark.parametrize("packed,lens,Hq,Hkv", [(True, [2113] * 5, 12, 12), (True, [300, 31, 1], 4, 2), (False, [200] * 3, 8, 2)])
+def test_delta_is_what_the_header_says(ops, monkeypatch, packed, lens, Hq, Hkv):  # noqa: F811
+    """rowsum(dout * out) in the caller's tensor, whichever kernel reads it: within the rounding of its fp32 sum of 128 products."""
+    from mi355_attn import _lib
+    print(f"case: delta {packed} {lens} {Hq}/{Hkv}", flush=True)
+    lib, seen = _lib.load(), []
+    real, real_backward = lib.mi355_prefill_bwd_ds, inner._prefill_backward
+
+    def backward(q, k, v, out, dout, lse, *rest, **kw):
+        delta = torch.full_like(lse, float("nan"))
+        monkeypatch.setattr(lib, "mi355_prefill_bwd_ds", lambda *a: real(*a[:6], delta.data_ptr(), *a[7:]))
+        grads = real_backward(q, k, v, out, dout, lse, *rest, **kw)
+        seen.append((delta, out, dout))
+        return grads
+
+    monkeypatch.setattr(inner, "_prefill_backward", backward)
+    _both_forms(ops, monkeypatch, lens, lens, Hq, Hkv, True, packed)
+    delta, out, dout = seen[0]                                           # (the first form is the one with dS in memory)
+    products = out.double() * dout.double()
+    want, size = products.sum(-1), products.abs().sum(-1)
+    if packed:
+        want, size = want.T, size.T
+    assert bool(((delta.double() - want).abs() <= 128 * 2 ** -24 * size).all())
