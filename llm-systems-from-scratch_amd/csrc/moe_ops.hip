@@ -361,7 +361,7 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
 //                                               86 / 75 / 78                78 / 72 / 73                 222 / 215 / 222
 //                                               2640 x 1024, 32 of 512, 4   4108 x 1024, 16 of 1024, 4   2609 x 2048, 8 of 1024, 1
 //                                               97 / 90 / 88                173 / 167 / 188              84 / 82 / 104
-// TURN: the workgroups of an XCD begin 0, 8, 16 or 24 steps of k in.  Rows of whole 4096 bytes from step 0 on all want the same channels of its L2 (turn_of), and
+// TURN: the workgroups of an XCD begin 0, 8, 16 or 24 steps of k in, by their columns and expert, so that a row's sums do not depend on the tile it falls into.  Rows of whole 4096 bytes from step 0 on all want the same channels of its L2 (turn_of), and
 // weights that come from HBM wait for these: 32 experts of 2048 x 2048, 64 pairs an expert 200 -> 154 us, 16 of 2048 x 1024 32 pairs 54.5 -> 45.7, 128 pairs 78.1 -> 77.1,
 // 8 of 2048 x 2048 75 pairs 66 -> 56, 250 pairs 103.9 / 104.2.  Where an expert's row tiles share its weights in the L2 their steps had better go together, so
 // not behind 256 pairs an expert, and not in the 256 x 256 tiles (396 -> 399 to 409).
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_til
         w_off[j] = (uint32_t)((wr * p.k + piece * 8) * 2);
     }
     const uint32_t lds0 = lds_address(lds);
-    const int n_steps = p.k / BK, turn = TURN ? blockIdx.x / 8 % 4 * 8 : 0;
+    const int n_steps = p.k / BK, turn = TURN ? (e * n_tiles + n_tile) % 4 * 8 : 0;
     const auto turned = [&](int step) { return (TURN && step + turn >= n_steps ? step + turn - n_steps : step + turn) * BK; };
     const auto issue_a = [&](int step, int slot) {
 #pragma unroll
@@ -846,7 +846,7 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
     // none would read weights for nothing (one in seven at two).  Us of router, experts and norm, without / with: 16 experts of 2048 x 1024, top
     // 4, 8 tokens 51.2 / 49.9, 16 57.4 / 55.7, 32 59.8 / 58.0; at 16 pairs an expert, where most take two row tiles and one step
     // at a time, 73.9 / 74.1.
-    const int turn = TURN ? turn_of(p.k, 4) : 0;
+    const int turn = TURN ? turn_of(p.k, 4, e * n_tiles + (int)(blockIdx.x % n_tiles)) : 0;     // (an expert's columns: whichever pairs it has)
     const bool ahead = !FEW && p.n_pairs >= 2 * p.E && p.n_pairs < 16 * p.E;
     int n_rows = 0;
     if constexpr (FEW) {

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
     float sq[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) sq[m] = 0.f;
-    weight_stream<MT, WAVES, kRing, TURN>(p.w, w_off, p.x, x_off, p.k, TURN ? turn_of(p.k, WAVES) : 0, wave, ring + wave * kRing, acc, [&] {
+    weight_stream<MT, WAVES, kRing, TURN>(p.w, w_off, p.x, x_off, p.k, TURN ? turn_of(p.k, WAVES, (int)blockIdx.x) : 0, wave, ring + wave * kRing, acc, [&] {
         if constexpr (NORM) {
             for (int c = tid; c < (p.k + 63) / 64 * 64; c += 64 * WAVES) norm_l[c] = c < p.k ? p.norm[c] : 0.f;
             __syncthreads();

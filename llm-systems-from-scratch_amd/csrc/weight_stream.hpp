@@ -22,7 +22,8 @@ constexpr int kStreamBytes = 12 * 1024;
 // time: 16 experts of 2048 x 1024, 32 tokens 44.0 us, 5.1 TB/s with the steps begun somewhere else by every one of an XCD's workgroups (every eighth of a launch) 39.5.  The same
 // beginning within an XCD and another on each other one gives nothing (45.0); nor does any with rows of 2048 bytes (24.3 / 25.1), which have two sets of channels.
 inline bool turn_pays(int k) { return k % 2048 == 0; }
-__device__ __forceinline__ int turn_of(int k, int waves) { return (int)(blockIdx.x / 8 * waves) % (k / 64); }
+// (at: the workgroup among those that read other weights, so that a row's sums do not depend on what else the launch has)
+__device__ __forceinline__ int turn_of(int k, int waves, int at) { return at / 8 * waves % (k / 64); }
 
 // The weights of a wavefront's first step, requested while the rows are still being looked for (slot 0 begins with them, whatever MT);
 // k a multiple of 64.

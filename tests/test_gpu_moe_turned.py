@@ -26,6 +26,25 @@ def test_large_tiles_of_whole_pages(T, E, top, k, ff, n):
     _products(T, E, top, k, ff, n, "large")
 
 
+@pytest.mark.parametrize("tiling,T,E,top,k,ff,n", [("direct", 32, 33, 1, 2048, 960, 72), ("direct", 15, 40, 2, 64, 2048, 2000), ("direct", 70, 4, 2, 2048, 192, 72), ("large", 400, 2, 1, 2048, 2048, 136),
+                                                   ("large", 700, 3, 1, 4096, 192, 2048)])
+def test_a_tokens_result_does_not_depend_on_its_place(tiling, T, E, top, k, ff, n):
+    """The same tokens in another order, so that a token's pair, row tile and workgroup are others: the same bits."""
+    import mi355_attn as ma
+    print(f"case: place {tiling} {T} {E} {top} {k} {ff} {n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+
+    def t(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g, device="cuda") * std).bfloat16()
+
+    h, up, down = t(T, k), t(E, 2 * ff, k, std=k ** -0.5), t(E, n, ff, std=ff ** -0.5)
+    ids = torch.rand(T, E, generator=g, device="cuda").argsort(-1)[:, :top].to(torch.int32).contiguous()
+    weights, perm = torch.rand(T, top, generator=g, device="cuda"), torch.randperm(T, generator=g, device="cuda")
+    here = ma.moe_experts(h, ids, weights, up, down, tiling=tiling).view(T, top, n)
+    there = ma.moe_experts(h[perm], ids[perm], weights[perm], up, down, tiling=tiling).view(T, top, n)
+    assert torch.equal(there, here[perm])
+
+
 def _products(T, E, top, k, ff, n, tiling):
     import mi355_attn as ma
     print(f"case: {tiling} {T} {E} {top} {k} {ff} {n}", flush=True)
