@@ -41,7 +41,7 @@ class CachedLM:
         self.context_length = engine.context_length
         self._next_id = 0
         self.decode_graphs = decode_graphs
-        self._graphs = {}                      # batch size -> [static step tensors, captured graph, what _decode_body left]
+        self._graphs = {}                      # batch size -> [static step tensors, captured graph, (its result, what makes the step's logits of it)]
 
     @classmethod
     def from_pretrained(cls, config_path: str, checkpoint_path: str, **kwargs) -> "CachedLM":
@@ -153,15 +153,13 @@ class CachedLM:
             entry[1] = graph
             return logits
         entry[1].replay()
-        return self._decode_logits(entry[2])
+        out, logits_of = entry[2]
+        return logits_of(self, out)
 
     def _decode_body(self, token_ids, plan):
-        """What a decode graph holds of a step ..."""
-        return self._forward(token_ids, plan, self.engine.attend_decode)
-
-    def _decode_logits(self, out):
-        """... and the step's logits, the caller's own, from the graph's result."""
-        return out.clone()
+        """What a decode graph holds of a step, and what makes the step's logits, the caller's own, of its result (a function of the model
+        and that: no bound one, which would keep the model alive)."""
+        return self._forward(token_ids, plan, self.engine.attend_decode), lambda model, out: out.clone()
 
     def forward(self, token_ids):
         """Logits (batch, seq, vocab) of whole sequences, as TransformerLM.forward returns them
@@ -353,12 +351,11 @@ class CachedTransformerLM(CachedLM):
     def _decode_body(self, token_ids, plan):
         """Up to MAX_LINEAR_ROWS rows leave the head to a launch behind the graph: its logits go to the caller's tensor, where a copy of 8 x 10000 out of
         the graph's takes 2.4 us and the gap in front of it (a step of 4 layers of 512, 8 sequences 97.9 -> 93.8, 2 of 1024, 4 sequences 69.8 -> 64.3; where the host is what a step waits for, 2 layers of 256, 50.5 -> 51.5)."""
-        if self._rows_fuse and token_ids.shape[0] <= ops.MAX_LINEAR_ROWS:
-            return self._rows_body(token_ids, plan, self.engine.attend_decode)
+        # (a subclass's own forward is what its graphs hold)
+        T, own = token_ids.shape[0], all(getattr(getattr(self, n), "__func__", None) is getattr(CachedTransformerLM, n) for n in ("_forward", "_forward_rows"))
+        if own and self._rows_fuse and T <= ops.MAX_LINEAR_ROWS and self._rows_pay(T):
+            return self._rows_body(token_ids, plan, self.engine.attend_decode), type(self)._rows_head
         return super()._decode_body(token_ids, plan)
-
-    def _decode_logits(self, out):
-        return self._rows_head(out) if self._rows_fuse and out.shape[0] <= ops.MAX_LINEAR_ROWS else super()._decode_logits(out)
 
     def _forward_rows(self, token_ids, plan, attend, out_rows=None):
         return self._rows_head(self._rows_body(token_ids, plan, attend), out_rows)

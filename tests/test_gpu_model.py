@@ -237,6 +237,42 @@ def test_decode_steps_replayed_from_a_hip_graph_equal_eager_steps(ops, kv_dtype)
     assert bool((err <= (0.15 if kv_dtype == "fp8" else 8e-2) + 5e-2 * ref.abs()).all()), float(err.max())
 
 
+@pytest.mark.parametrize("name", ["_forward", "_forward_rows"])
+def test_decode_graphs_of_a_subclass_hold_its_own_forward(ops, name):
+    """A step's first run is eager and the others are replayed: both are what the subclass makes of it."""
+    print(f"case: decode graphs of a subclass, {name}", flush=True)
+    doubled = type("Doubled", (ops.CachedTransformerLM,), {
+        name: lambda self, *a, **kw: getattr(super(type(self), self), name)(*a, **kw) * 2})
+    cfg = dict(CFG, num_layers=2, num_heads=2, d_model=128)
+    params, ids = _bf16_params(cfg, seed=51), [[3, 1, 4], [1, 5]]
+    models = [ops.CachedTransformerLM(cfg, params, max_batch=2), doubled(cfg, params, max_batch=2, decode_graphs=True)]
+    sids = [[m.new_sequence() for _ in ids] for m in models]
+    for m, s in zip(models, sids):
+        m.prefill(s, ids)
+    for t in range(5):
+        plain, twice = (m.decode(s, [t, 2 * t]) for m, s in zip(models, sids))
+        torch.cuda.synchronize()
+        _logit_close(twice / 2, plain.cpu())
+
+
+@pytest.mark.parametrize("B", [1, 32, 33])
+def test_replayed_logits_are_the_callers_own(ops, B):
+    """On either side of the rows whose head may run behind the graph: what one step returned stays when later steps are replayed, and is an eager twin's."""
+    print(f"case: replayed logits, {B} rows", flush=True)
+    cfg = dict(CFG, num_layers=3, num_heads=2, d_model=128)
+    params = _bf16_params(cfg, seed=61)
+    models = [ops.CachedTransformerLM(cfg, params, max_batch=B, decode_graphs=g) for g in (False, True)]
+    tokens = torch.randint(0, cfg["vocab_size"], (B, 8), generator=torch.Generator().manual_seed(62))
+    sids = [[m.new_sequence() for _ in range(B)] for m in models]
+    for m, s in zip(models, sids):
+        m.prefill(s, list(tokens[:, :3]))
+    got = [[m.decode(s, tokens[:, t].tolist()) for t in range(3, 8)] for m, s in zip(models, sids)]
+    torch.cuda.synchronize()
+    assert len({t.data_ptr() for t in got[1]}) == 5
+    for a, b in zip(*got):
+        _logit_close(b[None], a[None].cpu())
+
+
 def test_decode_steps_ask_the_attention_they_are_given(ops):
     """An engine whose attend_decode is replaced (to look at queries and keys, say) is asked in every layer of a decode step."""
     print("case: replaced attend_decode", flush=True)
