@@ -166,6 +166,8 @@ def check_scalar_address_hazards(src: str) -> str:
                         break
                 states += 1
             j -= 1
+    if n_checked == 0:
+        raise RuntimeError("%s: no memory instruction found in inline assembly" % src)
     if bad:
         raise RuntimeError("scalar address hazard in inline assembly:\n" + "\n".join(bad[:20]))
     return "%s: %d inline-assembly memory instructions, none reads a scalar register within five wait states of a vector write" % (src, n_checked)
@@ -182,15 +184,15 @@ def _vregs(text):
     return out
 
 
-def check_mfma_hazards(src: str) -> str:
-    """An MFMA may read a register two wait states after a vector instruction wrote it, and its result is there eleven behind an MFMA of eight passes.  The compiler
-    sees to that for its own instructions, not for MFMAs in inline assembly: this fails the build if, on the straight-line path, such an MFMA reads what a
-    vector instruction has just written, or another instruction touches its result too early (an MFMA counts as one state here, and takes eight)."""
-    with tempfile.TemporaryDirectory() as tmp:
-        asm = os.path.join(tmp, "k.s")
-        _run([HIPCC, *FLAGS, *EXTRA_FLAGS.get(src, []), "-S", "--cuda-device-only", os.path.join(CSRC, src), "-o", asm])
-        lines = open(asm).read().splitlines()
-    code, inside, bad, n_checked = [], False, [], 0
+_TRANS = ("v_exp_", "v_log_", "v_rcp_", "v_rsq_", "v_sqrt_", "v_sin_", "v_cos_")
+
+
+def asm_hazards(lines):
+    """Vector instructions in inline assembly (`lines` of compiler output), whose wait states the compiler does not see to: (MFMAs, others, what is wrong).  On
+    the straight-line path in front of each: an MFMA may read a register two wait states after a vector instruction wrote it, another one's operand may come
+    from a transcendental instruction two instructions earlier, and an MFMA's result is there eleven states behind one of eight passes (it counts as one
+    state here, and takes eight), for the compiler's instructions too where the MFMA is in assembly."""
+    code, inside, bad, n_mfma, n_other = [], False, [], 0, 0
     for no, raw in enumerate(lines, 1):
         if "#ASMSTART" in raw or "#ASMEND" in raw:
             inside = "#ASMSTART" in raw
@@ -200,22 +202,77 @@ def check_mfma_hazards(src: str) -> str:
             ops = text.split(None, 1)[1].split(",") if " " in text or "\t" in text else []
             code.append((no, text.split()[0], ops, inside))
     for i, (no, op, ops, in_asm) in enumerate(code):
-        own = in_asm and op.startswith("v_mfma")
-        n_checked += own
-        reads = _vregs(",".join(ops[1:] if own else ops)) if own or not in_asm else set()
+        own, other = in_asm and op.startswith("v_mfma"), in_asm and op.startswith("v_") and not op.startswith("v_mfma")
+        n_mfma += own
+        n_other += other
+        reads = _vregs(",".join(ops[1:] if own else ops)) if own or other or not in_asm else set()
         states, j = 0, i - 1
         while reads and j >= 0 and states < (2 if own else 11):
             _, prev, prev_ops, prev_asm = code[j]
             written = _vregs(prev_ops[0]) if prev.startswith("v_") and prev_ops else set()
             mfma = prev.startswith("v_mfma")
-            if written & reads and ((own and not mfma) or (not own and mfma and prev_asm and not op.startswith("v_mfma"))):
-                bad.append("%s:%d: %s reads or writes %s, written %d wait state(s) earlier by %s" % (src, no, op, sorted(written & reads)[:4], states, prev))
+            if written & reads and (not mfma if own else mfma and (prev_asm or other) and not op.startswith("v_mfma") or other and states < 1 and prev.startswith(_TRANS)):
+                bad.append("%d: %s reads or writes %s, written %d wait state(s) earlier by %s" % (no, op, sorted(written & reads)[:4], states, prev))
                 break
             states += int(prev_ops[0], 0) + 1 if prev == "s_nop" else 1
             j -= 1
+    return n_mfma, n_other, bad
+
+
+def scratch_before_products(lines, kernel):
+    """Accesses to scratch memory in `kernel` (a part of its symbol) from which an MFMA can still be reached: what the loop spills.  None where there is no such
+    kernel or it has no MFMA."""
+    code, labels, inside = [], {}, False
+    for no, raw in enumerate(lines, 1):
+        text = raw.split(";")[0].strip()
+        if text.endswith(":") and not text.startswith(".L"):
+            inside = kernel in text
+        elif text.startswith(".Lfunc_end") and inside:
+            break
+        if not inside:
+            continue
+        if text.endswith(":"):
+            labels[text[:-1]] = len(code)
+        elif text and not text.startswith("."):
+            code.append((no, text))
+    if not any(text.startswith("v_mfma") for _, text in code):
+        return None
+    follows = [[] for _ in code]                   # instruction -> those that come in front of it
+    for i, (_, text) in enumerate(code):
+        op = text.split()[0]
+        to = [] if op in ("s_branch", "s_endpgm") else [i + 1]
+        if op == "s_branch" or op.startswith("s_cbranch"):
+            to.append(labels[text.split()[1]])
+        for j in to:
+            if j < len(code):
+                follows[j].append(i)
+    reach, todo = set(), [i for i, (_, text) in enumerate(code) if text.startswith("v_mfma")]
+    while todo:
+        for i in follows[todo.pop()]:
+            if i not in reach:
+                reach.add(i)
+                todo.append(i)
+    return ["%d: %s" % (no, text) for i, (no, text) in enumerate(code) if text.startswith("scratch_") and i in reach]
+
+
+def check_wide_backward() -> str:
+    """bwd_dkv_wide_kernel has MFMAs and conversions in inline assembly, and all registers taken: no hazard of theirs, and nothing spilled before the last product,
+    where a reload would wait for all rows that are on their way."""
+    src = "prefill_bwd.hip"
+    with tempfile.TemporaryDirectory() as tmp:
+        asm = os.path.join(tmp, "k.s")
+        _run([HIPCC, *FLAGS, *EXTRA_FLAGS.get(src, []), "-S", "--cuda-device-only", os.path.join(CSRC, src), "-o", asm])
+        lines = open(asm).read().splitlines()
+    n_mfma, n_other, bad = asm_hazards(lines)
+    if n_mfma < 2 * 64 or n_other < 2 * 64:                           # (two instances: dV, dV and dK, dK of a step; P and dS of two steps)
+        raise RuntimeError("%s: %d MFMAs and %d other vector instructions found in inline assembly" % (src, n_mfma, n_other))
     if bad:
-        raise RuntimeError("MFMA hazard in inline assembly:\n" + "\n".join(bad[:20]))
-    return "%s: %d MFMAs in inline assembly, none reads a register that a vector instruction has just written" % (src, n_checked)
+        raise RuntimeError("hazards in inline assembly of %s:\n" % src + "\n".join(bad[:20]))
+    for mode in (0, 1):
+        spilled = scratch_before_products(lines, "bwd_dkv_wide_kernelILi%dE" % mode)
+        if spilled is None or spilled:
+            raise RuntimeError("%s: bwd_dkv_wide_kernel<%d> %s" % (src, mode, "not found" if spilled is None else "spills in its loop:\n" + "\n".join(spilled[:20])))
+    return "%s: %d MFMAs and %d other vector instructions in inline assembly without a hazard, nothing spilled before the last product" % (src, n_mfma, n_other)
 
 
 def _compile_all(srcs, tag=""):
@@ -275,7 +332,7 @@ def build_library(verbose: bool = True) -> str:
         calls = ex.submit(compile_calls)
         check = ex.submit(check_w64_registers)
         hazards = [ex.submit(check_scalar_address_hazards, s) for s in srcs if issues_memory_from_assembly(s)]
-        hazards.append(ex.submit(check_mfma_hazards, "prefill_bwd.hip"))
+        hazards.append(ex.submit(check_wide_backward))
         results = _compile_all(srcs)
         notes = [check.result()] + [h.result() for h in hazards]
     if verbose:
