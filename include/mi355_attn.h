@@ -270,6 +270,14 @@ int mi355_prefill_bwd_typed(const void* q, const void* k, const void* v, const v
  * the workspace still has room for their dS (it counts with the longest everywhere), else their gradients are zero. */
 int64_t mi355_prefill_bwd_ds_workspace(int B, int Hq, int Hkv, int Sq_max, int Sk_max, int D, int mask_mode, int packed, int same_bounds,
                                        int64_t total_q, int64_t total_k);
+/* Which kernel computes dK, dV and dS of such a call, for tests and for reading profiles; 0: no such form.  shares (may be NULL): into how many shares the row tiles
+ * of a key tile are dealt out. */
+enum {
+    MI355_BWD_DS_ROLES = 1, /* dV and dK on different wavefronts */
+    MI355_BWD_DS_WIDE = 2   /* 64 keys per wavefront, head_dim 128 */
+};
+int mi355_prefill_bwd_ds_kernel(int B, int Hq, int Hkv, int Sq_max, int Sk_max, int D, int mask_mode, int packed, int same_bounds, int64_t total_q, int64_t total_k,
+                                int* shares);
 int mi355_prefill_bwd_ds(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse, float* delta,
                          void* dq, void* dk, void* dv, const int64_t q_strides[3], const int64_t k_strides[3], const int64_t v_strides[3],
                          const int64_t o_strides[3], const int64_t do_strides[3], const int64_t dq_strides[3],

@@ -972,7 +972,8 @@ __global__ __launch_bounds__(kDqWaves * 64, 2) void bwd_dq_ds_kernel(BwdParams p
 #pragma unroll
             for (int j = 0; j < 16; ++j) dq[t][i][j] = 0.f;
     // Column n of half t is row 32 t + my_row of the sequence.  From step `diagonal` on some row does not see all keys of the step: dS is zero there
-    // unless its dP overflowed (0 * inf), so it is set to zero here, where there is time (the dK/dV kernel takes 5 % longer with it).
+    // unless its dP overflowed (0 * inf), so it is set to zero here, where there is time (the dK/dV kernel takes 5 % longer with it).  It may also never have been
+    // written: bwd_dkv_wide_kernel stores nothing of a half of a row tile of which no row sees any of a wavefront's 64 keys.
     const int my_row = kBwRows * rt + 16 * (n >> 4) + 8 * ((n >> 2) & 1) + 4 * ((n >> 3) & 1) + (n & 3);
     const int diagonal = (kBwRows * rt + sk - sq + 1) >> 5;
     if (n_steps > 0) {
@@ -1363,6 +1364,7 @@ struct DsPasses {
     int64_t plan_bytes = 0;       // lists, in front of dS
     int n_units = 0, units_per_pass = 0;
     int shares = 1;
+    bool wide = false;            // dK, dV and dS by bwd_dkv_wide_kernel
     int64_t part_rows = 0, part_bytes = 0;       // fp32 shares of dk and dv, behind the lists
     int64_t ds_room = 0, k_room = 0, q_room = 0, most_q = 0, most_k = 0;
     int64_t bytes() const { return plan_bytes + part_bytes + unit_bytes * units_per_pass; }
@@ -1435,6 +1437,12 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
         out.part_rows = rows_k;
         out.part_bytes = round_up(2 * out.shares * rows_k * Hkv * D * 4, kDsBlock);
     }
+    // Wavefronts of 64 keys: key tiles with sixteen steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
+    // 56 / 70; 4 x 602, 16 heads (5) 32 / 37; 16 x 920 (7) 231 / 243; 4 packed of 324 to 5199, 4 / 2 heads, 4 shares (11) 116 / 120; 51 packed of 1701, one head (13) all kernels
+    // 258 / 262; 21 packed of 995, 16 / 8 (15.5) all kernels 548 / 554; 2 x 2048, 32 heads (16) 186 / 175; 3000
+    // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
+    const double row_tiles = (double)(packed ? total_q : (int64_t)B * Sq) / kBwRows / B;
+    out.wide = D == 128 && row_tiles * G * (causal ? 0.5 : 1.0) >= 16.0 * out.shares;
     out.unit_bytes = out.ds_room * G * kDsBlock;
     const int64_t fit = out.unit_bytes > 0 ? kDsMost / out.unit_bytes : out.n_units;
     if (fit < 1) return false;
@@ -1483,12 +1491,7 @@ static int launch_bwd_ds(BwdParams p, const DsPasses& d, int64_t total_q, unsign
     const int64_t q_jobs = p.cu_q ? d.q_room : ((int64_t)(p.Sq + kBwRows - 1) / kBwRows * G + kDqWaves - 1) / kDqWaves;
     if (delta_wgs > 0x7fffffffLL || k_jobs * d.units_per_pass * d.shares > 0x7fffffffLL || q_jobs * d.units_per_pass > 0x7fffffffLL)
         return (int)hipErrorInvalidValue;
-    // Key tiles with sixteen steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
-    // 56 / 70; 4 x 602, 16 heads (5) 32 / 37; 16 x 920 (7) 231 / 243; 4 packed of 324 to 5199, 4 / 2 heads, 4 shares (11) 116 / 120; 51 packed of 1701, one head (13) all kernels
-    // 258 / 262; 21 packed of 995, 16 / 8 (15.5) all kernels 548 / 554; 2 x 2048, 32 heads (16) 186 / 175; 3000
-    // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
-    const double row_tiles = (double)(p.cu_q ? total_q : (int64_t)p.B * p.Sq) / kBwRows / p.B;
-    p.wide = D == 128 && row_tiles * G * (MODE == MI355_MASK_CAUSAL ? 0.5 : 1.0) >= 16.0 * p.shares;
+    p.wide = d.wide;
     hipLaunchKernelGGL((bwd_delta_kernel<D, MODE>), dim3((unsigned)delta_wgs), dim3(kPlanThreads), p.cu_q ? plan_lds_bytes(plan, p.B) : 0, stream, p, plan);
     for (p.unit0 = 0; p.unit0 < d.n_units; p.unit0 += p.n_units) {
         p.n_units = std::min(d.units_per_pass, d.n_units - p.unit0);
@@ -1685,6 +1688,16 @@ extern "C" int64_t mi355_prefill_bwd_ds_workspace(int B, int Hq, int Hkv, int Sq
     if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Sq_max <= 0 || Sk_max <= 0) return 0;
     DsPasses d;
     return ds_passes(B, Hq, Hkv, Sq_max, Sk_max, D, mask_mode, packed != 0, same_bounds != 0, total_q, total_k, d) ? d.bytes() : 0;
+}
+
+extern "C" int mi355_prefill_bwd_ds_kernel(int B, int Hq, int Hkv, int Sq_max, int Sk_max, int D, int mask_mode, int packed, int same_bounds, int64_t total_q,
+                                           int64_t total_k, int* shares) {
+    DsPasses d;
+    if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Sq_max <= 0 || Sk_max <= 0 ||
+        !ds_passes(B, Hq, Hkv, Sq_max, Sk_max, D, mask_mode, packed != 0, same_bounds != 0, total_q, total_k, d))
+        return 0;
+    if (shares) *shares = d.shares;
+    return d.wide ? MI355_BWD_DS_WIDE : MI355_BWD_DS_ROLES;
 }
 
 extern "C" int mi355_prefill_bwd_ds(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,

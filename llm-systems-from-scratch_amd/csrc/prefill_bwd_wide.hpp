@@ -100,6 +100,7 @@ __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParam
         return lowest > r_top ? 0 : ((r_top - lowest) / apart + 1) * G;
     };
     const int n_steps = __builtin_amdgcn_readfirstlane(steps_from(k0, kBwRows - 1));
+    // (Behind these no row of this half sees a key of this wavefront, and its dS is not written: bwd_dq_ds_kernel takes what a row does not see as zero.)
     const int my_steps = __builtin_amdgcn_readfirstlane(steps_from(kw0, kWdRows * rows + kWdRows - 1));
 
     // ---- what a step is: worked out 32 steps at a time, a lane each, and kept in LDS ----

@@ -8,7 +8,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmi355attn.so")
 # the same library without the training kernels: what a served model needs, built by the command line tools in a fresh checkout
 SERVING_LIB_PATH = os.path.join(_HERE, "libmi355attn_serving.so")
-TRAINING_ONLY = ("mi355_prefill_bwd", "mi355_prefill_bwd_mask", "mi355_prefill_bwd_typed", "mi355_prefill_bwd_ds", "mi355_prefill_bwd_ds_workspace")
+TRAINING_ONLY = ("mi355_prefill_bwd", "mi355_prefill_bwd_mask", "mi355_prefill_bwd_typed", "mi355_prefill_bwd_ds", "mi355_prefill_bwd_ds_workspace", "mi355_prefill_bwd_ds_kernel")
 
 MI355_BF16 = 0
 MI355_FP8_E4M3 = 1
@@ -38,6 +38,7 @@ EXPORTS = (
     "mi355_prefill_bwd_typed",
     "mi355_prefill_bwd_ds",
     "mi355_prefill_bwd_ds_workspace",
+    "mi355_prefill_bwd_ds_kernel",
     "mi355_paged_decode_fwd",
     "mi355_paged_decode_fwd_static",
     "mi355_paged_decode_workspace_bytes",
@@ -175,6 +176,8 @@ def load():
                                                                     i64, i64, vp, i64, vp]
     lib.mi355_prefill_bwd_ds_workspace.restype = i64
     lib.mi355_prefill_bwd_ds_workspace.argtypes = [i32] * 9 + [i64, i64]
+    lib.mi355_prefill_bwd_ds_kernel.restype = i32
+    lib.mi355_prefill_bwd_ds_kernel.argtypes = [i32] * 9 + [i64, i64, vp]
     lib.mi355_prefill_paged_fwd.restype = i32
     lib.mi355_prefill_paged_fwd.argtypes = [vp, vp, vp, vp, i64, i64, vp, vp, i64, i64, vp,
                                             i32, i32, i32, i32, i32, i32, i64, f32, i32, i32, i64, vp, sz, vp]
