@@ -61,3 +61,29 @@ def test_mixed_operands(B, H, Hkv, S, D, f32, layout, train):
         for a, b, t in zip(torch.autograd.grad(got, mixed, dout), torch.autograd.grad(want, ref, dout), mixed):
             assert a.dtype == t.dtype
             close(a, b)
+
+
+@pytest.mark.parametrize("lens,H,Hkv,D,f32", [([33, 1, 200], 4, 2, 128, "qk"), ([100, 64], 3, 3, 64, "q"), ([257, 30], 2, 1, 32, "kv")])
+@pytest.mark.parametrize("layout", ["whole", "sliced"])
+@pytest.mark.parametrize("train", [False, True])
+def test_mixed_packed_operands(lens, H, Hkv, D, f32, layout, train):
+    """Packed sequences, operands of their own or slices of one projection (not whole memory: torch's conversion): the kernels of the rounded operands, so the same bits."""
+    import mi355_attn as ma
+    print(f"case: mixed packed {lens} {H}/{Hkv} {D} {f32} {layout} {train}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(sum(lens))
+    T, cu = sum(lens), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device="cuda")
+    if layout == "sliced":
+        x = torch.randn(T, H + 2 * Hkv, D, generator=g, device="cuda")
+        q, k, v = x[:, :H], x[:, H:H + Hkv], x[:, H + Hkv:]
+    else:
+        q, k, v = (torch.randn(T, h, D, generator=g, device="cuda") for h in (H, Hkv, Hkv))
+    mixed = [t.detach() if name in f32 else t.bfloat16() for name, t in zip("qkv", (q, k, v))]
+    ref = [t.bfloat16() for t in mixed]
+    for t in (*mixed, *ref):
+        t.requires_grad_(train)
+    got, want = (ma.flash_attn_varlen_prefill(*t, cu, cu, max(lens), max(lens)) for t in (mixed, ref))
+    assert torch.equal(got, want)
+    if train:
+        dout = torch.randn(got.shape, generator=g, device="cuda").bfloat16()
+        for a, b, t in zip(torch.autograd.grad(got, mixed, dout), torch.autograd.grad(want, ref, dout), mixed):
+            assert a.dtype == t.dtype and torch.equal(a.bfloat16(), b)
