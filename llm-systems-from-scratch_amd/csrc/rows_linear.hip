@@ -208,10 +208,17 @@ __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
 }
 
 // Eight wavefronts with two steps each, one workgroup per compute unit, where every workgroup has one to itself and k is long: four have their steps one or
-// two at a time, a wait on memory each.  Us, four / eight (k x n): 2048 x 512, 8 rows 3.66 / 3.47, 17 rows 4.75 / 4.39, 100 rows 4.85 / 4.52; 4096 x 1024, 8 rows 5.3 /
-// 4.9, 32 rows 7.4 / 6.4; norm and 2048 x 6144, 8 rows 7.3 / 5.8; 14336 x 4096, 17 rows 33.7 / 20.4, 32 rows 33.4 / 24.1.  At k = 512 both are the launch (2.41 / 2.48,
+// two at a time, a wait on memory each.  Us, four / eight (k x n): 17 rows and more, whose ring of four has one step: 1024 x 1024 4.8 / 4.1, 2048 x 512 4.75 / 4.39, 100 rows 4.85 / 4.52,
+// 4096 x 1024, 32 rows 7.4 / 6.4, 14336 x 4096 50 / 34 to 38; norm and 2048 x 6144, 8 rows 10.0 / 9.3, and 1280 x 1280 5.3 / 5.0.  At k = 512 both are the launch (2.41 / 2.48,
 // with a norm 3.24 / 3.14 and 17 rows 3.73 / 3.76), at 256 eight lose 0.1 to 0.25; with more workgroups than units a second one hides the waits (300 rows,
-// 2688 x 1024 7.0 / 7.1).
+// 2688 x 1024 7.0 / 7.1).  Up to 16 rows without a norm have two steps of four wavefronts as well, and less to gain: one row of 2048 x 512 8 % and of 4096 x 512 11 %, 12 and 16 rows of
+// 1024 to 1536 lose 1 to 2 %, and 256 workgroups, which fill the chip by themselves, lose up to 5 (k = 1024, 8 rows 3.75 / 3.92; 1536 3, 3072 2.7) but for rows of whole 4096 bytes (2048 and 4096 gain 3).
+template <int MODE, int MT, bool NORM>
+static bool eight_pay(const RowsParams& p, int64_t workgroups) {
+    if (p.k < 1024 || workgroups > 256) return false;
+    if (MT > 1 || NORM) return true;
+    return p.k >= 1280 && (workgroups <= 128 ? p.T <= 8 || p.k >= 2048 : p.k % 2048 == 0);
+}
 // More workgroups than units over rows of whole 4096 bytes begin with steps of their own (turn_of): norm and 4096 x 12288, 8 rows 27.5 -> 23.6, 8192 x 8448 20 % less, 2048 x 16384 12;
 // with fewer it costs 1 to 2 %.  Gate and up, two runs of rows a workgroup, only at k = 2048 (5632 11.5 -> 11.0, 8192 10 % less): at 4096 they are -5 to +11 % (5120 +1, 6144 +7, 7168 -3, 8192 +8, 9216
 // -3, 11008 0, 14336 +10).
@@ -221,8 +228,9 @@ static bool rows_turn(const RowsParams& p, int64_t workgroups) {
 }
 template <int MODE, int MT, bool NORM>
 static void launch_rows_as(const RowsParams& p, const dim3& grid, hipStream_t s) {
-    if (p.k >= 1024 && (int64_t)grid.x * grid.y <= 256) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 8, false>), grid, dim3(512), 0, s, p);
-    else if (rows_turn<MODE>(p, (int64_t)grid.x * grid.y)) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4, true>), grid, dim3(256), 0, s, p);
+    const int64_t workgroups = (int64_t)grid.x * grid.y;
+    if (eight_pay<MODE, MT, NORM>(p, workgroups)) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 8, false>), grid, dim3(512), 0, s, p);
+    else if (rows_turn<MODE>(p, workgroups)) hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4, true>), grid, dim3(256), 0, s, p);
     else hipLaunchKernelGGL((rows_linear_kernel<MODE, MT, NORM, 4, false>), grid, dim3(256), 0, s, p);
 }
 

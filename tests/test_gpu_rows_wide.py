@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,k,n", [(1, 1016, 96), (1, 1024, 30), (16, 1032, 33), (17, 1024, 512), (32, 1096, 36), (9, 2048, 8192), (31, 1352, 8196), (32, 4096, 64),
-                                   (8, 14336, 40), (33, 1024, 96), (70, 2056, 129), (3, 4096, 4112)])
+                                   (8, 14336, 40), (33, 1024, 96), (70, 2056, 129), (3, 4096, 4112), (8, 1280, 72), (9, 1280, 40), (16, 1536, 96), (16, 2048, 40),
+                                   (4, 1536, 4128), (4, 2048, 8192)])
 def test_rows_linear_on_eight_wavefronts(ops, T, k, n):  # noqa: F811
     print(f"case: rows on eight wavefronts {T} {k} {n}", flush=True)
     g, prompt = torch.Generator().manual_seed(T + k), T > 32
