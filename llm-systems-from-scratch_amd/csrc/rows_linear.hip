@@ -208,11 +208,11 @@ __global__ __launch_bounds__(64 * WAVES) void rows_linear_kernel(RowsParams p) {
 }
 
 // Eight wavefronts with two steps each, one workgroup per compute unit, where every workgroup has one to itself and k is long: four have their steps one or
-// two at a time, a wait on memory each.  Us, four / eight (k x n): 17 rows and more, whose ring of four has one step: 1024 x 1024 4.8 / 4.1, 2048 x 512 4.75 / 4.39, 100 rows 4.85 / 4.52,
-// 4096 x 1024, 32 rows 7.4 / 6.4, 14336 x 4096 50 / 34 to 38; norm and 2048 x 6144, 8 rows 10.0 / 9.3, and 1280 x 1280 5.3 / 5.0.  At k = 512 both are the launch (2.41 / 2.48,
+// two at a time, a wait on memory each.  Us, four / eight (k x n): 17 rows and more, whose ring of four has one step: 1024 x 2048 4.8 / 4.2, 2048 x 512 4.75 / 4.39, 100 rows 4.85 / 4.52,
+// 4096 x 1024, 32 rows 7.4 / 6.4, 14336 x 4096 50 / 34 to 38; norm and 2048 x 6144, 8 rows 10.2 / 9.4, and 1280 x 2048 5.3 / 5.0.  At k = 512 both are the launch (2.41 / 2.48,
 // with a norm 3.24 / 3.14 and 17 rows 3.73 / 3.76), at 256 eight lose 0.1 to 0.25; with more workgroups than units a second one hides the waits (300 rows,
 // 2688 x 1024 7.0 / 7.1).  Up to 16 rows without a norm have two steps of four wavefronts as well, and less to gain: one row of 2048 x 512 8 % and of 4096 x 512 11 %, 12 and 16 rows of
-// 1024 to 1536 lose 1 to 2 %, and 256 workgroups, which fill the chip by themselves, lose up to 5 (k = 1024, 8 rows 3.75 / 3.92; 1536 3, 3072 2.7) but for rows of whole 4096 bytes (2048 and 4096 gain 3).
+// 1024 to 1536 lose 1 to 2 %, and 256 workgroups, which fill the chip by themselves, lose up to 5 (8192 rows of w, 8 rows of 1024 5.2 / 5.4, of 1536 6.7 / 6.9, of 3072 10.6 / 10.8) but for rows of whole 4096 bytes (2048 and 4096 gain 3).
 template <int MODE, int MT, bool NORM>
 static bool eight_pay(const RowsParams& p, int64_t workgroups) {
     if (p.k < 1024 || workgroups > 256) return false;
