@@ -1589,18 +1589,20 @@ def _direct_pairs(experts: int, k: int, ff: int, n: int) -> int:
     """Up to how many pairs the expert products run without an order.  That saves a launch and the padding of 128-row tiles, and costs
     what the pairs' rows take up: each 32 weight rows read those of their expert (k wide, then ff wide, and n out), and the weights once
     more for every 32 of them.  So the line is drawn at 1.2 M elements in all pairs' rows, but not above 64 pairs per expert, where one expert with more than its
-    share would be waited for, and not below 16: 24 where the gate and up tiles of 128 rows are no more than three quarters of a set per compute unit (experts * ff up to
-    12288), or of up to twelve experts one set (16384); with more experts in one whole set the ordered form is the better one from 10 to 18 pairs on.  Us without and with an
+    share would be waited for, and not below a number per expert: 12 with more than 24 experts; else 16; and 24 where the gate and up tiles of 128 rows are no more
+    than three quarters of a set per compute unit (experts * ff up to 12288) or, of up to twelve experts, one set (16384).  Sets that are nearly whole are what the ordered form
+    is best at: with more experts it is the faster one from 10 to 18 pairs on.  Us without and with an
     order, uniform ids, weights from HBM (several sets of them in turn: one set of up to 256 MB stays in the last-level cache, and both forms are faster then):
         8 experts of 1024 x 1024 (line at 48 pairs per expert) 32 pairs 21 / 30, 48 25 / 32; 8 of 2048 x 1024 (29) 24 25 / 39, 32 34 / 40; 8 of 1024 x 3072 (29) 28 41 / 56, 32 47 / 57;
         8 of 2048 x 2048 24 43 / 52, 32 59 / 53; 8 of 4096 x 2048 24 87 / 96, 32 104 / 97; 12 of 2048 x 1024 24 36 / 42, 32 46 / 43; 12 of 2048 x 1344 24 45 / 49, 28 52 / 49;
         12 of 1792 x 896 24 33 / 37, 32 42 / 38; 16 of 1536 x 768 24 33 / 35, 28 37 / 36; 16 of 1024 x 1024 (24) 24 28 / 32, 32 33 / 32; 32 of 512 x 512 (24) 24 20 / 23, 32 24 / 23
-      where the line is at 16 (or a little more by the rows):
+      where the line is at 16 or 12 (or a little more by the rows):
         14 of 2048 x 1152 16 46 / 46, 24 50 / 46; 16 of 1792 x 896 14 37 / 38, 18 40 / 39, 24 44 / 39; 16 of 2048 x 1024 16 41 / 45, 20 46 / 45, 24 49 / 45; 32 of 1024 x 512 10 28 / 28,
         16 29 / 28, 24 32 / 29; 32 of 2048 x 512 14 46 / 45, 24 50 / 46; 32 of 1024 x 1024 12 45 / 45, 16 48 / 45; 32 of 2048 x 1024 12 77 / 78, 16 82 / 79, 24 89 / 81;
         32 of 2048 x 2048 16 146 / 146, 24 162 / 148; 16 of 2048 x 2048 16 76 / 78, 24 81 / 79; 24 of 1536 x 768 16 42 / 51, 24 44 / 52; 24 of 2048 x 1024 16 63 / 67, 24 68 / 68;
-        16 of 2560 x 1280 16 64 / 80, 28 84 / 83; 48 of 1024 x 768 16 52 / 57, 24 59 / 58; 64 of 768 x 384 16 34 / 34."""
-    at_least = 24 if experts * ff <= (16384 if experts <= 12 else 12288) else 16
+        16 of 2560 x 1280 16 64 / 80, 28 84 / 83; 48 of 1024 x 768 16 52 / 57, 24 59 / 58; 64 of 768 x 384 16 34 / 34; 64 of 1024 x 512 14 50 / 46;
+        128 of 1024 x 384 14 80 / 73."""
+    at_least = 12 if experts > 24 else 24 if experts * ff <= (16384 if experts <= 12 else 12288) else 16
     return min(_DIRECT_PAIRS, 64 * experts, max(at_least * experts, (9 << 17) // (k + ff + n)))
 
 

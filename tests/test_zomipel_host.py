@@ -309,7 +309,7 @@ def test_line_of_the_expert_products_without_an_order():
 
 @pytest.mark.parametrize("E,k,ff,direct,ordered", [(16, 1792, 896, 14, 18), (16, 2048, 1024, 16, 20), (32, 1024, 512, 9, 18), (32, 2048, 512, 12, 18), (32, 1024, 1024, 12, 18),
                                                    (14, 2048, 1152, 16, 20), (20, 1536, 768, 16, 20), (12, 2048, 1024, 24, 32), (12, 2048, 1344, 24, 32), (8, 2048, 2048, 24, 32),
-                                                   (8, 1024, 1024, 40, 64), (16, 1536, 768, 24, 28), (24, 1536, 768, 16, 32), (32, 2048, 2048, 14, 18)])
+                                                   (8, 1024, 1024, 40, 64), (16, 1536, 768, 24, 28), (24, 1536, 768, 16, 32), (32, 2048, 2048, 12, 18), (64, 1024, 512, 8, 14), (128, 1024, 384, 8, 14)])
 def test_line_of_the_expert_products_is_between_what_was_measured(E, k, ff, direct, ordered):
     """Pairs per expert at which the one form was the faster one, and the other."""
     assert direct * E <= mi355_attn.ops._direct_pairs(E, k, ff, k) < ordered * E
