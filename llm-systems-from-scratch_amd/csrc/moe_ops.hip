@@ -933,12 +933,14 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(MoeParams p, const int3
 
 // From twelve pairs an expert on most experts take two row tiles, of which the small ring holds one step: with the large one 8 experts of 2048 x 2048, top 2, 64 tokens
 // 46.5 -> 41.1 us, 16 of 2048 x 1024, top 4, 100 tokens 49.5 -> 45.8; below, three workgroups per compute unit are worth more (32 tokens 39.5 / 40.7), and so they are where a
-// wavefront has four steps (16 of 1024 x 1024, top 4, 64 tokens 25.3 / 25.8).  (24 of 1536 x 768, top 4, 96 tokens 42, in tiles of 128 rows 50.)
+// wavefront has four steps (16 of 1024 x 1024, top 4, 64 tokens 25.3 / 25.8).  (24 of 1536 x 768, top 4, 96 tokens 42, in tiles of 128 rows 50.)  With more workgroups than the
+// two per compute unit that it leaves, from sixteen: up to fifteen pairs the third one is worth as much or more.  Pairs an expert, small / large ring: 10 of 1792 x 1792 12 39.9 / 43.4, 15 42.0 / 43.2, 16
+// 46.0 / 44.9; 16 of 1792 x 896 15 35.0 / 36.3, 16 39.0 / 38.6; 16 of 2560 x 1280 12 60.4 / 62.1, 16 68.9 / 64.9; 4 of 2048 x 1024, 256 workgroups, 13 19.4 / 17.5.
 template <bool GATE_UP>
 static void launch_direct(const MoeParams& p, const int32_t* ids, hipStream_t s) {
     const int tiles = (p.n + (GATE_UP ? 15 : 31)) / (GATE_UP ? 16 : 32);
     const dim3 grid((unsigned)(tiles * p.E)), block(256);
-    const bool large = p.k >= 1536 && p.n_pairs >= 12 * p.E, turn = turn_pays(p.k);
+    const bool large = p.k >= 1536 && p.n_pairs >= (grid.x <= 512 ? 12 : 16) * p.E, turn = turn_pays(p.k);
     if (p.n_pairs < p.E && p.n_pairs <= kFewPairs) {
         const dim3 few((unsigned)(tiles * p.n_pairs));
         if (turn) hipLaunchKernelGGL((moe_direct_kernel<GATE_UP, kStreamBytes, true, true>), few, block, 0, s, p, ids, tiles);
