@@ -364,7 +364,8 @@ __device__ __forceinline__ void store4(const MoeParams& p, int64_t out_row, int 
 // TURN: the workgroups of an XCD begin 0, 8, 16 or 24 steps of k in, by their columns and expert, so that a row's sums do not depend on the tile it falls into.  Rows of whole 4096 bytes from step 0 on all want the same channels of its L2 (turn_of), and
 // weights that come from HBM wait for these: 32 experts of 2048 x 2048, 64 pairs an expert 200 -> 154 us, 16 of 2048 x 1024 32 pairs 54.5 -> 45.7, 128 pairs 78.1 -> 77.1,
 // 8 of 2048 x 2048 75 pairs 66 -> 56, 250 pairs 103.9 / 104.2.  Where an expert's row tiles share its weights in the L2 their steps had better go together, so
-// not behind 256 pairs an expert, and not in the 256 x 256 tiles (396 -> 399 to 409).
+// not behind 256 pairs an expert (longer rows: 96; pairs an expert, without / with: 16 of 4096 x 1024 64 11 % less, 128 4 % more, 4 of 4096 x 4096 64 10 % less, 128 7 % more), and not in the
+// 256 x 256 tiles (396 -> 399 to 409).
 template <bool GATE_UP, bool TURN>
 __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeParams p, int n_tiles, int chunk) {
     constexpr int BM = 128, BK = 64, kTile = 128 * BK * 2, NA = 2, NW = 3;
@@ -1039,7 +1040,7 @@ static int launch_moe(const MoeParams& p, int dtype, int tiling, hipStream_t s) 
     const int chunk = n_tiles * std::max(1, (wide ? 32 : 64) / n_tiles);
     if (dtype == MI355_FP32) hipLaunchKernelGGL(moe_f32_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     else if (wide) hipLaunchKernelGGL(moe_wide_kernel<GATE_UP>, dim3((unsigned)(n_tiles * m_tiles + 384)), block, 0, s, p, n_tiles, chunk);
-    else if (large && turn_pays(p.k) && p.n_pairs <= 256LL * p.E) hipLaunchKernelGGL((moe_gemm_kernel<GATE_UP, true>), grid, block, 0, s, p, n_tiles, chunk);
+    else if (large && turn_pays(p.k) && p.n_pairs <= (p.k == 2048 ? 256LL : 96LL) * p.E) hipLaunchKernelGGL((moe_gemm_kernel<GATE_UP, true>), grid, block, 0, s, p, n_tiles, chunk);
     else if (large) hipLaunchKernelGGL((moe_gemm_kernel<GATE_UP, false>), grid, block, 0, s, p, n_tiles, chunk);
     else hipLaunchKernelGGL(moe_skinny_kernel<GATE_UP>, grid, block, 0, s, p, n_tiles, m_tiles);
     return (int)hipGetLastError();
