@@ -379,10 +379,18 @@ Tensor forward_only(const Tensor& q, const Tensor& k, const Tensor& v, const int
     return out;
 }
 
-// forward_only of short heads with fp32 among q, k and v, which the kernel rounds on their way in; undefined: no such form of this call
+// Few heads of more keys than a wavefront or two have at once run on the kernel that deals keys to wavefronts, behind a launch that rounds.  us with fp32 Q and K, rounded
+// on their way in / like this: heads of 64, one of 128 keys 6.0 / 6.4, of 150 7.9 / 6.9, of 256 10.1 / 7.3, 32 of 128 6.2 / 7.2, of 150 8.2 / 7.9, of 256 10.5 / 8.4, 64 of 256 10.6 / 11.1; of 32,
+// one of 150 6.0 / 6.2, of 177 6.4 / 6.2, of 256 7.3 / 6.4, 32 of 177 6.8 / 6.8, of 256 7.8 / 7.0, 64 of 256 7.8 / 8.3.  (Causal; without a mask every wavefront has all keys.)
+bool keys_dealt(const Shape& s, const c10::Device& dev) {
+    return (int64_t)s.B * s.Hq <= (s.causal ? 32 : 64) && s.Sk > (s.D == 64 ? 128 : 176) &&
+           mi355_prefill_kernel(s.B, s.Hq, s.Hkv, s.D, s.Sq, s.Sk, s.mode(), 0, 0, 0, 1, 0, compute_units(dev), nullptr) == MI355_PREFILL_KEYS;
+}
+
+// forward_only of short heads with fp32 among q, k and v, which the kernel rounds on their way in; undefined: no such form of this call, or not the faster one
 Tensor forward_mixed(const Tensor& q, const Tensor& k, const Tensor& v, const Shape& s) {
     const int f32 = f32_bits(q, k, v);
-    if (f32 == 0 || !((float)s.scale > 0.f) || !mi355_prefill_fwd_rounds(s.Hq, s.Hkv, s.Sq, s.Sk, s.D, s.mode())) return {};
+    if (f32 == 0 || !((float)s.scale > 0.f) || !mi355_prefill_fwd_rounds(s.Hq, s.Hkv, s.Sq, s.Sk, s.D, s.mode()) || keys_dealt(s, q.device())) return {};
     for (const Tensor* t : {&q, &k, &v})
         if (!whole_rows(*t) || t->stride(2) <= 0 || t->stride(2) >= (1 << 24)) return {};
     const auto dev = q.device();

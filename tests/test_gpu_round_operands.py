@@ -26,7 +26,7 @@ def test_round_operands(sizes):
 
 
 @pytest.mark.parametrize("B,H,Hkv,S,D,f32", [(2, 3, 3, 33, 32, "qk"), (9, 8, 8, 256, 32, "kv"), (3, 4, 4, 100, 64, "qk"), (2, 4, 2, 100, 64, "qk"), (2, 6, 6, 300, 64, "q"), (1, 4, 4, 177, 128, "qk"),
-                                             (1, 2, 2, 70, 128, "kv")])
+                                             (1, 2, 2, 70, 128, "kv"), (4, 8, 8, 128, 64, "qk"), (4, 8, 8, 129, 64, "kv"), (3, 11, 11, 256, 64, "qk"), (1, 1, 1, 177, 32, "qk")])
 @pytest.mark.parametrize("layout", ["whole", "heads apart", "gap", "odd"])
 @pytest.mark.parametrize("train", [False, True])
 def test_mixed_operands(B, H, Hkv, S, D, f32, layout, train):
