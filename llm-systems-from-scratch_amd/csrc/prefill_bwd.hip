@@ -1437,12 +1437,16 @@ static bool ds_passes(int B, int Hq, int Hkv, int Sq, int Sk, int D, int mask_mo
         out.part_rows = rows_k;
         out.part_bytes = round_up(2 * out.shares * rows_k * Hkv * D * 4, kDsBlock);
     }
-    // Wavefronts of 64 keys: key tiles with sixteen steps and more on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
+    // Wavefronts of 64 keys: key tiles with many steps on average (packed: of the mean length).  us of dK/dV, roles apart / wide (steps): 40 packed of 50 to 800 tokens, 8 heads, (2)
     // 56 / 70; 4 x 602, 16 heads (5) 32 / 37; 16 x 920 (7) 231 / 243; 4 packed of 324 to 5199, 4 / 2 heads, 4 shares (11) 116 / 120; 51 packed of 1701, one head (13) all kernels
     // 258 / 262; 21 packed of 995, 16 / 8 (15.5) all kernels 548 / 554; 2 x 2048, 32 heads (16) 186 / 175; 3000
     // tokens, 16 heads (23) 103 / 93; 6 packed of 100 to 1500, 64 / 8 (50) 235 / 232; 8192, 8 / 1 (64) 307 / 278; 16 of 256 to 4096, 32 / 8 (43) 905 / 832; 8 x 4096 (128) 2553 / 2250
+    // From sixteen on where no rows are dealt out, and not few of them under the diagonal, else from 24 on.  us of the whole backward, packed sequences of one length, roles apart / wide
+    // (steps): one share, 5 x 2113, 12 heads (16.5) 305 / 298, 4 x 2200, 4 heads (17) 126 / 122, 2 x 1250 without a mask, 16 heads (19.5) 134 / 131, but 100 x 257, 16 / 2 (16) 277 / 298, 32 x 600,
+    // 32 / 8 (18.8) 563 / 572, 16 x 700, 32 / 8 (22) 329 / 333; two shares, 90 x 556, 8 / 1 (17.4) 387 / 408, 4500, 8 heads (17.6) 218 / 223, 16 x 1280, 8 / 2 (20) 259 / 262, 16 x 1536, 8 / 2
+    // (24) 346 / 331; four, 4 x 1100, 32 / 4 (17) 224 / 231; eight, 3000, 16 / 2 (23) 178 / 186, 4500, 16 / 2 (35) 359 / 355; sixteen, 4096, 8 / 1 (16) 185 / 190, without a mask (32) 256 / 250
     const double row_tiles = (double)(packed ? total_q : (int64_t)B * Sq) / kBwRows / B;
-    out.wide = D == 128 && row_tiles * G * (causal ? 0.5 : 1.0) >= 16.0 * out.shares;
+    out.wide = D == 128 && row_tiles * G * (causal ? 0.5 : 1.0) >= (out.shares == 1 && (!causal || row_tiles >= 24.0) ? 16.0 : 24.0) * out.shares;
     out.unit_bytes = out.ds_room * G * kDsBlock;
     const int64_t fit = out.unit_bytes > 0 ? kDsMost / out.unit_bytes : out.n_units;
     if (fit < 1) return false;

@@ -39,7 +39,7 @@ constexpr int kWdGroup = 1040, kWdTile = kBwRows / 4 * kWdGroup;
 // What brought it there, cycles a step: a table of steps in LDS in place of scalar arithmetic and branches, 4350 -> 3600 (a branch that is taken stands in the
 // only wavefront's way); lane offsets of stores worked out, not read, in front of them 300; tiles in groups of four rows 16 bytes apart, so that
 // constants in the reads take the place of exclusive ors; rare blocks out of line.
-// A workgroup costs 25 K cycles around its steps (first rows 10 K, sums and rows out 12 K), so this is for key tiles with many of them: see launch_bwd_ds.
+// A workgroup costs 25 K cycles around its steps (first rows 10 K, sums and rows out 12 K), so this is for key tiles with many of them: see ds_passes.
 template <int MODE>
 __global__ __launch_bounds__(kWdWaves * 64, 1) void bwd_dkv_wide_kernel(BwdParams p) {
     constexpr bool CAUSAL = MODE == MI355_MASK_CAUSAL;

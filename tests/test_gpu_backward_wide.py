@@ -1,4 +1,4 @@
-"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with sixteen steps and more on average) against the form without dS in memory: rows and keys
+"""dK, dV and dS at head size 128 on wavefronts of 64 keys (key tiles with sixteen or 24 steps and more on average) against the form without dS in memory: rows and keys
 around the tiles of 64 and 128 and their halves, a tile of rows that is the sequence's only one, wavefronts without keys or rows, more queries than keys
 and the other way round, one to many steps, shares, fp32 gradients, several passes.  Every case says which kernel it is for, and how many shares it has; calls next
 to them run on the other kernel.  Tolerance of test_gpu_backward.py: one rounding of the result over a tensor."""
@@ -15,16 +15,16 @@ ROLES, WIDE = 1, 2
 PACKED = [
     ([1, 900, 33, 0, 830, 64, 65], None, 8, 1, True, ROLES, 8), ([31, 32, 33, 1800, 97, 95, 96], None, 16, 2, True, ROLES, 8), ([1700, 1, 129, 1023], [1800, 300, 64, 900], 6, 2, True, ROLES, 8),
     ([800, 1, 63, 900], [129, 64, 1, 127], 3, 1, False, ROLES, 4), ([2100, 2000], [40, 2100], 4, 4, True, ROLES, 4), ([700, 900, 64], [66, 193, 32], 4, 2, False, ROLES, 2),
-    ([2113] * 5, None, 12, 12, True, WIDE, 1), ([1, 900, 33, 0, 830, 64, 65], None, 64, 1, True, WIDE, 8), ([31, 32, 33, 700, 97, 95, 96], None, 128, 1, True, WIDE, 8),
-    ([1700, 1, 129, 1023], [1800, 300, 64, 900], 96, 24, True, WIDE, 1), ([800, 1, 63, 900], [129, 64, 1, 127], 64, 2, False, WIDE, 8), ([2100, 2000], [40, 2100], 32, 32, True, WIDE, 1),
-    ([700, 900, 64], [66, 193, 32], 64, 4, False, WIDE, 8), ([1025, 700, 33], [97, 161, 225], 128, 64, False, WIDE, 1)]
+    ([2113] * 5, None, 12, 12, True, WIDE, 1), ([1, 900, 33, 0, 830, 64, 65], None, 96, 1, True, WIDE, 8), ([31, 32, 33, 700, 97, 95, 96], None, 160, 1, True, WIDE, 8),
+    ([1700, 1, 129, 1023], [1800, 300, 64, 900], 144, 24, True, WIDE, 1), ([800, 1, 63, 900], [129, 64, 1, 127], 64, 2, False, WIDE, 8), ([2100, 2000], [40, 2100], 32, 32, True, WIDE, 1),
+    ([700, 900, 64], [66, 193, 32], 96, 4, False, WIDE, 8), ([1025, 700, 33], [97, 161, 225], 128, 64, False, WIDE, 1)]
 # batch, query heads, kv heads, queries, keys, causal, fp32 gradients | kernel, shares
 DENSE = [
     (3, 16, 2, 289, 289, True, True, ROLES, 4), (1, 12, 12, 2625, 2625, True, False, ROLES, 2), (2, 24, 3, 600, 130, False, False, ROLES, 8), (5, 8, 8, 1700, 65, False, True, ROLES, 2),
-    (9, 16, 1, 321, 500, True, False, ROLES, 4), (1, 32, 1, 1217, 1217, True, True, WIDE, 16), (30, 64, 8, 289, 289, True, True, WIDE, 1), (1, 24, 24, 2625, 2625, True, False, WIDE, 1),
-    (2, 64, 2, 600, 130, False, False, WIDE, 8), (64, 8, 8, 1025, 97, False, True, WIDE, 1), (64, 8, 8, 1025, 161, False, False, WIDE, 1), (17, 64, 4, 321, 500, True, False, WIDE, 2),
+    (9, 16, 1, 321, 500, True, False, ROLES, 4), (1, 32, 1, 1217, 1217, True, True, ROLES, 16), (1, 48, 1, 1217, 1217, True, True, WIDE, 16), (30, 96, 8, 289, 289, True, True, WIDE, 1), (1, 24, 24, 2625, 2625, True, False, WIDE, 1),
+    (2, 64, 2, 600, 130, False, False, WIDE, 8), (64, 8, 8, 1025, 97, False, True, WIDE, 1), (64, 8, 8, 1025, 161, False, False, WIDE, 1), (17, 80, 4, 321, 500, True, False, WIDE, 2), (9, 160, 4, 321, 500, True, False, WIDE, 4), (3, 32, 8, 1600, 1600, True, False, WIDE, 2),
     (1, 16, 16, 2090, 2050, True, False, WIDE, 1)]
-PASSES = [(1000, ROLES), (1100, WIDE)]
+PASSES = [(1000, ROLES), (1600, WIDE)]
 UNSEEN = [(2050, 2050), (2050, 2090), (2090, 2050)]
 
 
@@ -47,7 +47,7 @@ def test_cases_run_on_the_kernel_that_they_are_for():
             assert _kernel([n] * 3, [n] * 3, 28, 14, True, packed) == (want, 1)
     for Sq, Sk in UNSEEN:
         assert _kernel([Sq], [Sk], 16, 16, True, False) == (WIDE, 1)
-    assert {shares for *_, kernel, shares in PACKED + DENSE if kernel == WIDE} == {1, 2, 8, 16}
+    assert {shares for *_, kernel, shares in PACKED + DENSE if kernel == WIDE} == {1, 2, 4, 8, 16}
     assert _kernel([4096], [4096], 32, 8, True, False)[0] == WIDE and _kernel([64], [64], 8, 8, True, False) == (0, 0)
 
 
