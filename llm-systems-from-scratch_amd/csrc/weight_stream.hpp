@@ -9,17 +9,12 @@
 
 namespace mi355 {
 
-// per wavefront: 2 steps of 32 + 16 rows, or one of 32 + 32; three workgroups of four per compute unit, two where a norm's 16 KB come on top
+// The ring of a wavefront where three workgroups of four share a compute unit (two where a norm's 16 KB come on top): two steps of 32 + 16 rows, or one of 32 + 32.
+// Others: kWideStreamBytes of eight wavefronts (rows_linear.hip), kDirectRing of experts with many pairs (moe_ops.hip).
 constexpr int kStreamBytes = 12 * 1024;
 
-// w_off, a_off: byte offsets of this lane's 16 bytes in step 0: rows 8 j + lane / 8 of the weights (32) and of the activations
-// (16 * MT), piece (lane % 8) ^ (lane / 8) of the row's eight, so that the LDS row holds piece q at q ^ (row % 8).
-// k: row length in elements, a multiple of 8; meanwhile() runs when the first steps have been requested; on_rows(t, s, m, fragment) may
-// change a fragment of activations: lane holds row 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
-// sent: first_weights has been called (its requests are older than all of these, so the waits count the same).
-// acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
 // Workgroups that stream rows of whole 4096 bytes side by side, all from step 0 on, want the same few of an L2's sixteen channels (256 bytes each in turn) at any
-// time: 16 experts of 2048 x 1024, 32 tokens 44.0 us, 5.1 TB/s with the steps begun somewhere else by every one of an XCD's workgroups (every eighth of a launch) 39.5.  The same
+// time: 16 experts of 2048 x 1024, 32 tokens 44.0 us, 4.6 TB/s; 39.5, 5.1 TB/s, with the steps begun somewhere else by every one of an XCD's workgroups (every eighth of a launch).  The same
 // beginning within an XCD and another on each other one gives nothing (45.0); nor does any with rows of 2048 bytes (24.3 / 25.1), which have two sets of channels.
 inline bool turn_pays(int k) { return k % 2048 == 0; }
 // (at: the workgroup among those that read other weights, so that a row's sums do not depend on what else the launch has)
@@ -34,7 +29,14 @@ __device__ __forceinline__ void first_weights(const void* w, const uint32_t (&w_
     for (int j = 0; j < 4; ++j) dma_to_lds_16((const char*)w + 128 * (int64_t)t, w_off[j], lds_address(ring) + j * 1024);
 }
 
-// turn: the step that the wavefronts begin with (TURN; else 0)
+// w_off, a_off: byte offsets of this lane's 16 bytes in step 0: rows 8 j + lane / 8 of the weights (32) and of the activations
+// (16 * MT), piece (lane % 8) ^ (lane / 8) of the row's eight, so that the LDS row holds piece q at q ^ (row % 8).
+// k: row length in elements, a multiple of 8; meanwhile() runs when the first steps have been requested; on_rows(t, s, m, fragment) may
+// change a fragment of activations: lane holds row 16 m + lane % 16, elements 64 t + 32 s + 8 (lane / 16) .. + 7 (zeros from k on).
+// sent: first_weights has been called (its requests are older than all of these, so the waits count the same).
+// acc[m][i]: lane holds row 16 m + lane % 16 of the activations, rows 16 i + 4 (lane / 16) .. + 3 of the weights.
+// turn: the step that the wavefronts begin with, 0 <= turn < steps of k (TURN, with k a multiple of 64; else 0).  WAVES wavefronts share the steps; RING: bytes at `ring`, which
+// hold one to three steps.
 template <int MT, int WAVES, int RING, bool TURN, typename G, typename F>
 __device__ __forceinline__ void weight_stream(const void* w, const uint32_t (&w_off)[4], const void* a, const uint32_t (&a_off)[2 * MT],
                                               int k, int turn, int wave, unsigned char* ring, f32x4 (&acc)[MT][2], G&& meanwhile, F&& on_rows, bool sent = false) {
