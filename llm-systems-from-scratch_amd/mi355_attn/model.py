@@ -350,7 +350,8 @@ class CachedTransformerLM(CachedLM):
 
     def _decode_body(self, token_ids, plan):
         """Up to MAX_LINEAR_ROWS rows leave the head to a launch behind the graph: its logits go to the caller's tensor, where a copy of 8 x 10000 out of
-        the graph's takes 2.4 us and the gap in front of it (a step of 4 layers of 512, 8 sequences 97.9 -> 93.8, 2 of 1024, 4 sequences 69.8 -> 64.3; where the host is what a step waits for, 2 layers of 256, 50.5 -> 51.5)."""
+        the graph's takes 2.4 us and the gap in front of it (a step of 4 layers of 512, 8 sequences 100.2 -> 96.3, 2 of 1024 72.2 -> 66.3; where the host is what a
+        step waits for, 2 layers of 256, the same within the runs: 4.7 us of the host here, 4.5 for the copy)."""
         # (a subclass's own forward is what its graphs hold)
         T, own = token_ids.shape[0], all(getattr(getattr(self, n), "__func__", None) is getattr(CachedTransformerLM, n) for n in ("_forward", "_forward_rows"))
         if own and self._rows_fuse and T <= ops.MAX_LINEAR_ROWS and self._rows_pay(T):

@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 8, 1, 2048, 64, 2048), (5, 8, 2, 2048, 1024, 72), (47, 4, 1, 2048, 192, 2048), (48, 4, 1, 2048, 192, 100), (50, 3, 3, 4096, 128, 36),
-                                            (96, 4, 1, 2048, 2048, 2048), (97, 4, 1, 2048, 2048, 40), (300, 6, 2, 2048, 64, 64), (33, 4, 2, 1536, 2048, 96)])
+                                            (96, 4, 1, 2048, 2048, 2048), (97, 4, 1, 2048, 2048, 40), (300, 6, 2, 2048, 64, 64), (33, 4, 2, 1536, 2048, 96), (127, 8, 1, 1536, 1088, 64),
+                                            (128, 8, 1, 1536, 1088, 64)])
 def test_direct_products_of_whole_pages(T, E, top, k, ff, n):
     _products(T, E, top, k, ff, n, "direct")
 
@@ -20,9 +21,10 @@ def test_fewer_pairs_than_experts(T, E, top, k, ff, n):
     _products(T, E, top, k, ff, n, "direct")
 
 
-@pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 2, 1, 2048, 64, 2048), (130, 3, 1, 2048, 2048, 136), (200, 8, 2, 4096, 192, 2048), (513, 2, 1, 2048, 128, 128), (512, 2, 1, 2048, 2048, 96)])
+@pytest.mark.parametrize("T,E,top,k,ff,n", [(1, 2, 1, 2048, 64, 2048), (130, 3, 1, 2048, 2048, 136), (200, 8, 2, 4096, 192, 2048), (513, 2, 1, 2048, 128, 128), (512, 2, 1, 2048, 2048, 96), (192, 2, 1, 4096, 128, 72),
+                                            (193, 2, 1, 4096, 128, 72)])
 def test_large_tiles_of_whole_pages(T, E, top, k, ff, n):
-    """(128 x 128 tiles, up to 256 pairs an expert and one more)"""
+    """(128 x 128 tiles, up to 256 pairs an expert and one more, 96 with longer rows)"""
     _products(T, E, top, k, ff, n, "large")
 
 
