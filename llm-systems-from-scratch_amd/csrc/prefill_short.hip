@@ -25,14 +25,14 @@ __device__ __forceinline__ u32x4 rounded8(const float* x) {
 // ROUND (one query tile, a key head per query head): fp32 operands are rounded on their way in, and what a backward will read in bf16 leaves from here.  64 x 16 heads of 32, 256 tokens, fp32 Q and K, without a backward: two conversions and this kernel without it 38.7 us, like
 // this 24.9; 8 x 32 heads, 128 tokens 15.3 / 5.7; 64 x 16 heads of 64, 256 tokens 69.7 / 49.2.
 template <int D, bool CAUSAL, bool ROUND>
-__global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(PrefillParams p, int n_qtiles, int chunk, RoundedInputs r) {
+__global__ __launch_bounds__(256, D == 32 ? 4 : 2) void prefill_short_kernel(PrefillParams p, int n_qtiles, int group, int chunk, RoundedInputs r) {
     using R = TileReads<D>;
     constexpr int NS = R::NS, NDT = R::NDT, kRow = R::kRow, kTile = 64 * kRow, CPR = D / 8;
     __shared__ __attribute__((aligned(1024))) unsigned char k_lds[kShKeys / 64 * kTile];
     __shared__ __attribute__((aligned(1024))) unsigned char v_lds[kShKeys / 64 * kTile];
     // (the query tiles and query heads that read one key head's rows, and heads that share lines, run on one XCD)
     const int id = xcd_chunked_id(blockIdx.x, gridDim.x, chunk);
-    const int q0 = id % n_qtiles * kShRows, h = id / n_qtiles % p.Hq, b = id / (n_qtiles * p.Hq), hk = h / (p.Hq / p.Hkv);
+    const int q0 = id % n_qtiles * kShRows, h = id / n_qtiles % p.Hq, b = id / (n_qtiles * p.Hq), hk = h / group;
     const int rows = min(kShRows, p.Sq - q0), coff = p.Sk - p.Sq;
     const __bf16* qb = p.q + (int64_t)b * p.qs[0] + (int64_t)h * p.qs[1];
     const __bf16* kb = p.k + (int64_t)b * p.ks[0] + (int64_t)hk * p.ks[1];
@@ -246,8 +246,8 @@ static void launch_short(const PrefillParams& p, const RoundedInputs& r, hipStre
     const dim3 grid((unsigned)(n_qtiles * p.Hq * p.B));
     // Heads that are neighbours run on one XCD, see short_heads
     const int group = p.Hq / p.Hkv, chunk = n_qtiles * ((short_heads(D) + group - 1) / group * group);
-    if (p.mask_mode == MI355_MASK_CAUSAL) hipLaunchKernelGGL((prefill_short_kernel<D, true, ROUND>), grid, dim3(256), 0, s, p, n_qtiles, chunk, r);
-    else hipLaunchKernelGGL((prefill_short_kernel<D, false, ROUND>), grid, dim3(256), 0, s, p, n_qtiles, chunk, r);
+    if (p.mask_mode == MI355_MASK_CAUSAL) hipLaunchKernelGGL((prefill_short_kernel<D, true, ROUND>), grid, dim3(256), 0, s, p, n_qtiles, group, chunk, r);
+    else hipLaunchKernelGGL((prefill_short_kernel<D, false, ROUND>), grid, dim3(256), 0, s, p, n_qtiles, group, chunk, r);
 }
 
 int launch_prefill_short(const PrefillParams& p, int D, hipStream_t s) {
